@@ -52,14 +52,18 @@ __device__ __forceinline__ gcu8* global_bytes(const void* p) {
     return (gcu8*)uniform64(reinterpret_cast<uintptr_t>(p));
 }
 
-/* 16 bytes from / to global memory at any alignment. */
+/* 16 bytes from / to global memory at any alignment. The access keeps the
+ * global address space: through a generic pointer a select of two addresses
+ * becomes a flat load, which waits with the LDS reads. */
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(1)));
+typedef __attribute__((address_space(1))) u32x4 gu32x4;
+typedef __attribute__((address_space(1))) const u32x4 gcu32x4;
 __device__ __forceinline__ uint4 gload16(gcu8* p) {
-    uint4 v;
-    __builtin_memcpy(&v, (const void*)p, 16);
-    return v;
+    const u32x4 v = *(gcu32x4*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
 }
 __device__ __forceinline__ void gstore16(gu8* p, const uint4& v) {
-    __builtin_memcpy((void*)p, &v, 16);
+    *(gu32x4*)p = u32x4{v.x, v.y, v.z, v.w};
 }
 
 /* Orders this wave's global-memory writes before its later reads of the

@@ -52,26 +52,16 @@
 namespace cudec_amd {
 namespace {
 
-/* Candidates per lane: a window spans kC * 64 candidate positions. The
- * LZ4 two-wave form parses wider windows than the one-wave form: its
- * parser runs beside the copier, and a wider window fills more lanes of
- * every lane-parallel step, while a lone wave pays the wider speculation
- * on its own critical path. Snappy's two-wave windows are 448 candidates:
- * a window holds at most 64 members, and Snappy elements (2 to 5 bytes of
- * the source, mostly) fill those within a few hundred bytes, so wider
- * windows only add speculation to the busier parser wave (768: 35.2 ms,
- * 576: 32.1, 448: 30.7, 384: 31.9 on the uneven batch); its two-wave path
- * fits 96 VGPRs, so Snappy launches run five waves per SIMD throughout. */
+/* Candidates per lane of the one-wave form: a window spans kCandSplit * 64
+ * candidate positions. */
 constexpr uint32_t kCandSplit = 8;
-constexpr uint32_t kCandPipe = 16;
-constexpr uint32_t kCandPipeSnappy = 7;
-/* staged bytes a window of kC candidates per lane reads: the window plus
+/* staged bytes of a window of `window` positions: the window plus
  * the longest candidate that starts in it (an LZ4 sequence with one
  * extension byte per length reads 275 bytes, a Snappy literal window 277),
  * in whole 16-byte blocks. (A 512-byte margin staged 1.5 KiB a window; this
  * one takes the one-wave form 2.8% faster.) */
-constexpr uint32_t stage_bytes(uint32_t kc) { return kc * 64u + 304u; }
-constexpr uint32_t kStageBuf = stage_bytes(kCandPipe) + 16;
+constexpr uint32_t stage_bytes(uint32_t window) { return window + 304u; }
+constexpr uint32_t kStageBuf = stage_bytes(kCandSplit * 64) + 16;
 constexpr uint32_t kRing = 4096;          /* per-wave output ring */
 constexpr uint32_t kBatchMax = 2048;      /* output bytes of one batch, one-wave form */
 constexpr uint32_t kStop = 0xFFFFu;       /* link of an unresolvable candidate */
@@ -87,36 +77,38 @@ constexpr uint64_t kDefaultPipeMinCost = 512u << 10;
 constexpr int kKeys = 2 * kBins;
 
 static_assert(kBatchMax + 32 <= kRing, "ring must hold a batch and a margin");
+static_assert(kBatchMax <= 64 * kWave, "CoverLds marks a batch");
 static_assert((kRing & (kRing - 1)) == 0, "rings are powers of two");
 static_assert(kLaneMatch <= 64, "a lane match copies at most four 16-byte blocks");
-static_assert(kCandSplit * 64 + 2 + 269 + 3 <= stage_bytes(kCandSplit) &&
-                  kCandPipe * 64 + 2 + 269 + 3 <= stage_bytes(kCandPipe),
-              "a window's last candidate fits the stage");
+static_assert(2 + 269 + 3 <= stage_bytes(0), "a window's last candidate fits the stage");
 
-/* A wave's output ring (kR bytes, a power of two) and a stage buffer. The
- * one-wave decoders keep a 4 KiB ring each and the link table of their
- * window (walk_doubling); the two-wave form's copier an 8 KiB ring in the
- * same LDS (the two never run at once in a block). */
+/* An output ring of kR bytes (a power of two). */
 template <uint32_t kR>
 struct alignas(16) RingLds {
     static constexpr uint32_t kSize = kR;
     uint8_t ring[kR];
-    uint8_t stage[kStageBuf];
     uint8_t sink[kWave]; /* stores of lanes with nothing to store */
 };
-struct alignas(16) WaveLds : RingLds<kRing> {
-    uint16_t jump[kCandSplit * kWave];
+/* Which members of a group cover given bytes of its output: a bit for each
+ * member's first byte and, per 64 bytes, the members before them. */
+struct alignas(16) CoverLds {
+    uint64_t starts[kWave];
+    uint8_t before[kWave];
 };
-constexpr uint32_t kPipeRing = 8192;
-using PipeRing = RingLds<kPipeRing>;
-/* Output bytes of one batch in the two-wave form. Windows of token data
- * produce under 2 KiB; a window of long short-offset matches (64 members
- * of about 90 bytes each) fills up to 6 KiB, which its 8 KiB ring holds
- * with 2 KiB of history. */
-constexpr uint32_t kBatchMaxPipe = 6144;
-static_assert(kBatchMaxPipe + 32 <= kPipeRing, "the two-wave ring holds a batch and a margin");
-/* a batch's limit: the one-wave form walks by pointer doubling */
-constexpr uint32_t batch_max(bool one_wave) { return one_wave ? kBatchMax : kBatchMaxPipe; }
+
+/* A one-wave decoder's LDS: its ring, the stage of its window and the
+ * window's link table (walk_doubling). */
+struct alignas(16) WaveLds : RingLds<kRing> {
+    uint8_t stage[kStageBuf];
+    uint16_t jump[kCandSplit * kWave];
+    CoverLds cover;
+};
+/* A pipelined block's ring, the output bytes of one of its groups (64
+ * members of token data give under 2 KiB), and the history before a group
+ * that the group may read in the ring. */
+constexpr uint32_t kPipeRing = 16384;
+constexpr uint32_t kPipeBatch = 2560;
+constexpr uint32_t kPipeHistory = kPipeRing - 3 * kPipeBatch - 64;
 
 /* The decode queue hands out positions of the cost-sorted chunk order in
  * up to kSubQueues interleaved sub-queues (of k: sub-queue s holds
@@ -161,42 +153,51 @@ __device__ __forceinline__ uint32_t ring_index(uintptr_t dst_addr, uint64_t pos)
 
 /* ------------------------------------------------------------ staging */
 
-/* Loads compressed bytes [sp, sp + stage_bytes(kC)) of the chunk into stage and
+/* Loads compressed bytes [sp, sp + bytes) of the chunk into stage and
  * returns the offset of byte sp inside it. Only aligned 16-byte blocks that
- * start before the chunk end are read (each holds at least one byte of the
- * chunk, so none leaves the chunk's pages); later blocks are zero-filled.
- * Bytes past src_size are never trusted: every member is validated against
- * src_size before anything it read is used. */
-template <uint32_t kC>
+ * hold a byte of [sp, src_size) are read (so none leaves the chunk's
+ * pages); later blocks are zero-filled. Every load of the kRounds of 64
+ * blocks is issued before the first is stored, with no branch around it
+ * (a lane without a block reads the first one again): a load a round took
+ * a memory latency a round. Bytes past src_size are never trusted: every
+ * member is validated against src_size before anything it read is used. */
+template <uint32_t kRounds>
 __device__ __forceinline__ uint32_t stage_into(uint8_t* stage, gcu8* src,
                                                uint64_t src_size, uint64_t sp,
-                                               uint32_t lane) {
+                                               uint32_t bytes, uint32_t lane) {
     const uintptr_t a = (uintptr_t)(src + sp);
     const uintptr_t base = a & ~(uintptr_t)15;
-    const uintptr_t lo = (uintptr_t)src;
-    const uintptr_t end = lo + src_size;
-    for (uint32_t blk = lane; blk < stage_bytes(kC) / 16 + 1; blk += kWave) {
-        const uintptr_t g = base + 16u * blk;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        /* only a block that holds at least one byte of [src, src_size) */
-        if (g < end && g + 16 > lo) {
-            v = gload16((gcu8*)g);
+    const uintptr_t end = (uintptr_t)src + src_size;
+    const uint32_t blocks = bytes / 16 + 1;
+    uint4 v[kRounds];
+    if (sp < src_size) {
+#pragma unroll
+        for (uint32_t i = 0; i < kRounds; i++) {
+            const uint32_t blk = lane + i * kWave;
+            const uintptr_t g = base + 16u * blk;
+            v[i] = gload16((gcu8*)(blk < blocks && g < end ? g : base));
         }
-        *reinterpret_cast<uint4*>(&stage[16u * blk]) = v;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kRounds; i++) {
+        const uint32_t blk = lane + i * kWave;
+        if (blk < blocks) {
+            const bool in = sp < src_size && base + 16u * blk < end;
+            *reinterpret_cast<uint4*>(&stage[16u * blk]) = in ? v[i] : make_uint4(0, 0, 0, 0);
+        }
     }
     wave_order();
     return (uint32_t)(a - base);
 }
 
-/* Loads one dword per lane of the 1 KiB after the window staged at sp
- * (16 bytes apart, every one inside the source), so that the next window's
+/* Loads one dword per lane, `step` bytes apart, of what follows the `bytes`
+ * staged at sp (every one inside the source), so that the next window's
  * stage finds those bytes in L2. The caller holds the value until the
  * window is parsed, which keeps the loads off its critical path. */
-template <uint32_t kC>
 __device__ __forceinline__ uint32_t touch_ahead(gcu8* src, uint64_t src_size, uint64_t sp,
-                                                uint32_t lane) {
+                                                uint32_t bytes, uint32_t step, uint32_t lane) {
     const uintptr_t base = (uintptr_t)(src + sp) & ~(uintptr_t)15;
-    const uintptr_t g = base + 16u * (stage_bytes(kC) / 16 + 1) + 16u * lane;
+    const uintptr_t g = base + 16u * (bytes / 16 + 1) + step * lane;
     const uintptr_t end = (uintptr_t)src + src_size;
     return g + 4 <= end ? *(gcu32*)g : 0u;
 }
@@ -322,40 +323,47 @@ __device__ __forceinline__ uint32_t block_byte(const uint4& v, uint32_t i) {
     return (x >> ((i & 3) * 8)) & 0xFF;
 }
 
+/* Exactly n (0..15) bytes of v to ring position r, where they do not wrap:
+ * 8/4/2/1-byte stores, so no byte past n is touched. */
+template <class W>
+__device__ __forceinline__ void ring_tail(W& w, uint32_t r, const uint4& v, uint32_t n) {
+    uint8_t* p = &w.ring[r];
+    uint64_t lo = ((uint64_t)v.y << 32) | v.x;
+    const uint64_t hi = ((uint64_t)v.w << 32) | v.z;
+    if (n & 8) {
+        __builtin_memcpy(p, &lo, 8);
+        p += 8;
+        lo = hi;
+    }
+    if (n & 4) {
+        const uint32_t q = (uint32_t)lo;
+        __builtin_memcpy(p, &q, 4);
+        p += 4;
+        lo >>= 32;
+    }
+    if (n & 2) {
+        const uint16_t q = (uint16_t)lo;
+        __builtin_memcpy(p, &q, 2);
+        p += 2;
+        lo >>= 16;
+    }
+    if (n & 1) {
+        *p = (uint8_t)lo;
+    }
+}
+
 /* Exactly n (0..16) bytes of v to ring position r, wrapping at the ring's
- * end: 8/4/2/1-byte stores, so no byte past n is touched. */
+ * end. */
 template <class W>
 __device__ __forceinline__ void ring_put(W& w, uint32_t r, const uint4& v, uint32_t n) {
     if (n == 0) {
         return;
     }
     if (r + n <= W::kSize) {
-        uint8_t* p = &w.ring[r];
         if (n == 16) {
-            __builtin_memcpy(p, &v, 16);
-            return;
-        }
-        uint64_t lo = ((uint64_t)v.y << 32) | v.x;
-        const uint64_t hi = ((uint64_t)v.w << 32) | v.z;
-        if (n & 8) {
-            __builtin_memcpy(p, &lo, 8);
-            p += 8;
-            lo = hi;
-        }
-        if (n & 4) {
-            const uint32_t q = (uint32_t)lo;
-            __builtin_memcpy(p, &q, 4);
-            p += 4;
-            lo >>= 32;
-        }
-        if (n & 2) {
-            const uint16_t q = (uint16_t)lo;
-            __builtin_memcpy(p, &q, 2);
-            p += 2;
-            lo >>= 16;
-        }
-        if (n & 1) {
-            *p = (uint8_t)lo;
+            __builtin_memcpy(&w.ring[r], &v, 16);
+        } else {
+            ring_tail(w, r, v, n);
         }
         return;
     }
@@ -382,26 +390,24 @@ __device__ __forceinline__ uint32_t gather16(const uint4& S, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, pick);
 }
 
-/* The source period of a lane match lies wholly in flushed history, so its
- * bytes can be loaded before the window's literals are placed. */
-__device__ __forceinline__ bool period_in_history(uint64_t m, uint32_t off, uint32_t len,
-                                                  uint64_t hist_lo, uint64_t cap) {
-    const uint64_t y = m - off;
-    const uint32_t need = len < off ? len : off;
-    return y + need <= hist_lo && y + ((need + 15) & ~15u) <= cap;
+/* Where the last piece of a copy of len bytes starts: copies go out in
+ * pieces of 16, 8 or 4 bytes (the largest that fits the length), the last
+ * one ending at the copy's end and so overlapping the one before. */
+__device__ __forceinline__ uint32_t last_piece(uint32_t len) {
+    return len >= 16 ? len - 16 : len >= 8 ? len - 8 : len >= 4 ? len - 4 : 0;
 }
 
-/* Four 16-byte global loads of a history period of need (1..64) bytes at
- * `at`, issued together: block k starts 16 k bytes in, or at the period's
- * last block where the period is shorter, so every load stays inside the
- * period's 16-byte blocks. Straight-line on purpose: a load under a
- * condition of its own leaves the compiler copying its result where the
+/* Four 16-byte global loads of the pieces of a history source of len
+ * (1..64) bytes at `at`, issued together: at 0, 16, 32 (or at the last
+ * piece where that comes before) and at the last piece, none of which reads
+ * more than 15 bytes past the source. Straight-line on purpose: a load under
+ * a condition of its own leaves the compiler copying its result where the
  * condition ends, and the copy waits for the load right there. */
 struct Period {
     uint4 h0, h1, h2, h3;
 };
-__device__ __forceinline__ Period load_period(gcu8* at, uint32_t need) {
-    const uint32_t last = (need - 1) & ~15u;
+__device__ __forceinline__ Period load_period(gcu8* at, uint32_t len) {
+    const uint32_t last = last_piece(len);
     Period p;
     p.h0 = gload16(at);
     p.h1 = gload16(at + (last < 16u ? last : 16u));
@@ -411,138 +417,6 @@ __device__ __forceinline__ Period load_period(gcu8* at, uint32_t need) {
 }
 /* What lanes with no history period load instead (never written). */
 __device__ __align__(16) uint8_t no_period[16];
-
-/* One lane copies a match of len (<= kLaneMatch) bytes at output position
- * m with offset off into the ring; every source byte precedes m or is
- * written earlier by this lane. Two steps:
- *  1. the period S = [m - off, m - off + min(len, off)) goes to the ring at
- *     m: from flushed history (from_history: hp holds it, loaded by the
- *     caller with up to four 16-byte loads issued together), or from the
- *     ring with independent 16-byte reads, or bytewise where it straddles
- *     the ring's floor or wraps;
- *  2. an overlapping match (off < len) repeats it: for off < 16 the first
- *     16 bytes are built in registers from S (byte k = S[k mod off]) and
- *     the rest is copied from D = off * floor(16 / off) bytes back, 8 or 16
- *     bytes a step; for off >= 16, 16 bytes a step from off back. Where the
- *     match wraps the ring, bytewise. */
-template <class W>
-__device__ __forceinline__ void lane_match_copy(W& w, gcu8* dst, uintptr_t da,
-                                                uint64_t m, uint32_t off, uint32_t len,
-                                                uint64_t hist_lo, uint64_t cap, bool from_history,
-                                                const Period& hp) {
-    const uint64_t y = m - off;
-    const uint32_t need = len < off ? len : off;
-    const uint32_t rd = ring_index<W::kSize>(da, m);
-    const uint32_t ry = ring_index<W::kSize>(da, y);
-    /* step 1 */
-    if (from_history || (y >= hist_lo && ry + need <= W::kSize)) {
-        uint4 h0, h1, h2, h3;
-        if (from_history) {
-            h0 = hp.h0;
-            h1 = hp.h1;
-            h2 = hp.h2;
-            h3 = hp.h3;
-        } else {
-            /* reads past `need` (at most 15 bytes, still inside this
-             * WaveLds) are never stored */
-            __builtin_memcpy(&h0, &w.ring[ry], 16);
-            h1 = h2 = h3 = make_uint4(0, 0, 0, 0);
-            if (need > 16) {
-                __builtin_memcpy(&h1, &w.ring[ry + 16], 16);
-            }
-            if (need > 32) {
-                __builtin_memcpy(&h2, &w.ring[ry + 32], 16);
-            }
-            if (need > 48) {
-                __builtin_memcpy(&h3, &w.ring[ry + 48], 16);
-            }
-        }
-        if (rd + need <= W::kSize) {
-            /* whole blocks, then one exact tail */
-            const uint32_t full = need >> 4;
-            if (full > 0) {
-                __builtin_memcpy(&w.ring[rd], &h0, 16);
-            }
-            if (full > 1) {
-                __builtin_memcpy(&w.ring[rd + 16], &h1, 16);
-            }
-            if (full > 2) {
-                __builtin_memcpy(&w.ring[rd + 32], &h2, 16);
-            }
-            if (full > 3) {
-                __builtin_memcpy(&w.ring[rd + 48], &h3, 16);
-            }
-            const uint4 t = full == 0 ? h0 : full == 1 ? h1 : full == 2 ? h2 : h3;
-            ring_put(w, rd + 16 * full, t, need & 15);
-        } else {
-            ring_put(w, rd, h0, need < 16 ? need : 16);
-            if (need > 16) {
-                ring_put(w, (rd + 16) & (W::kSize - 1), h1, need - 16 < 16 ? need - 16 : 16);
-            }
-            if (need > 32) {
-                ring_put(w, (rd + 32) & (W::kSize - 1), h2, need - 32 < 16 ? need - 32 : 16);
-            }
-            if (need > 48) {
-                ring_put(w, (rd + 48) & (W::kSize - 1), h3, need - 48);
-            }
-        }
-    } else {
-        for (uint32_t i = 0; i < need; i++) {
-            w.ring[(rd + i) & (W::kSize - 1)] = history_byte(w, dst, y + i, hist_lo);
-        }
-    }
-    if (need == len) {
-        return;
-    }
-    /* step 2: off < len */
-    if (off < 16 && rd + (len > 16 ? len : 16) <= W::kSize) {
-        uint4 S;
-        __builtin_memcpy(&S, &w.ring[rd], 16);
-        uint32_t p = off;
-        if (p <= 2) {
-            /* periods 1 and 2 as period 4 */
-            S.x = __builtin_amdgcn_perm(0u, S.x, p == 1 ? 0x00000000u : 0x01000100u);
-            p = 4;
-        }
-        const uint32_t pb = __builtin_amdgcn_perm(0u, p, 0u);
-        const uint32_t cp = __builtin_amdgcn_perm(0u, 0x80u - p, 0u);
-        uint32_t q[4];
-        uint32_t r = 0;
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-            q[t] = gather16(S, period_sel(r, pb, cp));
-            r += 4;
-            r = r >= p ? r - p : r;
-            r = r >= p ? r - p : r;
-        }
-        ring_put(w, rd, make_uint4(q[0], q[1], q[2], q[3]), len < 16 ? len : 16);
-        /* D - 1 for off = 1..15, a nibble each */
-        const uint32_t D = (uint32_t)((0x0EDCBA98FDBEFEFFull >> (4 * (off - 1))) & 15) + 1;
-        if (D == 16) {
-            for (uint32_t i = 16; i < len; i += 16) {
-                uint4 v;
-                __builtin_memcpy(&v, &w.ring[rd + i - 16], 16);
-                ring_put(w, rd + i, v, len - i < 16 ? len - i : 16);
-            }
-        } else {
-            for (uint32_t i = 16; i < len; i += 8) {
-                uint2 v;
-                __builtin_memcpy(&v, &w.ring[rd + i - D], 8);
-                ring_put(w, rd + i, make_uint4(v.x, v.y, 0, 0), len - i < 8 ? len - i : 8);
-            }
-        }
-    } else if (off >= 16 && rd + len <= W::kSize) {
-        for (uint32_t i = off; i < len; i += 16) {
-            uint4 v;
-            __builtin_memcpy(&v, &w.ring[rd + i - off], 16);
-            ring_put(w, rd + i, v, len - i < 16 ? len - i : 16);
-        }
-    } else {
-        for (uint32_t i = off; i < len; i++) {
-            w.ring[(rd + i) & (W::kSize - 1)] = w.ring[(rd + i - off) & (W::kSize - 1)];
-        }
-    }
-}
 
 /* --------------------------------------------------- global slow path */
 
@@ -785,40 +659,152 @@ struct Group {
     uint32_t end_rel;
 };
 
-/* One lane's literal of lit_len (<= kLaneLit) bytes, staged at cw + lit,
- * to the ring at output position lit_at: 16 bytes a step, the last step
- * exact (a Snappy literal has no match after it to absorb an overrun). */
-template <class W>
-__device__ __forceinline__ void put_literal(W& w, const uint8_t* cw, uint32_t lit,
-                                            uint32_t lit_len, uintptr_t da, uint64_t lit_at) {
-    uint32_t i0 = 0;
-    for (; i0 + 16 <= lit_len; i0 += 16) {
-        uint4 v;
-        __builtin_memcpy(&v, cw + lit + i0, 16);
-        const uint32_t r = ring_index<W::kSize>(da, lit_at + i0);
-        if (r <= W::kSize - 16) {
-            __builtin_memcpy(&w.ring[r], &v, 16);
-        } else {
-            for (uint32_t b = 0; b < 16; b++) {
-                w.ring[(r + b) & (W::kSize - 1)] = (uint8_t)block_byte(v, b);
-            }
-        }
+/* LDS bytes by 32-bit LDS address. */
+typedef __attribute__((address_space(3))) uint8_t lds_u8;
+__device__ __forceinline__ uint32_t lds_address(const uint8_t* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)p;
+}
+
+/* Exactly len (1..64) bytes to `to`, from `from` (both LDS; `to` is at
+ * least 16 bytes, or len, further on: pieces go out in order, so where the
+ * copy repeats its source a piece reads what the ones before it wrote) or,
+ * where kHist and from_history, from the loaded pieces hp. A
+ * lane's copy is at most four 16-byte pieces, or two of 8 or of 4, the last
+ * ending at the copy's end (load_period): no tail of 8, 4, 2 and 1 bytes,
+ * each under a branch of its own, which took about three times the
+ * instructions. */
+template <uint32_t kBytes>
+struct Piece;
+template <>
+struct Piece<16> {
+    using type = uint4;
+    static __device__ __forceinline__ type of(const uint4& v) { return v; }
+};
+template <>
+struct Piece<8> {
+    using type = uint2;
+    static __device__ __forceinline__ type of(const uint4& v) { return make_uint2(v.x, v.y); }
+};
+template <>
+struct Piece<4> {
+    using type = uint32_t;
+    static __device__ __forceinline__ type of(const uint4& v) { return v.x; }
+};
+template <uint32_t kBytes, bool kHist>
+__device__ __forceinline__ void put_piece(uint8_t* to, const uint8_t* from, bool from_history,
+                                          const uint4& h) {
+    typename Piece<kBytes>::type x = Piece<kBytes>::of(h);
+    if (!kHist || !from_history) {
+        __builtin_memcpy(&x, from, kBytes);
     }
-    if (i0 < lit_len) {
-        uint4 v;
-        __builtin_memcpy(&v, cw + lit + i0, 16);
-        ring_put(w, ring_index<W::kSize>(da, lit_at + i0), v, lit_len - i0);
+    __builtin_memcpy(to, &x, kBytes);
+}
+template <bool kHist>
+__device__ __forceinline__ void lane_copy(uint8_t* to, const uint8_t* from, uint32_t len,
+                                          bool from_history, const Period& hp) {
+    const uint32_t last = last_piece(len);
+    if (len >= 16) {
+        put_piece<16, kHist>(to, from, from_history, hp.h0);
+        if (len > 32) {
+            put_piece<16, kHist>(to + 16, from + 16, from_history, hp.h1);
+        }
+        if (len > 48) {
+            put_piece<16, kHist>(to + 32, from + 32, from_history, hp.h2);
+        }
+        put_piece<16, kHist>(to + last, from + last, from_history, hp.h3);
+    } else if (len >= 8) {
+        put_piece<8, kHist>(to, from, from_history, hp.h0);
+        put_piece<8, kHist>(to + last, from + last, from_history, hp.h3);
+    } else if (len >= 4) {
+        put_piece<4, kHist>(to, from, from_history, hp.h0);
+        put_piece<4, kHist>(to + last, from + last, from_history, hp.h3);
+    } else {
+        /* 1 to 3 bytes: the first, the middle and the last */
+        const uint32_t mid = len >> 1, end = len - 1;
+        uint8_t a = (uint8_t)hp.h0.x, b = (uint8_t)(hp.h0.x >> (8 * mid)),
+                c = (uint8_t)(hp.h0.x >> (8 * end));
+        if (!kHist || !from_history) {
+            a = from[0];
+            b = from[mid];
+            c = from[end];
+        }
+        to[0] = a;
+        to[mid] = b;
+        to[end] = c;
     }
 }
 
+/* One lane's literal of lit_len (1..kLaneLit) bytes, staged at `from`, to
+ * the ring at index r0. */
+template <class W>
+__device__ __forceinline__ void put_literal(W& w, const uint8_t* from, uint32_t lit_len,
+                                            uint32_t r0) {
+    if (r0 + lit_len <= W::kSize) {
+        lane_copy<false>(&w.ring[r0], from, lit_len, false, Period{});
+    } else {
+        for (uint32_t b = 0; b < lit_len; b++) {
+            w.ring[(r0 + b) & (W::kSize - 1)] = from[b];
+        }
+    }
+}
+
+/* How a wave that executes groups stands to the others of its chunk. Alone:
+ * it runs every group of the chunk itself, so everything before the group
+ * is final. InTurn: the copiers of a pipelined block run consecutive groups
+ * at once (below), so what lies between the output position that was final
+ * when the group began and the group itself may still be unwritten, and
+ * bytes that followers may overwrite in the ring count as gone. */
+struct Alone {
+    static constexpr bool kInTurn = false;
+    __device__ uint64_t final_below(uint64_t d0) const { return d0; }
+    __device__ bool wait_turn() const { return true; }
+};
+
+/* Lane's members a..b (as a mask) that cover bytes [from, to) of the group,
+ * relative to its start, below member `lane`; none for an empty range. Each
+ * active lane's member starts at `start` (all different, the first at 0). Two rank queries per lane replace
+ * a search over the members. */
+__device__ __forceinline__ uint64_t members_covering(CoverLds& c, bool active, uint32_t start,
+                                                     uint32_t from, uint32_t to, uint32_t lane) {
+    c.starts[lane] = 0;
+    wave_order();
+    if (active) {
+        atomicOr((unsigned long long*)&c.starts[start >> 6], 1ull << (start & 63));
+    }
+    wave_order();
+    const uint32_t mine = (uint32_t)__builtin_popcountll(c.starts[lane]);
+    c.before[lane] = (uint8_t)(wave_inclusive_sum(mine, lane) - mine);
+    wave_order();
+    if (from >= to) {
+        return 0;
+    }
+    const uint32_t last = to - 1;
+    const uint64_t upto_a = ~0ull >> (63 - (from & 63)), upto_b = ~0ull >> (63 - (last & 63));
+    const uint32_t a = c.before[from >> 6] +
+                       (uint32_t)__builtin_popcountll(c.starts[from >> 6] & upto_a) - 1;
+    const uint32_t b = c.before[last >> 6] +
+                       (uint32_t)__builtin_popcountll(c.starts[last >> 6] & upto_b) - 1;
+    const uint64_t below = (1ull << lane) - 1;
+    return below & (~0ull << (a & 63)) & (~0ull >> (63 - (b & 63)));
+}
+
+/* Matches longer than this go 16 bytes a lane (ring_match_wide) instead of
+ * a byte a lane and 64 a step. */
+constexpr uint32_t kWideMatch = 256;
+
 /* Executes group g of the window staged at cw into the ring at output
  * positions [dp, dp + g.end_rel), flushes whole 16-byte blocks (all of them
- * when the chunk is done) and advances dp. */
-template <class W>
-__device__ __forceinline__ void execute_group(W& w, const uint8_t* cw, const Group& g,
-                                              gu8* dst, uint64_t cap, uint64_t& dp,
-                                              uint64_t& flushed, uint64_t ring_lo, bool done,
-                                              uint32_t lane) {
+ * when the chunk is done) and advances dp. Returns false only when the
+ * wait for its turn was given up.
+ *
+ * Literals go first, a member a lane. Then the matches that repeat nothing
+ * and whose source is final, a member a lane. The others go in stream
+ * order, the wave fanned out over the bytes. */
+template <class W, class Order>
+__device__ __forceinline__ bool execute_group(W& w, CoverLds& cover_lds, const uint8_t* cw,
+                                              const Group& g, gu8* dst, uint64_t cap,
+                                              uint64_t& dp, uint64_t& flushed, uint64_t ring_lo,
+                                              bool done, uint32_t lane, const Order& order) {
     const uintptr_t da = (uintptr_t)dst;
     const uint32_t take = g.take;
     const bool full = lane < take;
@@ -827,120 +813,206 @@ __device__ __forceinline__ void execute_group(W& w, const uint8_t* cw, const Gro
                    offset = g.offset, drel = g.drel;
     const uint64_t D0 = dp;
     const uint64_t D1 = dp + g.end_rel;
-    const uint64_t ring_floor = D1 + 16 > W::kSize ? D1 + 16 - W::kSize : 0;
+    const uint64_t final_lo = order.final_below(D0);
+    uint64_t ring_floor;
+    if constexpr (Order::kInTurn) {
+        ring_floor = D0 > kPipeHistory ? D0 - kPipeHistory : 0;
+    } else {
+        ring_floor = D1 + 16 > W::kSize ? D1 + 16 - W::kSize : 0;
+    }
     const uint64_t hist_lo = ring_lo > ring_floor ? ring_lo : ring_floor;
-    const uint64_t lit_at = D0 + drel;
-    const uint64_t m_at = lit_at + lit_len;
-    /* a literal the whole wave copies in stream order */
-    const bool wide_lit = lit_len > kLaneLit;
-    /* matches that read only history or their own literals go by their own
-     * lane; the history ones load their period now, so the load overlaps
-     * the literal phase */
-    const uint64_t y = m_at - offset;
-    const uint64_t need = match_len < offset ? match_len : offset;
-    const bool independent = y + need <= D0 || y >= lit_at;
-    const bool lane_match = full && !wide_lit && match_len <= kLaneMatch && independent;
-    const bool from_history =
-        lane_match && period_in_history(m_at, offset, match_len, hist_lo, cap);
-    /* every lane loads, with no branch around the loads (whose results
+    /* positions from here on are 32-bit and relative to the group's start:
+     * the group and the ring's history are a few KiB, and a source further
+     * back than 2^30 bytes is as good as one that far back */
+    const int hist_rel = (int)(hist_lo - D0);
+    const int final_rel = (int)(final_lo - D0);
+    const uint32_t ring_at = (uint32_t)(da + D0); /* ring index of the group's start, unmasked */
+    const uint32_t m_rel = drel + lit_len;
+    const int y_rel = offset > 1u << 30 ? -(1 << 30) : (int)(m_rel - offset);
+    const uint32_t need = match_len < offset ? match_len : offset;
+    const int src_end = y_rel + (int)need;
+    const bool has_match = full && match_len != 0;
+    const uint32_t rd = (ring_at + m_rel) & (W::kSize - 1);
+    const uint32_t ry = (ring_at + m_rel - offset) & (W::kSize - 1);
+    const bool short_fit = has_match && match_len <= kLaneMatch && rd + match_len <= W::kSize;
+    const bool src_fit = y_rel >= hist_rel && ry + need <= W::kSize;
+    /* matches that a lane copies by itself: those that repeat nothing, with
+     * a final source, in the ring or in flushed history (whose 16-byte loads
+     * may run up to 15 bytes past the source) */
+    const bool simple =
+        short_fit && offset >= match_len && (src_end <= final_rel || y_rel >= (int)drel);
+    const bool from_history = simple && src_end <= hist_rel && hist_lo + 15 <= cap;
+    const bool by_lane = from_history || (simple && src_fit);
+    /* history periods are loaded now, so the loads overlap the literal
+     * phase: every lane loads, with no branch around the loads (whose results
      * would then be copied, waiting for them here); a lane without a
      * history period reads the zero block no_period */
-    const Period hp = load_period(from_history ? dst + y : (gcu8*)no_period,
-                                  from_history ? (uint32_t)need : 1u);
-    /* phase 1: the lanes' literals */
-    if (active && !wide_lit) {
-        put_literal(w, cw, lit, lit_len, da, lit_at);
+    const Period hp =
+        load_period(from_history ? dst + (D0 + m_rel - offset) : (gcu8*)no_period,
+                    from_history ? need : 1u);
+    /* the literals */
+    const bool wide_lit = lit_len > kLaneLit;
+    if (active && !wide_lit && lit_len != 0) {
+        put_literal(w, cw + lit, lit_len, (ring_at + drel) & (W::kSize - 1));
+    }
+    for (uint64_t wide = __ballot(active && wide_lit); wide != 0;) {
+        const uint32_t j = __builtin_ctzll(wide);
+        clear_bit(wide, j);
+        const uint32_t jl = __builtin_amdgcn_readlane(lit_len, j);
+        const uint32_t jlit = __builtin_amdgcn_readlane(lit, j);
+        const uint32_t jr = ring_at + __builtin_amdgcn_readlane(drel, j);
+        for (uint32_t i = lane; i < jl; i += kWave) {
+            w.ring[(jr + i) & (W::kSize - 1)] = cw[jlit + i];
+        }
     }
     wave_order();
-    /* phase 2: the lane matches */
-    if (lane_match) {
-        lane_match_copy(w, dst, da, m_at, offset, match_len, hist_lo, cap, from_history, hp);
+    /* the members each of the other matches waits for: those that cover its
+     * source between the group's start and its own literals */
+    const bool rest = has_match && !by_lane;
+    const uint32_t src_from = y_rel > 0 ? (uint32_t)y_rel : 0;
+    const uint32_t src_to = !rest || src_end <= 0       ? 0
+                            : (uint32_t)src_end < drel ? (uint32_t)src_end
+                                                       : drel;
+    const uint64_t waits_for =
+        members_covering(cover_lds, full, drel, src_from, src_to, lane);
+    const bool held = Order::kInTurn && rest && y_rel < 0 && src_end > final_rel;
+    if (by_lane) {
+        lane_copy<true>(&w.ring[rd], &w.ring[ry], match_len, from_history, hp);
     }
     wave_order();
-    /* phase 3: the rest, in stream order, whole wave. The common member, a
-     * short match (<= 64 bytes) whose period is in the ring, is described by
-     * its lane up front in two words, so the loop pays two v_readlane and a
-     * byte a lane for it: fast_a = ring index of the match (13 bits), of
-     * its period (13 bits), length - 1 (6 bits); fast_b = o = min(offset,
-     * 64) in bits 0-7 and ceil(4096 / o) above them. Byte i copies period
-     * byte i mod offset, which precedes the match, so the lanes do not
-     * depend on each other. For i <= 64 the quotient floor(i / o) is
+    /* The common member of a level, a short match (<= 64 bytes) whose period
+     * is in the ring and which does not wrap there, is described by its lane
+     * up front in two words, so it costs two v_readlane and a byte a lane:
+     * fast_a = LDS address of the match (16 bits) and of its period; fast_b
+     * = its length (8 bits), o = min(offset, 64) (8 bits) and
+     * ceil(4096 / o). Where the match repeats its period, byte i copies
+     * period byte i mod offset, which precedes the match, so the lanes do
+     * not depend on each other. For i <= 64 the quotient floor(i / o) is
      * (i * ceil(4096 / o)) >> 12: with ceil(4096 / o) = (4096 + e) / o,
      * 0 <= e < o, the scaled product is i / o + i * e / (4096 o), and
      * i * e < 64 * 64 keeps the excess below the 1 / o that separates i / o
      * from the next integer. Two 24-bit multiplies and a shift replace a
      * reciprocal and its correction. */
-    const bool rest_fast = full && !lane_match && !wide_lit && match_len != 0 &&
-                           match_len <= kWave && y >= hist_lo;
-    static_assert(W::kSize <= 8192, "ring indices are packed in 13 bits");
-    const uint32_t fast_a = ring_index<W::kSize>(da, m_at) | ring_index<W::kSize>(da, y) << 13 |
-                            (match_len - 1) << 26;
+    const bool fast_member = rest && short_fit && src_fit;
+    /* (a source that runs on into the match must not wrap between them) */
+    const bool by_pieces = offset >= match_len || (offset >= 16 && ry < rd);
+    const uint64_t once_mask = __ballot(fast_member && by_pieces);
+    const uint64_t again_mask = __ballot(fast_member && !by_pieces);
+    const uint32_t lds_ring = lds_address(w.ring);
+    const uint32_t fast_a = (lds_ring + rd) | (lds_ring + ry) << 16;
     const uint32_t fast_o = offset - 1 < kWave ? offset : kWave;
-    const uint32_t fast_b = fast_o | ((4096u + fast_o - 1) / fast_o) << 8;
-    /* in stream order: runs of short ring matches (one straight-line step
-     * each, in a loop with no other branch), each run ended by the next
-     * other member */
-    uint64_t fast = __ballot(rest_fast);
-    uint64_t other = __ballot(active && (wide_lit || (full && !lane_match))) & ~fast;
+    const uint32_t fast_b = (match_len & 255) | fast_o << 8 | ((4096u + fast_o - 1) / fast_o) << 16;
+    const uint32_t sink = lds_address(w.sink) + lane;
+    /* lanes past the match write their own sink byte, so no lane is masked */
+    auto again_from = [&](uint32_t ja, uint32_t jb) {
+        const uint32_t r = __umul24(__umul24(lane, jb >> 16) >> 12, (jb >> 8) & 255);
+        return *(lds_u8*)(uintptr_t)((ja >> 16) + lane - r);
+    };
+    auto put = [&](uint32_t ja, uint32_t jb, uint8_t byte) {
+        const uint32_t at = (ja & 0xFFFF) + lane;
+        *(lds_u8*)(uintptr_t)(lane < (jb & 255) ? at : sink) = byte;
+    };
+    uint64_t undone = __ballot(rest);
+    /* InTurn: the members that need bytes of groups still running, or of
+     * such a member of this group, wait for this group's turn */
+    uint64_t later = Order::kInTurn ? __ballot(held) : 0;
+    if (Order::kInTurn && later != 0) {
+        for (uint64_t more = later;;) {
+            more = __ballot(rest && (waits_for & more) != 0) & ~later;
+            if (more == 0) {
+                break;
+            }
+            later |= more;
+        }
+    }
+    bool turn = false;
     for (;;) {
-        /* the fast members before the next other one */
-        uint64_t run = other != 0 ? fast & ((other & (0 - other)) - 1) : fast;
-        fast &= ~run;
-        while (run != 0) {
-            const uint32_t j = __builtin_ctzll(run);
-            clear_bit(run, j);
-            const uint32_t ja = __builtin_amdgcn_readlane(fast_a, j);
-            const uint32_t jb = __builtin_amdgcn_readlane(fast_b, j);
-            const uint32_t jo = jb & 255;
-            const uint32_t rm = ja & 8191;
-            const uint32_t rs = (ja >> 13) & 8191;
-            const uint32_t jm = (ja >> 26) + 1;
-            /* lane mod jo (lanes below jo get a zero quotient); lanes past
-             * the match write their own sink byte, so no lane is masked */
-            const uint32_t r = lane - __umul24(__umul24(lane, jb >> 8) >> 12, jo);
-            uint8_t* at = lane < jm ? &w.ring[(rm + lane) & (W::kSize - 1)] : &w.sink[lane];
-            *at = w.ring[(rs + r) & (W::kSize - 1)];
+        uint64_t todo = undone & ~later;
+        /* copies that go by pieces and wait for none: a member a lane
+         * where there are several, which costs about what four of them cost
+         * one by one */
+        const uint64_t lanes =
+            todo & once_mask & __ballot((waits_for & undone) == 0);
+        if (__builtin_popcountll(lanes) >= 4) {
+            if (((lanes >> lane) & 1) != 0) {
+                lane_copy<false>(&w.ring[rd], &w.ring[ry], match_len, false, hp);
+            }
+            todo &= ~lanes;
+            undone &= ~lanes;
             wave_order();
         }
-        if (other == 0) {
-            break;
-        }
-        /* a wide literal, then the match unless the member
-         * is the terminal literal (no rest member is a lane match) */
-        const uint32_t j = __builtin_ctzll(other);
-        clear_bit(other, j);
-        const uint32_t jl = __builtin_amdgcn_readlane(lit_len, j);
-        const uint32_t jlit = __builtin_amdgcn_readlane(lit, j);
-        const uint32_t jd = __builtin_amdgcn_readlane(drel, j);
-        const uint64_t jd0 = D0 + jd;
-        if (jl > kLaneLit) {
-            for (uint32_t i = lane; i < jl; i += kWave) {
-                w.ring[ring_index<W::kSize>(da, jd0 + i)] = cw[jlit + i];
+        /* the others in stream order, two at a time where the second does
+         * not touch the first */
+        const uint64_t below = todo & ((1ull << lane) - 1);
+        const uint64_t before = below == 0 ? 0 : 1ull << (63 - __builtin_clzll(below));
+        const uint64_t tied = __ballot((waits_for & before) != 0) | ~(once_mask | again_mask);
+        undone &= ~todo;
+        while (todo != 0) {
+            const uint32_t j = __builtin_ctzll(todo);
+            clear_bit(todo, j);
+            const uint32_t a0 = __builtin_amdgcn_readlane(fast_a, j);
+            const uint32_t b0 = __builtin_amdgcn_readlane(fast_b, j);
+            if ((((once_mask | again_mask) >> j) & 1) != 0) {
+                if ((todo & (0 - todo) & ~tied) != 0) {
+                    const uint32_t j1 = __builtin_ctzll(todo);
+                    clear_bit(todo, j1);
+                    const uint32_t a1 = __builtin_amdgcn_readlane(fast_a, j1);
+                    const uint32_t b1 = __builtin_amdgcn_readlane(fast_b, j1);
+                    const uint8_t x0 = again_from(a0, b0);
+                    const uint8_t x1 = again_from(a1, b1);
+                    put(a0, b0, x0);
+                    put(a1, b1, x1);
+                } else {
+                    put(a0, b0, again_from(a0, b0));
+                }
+                wave_order();
+                continue;
             }
-        }
-        wave_order();
-        if (j < take) {
             const uint32_t jm = __builtin_amdgcn_readlane(match_len, j);
             const uint32_t joff = __builtin_amdgcn_readlane(offset, j);
-            const uint64_t jm0 = jd0 + jl;
+            const uint64_t jm0 = D0 + __builtin_amdgcn_readlane(m_rel, j);
             const uint64_t jfrom = jm0 - joff;
+            if (jm > kWideMatch && jfrom >= hist_lo) {
+                ring_match_wide(w, da, jm0, joff, jm, lane);
+                wave_order();
+                continue;
+            }
             /* byte i copies period byte i mod joff, kept per lane as i
-             * steps by 64; lane mod joff and 64 mod joff as in the fast
-             * loop (for joff > 64 they are lane and 64) */
-            const uint32_t jb = __builtin_amdgcn_readlane(fast_b, j);
-            const uint32_t jo = jb & 255;
-            const uint32_t jq = jb >> 8;
+             * steps by 64; lane mod joff and 64 mod joff as above (for
+             * joff > 64 they are lane and 64) */
+            const uint32_t jo = (b0 >> 8) & 255;
+            const uint32_t jq = b0 >> 16;
             uint32_t r = lane - __umul24(__umul24(lane, jq) >> 12, jo);
             const uint32_t step =
                 joff > kWave ? kWave : kWave - __umul24(__umul24(kWave, jq) >> 12, jo);
-            for (uint32_t i = lane; i < jm; i += kWave) {
-                w.ring[ring_index<W::kSize>(da, jm0 + i)] =
-                    history_byte(w, dst, jfrom + r, hist_lo);
-                r += step;
-                r = r >= joff ? r - joff : r;
+            if (jfrom >= hist_lo) {
+                const uint32_t jd = (uint32_t)(da + jm0), js = (uint32_t)(da + jfrom);
+                for (uint32_t i = lane; i < jm; i += kWave) {
+                    w.ring[(jd + i) & (W::kSize - 1)] = w.ring[(js + r) & (W::kSize - 1)];
+                    r += step;
+                    r = r >= joff ? r - joff : r;
+                }
+            } else {
+                for (uint32_t i = lane; i < jm; i += kWave) {
+                    w.ring[ring_index<W::kSize>(da, jm0 + i)] =
+                        history_byte(w, dst, jfrom + r, hist_lo);
+                    r += step;
+                    r = r >= joff ? r - joff : r;
+                }
             }
+            wave_order();
         }
-        wave_order();
+        if (!Order::kInTurn || turn) {
+            break;
+        }
+        if (!order.wait_turn()) {
+            return false;
+        }
+        if (later == 0) {
+            break;
+        }
+        turn = true;
+        later = 0;
     }
     dp = D1;
     const uintptr_t a_end = done ? da + dp : ((da + dp) & ~(uintptr_t)15);
@@ -949,261 +1021,13 @@ __device__ __forceinline__ void execute_group(W& w, const uint8_t* cw, const Gro
         flush_ring(w, dst, flushed, to, lane);
         flushed = to;
     }
+    return true;
 }
 
 /* ------------------------------------------------- window parse */
 
-/* Follows the links from `start` (a scalar chain: each step reads the next
- * position out of the lane that holds the current one). Lane j of `member`
- * receives member j's position. The walk ends at a stop link (that position
- * is not a member), past the window, or after 64 members; it returns the
- * position after the last member and the member count. */
-template <uint32_t kC, uint32_t kMinStep, bool kStraight>
-__device__ __forceinline__ uint32_t walk_chain_regions(const uint32_t (&link)[kC],
-                                                       uint32_t start, uint32_t& count_out,
-                                                       uint32_t& member) {
-    static_assert(kStop >= kC * kWave + kWave, "a stop link must leave every region");
-    static_assert(kMinStep >= 2, "links go forward");
-    /* most members one region can hold, and the count at or below which
-     * the walk takes the unchecked loop there */
-    constexpr uint32_t kRegionMax = (kWave - 1) / kMinStep + 1;
-    constexpr uint32_t kFastMax = kWave - kRegionMax;
-    /* A straight run of guarded regions with no early exit (an exit edge
-     * out of the unrolled loop has the compiler re-materialise live values
-     * at every region), whatever kStraight says. A region is entered only
-     * while pos lies in it and fewer than 64 members are held; a stop link
-     * lies past every region, so the walk's end needs no flag of its own
-     * and is settled once, after the last region. */
-    uint32_t pos = start, count = 0, prev = kStop;
-#pragma unroll
-    for (uint32_t k = 0; k < kC; k++) {
-        uint32_t rel = pos - k * kWave;
-        if ((rel | count) >= kWave) {
-            continue; /* pos lies in a later region, or the walk has ended */
-        }
-        /* Per member: read the link of pos out of its lane, record pos as
-         * member `count`, step. The loop leaves once pos is outside this
-         * region (a stop link lands far outside) or 64 members are held.
-         * Only scalar registers are written apart from `member`. Two
-         * members a turn, the current position alternating between pos and
-         * nx, so that no step moves it.
-         * Links only go forward, by kMinStep bytes or more (an LZ4
-         * sequence takes 3, a Snappy element 2), so a region holds at most
-         * kRegionMax members and "pos < base + 64" is the whole region
-         * check. Entered with at most kFastMax members, the walk cannot
-         * pass 64 inside the region and takes the fast loop: the position itself selects
-         * the lane (a wave64 v_readlane uses bits [5:0] of the select), and
-         * a member costs a compare, a branch and the count. Otherwise the
-         * checked loop tests the count as well. In the fast loop four
-         * instructions separate a v_readlane from the one that uses its
-         * result as the select, the 4 wait states that use needs. */
-        uint32_t nx, t;
-        /* The count is an operand bound to m0 ("{m0}"), so the compiler
-         * moves it in and out and keeps its own uses of m0 apart:
-         * v_writelane takes its value and lane select from scalar
-         * registers, and only m0 as the lane select keeps it within one
-         * constant-bus read. The leading s_nop covers a lane select (rel)
-         * that the compiler may have just written from a vector
-         * instruction, and m0 written just before its first use. */
-        asm volatile(
-            "s_nop 4\n\t"
-            "s_cmp_gt_u32 %[cnt], %[fmax]\n\t"
-            "s_cbranch_scc1 walk_loop_%=\n"
-            "walk_fast_%=:\n\t"
-            "v_readlane_b32 %[nx], %[lk], %[pos]\n\t"
-            "v_writelane_b32 %[mem], %[pos], m0\n\t"
-            "s_add_u32 m0, m0, 1\n\t"
-            "s_cmp_lt_u32 %[nx], %[lim]\n\t"
-            "s_cbranch_scc0 walk_out_nx_%=\n\t"
-            "v_readlane_b32 %[pos], %[lk], %[nx]\n\t"
-            "v_writelane_b32 %[mem], %[nx], m0\n\t"
-            "s_add_u32 m0, m0, 1\n\t"
-            "s_cmp_lt_u32 %[pos], %[lim]\n\t"
-            "s_cbranch_scc1 walk_fast_%=\n\t"
-            "s_mov_b32 %[prev], %[nx]\n\t"
-            "s_branch walk_done_%=\n"
-            "walk_loop_%=:\n\t"
-            "v_readlane_b32 %[nx], %[lk], %[rel]\n\t"
-            "v_writelane_b32 %[mem], %[pos], m0\n\t"
-            "s_sub_u32 %[rel], %[nx], %[base]\n\t"
-            "s_add_u32 m0, m0, 1\n\t"
-            "s_or_b32 %[t], %[rel], m0\n\t"
-            "s_cmp_lt_u32 %[t], 64\n\t"
-            "s_cbranch_scc0 walk_out_nx_%=\n\t"
-            "v_readlane_b32 %[pos], %[lk], %[rel]\n\t"
-            "v_writelane_b32 %[mem], %[nx], m0\n\t"
-            "s_sub_u32 %[rel], %[pos], %[base]\n\t"
-            "s_add_u32 m0, m0, 1\n\t"
-            "s_or_b32 %[t], %[rel], m0\n\t"
-            "s_cmp_lt_u32 %[t], 64\n\t"
-            "s_cbranch_scc1 walk_loop_%=\n\t"
-            "s_mov_b32 %[prev], %[nx]\n\t"
-            "s_branch walk_done_%=\n"
-            "walk_out_nx_%=:\n\t"
-            "s_mov_b32 %[prev], %[pos]\n\t"
-            "s_mov_b32 %[pos], %[nx]\n"
-            "walk_done_%=:"
-            : [mem] "+v"(member), [pos] "+s"(pos), [cnt] "+{m0}"(count), [rel] "+s"(rel),
-              [prev] "=&s"(prev), [nx] "=&s"(nx), [t] "=&s"(t)
-            : [lk] "v"(link[k]), [base] "s"(k * kWave), [lim] "s"(k * kWave + kWave),
-              [fmax] "s"(kFastMax)
-            : "scc");
-    }
-    /* a stop link: the member that read it (prev, the last member) is no
-     * member, and the walk ends there; a walk that started on a stop link
-     * holds no member and stays as it is */
-    if (pos == kStop && count != 0) {
-        pos = prev;
-        count -= 1;
-    }
-    count_out = uniform32(count);
-    return uniform32(pos);
-}
-
-/* One region k of the walk (positions [64 k, 64 k + 64), links in lk<k>):
- * per member, read the link of pos out of its lane, record pos as member
- * m0, step; two members a turn, the current position alternating between
- * pos and nx so that no step moves it. Links only go forward by kMinStep
- * bytes or more, so a region holds at most kRegionMax members and
- * "pos < 64 k + 64" is the whole region check; entered with at most
- * kFastMax members the walk cannot pass 64 inside the region and takes the
- * fast loop (the position itself selects the lane: a wave64 v_readlane
- * uses bits [5:0] of the select), else the checked loop, which tests the
- * count as well. Four instructions separate a v_readlane from the one that
- * uses its result as the select (the 4 wait states that use needs), and
- * three separate an m0 update from the v_writelane that reads it. A
- * region is entered only while pos lies in it and fewer than 64 members are
- * held ((pos - base) | count below 64); leaving it (pos = the next position)
- * falls into the next region's check. A stop link lies past every region,
- * so the walk's end is settled once, in WALK_END. */
-#define WALK_REGION(k, B, L, N)                                                             \
-    "r" #k "_%=:\n\t"                                                                       \
-    "s_sub_u32 %[rel], %[pos], " #B "\n\t"                                                  \
-    "s_or_b32 %[t], %[rel], m0\n\t"                                                         \
-    "s_cmp_lt_u32 %[t], 64\n\t"                                                             \
-    "s_cbranch_scc0 r" #N "_%=\n\t"                                                         \
-    "s_cmp_gt_u32 m0, %[fmax]\n\t"                                                          \
-    "s_cbranch_scc1 c" #k "_%=\n"                                                           \
-    "f" #k "_%=:\n\t"                                                                       \
-    "v_readlane_b32 %[nx], %[lk" #k "], %[pos]\n\t"                                         \
-    "v_writelane_b32 %[mem], %[pos], m0\n\t"                                                \
-    "s_add_u32 m0, m0, 1\n\t"                                                               \
-    "s_cmp_lt_u32 %[nx], " #L "\n\t"                                                        \
-    "s_cbranch_scc0 o" #k "_%=\n\t"                                                         \
-    "v_readlane_b32 %[pos], %[lk" #k "], %[nx]\n\t"                                         \
-    "v_writelane_b32 %[mem], %[nx], m0\n\t"                                                 \
-    "s_add_u32 m0, m0, 1\n\t"                                                               \
-    "s_cmp_lt_u32 %[pos], " #L "\n\t"                                                       \
-    "s_cbranch_scc1 f" #k "_%=\n\t"                                                         \
-    "s_mov_b32 %[prev], %[nx]\n\t"                                                          \
-    "s_branch x" #k "_%=\n"                                                                 \
-    "c" #k "_%=:\n\t"                                                                       \
-    "v_readlane_b32 %[nx], %[lk" #k "], %[rel]\n\t"                                         \
-    "v_writelane_b32 %[mem], %[pos], m0\n\t"                                                \
-    "s_sub_u32 %[rel], %[nx], " #B "\n\t"                                                   \
-    "s_add_u32 m0, m0, 1\n\t"                                                               \
-    "s_or_b32 %[t], %[rel], m0\n\t"                                                         \
-    "s_cmp_lt_u32 %[t], 64\n\t"                                                             \
-    "s_cbranch_scc0 o" #k "_%=\n\t"                                                         \
-    "v_readlane_b32 %[pos], %[lk" #k "], %[rel]\n\t"                                        \
-    "v_writelane_b32 %[mem], %[nx], m0\n\t"                                                 \
-    "s_sub_u32 %[rel], %[pos], " #B "\n\t"                                                  \
-    "s_add_u32 m0, m0, 1\n\t"                                                               \
-    "s_or_b32 %[t], %[rel], m0\n\t"                                                         \
-    "s_cmp_lt_u32 %[t], 64\n\t"                                                             \
-    "s_cbranch_scc1 c" #k "_%=\n\t"                                                         \
-    "s_mov_b32 %[prev], %[nx]\n\t"                                                          \
-    "s_branch x" #k "_%=\n"                                                                 \
-    "o" #k "_%=:\n\t"                                                                       \
-    "s_mov_b32 %[prev], %[pos]\n\t"                                                         \
-    "s_mov_b32 %[pos], %[nx]\n"                                                             \
-    "x" #k "_%=:\n"
-
-/* The walk's entry and exits around the regions: the count lives in m0
- * during the walk (saved and restored around it): v_writelane takes its
- * value and lane select from scalar registers, and only m0 as the lane
- * select keeps it within one constant-bus read. The leading s_nop covers a
- * lane select the compiler may have just written from a vector instruction,
- * and m0 written just before its first use. Past the last region: a stop
- * link (pos = 0xffff) read by the last member (prev) makes it no member, and
- * the walk ends there (a walk that started on a stop link holds none);
- * otherwise the walk ended past the window or at 64 members. */
-#define WALK_BEGIN                                                                          \
-    "s_mov_b32 %[m0s], m0\n\t"                                                              \
-    "s_mov_b32 m0, %[cnt]\n\t"                                                              \
-    "s_nop 4\n"
-#define WALK_END(N)                                                                         \
-    "r" #N "_%=:\n\t"                                                                       \
-    "s_cmpk_eq_u32 %[pos], 0xffff\n\t"                                                      \
-    "s_cbranch_scc0 end_%=\n\t"                                                             \
-    "s_cmp_eq_u32 m0, 0\n\t"                                                                \
-    "s_cbranch_scc1 end_%=\n\t"                                                             \
-    "s_mov_b32 %[pos], %[prev]\n\t"                                                         \
-    "s_sub_u32 m0, m0, 1\n"                                                                 \
-    "end_%=:\n\t"                                                                           \
-    "s_mov_b32 %[cnt], m0\n\t"                                                              \
-    "s_mov_b32 m0, %[m0s]"
-#define WALK_OPERANDS                                                                       \
-    : [mem] "+v"(member), [pos] "+s"(pos), [cnt] "+s"(count), [rel] "=&s"(rel),             \
-      [prev] "+s"(prev), [nx] "=&s"(nx), [t] "=&s"(t), [m0s] "=&s"(m0_saved)
-
-/* The walk of walk_chain_regions, with the same results: for windows of up
- * to eight regions as one asm block (WALK_REGION per region), else region
- * by region. */
-template <uint32_t kC, uint32_t kMinStep, bool kStraight>
-__device__ __forceinline__ uint32_t walk_chain(const uint32_t (&link)[kC], uint32_t start,
-                                               uint32_t& count_out, uint32_t& member) {
-    static_assert(kStop >= kC * kWave + kWave, "a stop link must leave every region");
-    static_assert(kMinStep >= 2, "links go forward");
-    (void)kStraight;
-    /* most members one region can hold, and the count at or below which
-     * the walk takes the unchecked loop there */
-    constexpr uint32_t kRegionMax = (kWave - 1) / kMinStep + 1;
-    constexpr uint32_t kFastMax = kWave - kRegionMax;
-    if constexpr (kC > 8) {
-        /* sixteen regions in one block keep all sixteen link registers live
-         * at once and spill (5% slower on LZ4 than a block per region) */
-        return walk_chain_regions<kC, kMinStep, kStraight>(link, start, count_out, member);
-    } else {
-        uint32_t pos = start, count = 0, rel, prev = kStop, nx, t, m0_saved;
-        /* one asm block for the whole walk: no compiler code between regions
-         * (Snappy's seven regions: 2% faster than a block per region) */
-        if constexpr (kC == 8) {
-            asm volatile(WALK_BEGIN WALK_REGION(0, 0, 64, 1) WALK_REGION(1, 64, 128, 2)
-                             WALK_REGION(2, 128, 192, 3) WALK_REGION(3, 192, 256, 4)
-                                 WALK_REGION(4, 256, 320, 5) WALK_REGION(5, 320, 384, 6)
-                                     WALK_REGION(6, 384, 448, 7) WALK_REGION(7, 448, 512, 8)
-                                         WALK_END(8)
-                         WALK_OPERANDS
-                         : [lk0] "v"(link[0]), [lk1] "v"(link[1]), [lk2] "v"(link[2]),
-                           [lk3] "v"(link[3]), [lk4] "v"(link[4]), [lk5] "v"(link[5]),
-                           [lk6] "v"(link[6]), [lk7] "v"(link[7]), [fmax] "s"(kFastMax)
-                         : "scc");
-        } else if constexpr (kC == 7) {
-            asm volatile(WALK_BEGIN WALK_REGION(0, 0, 64, 1) WALK_REGION(1, 64, 128, 2)
-                             WALK_REGION(2, 128, 192, 3) WALK_REGION(3, 192, 256, 4)
-                                 WALK_REGION(4, 256, 320, 5) WALK_REGION(5, 320, 384, 6)
-                                     WALK_REGION(6, 384, 448, 7) WALK_END(7)
-                         WALK_OPERANDS
-                         : [lk0] "v"(link[0]), [lk1] "v"(link[1]), [lk2] "v"(link[2]),
-                           [lk3] "v"(link[3]), [lk4] "v"(link[4]), [lk5] "v"(link[5]),
-                           [lk6] "v"(link[6]), [fmax] "s"(kFastMax)
-                         : "scc");
-        } else {
-            static_assert(kC == 7, "walk regions are spelled out for these widths");
-        }
-        count_out = uniform32(count);
-        return uniform32(pos);
-    }
-}
-#undef WALK_REGION
-#undef WALK_BEGIN
-#undef WALK_END
-#undef WALK_OPERANDS
-
-/* The chain from `start`, as walk_chain decides it (members while in the
- * window and under 64; a position with a stop link is no member), by
- * pointer doubling over the window's links in LDS (jump, kC * 64 entries)
+/* The chain of links from `start` (members while in the window and under
+ * 64; a position with a stop link is no member), by pointer doubling over the window's links in LDS (jump, kC * 64 entries)
  * instead of one dependent step per member. Round r (r = 0..5) has the
  * table map a position to the one 2^r links on: lanes [2^r, 2^(r+1)) take
  * their member from lane (lane - 2^r) with one lookup, then every entry
@@ -1270,6 +1094,203 @@ __device__ __forceinline__ uint32_t walk_doubling(uint32_t (&link)[kC], uint32_t
     return uniform32(pos);
 }
 
+/* What resolving up to 64 members of a window decided: status not OK (the
+ * chunk fails); slow (the first member is one the window cannot hold); or
+ * the group g, whose `g.take` members (and a terminal literal) run, with
+ * done when the chunk ends after it. take < count: member take starts the
+ * next group. */
+struct Resolved {
+    int status;
+    bool slow;
+    bool done;
+    Group g;
+};
+
+/* The first flagged lane decides the group's end: `cut` (the group's output
+ * is full there), `held` (a member the window cannot hold), a status, or the
+ * chunk's end. */
+struct GroupEnd {
+    uint32_t take;
+    int status;
+    bool slow;
+    bool ended;
+};
+__device__ __forceinline__ GroupEnd group_end(uint32_t count, bool cut, bool hold, int ev,
+                                              bool ends) {
+    GroupEnd e{count, kOk, false, false};
+    const uint64_t flags = __ballot(cut || hold || ev != kOk || ends);
+    if (flags != 0) {
+        const uint32_t j = __builtin_ctzll(flags);
+        e.take = j;
+        const uint32_t what =
+            uniform32(__builtin_amdgcn_readlane((uint32_t)ev << 2 | (hold ? 2u : 0u) |
+                                                    (cut ? 1u : 0u), j));
+        if ((what & 2) != 0) {
+            e.slow = j == 0;
+        } else if ((what >> 2) != 0) {
+            e.status = (int)(what >> 2);
+        } else if ((what & 1) != 0) {
+            e.slow = j == 0;
+        } else {
+            e.ended = true;
+        }
+    }
+    e.take = uniform32(e.take);
+    e.slow = uniform32(e.slow) != 0;
+    e.ended = uniform32(e.ended) != 0;
+    e.status = (int)uniform32((uint32_t)e.status);
+    return e;
+}
+
+/* Source bytes from the window start, clamped: no window reaches
+ * kMaxWindow, so a position there stands for the source end. */
+constexpr uint32_t kMaxWindow = 0x7FFF0000u;
+__device__ __forceinline__ uint32_t window_limit(uint64_t src_size, uint64_t base) {
+    const uint64_t left = src_size - base;
+    return left >= kMaxWindow ? kMaxWindow : (uint32_t)left;
+}
+
+/* Extension bytes after the first that a length may have and still be
+ * followed in a window: matches of up to 2058 bytes, which a group holds. */
+constexpr uint32_t kWalkExtra = 7;
+static_assert(4 + 15 + 255 * (kWalkExtra + 1) + 270 <= kPipeBatch, "a group holds any such member");
+
+/* More than a sequence with one extension byte per length (275 bytes) and
+ * the margins of every rung reach past its start, and than the margins of
+ * the destination. */
+constexpr uint32_t kLz4Inside = 320;
+
+/* Resolves the members of an LZ4 window (lane j < count holds member j's
+ * position, relative to the window start `base` whose bytes are at cw;
+ * kLong: a match length may have up to kWalkExtra + 1 extension bytes): a
+ * prefix sum places each member's output from dp on and the exact ladder
+ * (src/lz4_block.h:95-258) runs per lane. A group's output stays within
+ * `batch` bytes. A position at or past the source end is CORRUPT (nothing
+ * at cw is used for it). */
+template <bool kLong>
+__device__ __forceinline__ Resolved resolve_lz4(const uint8_t* cw, uint32_t member,
+                                                uint32_t count, uint64_t base,
+                                                uint64_t src_size, uint64_t cap, uint64_t dp,
+                                                uint32_t batch, uint32_t lane) {
+    const bool is_member = lane < count;
+    uint64_t s = base + member; /* absolute source position */
+    const bool past = s >= src_size || member >= kMaxWindow;
+    Cand c = parse_candidate(cw, is_member && !past ? member : 0);
+    /* away from both ends of the chunk only the offset can be wrong */
+    const uint32_t last_member = uniform32(__builtin_amdgcn_readlane(member, count - 1));
+    const bool inside = last_member < kMaxWindow && src_size - base > last_member + kLz4Inside;
+    if (kLong && inside && is_member && c.complex && c.lit_len < 15 + 255) {
+        /* a match length of two to kWalkExtra + 1 extension bytes */
+        uint32_t q = c.next;
+        uint32_t e = 255;
+        for (uint32_t i = 0; i < kWalkExtra && e == 255; i++) {
+            e = cw[q++];
+            c.match_len += e;
+        }
+        c.complex = e == 255;
+    }
+    const bool hold = is_member && !past && c.complex;
+    const uint32_t out_len = is_member && !hold && !past ? c.lit_len + c.match_len : 0;
+    const uint32_t incl = wave_inclusive_sum(out_len, lane);
+    const uint32_t drel = incl - out_len;
+    const uint64_t d0 = dp + drel; /* absolute destination */
+    int ev = kOk;
+    bool terminal = false;
+    const bool long_match = c.match_len > 4 + 15 + 255 - 1;
+    const uint32_t all = uniform32(__builtin_amdgcn_readlane(incl, kWave - 1));
+    if (inside && cap - dp > all + kLz4Inside) {
+        const uint32_t before = (dp < kMaxWindow ? (uint32_t)dp : kMaxWindow) + drel + c.lit_len;
+        if (is_member && !hold && (c.offset == 0 || c.offset > before)) {
+            ev = kCorrupt;
+        }
+    } else if (is_member && !hold && !long_match) {
+        if (past) {
+            ev = kCorrupt;
+        } else {
+            s++;
+            if ((c.tok >> 4) == 15) {
+                if (s + 15 >= src_size) {
+                    ev = kCorrupt;
+                } else if (15 > cap - d0) {
+                    ev = kTooSmall;
+                } else {
+                    s++;
+                    if (s + 15 > src_size) {
+                        ev = kCorrupt;
+                    }
+                }
+            }
+            const uint64_t L = c.lit_len;
+            if (ev == kOk) {
+                if (L > src_size - s) {
+                    ev = kCorrupt;
+                } else if (L > cap - d0) {
+                    ev = kTooSmall;
+                } else if (cap - d0 - L < kLz4SlackDst || src_size - s - L < kLz4SlackSrc) {
+                    if (s + L != src_size) {
+                        ev = kCorrupt;
+                    } else if (cap == 0 && c.tok != 0) {
+                        ev = kCorrupt;
+                    } else {
+                        terminal = true;
+                    }
+                } else {
+                    const uint64_t dl = d0 + L;
+                    uint64_t M = (c.tok & 15) + 4;
+                    s += L + 2;
+                    if (c.offset == 0 || c.offset > dl) {
+                        ev = kCorrupt;
+                    } else {
+                        if ((c.tok & 15) == 15) {
+                            if (s >= src_size) {
+                                ev = kCorrupt;
+                            } else if (M > cap - dl) {
+                                ev = kTooSmall;
+                            } else {
+                                s++;
+                                M = c.match_len;
+                                if (s + kLz4MatchMargin > src_size) {
+                                    ev = kCorrupt;
+                                }
+                            }
+                        }
+                        if (ev == kOk) {
+                            if (M > cap - dl) {
+                                ev = kTooSmall;
+                            } else if (M > cap - dl - kLz4LastLiterals) {
+                                ev = kCorrupt;
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+    const uint32_t mine = terminal ? c.lit_len : out_len;
+    /* a full group ends before anything its next member would decide */
+    const bool cut = is_member && drel + mine > batch;
+    const bool inner = inside && cap - dp > all + kLz4Inside;
+    const GroupEnd e = group_end(count, cut, hold || (is_member && long_match && !inner),
+                                 cut ? kOk : ev, terminal);
+    Resolved r;
+    r.status = e.status;
+    r.slow = e.slow || count == 0;
+    r.done = e.ended;
+    r.g.lit = c.lit;
+    r.g.lit_len = c.lit_len;
+    r.g.match_len = c.match_len;
+    r.g.offset = c.offset;
+    r.g.drel = drel;
+    r.g.take = e.take;
+    r.g.terminal = e.ended;
+    const uint32_t last = e.ended ? e.take : e.take - 1;
+    r.g.end_rel = e.take == 0 && !e.ended
+                      ? 0u
+                      : uniform32(__builtin_amdgcn_readlane(incl, last) -
+                                  (e.ended ? __builtin_amdgcn_readlane(c.match_len, last) : 0));
+    return r;
+}
+
 /* What parsing one window decided. kGroup: execute `g` (staged at `delta`
  * in the stage buffer) and advance the source by `consumed`. kSlow: one
  * sequence the window cannot hold, by the scalar ladder (`q`, with the
@@ -1287,17 +1308,39 @@ struct Parsed {
     uint64_t lead_dp; /* output position after q */
 };
 
-/* Stages the window at sp into `stage`, speculates, walks and resolves it
- * (src/lz4_block.h:95-258 for every member, in parallel) and advances
- * sp and dp past what it decided. Reads the source only. kDoubling: walk
- * the chain by pointer doubling over `jump` (the one-wave form, where the
- * wave's own latency is the pace), else serially (the two-wave parser,
- * which leaves LDS and issue to the copier; `jump` is unused). */
-template <uint32_t kC, bool kDoubling>
+/* The group a window's chain resolved to, after a possible leading sequence
+ * already in `out`; pos: the position after the chain's last member. False
+ * when nothing of the window can run (its first member is slow). */
+__device__ __forceinline__ bool take_group(const Resolved& r, uint32_t count, uint32_t member,
+                                           uint32_t pos, uint64_t base, uint64_t src_size,
+                                           uint64_t& sp, uint64_t& dp, Parsed& out) {
+    if (r.status != kOk) {
+        out.kind = kParseFail;
+        out.status = r.status;
+        return true;
+    }
+    if (r.slow || (r.g.take == 0 && !r.done)) {
+        return false;
+    }
+    out.kind = kParseGroup;
+    out.g = r.g;
+    const uint64_t next_sp =
+        r.done ? src_size
+               : base + (r.g.take == count ? pos : __builtin_amdgcn_readlane(member, r.g.take));
+    sp = uniform64(next_sp);
+    dp = uniform64(dp + r.g.end_rel);
+    out.done = r.done;
+    return true;
+}
+
+/* The one-wave form's step: stages the window at sp into `stage`,
+ * speculates, walks the chain by pointer doubling over `jump` and resolves
+ * it, and advances sp and dp past what it decided. Reads the source only. */
 __device__ __forceinline__ Parsed parse_window(uint8_t* stage, uint16_t* jump, gcu8* src,
                                                uint64_t src_size, uint64_t cap, uint64_t& sp,
                                                uint64_t& dp, uint32_t lane,
                                                uint32_t& touch) {
+    constexpr uint32_t kC = kCandSplit;
     Parsed out;
     out.kind = kParseFail;
     out.status = kOk;
@@ -1305,12 +1348,12 @@ __device__ __forceinline__ Parsed parse_window(uint8_t* stage, uint16_t* jump, g
     out.lead = false;
     out.lead_dp = 0;
     const uint64_t base = sp; /* window start; member positions are relative to it */
-    out.delta = stage_into<kC>(stage, src, src_size, sp, lane);
-    touch = touch_ahead<kC>(src, src_size, sp, lane);
+    out.delta = stage_into<1>(stage, src, src_size, sp, stage_bytes(kC * kWave), lane);
+    touch = touch_ahead(src, src_size, sp, stage_bytes(kC * kWave), 16, lane);
     const uint8_t* cw = stage + out.delta;
     /* the scalar ladder reads a sequence's header from the stage while it
      * lies there (an LDS round trip per byte instead of a global one) */
-    const StagedBytes staged{src, cw, base, stage_bytes(kC) + 16 - out.delta};
+    const StagedBytes staged{src, cw, base, stage_bytes(kC * kWave) + 16 - out.delta};
 
     /* speculate: the link of each candidate position */
     uint32_t link[kC];
@@ -1349,132 +1392,11 @@ __device__ __forceinline__ Parsed parse_window(uint8_t* stage, uint16_t* jump, g
     /* walk the true chain */
     uint32_t count = 0;
     uint32_t member = 0; /* lane j: position of member j */
-    const uint32_t pos = kDoubling
-                             ? walk_doubling<kC>(link, start, jump, count, member, lane)
-                             : walk_chain<kC, 3, false>(link, start, count, member);
-
-    bool slow = count == 0;
-    if (!slow) {
-        /* resolve members: the exact ladder for each member's sequence */
-        const bool is_member = lane < count;
-        const Cand c = parse_candidate(cw, is_member ? member : 0);
-        const uint32_t out_len = is_member ? c.lit_len + c.match_len : 0;
-        const uint32_t incl = wave_inclusive_sum(out_len, lane);
-        const uint32_t drel = incl - out_len;
-        const uint64_t d0 = dp + drel; /* absolute destination */
-        int ev = kOk;
-        bool terminal = false;
-        if (is_member) {
-            uint64_t s = base + member;  /* absolute source position */
-            if (s >= src_size) {
-                ev = kCorrupt;
-            } else {
-                s++;
-                if ((c.tok >> 4) == 15) {
-                    if (s + 15 >= src_size) {
-                        ev = kCorrupt;
-                    } else if (15 > cap - d0) {
-                        ev = kTooSmall;
-                    } else {
-                        s++;
-                        if (s + 15 > src_size) {
-                            ev = kCorrupt;
-                        }
-                    }
-                }
-                const uint64_t L = c.lit_len;
-                if (ev == kOk) {
-                    if (L > src_size - s) {
-                        ev = kCorrupt;
-                    } else if (L > cap - d0) {
-                        ev = kTooSmall;
-                    } else if (cap - d0 - L < kLz4SlackDst || src_size - s - L < kLz4SlackSrc) {
-                        if (s + L != src_size) {
-                            ev = kCorrupt;
-                        } else if (cap == 0 && c.tok != 0) {
-                            ev = kCorrupt;
-                        } else {
-                            terminal = true;
-                        }
-                    } else {
-                        const uint64_t dl = d0 + L;
-                        uint64_t M = (c.tok & 15) + 4;
-                        s += L + 2;
-                        if (c.offset == 0 || c.offset > dl) {
-                            ev = kCorrupt;
-                        } else {
-                            if ((c.tok & 15) == 15) {
-                                if (s >= src_size) {
-                                    ev = kCorrupt;
-                                } else if (M > cap - dl) {
-                                    ev = kTooSmall;
-                                } else {
-                                    s++;
-                                    M = c.match_len;
-                                    if (s + kLz4MatchMargin > src_size) {
-                                        ev = kCorrupt;
-                                    }
-                                }
-                            }
-                            if (ev == kOk) {
-                                if (M > cap - dl) {
-                                    ev = kTooSmall;
-                                } else if (M > cap - dl - kLz4LastLiterals) {
-                                    ev = kCorrupt;
-                                }
-                            }
-                        }
-                    }
-                }
-            }
-        }
-        const uint32_t mine = terminal ? c.lit_len : out_len;
-        const bool cut = is_member && drel + mine > batch_max(kDoubling);
-        const bool flag = is_member && (cut || ev != kOk || terminal);
-        const uint64_t flags = __ballot(flag);
-        uint32_t take = count; /* members executed in full */
-        bool take_terminal = false;
-        int status = kOk;
-        if (flags != 0) {
-            const uint32_t j = __builtin_ctzll(flags);
-            take = j;
-            const bool j_cut = __builtin_amdgcn_readlane((uint32_t)cut, j) != 0;
-            const int j_ev = (int)__builtin_amdgcn_readlane((uint32_t)ev, j);
-            if (j_cut) {
-                slow = j == 0;
-            } else if (j_ev != kOk) {
-                status = j_ev;
-            } else {
-                take_terminal = true;
-            }
-        }
-        take = uniform32(take);
-        take_terminal = uniform32(take_terminal) != 0;
-        slow = uniform32(slow) != 0;
-        status = (int)uniform32((uint32_t)status);
-        if (status != kOk) {
-            out.status = status;
-            return out;
-        }
-        if (!slow && (take != 0 || take_terminal)) {
-            const uint32_t last = take_terminal ? take : take - 1;
-            out.kind = kParseGroup;
-            out.g.lit = c.lit;
-            out.g.lit_len = c.lit_len;
-            out.g.match_len = c.match_len;
-            out.g.offset = c.offset;
-            out.g.drel = drel;
-            out.g.take = take;
-            out.g.terminal = take_terminal;
-            out.g.end_rel = uniform32(__builtin_amdgcn_readlane(incl, last) -
-                                      (take_terminal ? __builtin_amdgcn_readlane(c.match_len, last)
-                                                     : 0));
-            const uint64_t next_sp =
-                take_terminal ? src_size
-                              : base + (take == count ? pos : __builtin_amdgcn_readlane(member, take));
-            sp = uniform64(next_sp);
-            dp = uniform64(dp + out.g.end_rel);
-            out.done = take_terminal;
+    const uint32_t pos = walk_doubling<kC>(link, start, jump, count, member, lane);
+    if (count != 0) {
+        const Resolved r =
+            resolve_lz4<false>(cw, member, count, base, src_size, cap, dp, kBatchMax, lane);
+        if (take_group(r, count, member, pos, base, src_size, sp, dp, out)) {
             return out;
         }
     }
@@ -1504,9 +1426,7 @@ __device__ __forceinline__ Parsed parse_window(uint8_t* stage, uint16_t* jump, g
 /* Longest literal a Snappy window resolves; longer ones take the scalar
  * ladder. A window literal therefore ends below kC * 64 + 5 + 256. */
 constexpr uint32_t kSnappyWinLit = 256;
-static_assert(kCandSplit * 64 + 5 + kSnappyWinLit + 16 <= stage_bytes(kCandSplit) + 16 &&
-                  kCandPipe * 64 + 5 + kSnappyWinLit + 16 <= stage_bytes(kCandPipe) + 16,
-              "stage covers a Snappy window");
+static_assert(5 + kSnappyWinLit + 16 <= stage_bytes(0) + 16, "stage covers a Snappy window");
 
 /* The element a tag at window position c would encode
  * (src/snappy_block.h:288-435): a literal (lit, lit_len; match_len 0) or a
@@ -1577,17 +1497,120 @@ __device__ __forceinline__ Cand parse_candidate_snappy(const uint8_t* cw, uint32
     return k;
 }
 
-/* As parse_window, for Snappy elements after the preamble: every member's
+/* More than a literal element with a copy element after it (271 bytes)
+ * reaches past its start. */
+constexpr uint32_t kSnappyInside = 320;
+
+/* As resolve_lz4, for Snappy elements after the preamble: every member's
  * rungs run in parallel (every reject is CORRUPT_INPUT, so the first
  * failing member in stream order decides), and the member whose position
  * is exactly the end of the source ends the chunk when the output so far
- * equals the declared length. kDoubling as for parse_window. */
-template <uint32_t kC, bool kDoubling>
+ * equals the declared length. */
+__device__ __forceinline__ Resolved resolve_snappy(const uint8_t* cw, uint32_t member,
+                                                   uint32_t count, uint64_t base,
+                                                   uint64_t src_size, uint64_t declared,
+                                                   uint64_t dp, uint32_t lim, uint32_t batch,
+                                                   uint32_t lane) {
+    const bool is_member = lane < count;
+    const uint64_t s = base + member;
+    const bool at_end = is_member && (s >= src_size || member >= kMaxWindow);
+    const Cand c = parse_candidate_snappy(cw, is_member && !at_end ? member : 0, lim);
+    const bool hold = is_member && !at_end && c.complex;
+    const uint32_t out_len = is_member && !at_end && !hold ? c.lit_len + c.match_len : 0;
+    const uint32_t incl = wave_inclusive_sum(out_len, lane);
+    const uint32_t drel = incl - out_len;
+    const uint64_t d0 = dp + drel;
+    int ev = kOk;
+    /* away from both ends of the chunk only the offset can be wrong */
+    const uint32_t last_member = uniform32(__builtin_amdgcn_readlane(member, count - 1));
+    const uint32_t all = uniform32(__builtin_amdgcn_readlane(incl, kWave - 1));
+    if (last_member < kMaxWindow && src_size - base > last_member + kSnappyInside &&
+        declared >= dp && declared - dp > all) {
+        const uint32_t before = (dp < kMaxWindow ? (uint32_t)dp : kMaxWindow) + drel + c.lit_len;
+        if (is_member && !hold && c.match_len != 0 && (c.offset == 0 || c.offset - 1 >= before) &&
+            (c.offset == 0 || (uint64_t)c.offset > d0 + c.lit_len)) {
+            ev = kCorrupt;
+        }
+    } else if (is_member && !hold) {
+        if (at_end) {
+            ev = s == src_size && d0 == declared ? kOk : kCorrupt;
+        } else if (d0 > declared) {
+            ev = kCorrupt;
+        } else if (c.lit_len != 0 || c.match_len == 0) {
+            /* a literal element (src/snappy_block.h:345-370), then, in a
+             * fused member, the copy element after it at (s2, d2) */
+            const uint64_t header = c.lit - member;
+            if (header > src_size - s) {
+                ev = kCorrupt;
+            } else if (c.lit_len > src_size - s - header) {
+                ev = kCorrupt;
+            } else if (c.lit_len > declared - d0) {
+                ev = kCorrupt;
+            } else if (c.match_len != 0) {
+                const uint64_t s2 = s + header + c.lit_len;
+                const uint64_t d2 = d0 + c.lit_len;
+                const uint64_t header2 = c.next - (c.lit + c.lit_len);
+                if (header2 > src_size - s2) {
+                    ev = kCorrupt;
+                } else if (c.offset == 0 || (uint64_t)c.offset > d2) {
+                    ev = kCorrupt;
+                } else if (c.match_len > declared - d2) {
+                    ev = kCorrupt;
+                }
+            }
+        } else {
+            /* a copy element (src/snappy_block.h:371-435) */
+            const uint64_t header = c.lit - member;
+            if (header > src_size - s) {
+                ev = kCorrupt;
+            } else if (c.offset == 0 || (uint64_t)c.offset > d0) {
+                ev = kCorrupt;
+            } else if (c.match_len > declared - d0) {
+                ev = kCorrupt;
+            }
+        }
+    }
+    const bool cut = is_member && !at_end && drel + out_len > batch;
+    const GroupEnd e = group_end(count, cut, hold, ev, at_end);
+    Resolved r;
+    r.status = e.status;
+    r.slow = e.slow || count == 0;
+    r.done = e.ended;
+    r.g.lit = c.lit;
+    r.g.lit_len = c.lit_len;
+    r.g.match_len = c.match_len;
+    r.g.offset = c.offset;
+    r.g.drel = drel;
+    r.g.take = e.take;
+    r.g.terminal = false;
+    r.g.end_rel =
+        e.take == 0 ? 0u : uniform32(__builtin_amdgcn_readlane(incl, e.take - 1));
+    return r;
+}
+
+/* One Snappy element by the exact scalar ladder, as a sequence of its own. */
+__device__ __forceinline__ int snappy_step(SnappyCursor& cur, Lz4Step& q, bool& last) {
+    SnappyStep e;
+    const int st = (int)uniform32((uint32_t)snappy_next(cur, e, last));
+    if (st != kOk) {
+        return st;
+    }
+    q.lit_src = e.is_copy ? 0 : e.from;
+    q.lit_dst = e.to;
+    q.lit_len = e.is_copy ? 0 : e.length;
+    q.match_dst = e.to + (e.is_copy ? 0 : e.length);
+    q.match_len = e.is_copy ? e.length : 0;
+    q.offset = e.is_copy ? (uint32_t)e.offset : 1u;
+    return st;
+}
+
+/* As parse_window, for Snappy. */
 __device__ __forceinline__ Parsed parse_window_snappy(uint8_t* stage, uint16_t* jump, gcu8* src,
                                                       uint64_t src_size, uint64_t cap,
                                                       uint64_t declared, uint64_t& sp,
                                                       uint64_t& dp, uint32_t lane,
                                                       uint32_t& touch) {
+    constexpr uint32_t kC = kCandSplit;
     Parsed out;
     out.kind = kParseFail;
     out.status = kOk;
@@ -1595,12 +1618,11 @@ __device__ __forceinline__ Parsed parse_window_snappy(uint8_t* stage, uint16_t* 
     out.lead = false;
     out.lead_dp = 0;
     const uint64_t base = sp;
-    out.delta = stage_into<kC>(stage, src, src_size, sp, lane);
-    touch = touch_ahead<kC>(src, src_size, sp, lane);
+    out.delta = stage_into<1>(stage, src, src_size, sp, stage_bytes(kC * kWave), lane);
+    touch = touch_ahead(src, src_size, sp, stage_bytes(kC * kWave), 16, lane);
     const uint8_t* cw = stage + out.delta;
-    /* source bytes from the window start, clamped: a fused copy must start
-     * before the source end */
-    const uint32_t lim = src_size - base >= 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)(src_size - base);
+    /* a fused copy must start before the source end */
+    const uint32_t lim = window_limit(src_size, base);
 
     uint32_t link[kC];
 #pragma unroll
@@ -1613,19 +1635,12 @@ __device__ __forceinline__ Parsed parse_window_snappy(uint8_t* stage, uint16_t* 
     uint32_t start = 0;
     if (uniform32(__builtin_amdgcn_readlane(link[0], 0)) == kStop) {
         SnappyCursor cur{src, src_size, cap, sp, dp, declared};
-        SnappyStep e;
         bool last = false;
-        const int st = (int)uniform32((uint32_t)snappy_next(cur, e, last));
+        const int st = snappy_step(cur, out.q, last);
         if (st != kOk) {
             out.status = st;
             return out;
         }
-        out.q.lit_src = e.is_copy ? 0 : e.from;
-        out.q.lit_dst = e.to;
-        out.q.lit_len = e.is_copy ? 0 : e.length;
-        out.q.match_dst = e.to + (e.is_copy ? 0 : e.length);
-        out.q.match_len = e.is_copy ? e.length : 0;
-        out.q.offset = e.is_copy ? (uint32_t)e.offset : 1u;
         sp = uniform64(cur.sp);
         dp = uniform64(cur.dp);
         out.lead = true;
@@ -1641,101 +1656,11 @@ __device__ __forceinline__ Parsed parse_window_snappy(uint8_t* stage, uint16_t* 
     }
     uint32_t count = 0;
     uint32_t member = 0;
-    const uint32_t pos = kDoubling
-                             ? walk_doubling<kC>(link, start, jump, count, member, lane)
-                             : walk_chain<kC, 2, true>(link, start, count, member);
-
-    bool slow = count == 0;
-    if (!slow) {
-        const bool is_member = lane < count;
-        const Cand c = parse_candidate_snappy(cw, is_member ? member : 0, lim);
-        const uint64_t s = base + member;
-        const bool at_end = is_member && s >= src_size;
-        const uint32_t out_len = is_member && !at_end ? c.lit_len + c.match_len : 0;
-        const uint32_t incl = wave_inclusive_sum(out_len, lane);
-        const uint32_t drel = incl - out_len;
-        const uint64_t d0 = dp + drel;
-        int ev = kOk;
-        if (is_member) {
-            if (at_end) {
-                ev = s == src_size && d0 == declared ? kOk : kCorrupt;
-            } else if (d0 > declared) {
-                ev = kCorrupt;
-            } else if (c.lit_len != 0 || c.match_len == 0) {
-                /* a literal element (src/snappy_block.h:345-370), then, in a
-                 * fused member, the copy element after it at (s2, d2) */
-                const uint64_t header = c.lit - member;
-                if (header > src_size - s) {
-                    ev = kCorrupt;
-                } else if (c.lit_len > src_size - s - header) {
-                    ev = kCorrupt;
-                } else if (c.lit_len > declared - d0) {
-                    ev = kCorrupt;
-                } else if (c.match_len != 0) {
-                    const uint64_t s2 = s + header + c.lit_len;
-                    const uint64_t d2 = d0 + c.lit_len;
-                    const uint64_t header2 = c.next - (c.lit + c.lit_len);
-                    if (header2 > src_size - s2) {
-                        ev = kCorrupt;
-                    } else if (c.offset == 0 || (uint64_t)c.offset > d2) {
-                        ev = kCorrupt;
-                    } else if (c.match_len > declared - d2) {
-                        ev = kCorrupt;
-                    }
-                }
-            } else {
-                /* a copy element (src/snappy_block.h:371-435) */
-                const uint64_t header = c.lit - member;
-                if (header > src_size - s) {
-                    ev = kCorrupt;
-                } else if (c.offset == 0 || (uint64_t)c.offset > d0) {
-                    ev = kCorrupt;
-                } else if (c.match_len > declared - d0) {
-                    ev = kCorrupt;
-                }
-            }
-        }
-        const bool cut = is_member && !at_end && drel + out_len > batch_max(kDoubling);
-        const bool flag = is_member && (cut || ev != kOk || at_end);
-        const uint64_t flags = __ballot(flag);
-        uint32_t take = count;
-        bool ended = false;
-        int status = kOk;
-        if (flags != 0) {
-            const uint32_t j = __builtin_ctzll(flags);
-            take = j;
-            const bool j_cut = __builtin_amdgcn_readlane((uint32_t)cut, j) != 0;
-            const int j_ev = (int)__builtin_amdgcn_readlane((uint32_t)ev, j);
-            if (j_ev != kOk) {
-                status = j_ev;
-            } else if (j_cut) {
-                slow = j == 0;
-            } else {
-                ended = true;
-            }
-        }
-        take = uniform32(take);
-        ended = uniform32(ended) != 0;
-        slow = uniform32(slow) != 0;
-        status = (int)uniform32((uint32_t)status);
-        if (status != kOk) {
-            out.status = status;
-            return out;
-        }
-        if (!slow && (take != 0 || ended)) {
-            out.kind = kParseGroup;
-            out.g.lit = c.lit;
-            out.g.lit_len = c.lit_len;
-            out.g.match_len = c.match_len;
-            out.g.offset = c.offset;
-            out.g.drel = drel;
-            out.g.take = take;
-            out.g.terminal = false;
-            out.g.end_rel = take == 0 ? 0u : uniform32(__builtin_amdgcn_readlane(incl, take - 1));
-            const uint32_t consumed = take == count ? pos : __builtin_amdgcn_readlane(member, take);
-            sp = uniform64(ended ? src_size : base + consumed);
-            dp = uniform64(dp + out.g.end_rel);
-            out.done = ended;
+    const uint32_t pos = walk_doubling<kC>(link, start, jump, count, member, lane);
+    if (count != 0) {
+        const Resolved r = resolve_snappy(cw, member, count, base, src_size, declared, dp, lim,
+                                          kBatchMax, lane);
+        if (take_group(r, count, member, pos, base, src_size, sp, dp, out)) {
             return out;
         }
     }
@@ -1746,38 +1671,31 @@ __device__ __forceinline__ Parsed parse_window_snappy(uint8_t* stage, uint16_t* 
     }
     /* one element by the exact scalar ladder */
     SnappyCursor cur{src, src_size, cap, sp, dp, declared};
-    SnappyStep e;
     bool last = false;
-    const int st = (int)uniform32((uint32_t)snappy_next(cur, e, last));
+    const int st = snappy_step(cur, out.q, last);
     if (st != kOk) {
         out.status = st;
         return out;
     }
     out.kind = kParseSlow;
     out.done = uniform32(last) != 0;
-    out.q.lit_src = e.is_copy ? 0 : e.from;
-    out.q.lit_dst = e.to;
-    out.q.lit_len = e.is_copy ? 0 : e.length;
-    out.q.match_dst = e.to + (e.is_copy ? 0 : e.length);
-    out.q.match_len = e.is_copy ? e.length : 0;
-    out.q.offset = e.is_copy ? (uint32_t)e.offset : 1u;
     sp = uniform64(cur.sp);
     dp = uniform64(cur.dp);
     return out;
 }
 
 /* A window of either format. */
-template <int kFormat, uint32_t kC, bool kDoubling>
+template <int kFormat>
 __device__ __forceinline__ Parsed parse_any(uint8_t* stage, uint16_t* jump, gcu8* src,
                                             uint64_t src_size,
                                             uint64_t cap, uint64_t declared, uint64_t& sp,
                                             uint64_t& dp, uint32_t lane,
                                             uint32_t& touch) {
     if (kFormat == kFormatSnappy) {
-        return parse_window_snappy<kC, kDoubling>(stage, jump, src, src_size, cap, declared, sp,
-                                                  dp, lane, touch);
+        return parse_window_snappy(stage, jump, src, src_size, cap, declared, sp, dp, lane,
+                                   touch);
     }
-    return parse_window<kC, kDoubling>(stage, jump, src, src_size, cap, sp, dp, lane, touch);
+    return parse_window(stage, jump, src, src_size, cap, sp, dp, lane, touch);
 }
 
 /* Start of a chunk: the Snappy preamble and its declared length against the
@@ -1868,84 +1786,526 @@ __device__ __forceinline__ void execute_slow(W& w, gcu8* src, gu8* dst,
     }
 }
 
-/* ------------------------------------------------- two-wave pipeline */
+/* ------------------------------------------------- pipelined blocks */
 
-/* The window record the parsing wave hands the copying wave: one Parsed,
- * laid out per lane in LDS. */
-struct alignas(16) PipeRec {
-    uint16_t lit[kWave];
-    uint16_t lit_len[kWave];
-    uint16_t match_len[kWave];
-    uint32_t offset[kWave];
-    uint16_t drel[kWave];
-    uint32_t kind;
-    int32_t status;
-    uint32_t done;
-    uint32_t delta;
-    uint32_t take;
-    uint32_t terminal;
-    uint32_t end_rel;
-    uint32_t lead;              /* kGroup: the slow sequence below runs first */
-    uint64_t lit_src, lit_dst, lit_len_s, match_dst, offset_s, match_len_s, dp_after;
+/* A pipelined block decodes one chunk with four waves. Wave 0, the parser,
+ * finds where the sequences (LZ4) or elements (Snappy) start, a window of
+ * the source at a time, and lists their positions; it decides nothing else.
+ * Waves 1 to 3, the copiers, take the listed members 64 at a time, in turn:
+ * a group is claimed (resolve_*, which decides every status), then executed
+ * while the next copier claims the next one.
+ *
+ * The parser's walk. A window is 64 segments, one a lane. Every lane first
+ * follows the chain from the first byte of its segment as if a member
+ * started there, counting members up to where it leaves the segment. Lane
+ * i's true entry is where lane i - 1 leaves, so each round hands the exits
+ * up one lane and a lane whose entry changed walks again. A wrong start
+ * meets the true chain after a few members (18 on 1 MiB LZ4 token chunks, 5
+ * to 7 on Snappy's and on 64 KiB ones), so the exits are mostly right at
+ * once and few rounds follow. A chain off the true one sometimes takes a
+ * byte for a long length and leaves far ahead; a lane takes an entry past
+ * its own segment only from a lane that is known to be right, so that such
+ * an exit does not cost the lanes behind it their chains. The wave takes 5
+ * steps for 64 members of 64 KiB LZ4 token chunks and of Snappy's, 13 on
+ * 1 MiB LZ4 token chunks. Speculating on every byte position and then
+ * following the links one by one, which this replaced, took 320 vector
+ * instructions and 64 dependent scalar steps for the same 64 members.
+ *
+ * Groups at once. A copier works on group k while groups k - 1 and k - 2
+ * are still running. What it needs of them it gets through `done`, the
+ * count of finished groups, and `done_dp`, the output position they reach;
+ * groups finish strictly in order. Literals, and matches whose source is
+ * final or lies in the group, run before the group's turn; the others wait
+ * for it. Three groups of at most kPipeBatch bytes may lie in the ring
+ * beside the history that a group reads there (kPipeHistory bytes before
+ * its start): a follower can overwrite nothing that a running group reads,
+ * and everything older than that history was flushed to memory by groups
+ * that have finished, because unfinished ones span at most two groups. */
+constexpr uint32_t kPipeWaves = 4;
+constexpr uint32_t kCopiers = kPipeWaves - 1;
+constexpr int kPipeBlock = kPipeWaves * kWave;
+static_assert(kPipeHistory + kCopiers * kPipeBatch + 64 <= kPipeRing &&
+                  (kCopiers - 1) * kPipeBatch <= kPipeHistory,
+              "running groups and their history share the ring");
+static_assert(kPipeBatch <= 64 * kWave, "CoverLds marks a batch");
+
+/* Bytes of a lane's segment: the window is 64 of them. A chunk's first
+ * window, and one after a window cut short, is a small one, so that its
+ * members reach the copiers early. */
+constexpr uint32_t kSegment = 128;
+constexpr uint32_t kSegmentFirst = 32;
+constexpr uint32_t kPipeStage = stage_bytes(kSegment * kWave) + 16;
+constexpr uint32_t stage_rounds(uint32_t bytes) { return (bytes / 16 + 1 + kWave - 1) / kWave; }
+constexpr uint32_t kStageRounds = stage_rounds(stage_bytes(kSegment * kWave));
+constexpr uint32_t kStageRoundsFirst = stage_rounds(stage_bytes(kSegmentFirst * kWave));
+static_assert(stage_rounds(stage_bytes(kCandSplit * kWave)) == 1, "one-wave stage");
+/* Members listed of one window; a window that holds more ends there. */
+constexpr uint32_t kListMax = 1280;
+constexpr uint32_t kListEnd = 0xFFFFu; /* a listed position at the source end */
+
+struct PipeWindow {
+    uint64_t base;   /* source position of the window */
+    uint32_t count;  /* listed members */
+    uint32_t delta;  /* where the window starts in its stage */
+    uint32_t staged; /* staged bytes from the window start */
 };
 
-/* A block's LDS. The two-wave form keeps kS window slots (a stage buffer
- * and a record each; slot 0's stage sits in the ring's LDS); the parser
- * fills them in turn and the copier runs them in the same order. */
-template <uint32_t kS>
+/* The claims' state: where the next group starts. */
+struct PipeClaim {
+    uint64_t dp;      /* output position */
+    uint64_t flushed; /* everything below is in memory (groups flush what follows) */
+    uint64_t ring_lo; /* the ring holds nothing below */
+    uint32_t win;     /* window, kNoWindow before the first */
+    uint32_t idx;     /* next member of it */
+};
+constexpr uint32_t kNoWindow = 0xFFFFFFFFu;
+constexpr uint32_t kClaimsOver = 0xFFFFFFFFu; /* `claim`: the chunk's end was decided */
+
 struct alignas(16) PipeLds {
     union {
         struct {
-            PipeRing w;                        /* copier's ring, slot 0's stage */
-            uint8_t stage[kS - 1][kStageBuf];  /* the other slots' stages */
-            PipeRec rec[kS];
-        } pipe;                                /* two-wave form */
-        struct {
-            WaveLds a, b;                      /* one wave each, once the block splits */
-        } split;
+            RingLds<kPipeRing> w;
+            uint8_t stage[2][kPipeStage];
+            uint16_t list[2][kListMax + 2];
+            CoverLds cover[kCopiers];
+        } pipe;                       /* pipelined */
+        WaveLds split[kPipeWaves];    /* one chunk a wave, once the block splits */
     };
+    PipeWindow window[2];
+    PipeClaim next;
+    uint64_t declared;    /* Snappy's preamble */
+    int32_t begun;        /* its verdict */
     uint32_t chunk_idx;
-    uint32_t fin;           /* lockstep: the step whose record ends the chunk */
-    uint32_t pub[kS];       /* slotted: 1 + sequence number of each slot's record */
-    uint32_t freed[kS];     /* slotted: 1 + sequence number of the record run last there */
-    uint32_t broken;        /* slotted: a wait ran out, and no wave waits any more */
-
-    __device__ uint8_t* stage_of(uint32_t slot) {
-        return slot == 0 ? pipe.w.stage : pipe.stage[slot - 1];
-    }
+    uint32_t published;   /* windows listed */
+    uint32_t retired;     /* windows whose members are all claimed */
+    uint32_t retired_k[2];/* the groups claimed by then */
+    uint32_t claim;       /* the group to be claimed next, or kClaimsOver */
+    uint32_t done;        /* groups finished */
+    uint32_t done_dp;     /* output position they reach (low 32 bits) */
+    uint32_t broken;      /* a wait ran out, and no wave waits any more */
 };
+static_assert(sizeof(PipeLds) <= 40960, "four blocks share a CU's 160 KiB");
 
-/* Slotted blocks signal through LDS words, each written by one wave and
- * polled by the other (s_sleep between reads). A wait longer than any
- * window could take (2^27 polls: seconds) marks the block broken, and a
- * broken block waits no more (false). */
+/* The waves signal through LDS words (s_sleep between reads). A wait longer
+ * than any work could take (2^27 polls: seconds) marks the block broken,
+ * and a broken block waits no more. */
 typedef __attribute__((address_space(3))) volatile uint32_t lds_flag;
-__device__ __forceinline__ bool await_flag(const lds_flag* flag, uint32_t want, lds_flag* broken) {
+enum Waited : uint32_t { kReached = 0, kOver = 1, kBroken = 2 };
+/* Until *flag is at least `want` (as a signed distance), or, with `over`
+ * given, until it says that the claims are over. */
+__device__ __forceinline__ Waited await_flag(const lds_flag* flag, uint32_t want,
+                                             const lds_flag* over, lds_flag* broken) {
     for (uint32_t i = 0;; i++) {
-        if (uniform32(*flag) == want) {
+        /* the end first: `flag` may be the claim itself */
+        if (over != nullptr && uniform32(*over) == kClaimsOver) {
+            return kOver;
+        }
+        if ((int32_t)(uniform32(*flag) - want) >= 0) {
             break;
         }
         if (uniform32(*broken) != 0) {
-            return false;
+            return kBroken;
         }
         if (i == (1u << 27)) {
             *broken = 1;
-            return false;
+            return kBroken;
         }
         __builtin_amdgcn_s_sleep(1);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    return true;
+    return kReached;
 }
 __device__ __forceinline__ void raise_flag(lds_flag* flag, uint32_t value) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     *flag = value;
 }
 
-static_assert(kLaneLit < 65536 && kBatchMaxPipe < 65536 && kStageBuf < 65536,
-              "window records hold 16-bit fields");
+/* A copier's group among the groups at once (execute_group's Order). */
+struct InTurn {
+    static constexpr bool kInTurn = true;
+    PipeLds& l;
+    uint32_t k;
+    /* everything below is final: done_dp is at most two groups behind */
+    __device__ uint64_t final_below(uint64_t d0) const {
+        const uint32_t reached = uniform32(*(const lds_flag*)&l.done_dp);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        return d0 - (uint32_t)((uint32_t)d0 - reached);
+    }
+    __device__ bool wait_turn() const {
+        return await_flag((const lds_flag*)&l.done, k, nullptr, (lds_flag*)&l.broken) == kReached;
+    }
+    __device__ void finish(uint64_t dp) const {
+        raise_flag((lds_flag*)&l.done_dp, (uint32_t)dp);
+        *(lds_flag*)&l.done = k + 1;
+    }
+};
 
-/* ------------------------------------------------------------- LZ4 */
+/* The position after the member at window position p, or kWalkStop | p
+ * where it cannot be told from the window: an LZ4 length of more than
+ * kWalkExtra + 1 extension bytes or one that runs past the stage (`limit`
+ * bytes from the window start), a Snappy literal past the window's
+ * longest. Positions past the source end (lim) are not walked from. */
+constexpr uint32_t kWalkStop = 0x80000000u;
+__device__ __forceinline__ uint32_t walk_long_lz4(const uint8_t* cw, uint32_t p, uint32_t limit) {
+    const uint32_t tok = cw[p];
+    uint32_t q = p + 1;
+    uint32_t lit = tok >> 4;
+    bool stop = false;
+    if (lit == 15) {
+        uint32_t e = 255;
+        for (uint32_t i = 0; i <= kWalkExtra && e == 255 && q < limit; i++) {
+            e = cw[q++];
+            lit += e;
+        }
+        stop = e == 255;
+    }
+    q += lit + 2;
+    if ((tok & 15) == 15) {
+        uint32_t e = 255;
+        for (uint32_t i = 0; i <= kWalkExtra && e == 255 && q < limit; i++) {
+            e = cw[q++];
+        }
+        stop = stop || e == 255;
+    }
+    return stop ? kWalkStop | p : q;
+}
+__device__ __forceinline__ uint32_t walk_step_lz4(const uint8_t* cw, uint32_t p, uint32_t limit) {
+    /* lengths of at most one extension byte without a branch, in two LDS
+     * round trips; bytes that are none are read but never used */
+    const uint32_t tok = cw[p];
+    const uint32_t e1 = cw[p + 1];
+    const bool x1 = tok >= 0xF0;
+    const uint32_t q = p + 3 + (x1 ? 16 + e1 : tok >> 4);
+    const uint32_t e2 = cw[q];
+    const bool x2 = (tok & 15) == 15;
+    uint32_t next = q + (x2 ? 1 : 0);
+    if ((x1 && e1 == 255) || (x2 && e2 == 255)) {
+        next = walk_long_lz4(cw, p, limit);
+    }
+    return next;
+}
+template <int kFormat>
+__device__ __forceinline__ uint32_t walk_step(const uint8_t* cw, uint32_t p, uint32_t limit,
+                                              uint32_t lim) {
+    if (kFormat == kFormatSnappy) {
+        const Cand c = parse_candidate_snappy(cw, p, lim);
+        return c.complex ? kWalkStop | p : c.next;
+    }
+    return walk_step_lz4(cw, p, limit);
+}
+
+/* Walks the window's chain (see above) from its first byte and lists its
+ * members; returns where it goes on: a window position, or kWalkStop | the
+ * last listed member, whose end the window cannot tell. */
+template <int kFormat>
+__device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segment,
+                                                uint32_t limit, uint32_t lim, uint16_t* list,
+                                                uint32_t& count, uint32_t lane) {
+    const uint32_t start = lane * segment;
+    const uint32_t end = start + segment < lim ? start + segment : lim;
+    uint32_t entry = start;
+    uint32_t exit, mine;
+    bool moves = true;
+    for (;;) {
+        if (moves) {
+            mine = 0;
+            exit = entry;
+            while (exit < end) {
+                exit = walk_step<kFormat>(cw, exit, limit, lim);
+                mine++;
+            }
+        }
+        const uint32_t before =
+            (uint32_t)__builtin_amdgcn_update_dpp(0, (int)exit, 0x138, 0xF, 0xF, false);
+        uint32_t from = lane == 0 ? 0 : before;
+        const uint64_t moved = __ballot(from != entry);
+        if (moved == 0) {
+            break;
+        }
+        /* up to the first lane that moves, entries and exits are final, and
+         * so is where the chain goes from there */
+        const uint32_t first = (uint32_t)__builtin_ctzll(moved);
+        const uint32_t reached = uniform32(__builtin_amdgcn_readlane(from, first));
+        if (reached >= lim) {
+            /* the chain stops, or leaves the source, before that lane */
+            if (lane >= first) {
+                entry = reached;
+                exit = reached;
+                mine = 0;
+            }
+            break;
+        }
+        const bool sure = lane >= first && reached >= start;
+        from = sure ? reached : from;
+        moves = from != entry && (sure || from < end);
+        entry = moves ? from : entry;
+    }
+    const uint32_t incl = wave_inclusive_sum(mine, lane);
+    const uint32_t total = uniform32(__builtin_amdgcn_readlane(incl, kWave - 1));
+    uint32_t i = incl - mine;
+    uint32_t p = entry;
+    uint32_t next = 0; /* the member after a full list, on its lane */
+    while (p < end) {
+        if (i < kListMax) {
+            list[i] = (uint16_t)p;
+        } else if (i == kListMax) {
+            next = p;
+        }
+        i++;
+        p = walk_step<kFormat>(cw, p, limit, lim);
+    }
+    if (total > kListMax) {
+        count = kListMax;
+        const uint64_t holder = __ballot(incl - mine <= kListMax && kListMax < incl);
+        return uniform32(__builtin_amdgcn_readlane(next, __builtin_ctzll(holder)));
+    }
+    count = total;
+    return uniform32(__builtin_amdgcn_readlane(exit, kWave - 1));
+}
+
+/* The parser's side of a chunk: window after window into the two window
+ * slots, a slot again once the groups of its window have finished. */
+template <int kFormat>
+__device__ __forceinline__ void run_parser(PipeLds& l, gcu8* src, uint64_t src_size, uint64_t cap,
+                                           uint32_t lane) {
+    uint64_t base = 0;
+    if (kFormat == kFormatSnappy) {
+        uint64_t declared = 0;
+        const int begun = chunk_begin<kFormat>(src, src_size, cap, base, declared);
+        l.declared = declared;
+        l.begun = begun;
+        if (begun != kOk) {
+            raise_flag((lds_flag*)&l.published, 1);
+            return;
+        }
+    }
+    uint32_t segment = kSegmentFirst;
+    for (uint32_t w = 0;; w++) {
+        const uint32_t b = w & 1;
+        const lds_flag* over = (const lds_flag*)&l.claim;
+        lds_flag* broken = (lds_flag*)&l.broken;
+        if (w >= 2) {
+            if (await_flag((const lds_flag*)&l.retired, w - 1, over, broken) != kReached) {
+                return;
+            }
+            const uint32_t groups = uniform32(*(const lds_flag*)&l.retired_k[b]);
+            if (await_flag((const lds_flag*)&l.done, groups, over, broken) != kReached) {
+                return;
+            }
+        }
+        uint8_t* stage = l.pipe.stage[b];
+        uint16_t* list = l.pipe.list[b];
+        const uint32_t lim = window_limit(src_size, base);
+        /* what is left of a short source is spread over the lanes */
+        const uint32_t spread = lim / kWave + 1;
+        segment = spread < segment ? spread : segment;
+        const uint32_t limit = stage_bytes(segment * kWave);
+        const uint32_t delta =
+            segment > kSegmentFirst
+                ? stage_into<kStageRounds>(stage, src, src_size, base, limit, lane)
+                : stage_into<kStageRoundsFirst>(stage, src, src_size, base, limit, lane);
+        const uint32_t touch = touch_ahead(src, src_size, base, limit, kSegment, lane);
+        const uint8_t* cw = stage + delta;
+        uint32_t count = 0;
+        const uint32_t next = walk_window<kFormat>(cw, segment, limit, lim, list, count, lane);
+        bool last = false;
+        uint64_t next_base = base + next;
+        segment = kSegment;
+        if ((next & kWalkStop) != 0) {
+            /* only where the member ends matters here (the copiers decide
+             * what it is worth): the exact ladder, with room for any output */
+            const uint64_t at = base + (next & ~kWalkStop);
+            const uint64_t room = 1ull << 62;
+            bool ends = false;
+            int st;
+            Lz4Step q;
+            if (kFormat == kFormatSnappy) {
+                SnappyCursor cur{src, src_size, room, at, room / 2, room};
+                st = snappy_step(cur, q, ends);
+                next_base = uniform64(cur.sp);
+            } else {
+                Lz4Cursor cur{src, src_size, room, at, room / 2};
+                const StagedBytes staged{src, cw, base, limit};
+                st = (int)uniform32((uint32_t)lz4_next<true>(cur, q, ends, staged));
+                next_base = uniform64(cur.sp);
+            }
+            last = st != kOk || uniform32(ends) != 0;
+            segment = kSegmentFirst;
+        } else if (next >= lim) {
+            last = true;
+        }
+        if (last) {
+            /* whatever comes after the last member lies at the source end */
+            list[count] = (uint16_t)kListEnd;
+            count++;
+        }
+        l.window[b].base = base;
+        l.window[b].count = count;
+        l.window[b].delta = delta;
+        l.window[b].staged = limit;
+        raise_flag((lds_flag*)&l.published, w + 1);
+        asm volatile("" ::"v"(touch));
+        if (last) {
+            return;
+        }
+        base = next_base;
+    }
+}
+
+/* A copier's side of a chunk: claims every kCopiers-th group, from group
+ * `c` on, and executes it. The copier whose claim decides the chunk's end
+ * returns true, with the status and the bytes produced. kParseOnly: claims
+ * only. */
+template <int kFormat, bool kParseOnly>
+__device__ __forceinline__ bool run_copier(PipeLds& l, uint32_t c, gcu8* src, uint64_t src_size,
+                                           gu8* dst, uint64_t cap, int& status, uint64_t& produced,
+                                           uint32_t lane) {
+    lds_flag* broken = (lds_flag*)&l.broken;
+    lds_flag* claim = (lds_flag*)&l.claim;
+    for (uint32_t k = c;; k += kCopiers) {
+        produced = 0;
+        const Waited got = await_flag(claim, k, claim, broken);
+        if (got == kOver) {
+            return false;
+        }
+        if (got == kBroken) {
+            status = CUDEC_ERR_CUDA;
+            return true;
+        }
+        const InTurn turn{l, k};
+        uint64_t dp = uniform64(l.next.dp);
+        uint64_t flushed = uniform64(l.next.flushed);
+        uint64_t ring_lo = uniform64(l.next.ring_lo);
+        uint32_t win = uniform32(l.next.win);
+        uint32_t idx = uniform32(l.next.idx);
+        if (win == kNoWindow || idx == uniform32(l.window[win & 1].count)) {
+            if (win != kNoWindow) {
+                l.retired_k[win & 1] = k;
+                raise_flag((lds_flag*)&l.retired, win + 1);
+            }
+            win++;
+            idx = 0;
+            if (await_flag((const lds_flag*)&l.published, win + 1, nullptr, broken) != kReached) {
+                status = CUDEC_ERR_CUDA;
+                return true;
+            }
+            if (kFormat == kFormatSnappy && win == 0 &&
+                uniform32((uint32_t)l.begun) != (uint32_t)kOk) {
+                status = (int)uniform32((uint32_t)l.begun);
+                raise_flag(claim, kClaimsOver);
+                return true;
+            }
+        }
+        const uint32_t b = win & 1;
+        const uint64_t base = uniform64(l.window[b].base);
+        const uint32_t listed = uniform32(l.window[b].count);
+        const uint8_t* cw = l.pipe.stage[b] + uniform32(l.window[b].delta);
+        const uint32_t lim = window_limit(src_size, base);
+        const uint32_t left = listed - idx;
+        const uint32_t count = left < kWave ? left : kWave;
+        uint32_t member = lane < count ? (uint32_t)l.pipe.list[b][idx + lane] : 0;
+        member = member == kListEnd ? lim : member;
+        const uint64_t declared = kFormat == kFormatSnappy ? uniform64(l.declared) : 0;
+        const Resolved r =
+            kFormat == kFormatSnappy
+                ? resolve_snappy(cw, member, count, base, src_size, declared, dp, lim, kPipeBatch,
+                                 lane)
+                : resolve_lz4<true>(cw, member, count, base, src_size, cap, dp, kPipeBatch, lane);
+        if (r.status != kOk) {
+            status = r.status;
+            raise_flag(claim, kClaimsOver);
+            return true;
+        }
+        if (!r.slow) {
+            if (r.done) {
+                raise_flag(claim, kClaimsOver);
+            } else {
+                l.next.dp = dp + r.g.end_rel;
+                l.next.flushed = flushed;
+                l.next.ring_lo = ring_lo;
+                l.next.win = win;
+                l.next.idx = idx + r.g.take;
+                raise_flag(claim, k + 1);
+            }
+            bool ran;
+            if (kParseOnly) {
+                dp += r.g.end_rel;
+                ran = turn.wait_turn();
+            } else {
+                /* what precedes the group is flushed by then, up to the last
+                 * whole 16 bytes */
+                const uint64_t whole = (((uintptr_t)dst + dp) & ~(uintptr_t)15) - (uintptr_t)dst;
+                if ((int64_t)whole > (int64_t)flushed) {
+                    flushed = whole;
+                }
+                ran = execute_group(l.pipe.w, l.pipe.cover[c], cw, r.g, dst, cap, dp, flushed, ring_lo, r.done,
+                                    lane, turn);
+            }
+            if (!ran) {
+                status = CUDEC_ERR_CUDA;
+                return true;
+            }
+            turn.finish(dp);
+            if (r.done) {
+                status = kOk;
+                produced = dp;
+                return true;
+            }
+            continue;
+        }
+        /* a member the window cannot hold: the exact scalar ladder, then the
+         * slow copies, alone in the block (they use the ring as they like) */
+        Lz4Step q;
+        bool last = false;
+        int st;
+        const uint64_t at = base + uniform32(__builtin_amdgcn_readlane(member, 0));
+        uint64_t dp_after;
+        if (kFormat == kFormatSnappy) {
+            SnappyCursor cur{src, src_size, cap, at, dp, declared};
+            st = snappy_step(cur, q, last);
+            dp_after = uniform64(cur.dp);
+        } else {
+            Lz4Cursor cur{src, src_size, cap, at, dp};
+            const StagedBytes staged{src, cw, base, uniform32(l.window[b].staged)};
+            st = (int)uniform32((uint32_t)lz4_next<true>(cur, q, last, staged));
+            dp_after = uniform64(cur.dp);
+        }
+        if (st != kOk) {
+            status = st;
+            raise_flag(claim, kClaimsOver);
+            return true;
+        }
+        last = uniform32(last) != 0;
+        if (!turn.wait_turn()) {
+            status = CUDEC_ERR_CUDA;
+            return true;
+        }
+        if (kParseOnly) {
+            dp = dp_after;
+        } else {
+            const uint64_t whole = (((uintptr_t)dst + dp) & ~(uintptr_t)15) - (uintptr_t)dst;
+            if ((int64_t)whole > (int64_t)flushed) {
+                flushed = whole;
+            }
+            execute_slow(l.pipe.w, src, dst, cap, q, dp_after, dp, flushed, ring_lo, last, lane);
+        }
+        turn.finish(dp);
+        if (last) {
+            raise_flag(claim, kClaimsOver);
+            status = kOk;
+            produced = dp;
+            return true;
+        }
+        l.next.dp = dp;
+        l.next.flushed = flushed;
+        l.next.ring_lo = ring_lo;
+        l.next.win = win;
+        l.next.idx = idx + 1;
+        raise_flag(claim, k + 1);
+    }
+}
+
+/* ------------------------------------------------------------- one wave */
 
 struct ChunkOut {
     int status;
@@ -1968,8 +2328,7 @@ __device__ __forceinline__ ChunkOut decode_chunk(WaveLds& w, gcu8* src,
         }
         uint32_t touch = 0;
         const Parsed pr =
-            parse_any<kFormat, kCandSplit, true>(w.stage, w.jump, src, src_size, cap, declared,
-                                                 sp, pdp, lane, touch);
+            parse_any<kFormat>(w.stage, w.jump, src, src_size, cap, declared, sp, pdp, lane, touch);
         if (pr.kind == kParseFail) {
             status = pr.status;
             break;
@@ -1981,8 +2340,8 @@ __device__ __forceinline__ ChunkOut decode_chunk(WaveLds& w, gcu8* src,
                 execute_slow(w, src, dst, cap, pr.q, pr.lead_dp, dp, flushed, ring_lo, false,
                              lane);
             }
-            execute_group(w, w.stage + pr.delta, pr.g, dst, cap, dp, flushed, ring_lo, pr.done,
-                          lane);
+            execute_group(w, w.cover, w.stage + pr.delta, pr.g, dst, cap, dp, flushed, ring_lo, pr.done,
+                          lane, Alone{});
         } else {
             execute_slow(w, src, dst, cap, pr.q, pdp, dp, flushed, ring_lo, pr.done, lane);
         }
@@ -1996,107 +2355,6 @@ __device__ __forceinline__ ChunkOut decode_chunk(WaveLds& w, gcu8* src,
     r.status = status;
     r.produced = dp;
     return r;
-}
-
-/* The parser's side of one window of the two-wave form: parse (or hand
- * over the chunk's failure) into record r and stage buffer `stage`;
- * returns whether this record ends the chunk. */
-template <int kFormat>
-__device__ __forceinline__ bool parse_into(PipeRec& r, uint8_t* stage, int begun, uint64_t& fuel,
-                                           gcu8* src, uint64_t src_size, uint64_t cap,
-                                           uint64_t declared, uint64_t& sp, uint64_t& dp,
-                                           uint32_t lane, uint32_t& touch) {
-    Parsed pr;
-    if (begun != kOk || fuel-- == 0) {
-        pr.kind = kParseFail;
-        pr.status = begun != kOk ? begun : kCorrupt;
-        pr.done = false;
-        pr.delta = 0;
-    } else {
-        constexpr uint32_t kC = kFormat == kFormatSnappy ? kCandPipeSnappy : kCandPipe;
-        pr = parse_any<kFormat, kC, false>(stage, nullptr, src, src_size, cap, declared, sp, dp,
-                                           lane, touch);
-    }
-    r.kind = pr.kind;
-    r.status = pr.status;
-    r.done = pr.done ? 1u : 0u;
-    r.lead = pr.lead ? 1u : 0u;
-    if (pr.kind == kParseSlow || pr.lead) {
-        r.lit_src = pr.q.lit_src;
-        r.lit_dst = pr.q.lit_dst;
-        r.lit_len_s = pr.q.lit_len;
-        r.match_dst = pr.q.match_dst;
-        r.offset_s = pr.q.offset;
-        r.match_len_s = pr.q.match_len;
-        r.dp_after = pr.lead ? pr.lead_dp : dp;
-    }
-    if (pr.kind == kParseGroup) {
-        r.lit[lane] = (uint16_t)pr.g.lit;
-        r.lit_len[lane] = (uint16_t)pr.g.lit_len;
-        r.match_len[lane] = (uint16_t)pr.g.match_len;
-        r.offset[lane] = pr.g.offset;
-        r.drel[lane] = (uint16_t)pr.g.drel;
-        r.delta = pr.delta;
-        r.take = pr.g.take;
-        r.terminal = pr.g.terminal ? 1u : 0u;
-        r.end_rel = pr.g.end_rel;
-    }
-    return pr.kind == kParseFail || pr.done;
-}
-
-/* The copier's side: run record r, whose window is staged in `stage`
- * (kParseOnly: only the output size advances); a failed record sets
- * status. Returns whether this record ends the chunk. */
-template <bool kParseOnly>
-__device__ __forceinline__ bool run_record(PipeRing& w, const PipeRec& r, const uint8_t* stage,
-                                           gcu8* src, gu8* dst, uint64_t cap, uint64_t& dp,
-                                           uint64_t& flushed, uint64_t& ring_lo, int& status,
-                                           uint32_t lane) {
-    /* every field read at once, before the kind decides which are used
-     * (one LDS round trip; a slow or failed record's group fields are
-     * stale and unused) */
-    Group g;
-    g.lit = r.lit[lane];
-    g.lit_len = r.lit_len[lane];
-    g.match_len = r.match_len[lane];
-    g.offset = r.offset[lane];
-    g.drel = r.drel[lane];
-    g.take = uniform32(r.take);
-    g.terminal = uniform32(r.terminal) != 0;
-    g.end_rel = uniform32(r.end_rel);
-    const uint32_t delta = uniform32(r.delta);
-    const uint32_t kind = uniform32(r.kind);
-    const bool done = uniform32(r.done) != 0;
-    const bool lead = uniform32(r.lead) != 0;
-    if (kind == kParseFail) {
-        status = (int)uniform32((uint32_t)r.status);
-        return true;
-    }
-    if (kParseOnly) {
-        /* the parse ceiling: the records' sizes, no bytes */
-        if (kind == kParseSlow || lead) {
-            dp = uniform64(r.dp_after);
-        }
-        if (kind == kParseGroup) {
-            dp += g.end_rel;
-        }
-        return done;
-    }
-    if (kind == kParseSlow || lead) {
-        Lz4Step s;
-        s.lit_src = uniform64(r.lit_src);
-        s.lit_dst = uniform64(r.lit_dst);
-        s.lit_len = uniform64(r.lit_len_s);
-        s.match_dst = uniform64(r.match_dst);
-        s.offset = (uint32_t)uniform64(r.offset_s);
-        s.match_len = uniform64(r.match_len_s);
-        execute_slow(w, src, dst, cap, s, uniform64(r.dp_after), dp, flushed, ring_lo,
-                     kind == kParseSlow && done, lane);
-    }
-    if (kind == kParseGroup) {
-        execute_group(w, stage + delta, g, dst, cap, dp, flushed, ring_lo, done, lane);
-    }
-    return done;
 }
 
 /* ------------------------------------------------------------ kernels */
@@ -2231,160 +2489,14 @@ __device__ __forceinline__ uint32_t queue_pop(Queue* q, size_t n, QueueCursor& c
     return (uint32_t)n;
 }
 
-constexpr int kPipeBlock = 2 * kWave;
-constexpr uint32_t kNoFin = 0xFFFFFFFFu;
-
-/* Two waves per chunk. Wave 0 parses windows into the block's window
- * slots (a record and a stage buffer each) while wave 1 executes the
- * records in the same order. Parsing reads only the source and decides
- * every status; execution only writes the ring and the destination, so the
- * chunk's critical path is the longer of the two per window rather than
- * their sum. Slotted blocks (four slots) hand windows over through LDS
- * flags, so the parser may run three windows ahead; lockstep blocks (two
- * slots) take one barrier per window. Control flow around the barriers is
- * uniform for the block: both waves read the chunk index (and, lockstep,
- * the final step) from LDS after a barrier, and a barrier opens every
- * chunk so that no control word is rewritten while the other wave may
- * still read it. */
-/* kWaves: waves per SIMD the register budget is cut for. 4 (128 VGPRs) for
- * launches that pipeline chunks; 5 (96 VGPRs, some spills on the two-wave
- * path) for launches where every chunk runs on one wave, which are
- * throughput-bound and gain from a fifth wave. kSubs: decode sub-queues,
- * kSubQueues for launches of many chunks per wave, else 1 (the single
- * counter, whose code keeps the fewest scalar registers live). */
-template <int kFormat, int kWaves, uint32_t kSubs, bool kParseOnly>
-__global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu(kWaves)))
-    piped_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
-                const size_t* caps, size_t n, cudec_chunk_result* results, Queue* q,
-                const uint32_t* order, Plan plan) {
-    /* Slotted (four waves per SIMD): four window slots signalled through
-     * LDS flags, so the parser runs up to three windows ahead and neither
-     * wave waits on the other's slowest windows (a window's parse and copy
-     * times vary independently). Lockstep (five waves per SIMD, where ten
-     * blocks must fit a CU's LDS): two slots and a barrier per window. */
-    constexpr bool kSlotted = kWaves == 4;
-    constexpr uint32_t kS = kSlotted ? 4 : 2;
-    __shared__ PipeLds<kS> L;
-    const uint32_t lane = __lane_id();
-    const bool parser = uniform32(threadIdx.x / kWave) == 0;
-    uint32_t split_idx = 0xFFFFFFFFu; /* first chunk decoded one wave per chunk */
-    QueueCursor cursor{blockIdx.x % kSubs, kSubs};
-    if (kSlotted && parser && lane < kS) {
-        L.pub[lane] = 0;
-        L.freed[lane] = 0;
-        L.broken = 0;
-    }
-    uint32_t seq = 0; /* slotted: windows of this block so far, counted alike by both waves */
-    for (;;) {
-        /* both waves are done reading the previous chunk's control words
-         * (chunk_idx, fin) before the parser writes the next chunk's */
-        __syncthreads();
-        if (parser) {
-            L.chunk_idx = queue_pop<kSubs>(q, n, cursor, lane);
-            L.fin = kNoFin;
-        }
-        __syncthreads();
-        const uint32_t idx = uniform32(L.chunk_idx);
-        if (idx >= n) {
-            break;
-        }
-        const uint64_t chunk = order[idx];
-        gcu8* src = global_bytes(srcs[chunk]);
-        gu8* dst = global_bytes(dsts[chunk]);
-        const uint64_t src_size = uniform64(src_sizes[chunk]);
-        const uint64_t cap = uniform64(caps[chunk]);
-        if (!plan_two_wave(plan, cost_bin(src_size, cap))) {
-            /* the queue holds every two-wave chunk before the one-wave
-             * ones, so the block splits for good */
-            split_idx = idx;
-            break;
-        }
-        uint64_t sp = 0, declared = 0, dp = 0, flushed = 0, ring_lo = 0;
-        uint64_t fuel = src_size == UINT64_MAX ? UINT64_MAX : src_size + 2;
-        int status = kOk;
-        /* the parser's preamble verdict (Snappy), handed over as a failed
-         * window record when it is not OK */
-        const int begun = parser ? chunk_begin<kFormat>(src, src_size, cap, sp, declared) : kOk;
-        if constexpr (kSlotted) {
-            lds_flag* broken = (lds_flag*)&L.broken;
-            if (parser) {
-                /* each window: wait until its slot's previous record has
-                 * run, parse into the slot, publish */
-                for (;;) {
-                    const uint32_t sl = seq % kS;
-                    if (seq >= kS &&
-                        !await_flag((const lds_flag*)&L.freed[sl], seq - kS + 1, broken)) {
-                        break;
-                    }
-                    uint32_t touch = 0;
-                    const bool last =
-                        parse_into<kFormat>(L.pipe.rec[sl], L.stage_of(sl), begun, fuel, src,
-                                            src_size, cap, declared, sp, dp, lane, touch);
-                    raise_flag((lds_flag*)&L.pub[sl], seq + 1);
-                    seq++;
-                    /* the look-ahead loads land by now */
-                    asm volatile("" ::"v"(touch));
-                    if (last) {
-                        break;
-                    }
-                }
-            } else {
-                /* each window: wait for its record, run it, free the slot */
-                for (;;) {
-                    const uint32_t sl = seq % kS;
-                    if (!await_flag((const lds_flag*)&L.pub[sl], seq + 1, broken)) {
-                        status = CUDEC_ERR_CUDA;
-                        break;
-                    }
-                    const bool last =
-                        run_record<kParseOnly>(L.pipe.w, L.pipe.rec[sl], L.stage_of(sl), src, dst,
-                                               cap, dp, flushed, ring_lo, status, lane);
-                    raise_flag((lds_flag*)&L.freed[sl], seq + 1);
-                    seq++;
-                    if (last) {
-                        break;
-                    }
-                }
-            }
-        } else {
-            bool pdone = false;
-            /* step k: the parser fills slot k mod 2 while the copier runs
-             * step k - 1's record; one barrier a step */
-            for (uint32_t step = 0;; step++) {
-                const uint32_t b = step & 1;
-                if (parser) {
-                    if (!pdone) {
-                        uint32_t touch = 0;
-                        pdone = parse_into<kFormat>(L.pipe.rec[b], L.stage_of(b), begun, fuel, src,
-                                                    src_size, cap, declared, sp, dp, lane, touch);
-                        if (pdone) {
-                            L.fin = step;
-                        }
-                        /* the look-ahead loads land by now */
-                        asm volatile("" ::"v"(touch));
-                    }
-                } else if (step > 0 && status == kOk) {
-                    run_record<kParseOnly>(L.pipe.w, L.pipe.rec[b ^ 1], L.stage_of(b ^ 1), src,
-                                           dst, cap, dp, flushed, ring_lo, status, lane);
-                }
-                __syncthreads();
-                const uint32_t fin = uniform32(L.fin);
-                if (fin != kNoFin && step == fin + 1) {
-                    break;
-                }
-            }
-        }
-        if (!parser) {
-            write_result(results, chunk, status, dp);
-        }
-    }
-    if (split_idx == 0xFFFFFFFFu) {
-        return;
-    }
-    /* one wave per chunk from here: the parser decodes the chunk in hand,
-     * the other wave takes its own from the queue; no barrier follows */
-    WaveLds& w = parser ? L.split.a : L.split.b;
-    uint32_t idx = parser ? split_idx : queue_pop<kSubs>(q, n, cursor, lane);
+/* One chunk a wave, from queue position idx on, until the queue is dry. */
+template <int kFormat, uint32_t kSubs, bool kParseOnly>
+__device__ __forceinline__ void decode_alone(WaveLds& w, uint32_t idx, const void* const* srcs,
+                                             const size_t* src_sizes, void* const* dsts,
+                                             const size_t* caps, size_t n,
+                                             cudec_chunk_result* results, Queue* q,
+                                             const uint32_t* order, QueueCursor& cursor,
+                                             uint32_t lane) {
     while (idx < n) {
         const uint64_t chunk = order[idx];
         gcu8* src = global_bytes(srcs[chunk]);
@@ -2397,13 +2509,103 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
     }
 }
 
+/* The persistent decoder. A block takes the queue's pipelined chunks first,
+ * all four waves on one chunk (above); a barrier opens every chunk, so that
+ * no control word is reset while another wave may still read it. The queue
+ * holds every pipelined chunk before the others, so once a block meets one
+ * of the others it splits for good into four one-wave decoders.
+ *
+ * Four blocks fill a CU's LDS, sixteen waves at 128 VGPRs each. kSubs:
+ * decode sub-queues, kSubQueues for launches of many chunks per wave, else
+ * 1 (the single counter, whose code keeps the fewest scalar registers
+ * live). */
+template <int kFormat, uint32_t kSubs, bool kParseOnly>
+__global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu(4)))
+    piped_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
+                const size_t* caps, size_t n, cudec_chunk_result* results, Queue* q,
+                const uint32_t* order, Plan plan) {
+    __shared__ PipeLds l;
+    const uint32_t lane = __lane_id();
+    const uint32_t wave = uniform32(threadIdx.x / kWave);
+    QueueCursor cursor{blockIdx.x % kSubs, kSubs};
+    uint32_t idx;
+    if (wave == 0 && lane == 0) {
+        l.broken = 0;
+    }
+    for (;;) {
+        /* every wave is done with the previous chunk's control words */
+        __syncthreads();
+        if (wave == 0) {
+            l.chunk_idx = queue_pop<kSubs>(q, n, cursor, lane);
+            l.next.dp = 0;
+            l.next.flushed = 0;
+            l.next.ring_lo = 0;
+            l.next.win = kNoWindow;
+            l.next.idx = 0;
+            l.published = 0;
+            l.retired = 0;
+            l.claim = 0;
+            l.done = 0;
+            l.done_dp = 0;
+        }
+        __syncthreads();
+        idx = uniform32(l.chunk_idx);
+        if (idx >= n) {
+            return;
+        }
+        const uint64_t chunk = order[idx];
+        gcu8* src = global_bytes(srcs[chunk]);
+        gu8* dst = global_bytes(dsts[chunk]);
+        const uint64_t src_size = uniform64(src_sizes[chunk]);
+        const uint64_t cap = uniform64(caps[chunk]);
+        if (!plan_two_wave(plan, cost_bin(src_size, cap))) {
+            break;
+        }
+        if (wave == 0) {
+            run_parser<kFormat>(l, src, src_size, cap, lane);
+        } else {
+            int status = kOk;
+            uint64_t produced = 0;
+            if (run_copier<kFormat, kParseOnly>(l, wave - 1, src, src_size, dst, cap, status,
+                                                produced, lane)) {
+                write_result(results, chunk, (int)uniform32((uint32_t)status),
+                             uniform64(produced));
+            }
+        }
+    }
+    /* no barrier follows; the first wave decodes the chunk in hand */
+    if (wave != 0) {
+        idx = queue_pop<kSubs>(q, n, cursor, lane);
+    }
+    decode_alone<kFormat, kSubs, kParseOnly>(l.split[wave], idx, srcs, src_sizes, dsts, caps, n,
+                                             results, q, order, cursor, lane);
+}
+
+/* The persistent decoder of launches where every chunk runs on one wave:
+ * those are bound by throughput and gain from a fifth wave per SIMD (96
+ * VGPRs). */
+constexpr int kAloneBlock = 2 * kWave;
+template <int kFormat, uint32_t kSubs, bool kParseOnly>
+__global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_eu(5)))
+    alone_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
+                const size_t* caps, size_t n, cudec_chunk_result* results, Queue* q,
+                const uint32_t* order) {
+    __shared__ WaveLds w[kAloneBlock / kWave];
+    const uint32_t lane = __lane_id();
+    QueueCursor cursor{blockIdx.x % kSubs, kSubs};
+    const uint32_t idx = queue_pop<kSubs>(q, n, cursor, lane);
+    decode_alone<kFormat, kSubs, kParseOnly>(w[uniform32(threadIdx.x / kWave)], idx, srcs,
+                                             src_sizes, dsts, caps, n, results, q, order, cursor,
+                                             lane);
+}
+
 /* Launch geometry and a scratch pool, per device, set up on first use. The
  * pool keeps freed scratch (release threshold at its maximum) so that a
  * stream of launches does not return memory to the driver between them. */
 struct DeviceState {
     int cus = 0;
-    int pipe_blocks_per_cu = 0;  /* piped_batch<_, 4> (two-wave blocks) */
-    int split_blocks_per_cu = 0; /* piped_batch<_, 5>: no two-wave chunk, or Snappy */
+    int pipe_blocks_per_cu[2] = {0, 0};  /* piped_batch, per format */
+    int alone_blocks_per_cu[2] = {0, 0}; /* alone_batch */
     Plan plan[2];                /* per format (kFormatLz4, kFormatSnappy) */
     uint64_t min_cost[2];        /* the threshold each plan was last set from */
     hipMemPool_t pool = nullptr; /* made on the first allocating launch */
@@ -2456,19 +2658,24 @@ hipError_t device_state(DeviceState** out) {
         if (e != hipSuccess) {
             return e;
         }
-        int per = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, piped_batch<kFormatLz4, 4, 1, false>,
-                                                         kPipeBlock, 0);
-        if (e != hipSuccess) {
-            return e;
+        const void* kernels[2][2] = {
+            {reinterpret_cast<const void*>(&piped_batch<kFormatLz4, 1, false>),
+             reinterpret_cast<const void*>(&alone_batch<kFormatLz4, 1, false>)},
+            {reinterpret_cast<const void*>(&piped_batch<kFormatSnappy, 1, false>),
+             reinterpret_cast<const void*>(&alone_batch<kFormatSnappy, 1, false>)}};
+        for (int f = 0; f < 2; f++) {
+            int per = 0;
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernels[f][0], kPipeBlock, 0);
+            if (e != hipSuccess) {
+                return e;
+            }
+            d.pipe_blocks_per_cu[f] = per > 0 ? per : 1;
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernels[f][1], kAloneBlock, 0);
+            if (e != hipSuccess) {
+                return e;
+            }
+            d.alone_blocks_per_cu[f] = per > 0 ? per : 1;
         }
-        d.pipe_blocks_per_cu = per > 0 ? per : 1;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, piped_batch<kFormatLz4, 5, 1, false>,
-                                                         kPipeBlock, 0);
-        if (e != hipSuccess) {
-            return e;
-        }
-        d.split_blocks_per_cu = per > 0 ? per : 1;
         for (int f = 0; f < 2; f++) {
             d.plan[f] = plan_from_threshold(kDefaultPipeMinCost);
             d.min_cost[f] = kDefaultPipeMinCost;
@@ -2606,40 +2813,39 @@ hipError_t queue_and_decode(DeviceState* dev, int format, const void* const* src
     for (int w = 0; w < kBins / 64; w++) {
         any_two_wave = any_two_wave || plan.two_wave[w] != 0;
     }
-    /* two-wave blocks; a block splits into two one-wave decoders when it
-     * meets a one-wave chunk. The five-wave build runs where no chunk is
-     * two-wave (every block splits at once) and for Snappy, whose two-wave
-     * path fits its 96 VGPRs. */
-    const bool five_waves = !any_two_wave || format == kFormatSnappy;
+    /* pipelined blocks, each of which splits into one-wave decoders when it
+     * meets a one-wave chunk; or, where the plan pipelines no chunk, the
+     * one-wave kernel */
+    const int f = format == kFormatSnappy ? 1 : 0;
+    const int waves = any_two_wave ? (int)kPipeWaves : kAloneBlock / (int)kWave;
     size_t grid = (size_t)dev->cus *
-                  (size_t)(five_waves ? dev->split_blocks_per_cu : dev->pipe_blocks_per_cu);
+                  (size_t)(any_two_wave ? dev->pipe_blocks_per_cu[f] : dev->alone_blocks_per_cu[f]);
     if (grid > n) {
         grid = n;
     }
-    const dim3 gd((unsigned)grid), bd(kPipeBlock);
-    const bool many = (uint64_t)n >= kSubQueueMinPerWave * 2 * (uint64_t)grid;
-    const int shape = (parse_only ? 8 : 0) | (format == kFormatSnappy ? 4 : 0) |
-                      (five_waves ? 2 : 0) | (many ? 1 : 0);
+    const dim3 gd((unsigned)grid), bd((unsigned)(waves * (int)kWave));
+    const bool many = (uint64_t)n >= kSubQueueMinPerWave * (uint64_t)waves * (uint64_t)grid;
+    const int shape = (parse_only ? 8 : 0) | (f ? 4 : 0) | (any_two_wave ? 0 : 2) | (many ? 1 : 0);
     switch (shape) {
-#define CUDEC_PIPED(kShape, kFmt, kW, kS, kP)                                             \
+#define CUDEC_PIPED(kShape, kFmt, kS, kP)                                                 \
     case kShape:                                                                          \
-        hipLaunchKernelGGL((piped_batch<kFmt, kW, kS, kP>), gd, bd, 0, stream, srcs,      \
+        hipLaunchKernelGGL((piped_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
                            src_sizes, dsts, caps, n, results, q, order, plan);            \
+        break;                                                                            \
+    case kShape + 2:                                                                      \
+        hipLaunchKernelGGL((alone_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
+                           src_sizes, dsts, caps, n, results, q, order);                  \
         break;
-        CUDEC_PIPED(0, kFormatLz4, 4, 1, false)
-        CUDEC_PIPED(1, kFormatLz4, 4, kSubQueues, false)
-        CUDEC_PIPED(2, kFormatLz4, 5, 1, false)
-        CUDEC_PIPED(3, kFormatLz4, 5, kSubQueues, false)
-        CUDEC_PIPED(6, kFormatSnappy, 5, 1, false)
-        CUDEC_PIPED(7, kFormatSnappy, 5, kSubQueues, false)
-        CUDEC_PIPED(8, kFormatLz4, 4, 1, true)
-        CUDEC_PIPED(9, kFormatLz4, 4, kSubQueues, true)
-        CUDEC_PIPED(10, kFormatLz4, 5, 1, true)
-        CUDEC_PIPED(11, kFormatLz4, 5, kSubQueues, true)
-        CUDEC_PIPED(14, kFormatSnappy, 5, 1, true)
-        CUDEC_PIPED(15, kFormatSnappy, 5, kSubQueues, true)
+        CUDEC_PIPED(0, kFormatLz4, 1, false)
+        CUDEC_PIPED(1, kFormatLz4, kSubQueues, false)
+        CUDEC_PIPED(4, kFormatSnappy, 1, false)
+        CUDEC_PIPED(5, kFormatSnappy, kSubQueues, false)
+        CUDEC_PIPED(8, kFormatLz4, 1, true)
+        CUDEC_PIPED(9, kFormatLz4, kSubQueues, true)
+        CUDEC_PIPED(12, kFormatSnappy, 1, true)
+        CUDEC_PIPED(13, kFormatSnappy, kSubQueues, true)
 #undef CUDEC_PIPED
-        default: /* Snappy always takes the five-wave build */
+        default:
             return hipErrorInvalidValue;
     }
     return hipGetLastError();
