@@ -70,9 +70,12 @@ constexpr uint32_t kLaneMatch = 64;       /* matches copied by their lane (<= 64
 constexpr uint32_t kOctaveBits = 2;       /* cost bins per octave: 4 */
 constexpr int kBins = 64 << kOctaveBits;
 static_assert(kBins == kCostBins, "the plan API names every bin");
-/* Default plan: chunks costing at least 512 KiB (capacity + capacity -
- * compressed) run on two waves. */
-constexpr uint64_t kDefaultPipeMinCost = 512u << 10;
+/* Default plans: chunks costing at least this (capacity + capacity -
+ * compressed) are pipelined. */
+constexpr uint64_t kDefaultPipeMinCost[2] = {128u << 10, 64u << 10};
+/* ... and in launches of few chunks (plan_launch): below this one wave is
+ * as fast (a 4 KiB token page alone: 36 us on one wave, 40 pipelined). */
+constexpr uint64_t kFewPipeMinCost = 8u << 10;
 /* Queue keys: a chunk's class (two-wave first), then its cost bin. */
 constexpr int kKeys = 2 * kBins;
 
@@ -2465,14 +2468,21 @@ __global__ void queue_fill(const size_t* sizes, const size_t* caps, size_t n, Qu
 }
 
 /* The next queue position for this wave from kSubs sub-queues (1: the
- * single counter), or at least n once every one is drained (n < 2^32).
+ * single counter; 0: no queue, the launch has a place for every chunk and
+ * gives each wave or block its own, `own`), or at least n once every one is
+ * drained (n < 2^32).
  * Every lane takes part in the atomic and only lane 0 adds: a
  * lane-0-only branch at a persistent loop's top and bottom lets the
  * compiler fold both into an exec-masked inner loop that only lane 0 can
  * leave. */
 template <uint32_t kSubs>
 __device__ __forceinline__ uint32_t queue_pop(Queue* q, size_t n, QueueCursor& c,
-                                              uint32_t lane) {
+                                              uint32_t lane, uint64_t own) {
+    if (kSubs == 0) {
+        const bool first = c.left == 0;
+        c.left = 1;
+        return first && own < n ? (uint32_t)own : (uint32_t)n;
+    }
     if (kSubs == 1) {
         return uniform32(atomicAdd(&q->next[0], lane == 0 ? 1u : 0u));
     }
@@ -2483,10 +2493,17 @@ __device__ __forceinline__ uint32_t queue_pop(Queue* q, size_t n, QueueCursor& c
         if (pos < n) {
             return (uint32_t)pos;
         }
-        c.sub = (c.sub + 1) % kSubs;
+        c.sub = (c.sub + 1) % (kSubs == 0 ? 1 : kSubs);
         c.left--;
     }
     return (uint32_t)n;
+}
+
+/* The chunk at a queue position: the cost order's, or, with no queue, the
+ * position itself. */
+template <uint32_t kSubs>
+__device__ __forceinline__ uint64_t chunk_at(const uint32_t* order, uint32_t idx) {
+    return kSubs == 0 ? idx : order[idx];
 }
 
 /* One chunk a wave, from queue position idx on, until the queue is dry. */
@@ -2498,16 +2515,17 @@ __device__ __forceinline__ void decode_alone(WaveLds& w, uint32_t idx, const voi
                                              const uint32_t* order, QueueCursor& cursor,
                                              uint32_t lane) {
     while (idx < n) {
-        const uint64_t chunk = order[idx];
+        const uint64_t chunk = chunk_at<kSubs>(order, idx);
         gcu8* src = global_bytes(srcs[chunk]);
         gu8* dst = global_bytes(dsts[chunk]);
         const uint64_t src_size = uniform64(src_sizes[chunk]);
         const uint64_t cap = uniform64(caps[chunk]);
         const ChunkOut o = decode_chunk<kFormat, kParseOnly>(w, src, src_size, dst, cap, lane);
         write_result(results, chunk, (int)uniform32((uint32_t)o.status), uniform64(o.produced));
-        idx = queue_pop<kSubs>(q, n, cursor, lane);
+        idx = queue_pop<kSubs>(q, n, cursor, lane, n);
     }
 }
+
 
 /* The persistent decoder. A block takes the queue's pipelined chunks first,
  * all four waves on one chunk (above); a barrier opens every chunk, so that
@@ -2516,9 +2534,9 @@ __device__ __forceinline__ void decode_alone(WaveLds& w, uint32_t idx, const voi
  * of the others it splits for good into four one-wave decoders.
  *
  * Four blocks fill a CU's LDS, sixteen waves at 128 VGPRs each. kSubs:
- * decode sub-queues, kSubQueues for launches of many chunks per wave, else
- * 1 (the single counter, whose code keeps the fewest scalar registers
- * live). */
+ * decode sub-queues, kSubQueues for launches of many chunks per wave, 0 for
+ * launches with a resident block for every chunk, else 1 (the single
+ * counter, whose code keeps the fewest scalar registers live). */
 template <int kFormat, uint32_t kSubs, bool kParseOnly>
 __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu(4)))
     piped_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
@@ -2527,7 +2545,7 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
     __shared__ PipeLds l;
     const uint32_t lane = __lane_id();
     const uint32_t wave = uniform32(threadIdx.x / kWave);
-    QueueCursor cursor{blockIdx.x % kSubs, kSubs};
+    QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
     uint32_t idx;
     if (wave == 0 && lane == 0) {
         l.broken = 0;
@@ -2536,7 +2554,7 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
         /* every wave is done with the previous chunk's control words */
         __syncthreads();
         if (wave == 0) {
-            l.chunk_idx = queue_pop<kSubs>(q, n, cursor, lane);
+            l.chunk_idx = queue_pop<kSubs>(q, n, cursor, lane, blockIdx.x);
             l.next.dp = 0;
             l.next.flushed = 0;
             l.next.ring_lo = 0;
@@ -2553,7 +2571,7 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
         if (idx >= n) {
             return;
         }
-        const uint64_t chunk = order[idx];
+        const uint64_t chunk = chunk_at<kSubs>(order, idx);
         gcu8* src = global_bytes(srcs[chunk]);
         gu8* dst = global_bytes(dsts[chunk]);
         const uint64_t src_size = uniform64(src_sizes[chunk]);
@@ -2575,7 +2593,7 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
     }
     /* no barrier follows; the first wave decodes the chunk in hand */
     if (wave != 0) {
-        idx = queue_pop<kSubs>(q, n, cursor, lane);
+        idx = queue_pop<kSubs>(q, n, cursor, lane, n);
     }
     decode_alone<kFormat, kSubs, kParseOnly>(l.split[wave], idx, srcs, src_sizes, dsts, caps, n,
                                              results, q, order, cursor, lane);
@@ -2592,9 +2610,11 @@ __global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_e
                 const uint32_t* order) {
     __shared__ WaveLds w[kAloneBlock / kWave];
     const uint32_t lane = __lane_id();
-    QueueCursor cursor{blockIdx.x % kSubs, kSubs};
-    const uint32_t idx = queue_pop<kSubs>(q, n, cursor, lane);
-    decode_alone<kFormat, kSubs, kParseOnly>(w[uniform32(threadIdx.x / kWave)], idx, srcs,
+    QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
+    const uint32_t wave = uniform32(threadIdx.x / kWave);
+    const uint32_t idx = queue_pop<kSubs>(
+        q, n, cursor, lane, (uint64_t)blockIdx.x * (kAloneBlock / kWave) + wave);
+    decode_alone<kFormat, kSubs, kParseOnly>(w[wave], idx, srcs,
                                              src_sizes, dsts, caps, n, results, q, order, cursor,
                                              lane);
 }
@@ -2677,8 +2697,8 @@ hipError_t device_state(DeviceState** out) {
             d.alone_blocks_per_cu[f] = per > 0 ? per : 1;
         }
         for (int f = 0; f < 2; f++) {
-            d.plan[f] = plan_from_threshold(kDefaultPipeMinCost);
-            d.min_cost[f] = kDefaultPipeMinCost;
+            d.plan[f] = plan_from_threshold(kDefaultPipeMinCost[f]);
+            d.min_cost[f] = kDefaultPipeMinCost[f];
         }
         /* this device is current: its own copy of the fixed scratch */
         d.fixed_status = hipGetSymbolAddress(&d.fixed, HIP_SYMBOL(scratch));
@@ -2788,62 +2808,97 @@ uint32_t host_cost_bin(uint64_t src_size, uint64_t cap) {
 
 namespace {
 
-/* Bins the batch into the queue held by `work` (a Queue, then order[n])
- * and launches the persistent decoder, all on `stream`; parse_only
- * launches its parse-only build. */
-hipError_t queue_and_decode(DeviceState* dev, int format, const void* const* srcs,
+/* How one launch runs: its plan, whether any chunk may be pipelined, its
+ * grid, and whether every chunk has a resident block (or wave) of its own,
+ * so that it needs no queue and no scratch. */
+struct Launch {
+    Plan plan;
+    bool pipes;
+    bool direct;
+    size_t grid;
+};
+
+/* A launch of few chunks leaves most of the chip idle whatever it does, and
+ * takes as long as its largest chunk: under the default plan all its chunks
+ * are pipelined (16 token chunks of 4 KiB to 1 MiB: 1.45 ms, against 2.38
+ * with the threshold alone), up to two chunks a resident block. The queue's
+ * four kernels and the scratch allocation cost about 35 us, so a launch
+ * that has a resident block for each chunk takes them in their own order. */
+Launch plan_launch(const DeviceState& dev, int f, size_t n) {
+    Launch r;
+    {
+        std::lock_guard<std::mutex> hold(g_devices_lock);
+        r.plan = dev.plan[f];
+    }
+    const size_t pipe_blocks = (size_t)dev.cus * (size_t)dev.pipe_blocks_per_cu[f];
+    const Plan usual = plan_from_threshold(kDefaultPipeMinCost[f]);
+    if (n <= 2 * pipe_blocks && std::memcmp(&r.plan, &usual, sizeof(Plan)) == 0) {
+        r.plan = plan_from_threshold(kFewPipeMinCost);
+    }
+    r.pipes = false;
+    for (int w = 0; w < kBins / 64; w++) {
+        r.pipes = r.pipes || r.plan.two_wave[w] != 0;
+    }
+    const size_t per = r.pipes ? 1 : kAloneBlock / kWave; /* chunks a block starts with */
+    const size_t blocks = r.pipes ? pipe_blocks : (size_t)dev.cus * (size_t)dev.alone_blocks_per_cu[f];
+    const size_t wanted = (n + per - 1) / per;
+    r.direct = wanted <= blocks;
+    r.grid = r.direct ? wanted : blocks;
+    return r;
+}
+
+/* Launches the persistent decoder on `stream`; parse_only launches its
+ * parse-only build. Unless the launch is direct, the batch is first binned
+ * into the queue held by `work` (a Queue, then order[n]). */
+hipError_t queue_and_decode(const Launch& launch, int format, const void* const* srcs,
                             const size_t* src_sizes, void* const* dsts, const size_t* caps,
                             size_t n, cudec_chunk_result* results, void* work,
                             hipStream_t stream, bool parse_only) {
-    Plan plan;
-    {
-        std::lock_guard<std::mutex> hold(g_devices_lock);
-        plan = dev->plan[format == kFormatSnappy ? kFormatSnappy : kFormatLz4];
-    }
+    const Plan plan = launch.plan;
     Queue* q = static_cast<Queue*>(work);
-    uint32_t* order = reinterpret_cast<uint32_t*>(q + 1);
-    const unsigned tb = 256;
-    const unsigned nb = (unsigned)((n + tb - 1) / tb);
-    hipLaunchKernelGGL(queue_reset, dim3(1), dim3(kKeys), 0, stream, q);
-    hipLaunchKernelGGL(queue_count, dim3(nb), dim3(tb), 0, stream, src_sizes, caps, n, q, plan);
-    hipLaunchKernelGGL(queue_scan, dim3(1), dim3(1), 0, stream, q);
-    hipLaunchKernelGGL(queue_fill, dim3(nb), dim3(tb), 0, stream, src_sizes, caps, n, q, order,
-                       plan);
-    bool any_two_wave = false;
-    for (int w = 0; w < kBins / 64; w++) {
-        any_two_wave = any_two_wave || plan.two_wave[w] != 0;
+    uint32_t* order = launch.direct ? nullptr : reinterpret_cast<uint32_t*>(q + 1);
+    if (!launch.direct) {
+        const unsigned tb = 256;
+        const unsigned nb = (unsigned)((n + tb - 1) / tb);
+        hipLaunchKernelGGL(queue_reset, dim3(1), dim3(kKeys), 0, stream, q);
+        hipLaunchKernelGGL(queue_count, dim3(nb), dim3(tb), 0, stream, src_sizes, caps, n, q,
+                           plan);
+        hipLaunchKernelGGL(queue_scan, dim3(1), dim3(1), 0, stream, q);
+        hipLaunchKernelGGL(queue_fill, dim3(nb), dim3(tb), 0, stream, src_sizes, caps, n, q,
+                           order, plan);
     }
     /* pipelined blocks, each of which splits into one-wave decoders when it
      * meets a one-wave chunk; or, where the plan pipelines no chunk, the
      * one-wave kernel */
     const int f = format == kFormatSnappy ? 1 : 0;
-    const int waves = any_two_wave ? (int)kPipeWaves : kAloneBlock / (int)kWave;
-    size_t grid = (size_t)dev->cus *
-                  (size_t)(any_two_wave ? dev->pipe_blocks_per_cu[f] : dev->alone_blocks_per_cu[f]);
-    if (grid > n) {
-        grid = n;
-    }
+    const int waves = launch.pipes ? (int)kPipeWaves : kAloneBlock / (int)kWave;
+    const size_t grid = launch.grid;
     const dim3 gd((unsigned)grid), bd((unsigned)(waves * (int)kWave));
     const bool many = (uint64_t)n >= kSubQueueMinPerWave * (uint64_t)waves * (uint64_t)grid;
-    const int shape = (parse_only ? 8 : 0) | (f ? 4 : 0) | (any_two_wave ? 0 : 2) | (many ? 1 : 0);
+    const int subs = launch.direct ? 2 : many ? 1 : 0;
+    const int shape = (parse_only ? 16 : 0) | (f ? 8 : 0) | (launch.pipes ? 0 : 4) | subs;
     switch (shape) {
 #define CUDEC_PIPED(kShape, kFmt, kS, kP)                                                 \
     case kShape:                                                                          \
         hipLaunchKernelGGL((piped_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
                            src_sizes, dsts, caps, n, results, q, order, plan);            \
         break;                                                                            \
-    case kShape + 2:                                                                      \
+    case kShape + 4:                                                                      \
         hipLaunchKernelGGL((alone_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
                            src_sizes, dsts, caps, n, results, q, order);                  \
         break;
         CUDEC_PIPED(0, kFormatLz4, 1, false)
         CUDEC_PIPED(1, kFormatLz4, kSubQueues, false)
-        CUDEC_PIPED(4, kFormatSnappy, 1, false)
-        CUDEC_PIPED(5, kFormatSnappy, kSubQueues, false)
-        CUDEC_PIPED(8, kFormatLz4, 1, true)
-        CUDEC_PIPED(9, kFormatLz4, kSubQueues, true)
-        CUDEC_PIPED(12, kFormatSnappy, 1, true)
-        CUDEC_PIPED(13, kFormatSnappy, kSubQueues, true)
+        CUDEC_PIPED(2, kFormatLz4, 0, false)
+        CUDEC_PIPED(8, kFormatSnappy, 1, false)
+        CUDEC_PIPED(9, kFormatSnappy, kSubQueues, false)
+        CUDEC_PIPED(10, kFormatSnappy, 0, false)
+        CUDEC_PIPED(16, kFormatLz4, 1, true)
+        CUDEC_PIPED(17, kFormatLz4, kSubQueues, true)
+        CUDEC_PIPED(18, kFormatLz4, 0, true)
+        CUDEC_PIPED(24, kFormatSnappy, 1, true)
+        CUDEC_PIPED(25, kFormatSnappy, kSubQueues, true)
+        CUDEC_PIPED(26, kFormatSnappy, 0, true)
 #undef CUDEC_PIPED
         default:
             return hipErrorInvalidValue;
@@ -2899,6 +2954,12 @@ hipError_t launch_tuned(int format, const void* const* srcs, const size_t* src_s
     if (e != hipSuccess) {
         return e;
     }
+    const int f = format == kFormatSnappy ? kFormatSnappy : kFormatLz4;
+    const Launch launch = plan_launch(*dev, f, n);
+    if (launch.direct) {
+        return queue_and_decode(launch, format, srcs, src_sizes, dsts, caps, n, results, nullptr,
+                                stream, parse_only);
+    }
     hipMemPool_t pool = scratch_pool(*dev, id);
     const size_t bytes = sizeof(Queue) + sizeof(uint32_t) * n;
     /* under stream capture the scratch becomes a graph allocation node of
@@ -2915,10 +2976,10 @@ hipError_t launch_tuned(int format, const void* const* srcs, const size_t* src_s
     if (e != hipSuccess) {
         return e;
     }
-    e = queue_and_decode(dev, format, srcs, src_sizes, dsts, caps, n, results, mem, stream,
+    e = queue_and_decode(launch, format, srcs, src_sizes, dsts, caps, n, results, mem, stream,
                          parse_only);
-    const hipError_t f = hipFreeAsync(mem, stream);
-    return e != hipSuccess ? e : f;
+    const hipError_t freed = hipFreeAsync(mem, stream);
+    return e != hipSuccess ? e : freed;
 }
 
 hipError_t launch_tuned_fixed(int format, const void* const* srcs, const size_t* src_sizes,
@@ -2935,8 +2996,9 @@ hipError_t launch_tuned_fixed(int format, const void* const* srcs, const size_t*
     if (dev->fixed == nullptr) {
         return dev->fixed_status != hipSuccess ? dev->fixed_status : hipErrorInvalidSymbol;
     }
-    return queue_and_decode(dev, format, srcs, src_sizes, dsts, caps, n, results, dev->fixed,
-                            stream, false);
+    const int f = format == kFormatSnappy ? kFormatSnappy : kFormatLz4;
+    return queue_and_decode(plan_launch(*dev, f, n), format, srcs, src_sizes, dsts, caps, n,
+                            results, dev->fixed, stream, false);
 }
 
 }  // namespace cudec_amd
