@@ -61,7 +61,7 @@ __device__ __forceinline__ uint32_t stage_into(uint8_t* stage, gcu8* src,
     const uintptr_t a = (uintptr_t)(src + sp);
     const uintptr_t base = a & ~(uintptr_t)15;
     const uintptr_t end = (uintptr_t)src + src_size;
-    const uint32_t blocks = bytes / 16 + 1;
+    const uint32_t blocks = (bytes + 30) / 16; /* whatever the alignment of sp */
     uint4 v[kRounds];
     if (sp < src_size) {
 #pragma unroll

@@ -1,16 +1,30 @@
-/* The Zstandard batch decoder for gfx950: one wave per frame, frames taken
- * costliest first (the LZ4 decoder's cost queue: output plus what matches
- * add) from a device counter by a persistent grid.
+/* The Zstandard batch decoder for gfx950: a block of two waves per frame,
+ * frames taken costliest first (the LZ4 decoder's cost queue: output plus
+ * what matches add) from a device counter by a persistent grid.
  *
- * A frame's decode (zstd_decode.h) keeps its Huffman and FSE tables in the
- * wave's LDS (FrameTables, about 10 KiB), so a table built for one block is
- * there for the next block's Treeless or Repeat mode. Huffman-coded
- * literals are decoded four streams at a time, one lane a stream, into the
- * wave's 128 KiB literals slot in global scratch; the sequences are decoded
- * in order on every lane (the FSE states are one serial chain), 64 at a
- * time, and each batch is executed straight into the frame's output: short
- * literals and matches from before the batch one lane a sequence, the rest
- * wave-wide (zstd_decode.h, execute_batch).
+ * The entropy wave walks the frame (zstd_decode.h, walk_frame), builds the
+ * FSE tables and decodes the sequences, 64 at a time, into jobs: slots in
+ * LDS that the copy wave takes in order. The copy wave decodes the
+ * Huffman-coded literals (one lane a stream) into the block's 128 KiB slot
+ * in global scratch and executes the sequences through an LDS ring
+ * (execute.h, the same code that writes LZ4 output). Neither waits for the
+ * other beyond the slots, so a frame's time is the longer of the two.
+ *
+ * What bounds it is the FSE chain: a sequence's three states give the bits
+ * that give the next states. The entropy wave spends a lane on each of the
+ * three fields (every quad of lanes does the same): one LDS read takes the
+ * three cells, sums over the quad place each lane's bits, and two reads of
+ * the staged bitstream give its extra bits and its next state, two LDS round
+ * trips and about 45 instructions a sequence. Everything that does not feed
+ * the next state (code baselines, repeat offsets, limits, positions) is done
+ * per 64 sequences, a lane each. Measured alone, a sequence costs 390 cycles
+ * of FSE chain, 208 of finishing and 211 of copies on the other wave. One
+ * wave a frame with one sequence decoded and executed after the other took
+ * 13.72 ms for 4096 frames of 64 KiB and 284 ms for 20 000 uneven frames;
+ * this takes 6.27 and 78.9 ms.
+ *
+ * The first error in stream order decides a frame: the entropy wave's
+ * verdicts travel as jobs, behind the literals that precede them.
  *
  * The content checksum of a frame is checked by a second kernel, four
  * lanes a frame (xxhash.h), over every frame that decoded and carries one:
@@ -20,6 +34,7 @@
 
 #include "common.h"
 #include "cudec_zstd.h"
+#include "execute.h"
 #include "xxhash.h"
 #include "zstd_decode.h"
 
@@ -29,40 +44,14 @@ namespace {
 constexpr int kVerifyBlock = 256;
 constexpr uint64_t kPoolKeep = 512ull << 20; /* scratch kept between launches */
 
+/* The Wave policy of the shared Huffman code. */
 struct Wave {
     static constexpr uint32_t kLanes = kWave;
     uint32_t lane;
     __device__ void sync() const { wave_order(); }
-    __device__ uint32_t uniform(uint32_t v) const { return uniform32(v); }
-    /* a reader every lane runs on the same stream. Its words stay in vector
-     * registers: made wave-uniform, the sequence decode ran on the CU's
-     * one scalar unit, which the CU's resident waves then shared, and it
-     * was 29% slower (4.3e7 against 3.4e7 clocks a wave on 64 KiB frames) */
+    /* a reader every lane runs on the same stream */
     struct Same {
         static __device__ uint64_t fix64(uint64_t v) { return v; }
-    };
-    /* a batch's sequence records: lane k holds record k in registers */
-    struct Records {
-        zstd::Rec mine;
-        __device__ void put(uint32_t lane, uint32_t k, const zstd::Rec& v) {
-            const bool me = lane == k; /* a select, not a branch */
-            mine.d = me ? v.d : mine.d;
-            mine.ll = me ? v.ll : mine.ll;
-            mine.ml = me ? v.ml : mine.ml;
-            mine.lit = me ? v.lit : mine.lit;
-            mine.at = me ? v.at : mine.at;
-        }
-        __device__ zstd::Rec get(uint32_t k) const { /* k is the same on every lane */
-            zstd::Rec r;
-            r.d = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mine.d >> 32), (int)k) << 32) |
-                  (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)mine.d, (int)k);
-            r.ll = (uint32_t)__builtin_amdgcn_readlane((int)mine.ll, (int)k);
-            r.ml = (uint32_t)__builtin_amdgcn_readlane((int)mine.ml, (int)k);
-            r.lit = (uint32_t)__builtin_amdgcn_readlane((int)mine.lit, (int)k);
-            r.at = (uint32_t)__builtin_amdgcn_readlane((int)mine.at, (int)k);
-            return r;
-        }
-        __device__ zstd::Rec own(uint32_t, uint32_t) const { return mine; }
     };
 };
 
@@ -73,8 +62,566 @@ struct FrameCheck {
     uint32_t verify; /* 1: the frame decoded and carries a content checksum */
 };
 
+/* What the entropy wave asks of the copy wave, in stream order. */
+enum JobKind : uint32_t {
+    kJobFrame,     /* a frame begins: chunk index a, output b, capacity c */
+    kJobBlock,     /* n output bytes: a copy of a, or (a null) the byte x */
+    kJobLiterals,  /* the block's literals: at a, or (a null) n times x */
+    kJobHuffman,   /* the block's literals: payload a of b bytes, n symbols */
+    kJobSequences, /* n sequences, literals from c on */
+    kJobTail,      /* n literals from c on */
+    kJobFail,      /* the frame ends with status x */
+    kJobEnd,       /* the frame ends: written a, checksum x (y: it has one) */
+    kJobQuit,
+};
+constexpr uint32_t kJobs = 3; /* slots: the entropy wave may run two ahead */
+struct alignas(16) Job {
+    uint32_t ll[kWave], ml[kWave], off[kWave]; /* kJobSequences, a lane each */
+    uint64_t a, b, c;
+    uint32_t kind, n, x, y;
+};
+static_assert(sizeof(Job) % 16 == 0, "slots keep their alignment");
+
+/* An FSE cell of a sequence field in one word: symbol (6 bits), state bits
+ * (4), extra bits of the symbol's code (5), next-state base (16). */
+constexpr uint32_t kCellBits = 6, kCellExtra = 10, kCellBase = 16;
+constexpr uint32_t kCodes = (zstd::kLitLenMax + 1) + (zstd::kMatchLenMax + 1);
+
+/* Staged bitstream of one batch: at most 712 bytes (zstd::kWindowBytes). */
+struct alignas(16) EntropyLds {
+    uint32_t litlen[1u << zstd::kLitLenLog];
+    uint32_t matchlen[1u << zstd::kMatchLenLog];
+    uint32_t offset[1u << zstd::kOffsetLog];
+    uint32_t code[kCodes]; /* baseline, extra bits above it (24) */
+    int16_t counts[zstd::kMatchLenMax + 1];
+    uint16_t next[zstd::kMatchLenMax + 1];
+    alignas(16) uint8_t window[zstd::kWindowBytes + 16];
+};
+constexpr uint32_t kHeaderStage = 512; /* of the window: table descriptions */
+static_assert(kHeaderStage + (1u << zstd::kLitLenLog) <= zstd::kWindowBytes,
+              "a field's symbol order lies behind the descriptions");
+static_assert(zstd::kBatch == kWave, "a batch holds a sequence a lane");
+
+struct alignas(16) CopyLds : RingLds<kRing> {
+    CoverLds cover;
+    uint16_t huffman[zstd::kHufCells];
+    zstd::HufScratch huf;
+    uint32_t stream_bad[4];
+    alignas(16) uint8_t stage[zstd::kWindowBytes + 16]; /* literals of a group; Huffman windows */
+};
+constexpr uint32_t kLitStage = zstd::kWindowBytes - 16; /* literal bytes of a group */
+
+struct alignas(16) FrameLds {
+    EntropyLds e;
+    CopyLds c;
+    Job job[kJobs];
+    uint32_t published; /* jobs written */
+    uint32_t consumed;  /* jobs done */
+    uint32_t broken;    /* a wait ran out, and no wave waits any more */
+};
+static_assert(sizeof(FrameLds) <= 20480, "eight blocks share a CU's 160 KiB");
+
+/* ------------------------------------------------------------ entropy */
+
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+template <class T>
+__device__ __forceinline__ uint32_t lds_at(const T* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const T*)p;
+}
+
+/* Lane `from` of every quad, on its whole quad. */
+template <uint32_t kFrom>
+__device__ __forceinline__ uint32_t quad(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kFrom * 0x55, 0xF, 0xF, true);
+}
+
+/* n (0..31) bits of the staged stream from window bit `at` on, in stream
+ * order lowest first. A position before the window (a stream that ran out:
+ * its batch is refused) reads the window's start. */
+__device__ __forceinline__ uint32_t window_bits(uint32_t window, int at, uint32_t n) {
+    const uint32_t p = at < 0 ? 0u : (uint32_t)at;
+    const uint32_t a = window + ((p >> 5) << 2);
+    const uint32_t lo = *(lds_u32*)(uintptr_t)a, hi = *(lds_u32*)(uintptr_t)(a + 4);
+    return __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(hi, lo, p & 31), 0, n);
+}
+
+/* Builds a field's cells from counts[0..last] at accuracy `log` (RFC 8878
+ * 4.1.1), as zstd::build_fse_table does one cell after the other: "less
+ * than one" symbols take the top cells; the others, in symbol order, the
+ * cells 0, step, 2 step, ... that lie below those; then, in cell order, each
+ * symbol's cells count up from its probability. Cells go 64 at a time: a
+ * cell's rank among its symbol's comes from ballots on the symbol's bits.
+ * `order` is scratch of 1 << log bytes. False if the counts do not fill the
+ * table exactly. */
+__device__ __forceinline__ bool build_cells(EntropyLds& e, uint32_t* cells, uint8_t* order,
+                                            uint32_t last, uint32_t log, const uint32_t* codes,
+                                            uint32_t lane) {
+    const uint32_t size = 1u << log;
+    const uint32_t mask = size - 1;
+    const int count = lane <= last ? e.counts[lane] : 0;
+    const uint64_t lows = __ballot(count < 0);
+    const uint32_t low = (uint32_t)__builtin_popcountll(lows);
+    const uint32_t mine = count > 0 ? (uint32_t)count : 0;
+    const uint32_t incl = wave_inclusive_sum(mine, lane);
+    const uint32_t placed = uniform32(__builtin_amdgcn_readlane(incl, kWave - 1));
+    if (placed + low != size) {
+        return false;
+    }
+    const uint64_t below = (1ull << lane) - 1;
+    if (count < 0) {
+        cells[size - 1 - (uint32_t)__builtin_popcountll(lows & below)] = lane;
+    }
+    if (lane <= last) {
+        e.next[lane] = (uint16_t)(count < 0 ? 1 : count);
+    }
+    for (uint32_t t = 0; t < mine; t++) {
+        order[incl - mine + t] = (uint8_t)lane;
+    }
+    wave_order();
+    const uint32_t step = (size >> 1) + (size >> 3) + 3;
+    uint32_t run = 0;
+    for (uint32_t i0 = 0; i0 < size; i0 += kWave) {
+        const uint32_t i = i0 + lane;
+        const uint32_t at = (i * step) & mask;
+        const bool fits = i < size && at + low < size;
+        const uint64_t all = __ballot(fits);
+        if (fits) {
+            cells[at] = order[run + (uint32_t)__builtin_popcountll(all & below)];
+        }
+        run += (uint32_t)__builtin_popcountll(all);
+    }
+    wave_order();
+    for (uint32_t c0 = 0; c0 < size; c0 += kWave) {
+        const uint32_t c = c0 + lane;
+        const uint32_t s = c < size ? cells[c] : 0;
+        uint64_t same = __ballot(c < size);
+#pragma unroll
+        for (uint32_t b = 0; b < 6; b++) {
+            const uint64_t set = __ballot(((s >> b) & 1) != 0);
+            same &= ((s >> b) & 1) != 0 ? set : ~set;
+        }
+        const uint32_t first = e.next[s];
+        const uint32_t state = first + (uint32_t)__builtin_popcountll(same & below);
+        wave_order();
+        if (c < size) {
+            if ((same >> lane) == 1) { /* the symbol's last cell here */
+                e.next[s] = (uint16_t)(state + 1);
+            }
+            const uint32_t bits = log - zstd::high_bit(state);
+            const uint32_t extra = codes == nullptr ? s : codes[s] >> 24;
+            cells[c] = s | bits << kCellBits | extra << kCellExtra |
+                       ((state << bits) - size) << kCellBase;
+        }
+        wave_order();
+    }
+    return true;
+}
+
+/* One sequence field's table. */
+struct Field {
+    uint32_t* cells;
+    const uint32_t* codes; /* null: the offset field, whose extra bits are its symbol */
+    uint32_t log;
+    bool present;
+};
+
+/* walk_frame's flow of the entropy wave. */
+struct EntropyFlow {
+    FrameLds& l;
+    uint32_t lane;
+    uint32_t seq;  /* jobs so far */
+    bool alive;    /* no wait has run out */
+    Field ll, of, ml;
+    uint32_t r0, r1, r2; /* the frame's repeat offsets */
+
+    __device__ uint64_t u64(uint64_t v) const { return uniform64(v); }
+
+    /* The next slot, once the copy wave is done with it. */
+    __device__ __forceinline__ Job& slot() {
+        if (seq >= kJobs && alive) {
+            alive = await_flag((const lds_flag*)&l.consumed, seq - kJobs + 1, nullptr,
+                               (lds_flag*)&l.broken) == kReached;
+        }
+        return l.job[seq % kJobs];
+    }
+    __device__ __forceinline__ void post(Job& j, uint32_t kind, uint32_t n, uint64_t a, uint64_t b,
+                                         uint64_t c, uint32_t x, uint32_t y) {
+        j.kind = kind;
+        j.n = n;
+        j.a = a;
+        j.b = b;
+        j.c = c;
+        j.x = x;
+        j.y = y;
+        seq++;
+        raise_flag((lds_flag*)&l.published, seq);
+    }
+    __device__ __forceinline__ void ask(uint32_t kind, uint32_t n, uint64_t a, uint64_t b,
+                                        uint64_t c, uint32_t x, uint32_t y) {
+        Job& j = slot();
+        post(j, kind, n, a, b, c, x, y);
+    }
+    __device__ __forceinline__ void begin(uint64_t chunk, gu8* dst, uint64_t cap) {
+        ll.present = of.present = ml.present = false;
+        r0 = 1;
+        r1 = 4;
+        r2 = 8;
+        ask(kJobFrame, 0, chunk, (uint64_t)(uintptr_t)dst, cap, 0, 0);
+    }
+    __device__ void block(const ZG uint8_t* from, uint8_t fill, uint64_t n) {
+        ask(kJobBlock, (uint32_t)n, (uint64_t)(uintptr_t)from, 0, 0, fill, 0);
+    }
+    __device__ void literals(const ZG uint8_t* from, uint8_t fill, uint64_t n) {
+        ask(kJobLiterals, (uint32_t)n, (uint64_t)(uintptr_t)from, 0, 0, fill, 0);
+    }
+    __device__ bool huffman(const ZG uint8_t* payload, uint64_t size, uint64_t regen,
+                            uint32_t streams, bool treeless) {
+        ask(kJobHuffman, (uint32_t)regen, (uint64_t)(uintptr_t)payload, size, 0, streams,
+            treeless ? 1u : 0u);
+        return true; /* the copy wave refuses it */
+    }
+    __device__ void tail(uint64_t lp, uint64_t n) {
+        if (n != 0) {
+            ask(kJobTail, (uint32_t)n, 0, 0, lp, 0, 0);
+        }
+    }
+
+    /* Loads one field's table (RFC 8878 3.1.1.3.2.1): 0 predefined, 1
+     * run-length, 2 an FSE description, 3 repeat; `head` holds the staged
+     * section from its current position on, `left` the section's bytes. */
+    __device__ __forceinline__ bool load(Field& f, uint32_t mode, const uint8_t* head,
+                                         uint64_t left, uint32_t max_symbol, uint32_t log_max,
+                                         const int16_t* defaults, uint32_t default_last,
+                                         uint32_t default_log, uint32_t& used) {
+        used = 0;
+        if (mode == 3) {
+            return f.present;
+        }
+        if (mode == 1) {
+            const uint32_t s = left == 0 ? 255u : uniform32(head[0]);
+            if (s > max_symbol) {
+                return false;
+            }
+            f.cells[0] = s | (f.codes == nullptr ? s : f.codes[s] >> 24) << kCellExtra;
+            wave_order();
+            f.log = 0;
+            f.present = true;
+            used = 1;
+            return true;
+        }
+        uint32_t last = default_last, log = default_log;
+        if (mode == 0) {
+            if (lane <= default_last) {
+                l.e.counts[lane] = defaults[lane];
+            }
+        } else {
+            uint64_t u = 0;
+            if (!zstd::read_fse_description((const ZL uint8_t*)head, left, max_symbol, log_max,
+                                            (ZL int16_t*)l.e.counts, last, log, u)) {
+                return false;
+            }
+            last = uniform32(last);
+            log = uniform32(log);
+            used = uniform32((uint32_t)u);
+        }
+        wave_order();
+        if (!build_cells(l.e, f.cells, &l.e.window[kHeaderStage], last, log, f.codes, lane)) {
+            used = 0;
+            return false;
+        }
+        f.log = log;
+        f.present = true;
+        return true;
+    }
+
+    __device__ int sequences(const ZG uint8_t* sec, uint64_t left, uint32_t modes, uint32_t count,
+                             uint64_t regen, uint64_t window, uint64_t cap, uint64_t& lp,
+                             uint64_t& o) {
+        /* the three descriptions, whose readers stay below kHeaderStage: a
+         * field's is at most 53 probabilities of 10 bits and as many 2-bit
+         * repeat fields */
+        EntropyLds& e = l.e;
+        const uint32_t staged = left < kHeaderStage - 16 ? (uint32_t)left : kHeaderStage - 16;
+        const uint32_t delta = stage_into<1>(e.window, (gcu8*)sec, staged, 0, staged, lane);
+        const uint8_t* head = e.window + delta;
+        uint32_t u = 0;
+        if (!load(ll, modes >> 6, head, left, zstd::kLitLenMax, zstd::kLitLenLog,
+                  zstd::kLitLenDefault, 35, 6, u)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        head += u;
+        left -= u;
+        sec += u;
+        if (!load(of, (modes >> 4) & 3u, head, left, zstd::kOffsetMax, zstd::kOffsetLog,
+                  zstd::kOffsetDefault, 28, 5, u)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        head += u;
+        left -= u;
+        sec += u;
+        if (!load(ml, (modes >> 2) & 3u, head, left, zstd::kMatchLenMax, zstd::kMatchLenLog,
+                  zstd::kMatchLenDefault, 52, 6, u)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        left -= u;
+        sec += u;
+        /* the backward bitstream (RFC 8878 4.1): `bits` left of it */
+        const uint32_t marker = left == 0 ? 0u : uniform32(sec[left - 1]);
+        if (marker == 0) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        int bits = 8 * (int)(left - 1) + (int)zstd::high_bit(marker);
+
+        /* this lane's field: 0 literal length, 1 match length, 2 (and 3)
+         * offset; masks of what precedes its bits */
+        const uint32_t f = (lane & 3) < 2 ? lane & 3 : 2;
+        const uint32_t table = f == 0 ? lds_at(e.litlen) : f == 1 ? lds_at(e.matchlen)
+                                                                   : lds_at(e.offset);
+        const uint32_t is_of = f == 2 ? ~0u : 0u, is_ll = f == 0 ? ~0u : 0u;
+        uint32_t state = 0;
+        int pending = CUDEC_OK; /* the first execution error, reported once
+                                   the whole block decodes */
+        uint32_t k = 0;
+        for (;;) {
+            /* stage what the batch reads: its bytes end where `bits` does */
+            const uint32_t hi = ((uint32_t)bits + 7) >> 3;
+            const uint32_t lo = hi > zstd::kWindowBytes - 32 ? hi - (zstd::kWindowBytes - 32) : 0;
+            wave_order();
+            const uint32_t skew =
+                stage_into<1>(e.window, (gcu8*)sec, hi, lo, hi - lo, lane);
+            const uint32_t win = lds_at(e.window);
+            const int base = 8 * ((int)skew - (int)lo); /* window bit of stream bit 0 */
+            if (k == 0) {
+                /* the initial states: literal length, offset, match length */
+                const uint32_t n = f == 0 ? ll.log : f == 1 ? ml.log : of.log;
+                const uint32_t upto = f == 0   ? ll.log
+                                      : f == 2 ? ll.log + of.log
+                                               : ll.log + of.log + ml.log;
+                state = window_bits(win, base + bits - (int)upto, n);
+                bits -= (int)(ll.log + of.log + ml.log);
+                if (bits < 0) {
+                    return CUDEC_ERR_CORRUPT_INPUT;
+                }
+            }
+            const uint32_t cnt = count - k < kWave ? count - k : kWave;
+            Job& j = slot();
+            const uint32_t raw = lds_at(j.ll) + 4 * f;
+            int at = base + bits; /* window bit above the next one */
+            for (uint32_t s = 0; s < cnt; s++) {
+                const uint32_t cell = *(lds_u32*)(uintptr_t)(table + 4 * state);
+                const uint32_t sym = cell & 63;
+                const uint32_t extra = (cell >> kCellExtra) & 31;
+                /* no state is read after the block's last sequence */
+                const uint32_t sb = k + s + 1 == count ? 0u : (cell >> kCellBits) & 15;
+                /* the offset's extra bits come first, then the match
+                 * length's, then the literal length's; the states: literal
+                 * length, match length, offset */
+                const uint32_t x0 = quad<0>(extra), x1 = quad<1>(extra), x2 = quad<2>(extra);
+                const uint32_t s0 = quad<0>(sb), s1 = quad<1>(sb), s2 = quad<2>(sb);
+                const uint32_t before = x2 + (x1 & ~is_of) + (x0 & is_ll);
+                const uint32_t extras = x0 + x1 + x2;
+                const uint32_t states = s0 + (s1 & ~is_ll) + (s2 & is_of);
+                const uint32_t ex = window_bits(win, at - (int)before, extra);
+                at -= (int)extras;
+                const uint32_t nx = window_bits(win, at - (int)states, sb);
+                at -= (int)(s0 + s1 + s2);
+                state = (cell >> kCellBase) + nx;
+                const uint32_t value = (is_of != 0 ? 1u << (sym & 31) : sym << 16) + ex;
+                *(lds_u32*)(uintptr_t)(raw + 12 * s) = value;
+            }
+            bits = (int)uniform32((uint32_t)(at - base));
+            if (bits < 0) {
+                return CUDEC_ERR_CORRUPT_INPUT;
+            }
+            wave_order();
+            if (pending == CUDEC_OK) {
+                pending = finish_batch(j, cnt, regen, window, cap, lp, o);
+            }
+            k += cnt;
+            if (k == count) {
+                break;
+            }
+        }
+        if (bits != 0) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        return pending;
+    }
+
+    /* A batch's raw values (three words a sequence, in the slot) to lengths
+     * and distances, a lane each, with every check of their execution; posts
+     * the job, or returns the first error in stream order. */
+    __device__ __forceinline__ int finish_batch(Job& j, uint32_t cnt, uint64_t regen,
+                                                uint64_t window, uint64_t cap, uint64_t& lp,
+                                                uint64_t& o) {
+        const uint32_t* raw = j.ll + 3 * lane;
+        const uint32_t v0 = raw[0], v1 = raw[1], value = raw[2];
+        wave_order();
+        const bool in = lane < cnt;
+        const uint32_t c0 = v0 >> 16, c1 = v1 >> 16;
+        const uint32_t llen =
+            in ? (l.e.code[c0 <= zstd::kLitLenMax ? c0 : 0] & 0xFFFFFF) + (v0 & 0xFFFF) : 0;
+        const uint32_t mlen =
+            in ? (l.e.code[zstd::kLitLenMax + 1 + (c1 <= zstd::kMatchLenMax ? c1 : 0)] & 0xFFFFFF) +
+                     (v1 & 0xFFFF)
+               : 0;
+        /* repeat offsets (RFC 8878 3.1.1.5), one sequence after the other on
+         * the scalar unit; zero: an error */
+        const uint64_t no_literals = __ballot(llen == 0);
+        uint32_t dist = 0;
+        uint32_t a = r0, b = r1, c = r2;
+        for (uint32_t i = 0; i < cnt; i++) {
+            const uint32_t v = __builtin_amdgcn_readlane(value, i);
+            uint32_t d;
+            if (v > 3) {
+                d = v - 3;
+                c = b;
+                b = a;
+                a = d;
+            } else {
+                const uint32_t which = v - 1 + (uint32_t)((no_literals >> i) & 1);
+                d = which == 0 ? a : which == 1 ? b : which == 2 ? c : a - 1;
+                if (which != 0 && d != 0) {
+                    c = which == 1 ? c : b;
+                    b = a;
+                    a = d;
+                }
+            }
+            dist = lane == i ? d : dist;
+        }
+        r0 = a;
+        r1 = b;
+        r2 = c;
+        /* positions: a block's regenerated literals and output fit 32 bits
+         * whatever the lengths claim (64 of at most 2^17 + 2^16 each) */
+        const uint32_t lit_incl = wave_inclusive_sum(llen, lane);
+        const uint32_t out_incl = wave_inclusive_sum(llen + mlen, lane);
+        const uint64_t m = o + (out_incl - mlen);
+        int ev = CUDEC_OK;
+        if (in) {
+            if (lit_incl > regen - lp || dist == 0 || dist > m || dist > window) {
+                ev = CUDEC_ERR_CORRUPT_INPUT;
+            } else if (m > cap || mlen > cap - m) {
+                ev = CUDEC_ERR_OUTPUT_TOO_SMALL;
+            }
+        }
+        const uint64_t bad = __ballot(ev != CUDEC_OK);
+        if (bad != 0) {
+            return (int)uniform32(__builtin_amdgcn_readlane((uint32_t)ev, __builtin_ctzll(bad)));
+        }
+        j.ll[lane] = llen;
+        j.ml[lane] = mlen;
+        j.off[lane] = dist;
+        post(j, kJobSequences, cnt, 0, 0, lp, 0, 0);
+        lp += uniform32(__builtin_amdgcn_readlane(lit_incl, kWave - 1));
+        o += uniform32(__builtin_amdgcn_readlane(out_incl, kWave - 1));
+        return CUDEC_OK;
+    }
+};
+
+/* ------------------------------------------------------------ copies */
+
+/* The copy wave's place in a frame's output. */
+struct CopyState {
+    gu8* dst;
+    uint64_t cap;
+    uint64_t dp;      /* output bytes so far */
+    uint64_t flushed; /* of them, in memory */
+    uint64_t ring_lo; /* the ring holds none before */
+    gcu8* lit;        /* the block's literals */
+};
+
+/* n bytes from memory to the output: a few through the ring, more around it. */
+__device__ __forceinline__ void copy_bytes(CopyLds& w, CopyState& s, gcu8* from, uint32_t n,
+                                           uint32_t lane) {
+    const uintptr_t da = (uintptr_t)s.dst;
+    if (n <= kBatchMax / 2) {
+        for (uint32_t i = lane; i < n; i += kWave) {
+            w.ring[ring_index<kRing>(da, s.dp + i)] = from[i];
+        }
+        wave_order();
+        s.dp += n;
+        const uintptr_t a_end = (da + s.dp) & ~(uintptr_t)15;
+        if (a_end > da + s.flushed) {
+            flush_ring(w, s.dst, s.flushed, (uint64_t)(a_end - da), lane);
+            s.flushed = (uint64_t)(a_end - da);
+        }
+        return;
+    }
+    flush_ring(w, s.dst, s.flushed, s.dp, lane);
+    wave_copy_global(s.dst + s.dp, from, n, lane);
+    s.dp += n;
+    s.flushed = s.dp;
+    s.ring_lo = s.dp;
+}
+
+/* n times the byte `fill` at `to`. */
+__device__ __forceinline__ void fill_bytes(gu8* to, uint32_t fill, uint32_t n, uint32_t lane) {
+    const uint32_t word = fill * 0x01010101u;
+    const uint4 v = make_uint4(word, word, word, word);
+    for (uint32_t i = 16 * lane; i + 16 <= n; i += 16 * kWave) {
+        gstore16(to + i, v);
+    }
+    const uint32_t done = n & ~15u;
+    if (lane < n - done) {
+        to[done + lane] = (uint8_t)fill;
+    }
+    wave_order();
+}
+
+/* A batch of cnt sequences, as groups that the ring and the literals' stage
+ * hold; a sequence that fits neither goes global to global. */
+__device__ __forceinline__ void run_sequences(CopyLds& w, CopyState& s, const Job& j, uint32_t cnt,
+                                              uint64_t lp, uint32_t lane) {
+    const uint32_t ll = j.ll[lane], ml = j.ml[lane], off = j.off[lane];
+    for (uint32_t i = 0; i < cnt;) {
+        /* sequence i + lane on this lane */
+        uint32_t gl = ll, gm = ml, go = off;
+        if (i != 0) {
+            gl = (uint32_t)__shfl((int)ll, (int)((i + lane) & (kWave - 1)));
+            gm = (uint32_t)__shfl((int)ml, (int)((i + lane) & (kWave - 1)));
+            go = (uint32_t)__shfl((int)off, (int)((i + lane) & (kWave - 1)));
+        }
+        const bool in = i + lane < cnt;
+        const uint32_t lit = in ? gl : 0, match = in ? gm : 0;
+        const uint32_t lit_incl = wave_inclusive_sum(lit, lane);
+        const uint32_t out_incl = wave_inclusive_sum(lit + match, lane);
+        const uint64_t over = __ballot(!in || lit_incl > kLitStage || out_incl > kBatchMax);
+        const uint32_t take = over == 0 ? kWave : (uint32_t)__builtin_ctzll(over);
+        if (take == 0) {
+            Lz4Step q;
+            q.lit_src = lp;
+            q.lit_dst = s.dp;
+            q.lit_len = uniform32(lit);
+            q.match_dst = s.dp + q.lit_len;
+            q.match_len = uniform32(match);
+            q.offset = uniform32(go);
+            execute_slow(w, s.lit, s.dst, s.cap, q, q.match_dst + q.match_len, s.dp, s.flushed,
+                         s.ring_lo, false, lane);
+            lp += q.lit_len;
+            i++;
+            continue;
+        }
+        const uint32_t lits = uniform32(__builtin_amdgcn_readlane(lit_incl, take - 1));
+        const uint32_t delta = stage_into<1>(w.stage, s.lit, lp + lits, lp, lits, lane);
+        Group g;
+        g.lit = lit_incl - lit;
+        g.lit_len = lit;
+        g.match_len = match;
+        g.offset = go;
+        g.drel = out_incl - (lit + match);
+        g.take = take;
+        g.terminal = false;
+        g.end_rel = uniform32(__builtin_amdgcn_readlane(out_incl, take - 1));
+        execute_group(w, w.cover, w.stage + delta, g, s.dst, s.cap, s.dp, s.flushed, s.ring_lo,
+                      false, lane, Alone{});
+        lp += lits;
+        i += take;
+    }
+}
+
 /* Scratch of one launch: the frame counter, the cost order, a FrameCheck
- * per frame, then a literals slot of kBlockCeiling bytes per wave of the
+ * per frame, then a literals slot of kBlockCeiling bytes per block of the
  * grid. */
 constexpr size_t kCounterBytes = 256;
 
@@ -84,41 +631,138 @@ __global__ void zstd_reset(unsigned long long* counter) {
     }
 }
 
-__global__ void __launch_bounds__(kWave)
+constexpr int kFrameBlock = 2 * kWave;
+__global__ void __launch_bounds__(kFrameBlock) __attribute__((amdgpu_waves_per_eu(4)))
     zstd_batch(const void* const* srcs, const size_t* sizes, void* const* dsts, const size_t* caps,
                size_t n, cudec_chunk_result* results, unsigned long long* counter,
                const uint32_t* order, FrameCheck* checks, uint8_t* lits_base) {
-    __shared__ zstd::FrameTables tables_lds;
-    ZL zstd::FrameTables& tables = *(ZL zstd::FrameTables*)&tables_lds;
-    const Wave w{__lane_id()};
-    ZG uint8_t* lits = (ZG uint8_t*)(lits_base + (size_t)blockIdx.x * zstd::kBlockCeiling);
-    /* The loop body has no lane-conditional region: every lane issues the
-     * atomic (lane 0 adds one, the others zero, so lane 0's old value is
-     * the frame's index whatever order the lanes are applied in) and every
-     * lane stores the same result. A lane-0-only atomic here let the
-     * compiler's structurizer send lanes 1..63 back to the index read
-     * without lane 0, which then read index 0 for ever. */
-    for (;;) {
-        const unsigned long long old = atomicAdd(counter, w.lane == 0 ? 1ull : 0ull);
-        const uint64_t k = uniform64(old);
-        if (k >= n) {
-            break;
+    __shared__ FrameLds l;
+    const uint32_t lane = __lane_id();
+    const bool entropy = uniform32(threadIdx.x / kWave) == 0;
+    if (entropy) {
+        for (uint32_t c = lane; c < kCodes; c += kWave) {
+            const uint32_t m = c - (zstd::kLitLenMax + 1);
+            l.e.code[c] = c <= zstd::kLitLenMax
+                              ? zstd::kLitLenBase[c] | (uint32_t)zstd::kLitLenBits[c] << 24
+                              : zstd::kMatchLenBase[m] | (uint32_t)zstd::kMatchLenBits[m] << 24;
         }
-        const uint64_t i = uniform32(order[k]);
-        const ZG uint8_t* src = (const ZG uint8_t*)uniform_ptr(static_cast<const uint8_t*>(srcs[i]));
-        ZG uint8_t* dst = (ZG uint8_t*)uniform_ptr(static_cast<uint8_t*>(dsts[i]));
-        const uint64_t size = uniform64(sizes[i]);
-        const uint64_t cap = uniform64(caps[i]);
-        zstd::FrameEnd end{0, 0, false};
-        const int st = (int)uniform32((uint32_t)zstd::decode_frame(w, src, size, dst, cap, tables,
-                                                                     lits, end));
-        write_result(results, i, st, st == CUDEC_OK ? uniform64(end.written) : 0);
-        FrameCheck c;
-        c.written = uniform64(end.written);
-        c.checksum = uniform32(end.checksum);
-        c.verify = st == CUDEC_OK && end.has_checksum ? 1u : 0u;
-        checks[i] = c;
-        wave_order();
+        l.published = 0;
+        l.consumed = 0;
+        l.broken = 0;
+    }
+    __syncthreads();
+    if (entropy) {
+        EntropyFlow f{l, lane, 0, true,
+                      Field{l.e.litlen, l.e.code, 0, false},
+                      Field{l.e.offset, nullptr, 0, false},
+                      Field{l.e.matchlen, l.e.code + zstd::kLitLenMax + 1, 0, false},
+                      1, 4, 8};
+        /* every lane issues the atomic (lane 0 adds one, the others zero, so
+         * lane 0's old value is the frame's index whatever order the lanes
+         * are applied in): a lane-0-only branch here let the compiler's
+         * structurizer send lanes 1..63 back to the read without lane 0 */
+        while (f.alive) {
+            const unsigned long long old = atomicAdd(counter, lane == 0 ? 1ull : 0ull);
+            const uint64_t k = uniform64(old);
+            if (k >= n) {
+                break;
+            }
+            const uint64_t i = uniform32(order[k]);
+            const ZG uint8_t* src =
+                (const ZG uint8_t*)uniform_ptr(static_cast<const uint8_t*>(srcs[i]));
+            gu8* dst = global_bytes(dsts[i]);
+            const uint64_t size = uniform64(sizes[i]);
+            const uint64_t cap = uniform64(caps[i]);
+            f.begin(i, dst, cap);
+            zstd::FrameEnd end{0, 0, false};
+            const int st = (int)uniform32((uint32_t)zstd::walk_frame(f, src, size, cap, end));
+            if (st != CUDEC_OK) {
+                f.ask(kJobFail, 0, 0, 0, 0, (uint32_t)st, 0);
+            } else {
+                f.ask(kJobEnd, 0, end.written, 0, 0, end.checksum, end.has_checksum ? 1u : 0u);
+            }
+        }
+        f.ask(kJobQuit, 0, 0, 0, 0, 0, 0);
+        return;
+    }
+    CopyLds& w = l.c;
+    const Wave wave{lane};
+    gu8* lits = (gu8*)(lits_base + (size_t)blockIdx.x * zstd::kBlockCeiling);
+    CopyState s{nullptr, 0, 0, 0, 0, lits};
+    uint64_t chunk = 0;
+    uint32_t huf_log = 0;
+    int status = CUDEC_OK;
+    bool open = false; /* a frame has begun and not ended */
+    for (uint32_t seq = 0;; seq++) {
+        if (await_flag((const lds_flag*)&l.published, seq + 1, nullptr, (lds_flag*)&l.broken) !=
+            kReached) {
+            if (open) {
+                write_result(results, chunk, CUDEC_ERR_CUDA, 0);
+                checks[chunk].verify = 0;
+            }
+            return;
+        }
+        const Job& j = l.job[seq % kJobs];
+        const uint32_t kind = uniform32(j.kind), num = uniform32(j.n), x = uniform32(j.x),
+                       y = uniform32(j.y);
+        const uint64_t a = uniform64(j.a), b = uniform64(j.b), c = uniform64(j.c);
+        if (kind == kJobQuit) {
+            return;
+        }
+        if (kind == kJobFrame) {
+            chunk = a;
+            s = CopyState{(gu8*)(uintptr_t)b, c, 0, 0, 0, lits};
+            huf_log = 0;
+            status = CUDEC_OK;
+            open = true;
+        } else if (kind == kJobFail || kind == kJobEnd) {
+            if (kind == kJobFail && status == CUDEC_OK) {
+                status = (int)x;
+            }
+            if (status == CUDEC_OK) {
+                flush_ring(w, s.dst, s.flushed, s.dp, lane);
+            }
+            write_result(results, chunk, status, status == CUDEC_OK ? a : 0);
+            FrameCheck fc;
+            fc.written = a;
+            fc.checksum = x;
+            fc.verify = status == CUDEC_OK && y != 0 ? 1u : 0u;
+            checks[chunk] = fc;
+            open = false;
+        } else if (status == CUDEC_OK) {
+            if (kind == kJobSequences) {
+                run_sequences(w, s, j, num, c, lane);
+            } else if (kind == kJobTail) {
+                copy_bytes(w, s, s.lit + c, num, lane);
+            } else if (kind == kJobLiterals) {
+                s.lit = (gcu8*)(uintptr_t)a;
+                if (a == 0) {
+                    fill_bytes(lits, x, num, lane);
+                    s.lit = lits;
+                }
+            } else if (kind == kJobHuffman) {
+                s.lit = lits;
+                if (!zstd::decode_huffman_section(wave, (const ZG uint8_t*)(uintptr_t)a, b, num, x,
+                                                  y != 0, *(ZL zstd::HufScratch*)&w.huf,
+                                                  (ZL uint16_t*)w.huffman, huf_log,
+                                                  (ZL uint32_t*)w.stream_bad, (ZL uint8_t*)w.stage,
+                                                  zstd::kWindowBytes, (ZG uint8_t*)lits)) {
+                    status = CUDEC_ERR_CORRUPT_INPUT;
+                }
+                status = (int)uniform32((uint32_t)status);
+                huf_log = uniform32(huf_log);
+                wave_order();
+            } else if (a != 0) { /* kJobBlock */
+                copy_bytes(w, s, (gcu8*)(uintptr_t)a, num, lane);
+            } else {
+                flush_ring(w, s.dst, s.flushed, s.dp, lane);
+                fill_bytes(s.dst + s.dp, x, num, lane);
+                s.dp += num;
+                s.flushed = s.dp;
+                s.ring_lo = s.dp;
+            }
+        }
+        raise_flag((lds_flag*)&l.consumed, seq + 1);
     }
 }
 
@@ -197,15 +841,15 @@ hipError_t launch_zstd(const void* const* srcs, const size_t* sizes, void* const
     if (e != hipSuccess) {
         return e;
     }
-    /* as many one-wave blocks as are resident at once (LDS and registers
-     * decide), on every CU */
+    /* as many blocks as are resident at once (LDS and registers decide), on
+     * every CU */
     int per_cu = 0;
-    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, zstd_batch, kWave, 0);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, zstd_batch, kFrameBlock, 0);
     if (e != hipSuccess) {
         return e;
     }
-    const size_t waves = (size_t)(cus > 0 ? cus : 1) * (size_t)(per_cu > 0 ? per_cu : 1);
-    const size_t grid = n < waves ? n : waves;
+    const size_t blocks = (size_t)(cus > 0 ? cus : 1) * (size_t)(per_cu > 0 ? per_cu : 1);
+    const size_t grid = n < blocks ? n : blocks;
     if (n > UINT32_MAX) {
         return hipErrorInvalidValue; /* the cost order indexes frames in 32 bits */
     }
@@ -236,7 +880,7 @@ hipError_t launch_zstd(const void* const* srcs, const size_t* sizes, void* const
         e = cost_order(sizes, caps, n, order_work, stream, &order);
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(zstd_batch, dim3((unsigned)grid), dim3(kWave), 0, stream, srcs, sizes,
+        hipLaunchKernelGGL(zstd_batch, dim3((unsigned)grid), dim3(kFrameBlock), 0, stream, srcs, sizes,
                            dsts, caps, n, results, counter, order, checks, lits);
         e = hipGetLastError();
     }

@@ -9,14 +9,14 @@
  * survive block boundaries: a Treeless literals section reuses the last
  * Huffman table and a Repeat sequence mode the last FSE table of its field.
  *
- * What runs in parallel is given by the Wave policy (kLanes, lane, sync,
- * uniform: a value every lane holds, as one register for all of them): a
- * wave of 64 lanes on the device, one lane on the host. The serial parts run
- * on every lane with the same values (uniform code); the lane-parallel parts
- * are the four Huffman streams of a literals section, the Huffman table
- * fill, and every byte copy. Lanes exchange results only through memory
- * after a sync(), never through a cross-lane vote, so no convergent
- * operation sits inside the decode's control flow.
+ * walk_frame reads a frame's and its blocks' headers and decides their
+ * verdicts in order; what the sections hold it hands to a Flow. The device
+ * kernel's Flow (zstd.hip) passes literals and copies on to a second wave
+ * and decodes the sequences with the whole wave; the Flow here (DirectFlow)
+ * decodes and executes everything on the spot, one sequence after the other,
+ * as the CPU build does. The Huffman parts, shared by both, take a Wave
+ * policy (kLanes, lane, sync): a wave of 64 lanes on the device, one lane on
+ * the host; their lanes exchange results only through memory after a sync().
  *
  * Accepted frames and verdicts follow the reference's v1 subset
  * (docs/MASTERPLAN.md:1172-1305, tests/zstd_twin_driver.h:178-390): one
@@ -243,8 +243,9 @@ using LaneBits = BackBitsT<PerLane>;
 
 /* A forward little-endian bitstream (FSE table descriptions, RFC 8878
  * 4.1.1): bits from the low end of each byte up. */
+template <class Bytes> /* a byte pointer, global or LDS */
 struct ForwardBits {
-    const ZG uint8_t* p;
+    Bytes p;
     uint64_t size;
     uint64_t byte;
     uint32_t bit;
@@ -280,7 +281,8 @@ struct FseCell {
  * that is truncated, whose accuracy log exceeds log_max, that names a
  * symbol past max_symbol, or whose probabilities do not sum to the table
  * size (tests/zstd_fse_twin.cpp pins these rungs in the reference). */
-ZD bool read_fse_description(const ZG uint8_t* src, uint64_t size, uint32_t max_symbol,
+template <class Bytes>
+ZD bool read_fse_description(Bytes src, uint64_t size, uint32_t max_symbol,
                              uint32_t log_max, ZL int16_t* counts, uint32_t& last_symbol,
                              uint32_t& log, uint64_t& used) {
     if (size == 0) {
@@ -290,7 +292,7 @@ ZD bool read_fse_description(const ZG uint8_t* src, uint64_t size, uint32_t max_
     for (uint32_t s = 0; s < alphabet; s++) {
         counts[s] = 0;
     }
-    ForwardBits in{src, size, 0, 0};
+    ForwardBits<Bytes> in{src, size, 0, 0};
     if (!in.available(4)) {
         return false;
     }
@@ -617,6 +619,64 @@ ZD bool decode_huffman_stream(const ZG uint8_t* src, uint64_t size, const ZL uin
     return in.at_end();
 }
 
+/* A Huffman-coded literals section's payload (RFC 8878 3.1.1.3.1): the tree
+ * description unless treeless (log holds the table of the block before, 0:
+ * none), then one or four streams of `regen` symbols in all, decoded into
+ * lits, one lane a stream. Each stream leaves its verdict in memory and
+ * every lane reads all four after the sync (no cross-lane vote). */
+template <class W>
+ZD bool decode_huffman_section(const W& w, const ZG uint8_t* payload, uint64_t psize,
+                               uint64_t regen, uint32_t streams, bool treeless, ZL HufScratch& s,
+                               ZL uint16_t* table, uint32_t& log, ZL uint32_t* bad,
+                               ZL uint8_t* window, uint32_t window_bytes, ZG uint8_t* lits) {
+    if (!treeless) {
+        uint32_t tree_log = 0;
+        uint64_t tree = 0;
+        if (!read_huffman_table(w, payload, psize, s, table, tree_log, tree)) {
+            return false;
+        }
+        log = tree_log;
+        payload += tree;
+        psize -= tree;
+    } else if (log == 0) {
+        return false; /* treeless with no table */
+    }
+    if (psize == 0) {
+        return false;
+    }
+    for (uint32_t k = w.lane; k < 4; k += W::kLanes) {
+        bad[k] = 0;
+    }
+    w.sync();
+    if (streams == 1) {
+        for (uint32_t k = w.lane; k < 1; k += W::kLanes) {
+            bad[0] = decode_huffman_stream(payload, psize, table, log, lits, regen, window,
+                                           window_bytes) ? 0u : 1u;
+        }
+    } else {
+        if (psize < 10 || regen < 6) {
+            return false;
+        }
+        const uint64_t s0 = read_le(payload, 2), s1 = read_le(payload + 2, 2),
+                       s2 = read_le(payload + 4, 2);
+        const uint64_t bytes = psize - 6;
+        if (s0 + s1 + s2 >= bytes) {
+            return false;
+        }
+        const uint64_t seg = (regen + 3) / 4;
+        for (uint32_t k = w.lane; k < 4; k += W::kLanes) {
+            const uint64_t from = 6 + (k > 0 ? s0 : 0) + (k > 1 ? s1 : 0) + (k > 2 ? s2 : 0);
+            const uint64_t len = k == 0 ? s0 : k == 1 ? s1 : k == 2 ? s2 : bytes - s0 - s1 - s2;
+            const uint64_t n = k < 3 ? seg : regen - 3 * seg;
+            bad[k] = decode_huffman_stream(payload + from, len, table, log, lits + k * seg, n,
+                                           window + k * (window_bytes / 4), window_bytes / 4)
+                         ? 0u : 1u;
+        }
+    }
+    w.sync();
+    return (bad[0] | bad[1] | bad[2] | bad[3]) == 0;
+}
+
 /* ------------------------------------------------------------- sequences */
 
 struct SeqTable {
@@ -625,18 +685,14 @@ struct SeqTable {
     bool present;
 };
 
-/* Up to kBatch decoded and checked sequences of a block are executed
- * together. One sequence's record: distance, literal length, match length,
- * where its literals start in the block's literals, and where its output
- * starts relative to the batch's first output byte. The Wave policy keeps
- * the records (W::Records: put(lane, k, rec), get(k) for every lane,
- * own(lane, k) for the lane that holds record k): on the device lane k
- * holds record k in registers. */
+/* The kernel decodes and checks kBatch sequences before it executes them,
+ * a lane each. */
 constexpr uint32_t kBatch = 64;
 /* A batch's bitstream is at most 64 x (31 + 16 + 16 extra bits + 9 + 9 + 8
  * state bits) = 712 bytes, so a window of this size staged at a batch's
  * start holds every byte its refills read. */
 constexpr uint32_t kWindowBytes = 1024;
+/* One sequence's record, for a policy that holds a batch of them. */
 struct Rec {
     uint64_t d;
     uint32_t ll, ml, lit, at;
@@ -798,177 +854,31 @@ struct FrameEnd {
     bool has_checksum;
 };
 
-/* Copies n literal bytes to out[0, n): from `lit` (raw or decoded), or the
- * byte `fill` when lit is null (a run-length section). */
-template <class W>
-ZD void put_literals(const W& w, ZG uint8_t* out, const ZG uint8_t* lit, uint8_t fill,
-                     uint64_t n) {
-    if (lit != nullptr) {
-        for (uint64_t i = w.lane; i < n; i += W::kLanes) {
-            out[i] = lit[i];
-        }
-    } else {
-        for (uint64_t i = w.lane; i < n; i += W::kLanes) {
-            out[i] = fill;
-        }
-    }
-    w.sync();
-}
-
-/* out[at + i] = out[at - d + (i mod d)] for i < n: every source byte lies
- * before `at`, so lanes need no order among themselves. */
-template <class W>
-ZD void put_match(const W& w, ZG uint8_t* out, uint64_t at, uint64_t d, uint64_t n) {
-    const ZG uint8_t* from = out + at - d;
-    if (d <= 0xFFFFFFFFull && n <= 0xFFFFFFFFull) {
-        const uint32_t d32 = (uint32_t)d;
-        for (uint32_t i = w.lane; i < (uint32_t)n; i += W::kLanes) {
-            out[at + i] = from[i % d32];
-        }
-    } else {
-        for (uint64_t i = w.lane; i < n; i += W::kLanes) {
-            out[at + i] = from[i % d];
-        }
-    }
-    w.sync();
-}
-
-/* The wave copies stream bytes [pos - cap, pos) (from 0 when pos < cap)
- * into buf, and the reader reads from there: a sequence batch's bits in one
- * round trip. */
-template <class W>
-ZD void stage_wave(const W& w, BackBitsT<typename W::Same>& in, ZL uint8_t* buf, uint32_t cap) {
-    const uint64_t lo = in.pos > cap ? in.pos - cap : 0;
-    const uint32_t len = (uint32_t)(in.pos - lo);
-    for (uint32_t i = w.lane * 16; i < len; i += W::kLanes * 16) {
-        if (i + 16 <= len) {
-            uint8_t v[16];
-            __builtin_memcpy(v, (const void*)(in.p + lo + i), 16);
-            for (uint32_t j = 0; j < 16; j++) {
-                buf[i + j] = v[j];
-            }
-        } else {
-            for (uint32_t j = i; j < len; j++) {
-                buf[j] = in.p[lo + j];
-            }
-        }
-    }
-    w.sync();
-    in.win = buf;
-    in.win_lo = lo;
-    in.win_hi = in.pos;
-}
-
-/* An FSE cell as one 32-bit load, made wave-uniform. */
-template <class W>
-ZD FseCell load_cell(const W& w, const ZL FseCell* cells, uint32_t state) {
-    const FseCell raw = cells[state];
-    uint32_t v;
-    __builtin_memcpy(&v, &raw, 4);
-    v = w.uniform(v);
-    FseCell c;
-    __builtin_memcpy(&c, &v, 4);
-    return c;
-}
-
-/* n bytes from src to dst on one lane: 16-byte steps, then single bytes
- * (never past dst + n: the bytes after belong to other lanes). */
-ZD void lane_copy(ZG uint8_t* dst, const ZG uint8_t* src, uint32_t n) {
-    uint32_t i = 0;
-    for (; i + 16 <= n; i += 16) {
-        uint8_t v[16];
-        __builtin_memcpy(v, (const void*)(src + i), 16);
-        __builtin_memcpy((void*)(dst + i), v, 16);
-    }
-    for (; i < n; i++) {
-        dst[i] = src[i];
-    }
-}
-
-/* Literals and matches a single lane takes alone. */
-constexpr uint32_t kLaneBytes = 64;
-
-/* Executes a batch of cnt sequences whose output starts at out[bo]:
- *   1. one lane a sequence: literals of up to kLaneBytes, and matches of up
- *      to kLaneBytes whose source period lies wholly before the batch (so
- *      already written): neither reads anything the batch writes;
- *   2. the wave, sequence by sequence: longer literals, and longer matches
- *      whose period lies before the batch;
- *   3. the wave, in sequence order: every other match, whose source may be
- *      the output of an earlier sequence of the batch (all of which steps 1
- *      and 2 wrote, or step 3 wrote before it).
- * A match's bytes depend only on bytes before its own start, so this order
- * writes what sequence-by-sequence execution writes. */
-template <class W>
-ZD void execute_batch(const W& w, ZG uint8_t* out, uint64_t bo, const ZG uint8_t* lit,
-                      uint8_t fill, const typename W::Records& recs, uint32_t cnt) {
-    ZG uint8_t* base = out + bo;
-    for (uint32_t k = w.lane; k < cnt; k += W::kLanes) {
-        const Rec r = recs.own(w.lane, k);
-        if (r.ll <= kLaneBytes) {
-            if (lit != nullptr) {
-                lane_copy(base + r.at, lit + r.lit, r.ll);
-            } else {
-                for (uint32_t i = 0; i < r.ll; i++) {
-                    base[r.at + i] = fill;
-                }
-            }
-        }
-        const uint64_t m = (uint64_t)r.at + r.ll;
-        const uint64_t span = r.d < r.ml ? r.d : r.ml;
-        if (r.ml <= kLaneBytes && r.d >= m + span) {
-            const ZG uint8_t* from = base + m - r.d; /* before the batch: d <= bo + m */
-            if (r.d >= r.ml) {
-                lane_copy(base + m, from, r.ml);
-            } else {
-                for (uint32_t i = 0; i < r.ml; i++) {
-                    base[m + i] = from[i % (uint32_t)r.d];
-                }
-            }
-        }
-    }
-    w.sync();
-    for (uint32_t k = 0; k < cnt; k++) {
-        const Rec r = recs.get(k);
-        if (r.ll > kLaneBytes) {
-            put_literals(w, base + r.at, lit != nullptr ? lit + r.lit : nullptr, fill, r.ll);
-        }
-        const uint64_t m = (uint64_t)r.at + r.ll;
-        const uint64_t span = r.d < r.ml ? r.d : r.ml;
-        if (r.ml > kLaneBytes && r.d >= m + span) {
-            put_match(w, out, bo + m, r.d, r.ml);
-        }
-    }
-    for (uint32_t k = 0; k < cnt; k++) {
-        const Rec r = recs.get(k);
-        const uint64_t m = (uint64_t)r.at + r.ll;
-        const uint64_t span = r.d < r.ml ? r.d : r.ml;
-        if (r.d < m + span) {
-            put_match(w, out, bo + m, r.d, r.ml);
-        }
-    }
-}
-
-/* Decodes one frame of `size` bytes into out[0, cap). `lits` is scratch of
- * kBlockCeiling bytes for Huffman-coded literals. Returns the status; on
- * CUDEC_OK `end` says how much was written and which checksum the output
- * must have. */
-template <class W>
-ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t* out,
-                    uint64_t cap, ZL FrameTables& t, ZG uint8_t* lits, FrameEnd& end) {
+/* Reads one frame's headers (RFC 8878 3.1.1) and takes its content through
+ * flow `f`, in stream order. Returns the frame's status; on CUDEC_OK `end`
+ * says how much was written and which checksum the output must have. A flow
+ * that decides a section later than it is handed on (returning true at once)
+ * must itself see to it that the first error in stream order wins. It has
+ *   block(from, fill, n): n output bytes, a copy or (from null) a fill;
+ *   literals(from, fill, n): the block's literals, likewise;
+ *   huffman(payload, size, regen, streams, treeless): the block's literals;
+ *   sequences(...): the block's sequences, advancing lp (literals consumed)
+ *     and o (output position), with the status of the section;
+ *   tail(lp, n): the literals after the last sequence;
+ *   u64(v): a value every lane holds, as one. */
+template <class Flow>
+ZD int walk_frame(Flow& f, const ZG uint8_t* src, uint64_t size, uint64_t cap, FrameEnd& end) {
     FrameHeader h;
-    int st = parse_frame_header(src, size, h);
+    const int st = parse_frame_header(src, size, h);
     if (st != CUDEC_OK) {
         return st;
     }
+    h.content_size = f.u64(h.content_size);
+    h.window = f.u64(h.window);
     if (h.content_size > cap) {
         return CUDEC_ERR_OUTPUT_TOO_SMALL;
     }
     const uint64_t block_max = h.window < kBlockCeiling ? h.window : kBlockCeiling;
-    SeqTable ll{t.litlen, 0, false}, of{t.offset, 0, false}, ml{t.matchlen, 0, false};
-    uint32_t huf_log = 0; /* 0: no Huffman table yet */
-    Repeats rep;
-    rep.reset();
     uint64_t pos = h.header_size;
     uint64_t o = 0; /* bytes written */
     for (;;) {
@@ -976,7 +886,7 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
         if (size - pos < 3) {
             return CUDEC_ERR_CORRUPT_INPUT;
         }
-        const uint32_t bh = (uint32_t)read_le(src + pos, 3);
+        const uint32_t bh = (uint32_t)f.u64(read_le(src + pos, 3));
         const bool last_block = (bh & 1u) != 0;
         const uint32_t type = (bh >> 1) & 3u;
         const uint32_t bsize = bh >> 3;
@@ -992,15 +902,16 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
             if (bsize > cap - o) {
                 return CUDEC_ERR_OUTPUT_TOO_SMALL;
             }
-            put_literals(w, out + o, type == 0 ? body : nullptr, type == 1 ? body[0] : 0, bsize);
+            f.block(type == 0 ? body : nullptr, type == 1 ? body[0] : (uint8_t)0, bsize);
             o += bsize;
         } else {
             /* literals section (RFC 8878 3.1.1.3.1) */
             if (body_size == 0) {
                 return CUDEC_ERR_CORRUPT_INPUT;
             }
-            const uint32_t ltype = body[0] & 3u;
-            const uint32_t sf = (body[0] >> 2) & 3u;
+            const uint64_t head = f.u64(read_le(body, body_size < 5 ? body_size : 5));
+            const uint32_t ltype = (uint32_t)head & 3u;
+            const uint32_t sf = (uint32_t)(head >> 2) & 3u;
             uint32_t lh = 0;
             uint64_t regen = 0, csize = 0;
             uint32_t streams = 0;
@@ -1009,14 +920,14 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
                 if (body_size < lh) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                regen = read_le(body, lh) >> (lh == 1 ? 3 : 4);
+                regen = (head & ((1ull << (8 * lh)) - 1)) >> (lh == 1 ? 3 : 4);
             } else {
                 lh = sf <= 1 ? 3u : sf == 2 ? 4u : 5u;
                 const uint32_t fb = sf <= 1 ? 10u : sf == 2 ? 14u : 18u;
                 if (body_size < lh) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                const uint64_t raw = read_le(body, lh);
+                const uint64_t raw = head & ((1ull << (8 * lh)) - 1);
                 regen = (raw >> 4) & ((1ull << fb) - 1);
                 csize = (raw >> (4 + fb)) & ((1ull << fb) - 1);
                 streams = sf == 0 ? 1u : 4u;
@@ -1025,80 +936,26 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
                 return CUDEC_ERR_CORRUPT_INPUT;
             }
             const uint64_t after = body_size - lh;
-            const ZG uint8_t* lit = nullptr; /* null: run-length literals */
-            uint8_t fill = 0;
             uint64_t lused = 0;
             if (ltype == 0) {
                 if (regen > after) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                lit = body + lh;
+                f.literals(body + lh, (uint8_t)0, regen);
                 lused = lh + regen;
             } else if (ltype == 1) {
                 if (after < 1) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                fill = body[lh];
+                f.literals(nullptr, body[lh], regen);
                 lused = lh + 1;
             } else {
                 if (csize > after) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                const ZG uint8_t* payload = body + lh;
-                uint64_t psize = csize;
-                if (ltype == 2) {
-                    uint32_t log = 0;
-                    uint64_t tree = 0;
-                    if (!read_huffman_table(w, payload, psize, t.huf, t.huffman, log, tree)) {
-                        return CUDEC_ERR_CORRUPT_INPUT;
-                    }
-                    huf_log = log;
-                    payload += tree;
-                    psize -= tree;
-                } else if (huf_log == 0) {
-                    return CUDEC_ERR_CORRUPT_INPUT; /* treeless with no table */
-                }
-                if (psize == 0) {
+                if (!f.huffman(body + lh, csize, regen, streams, ltype == 3)) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                /* one lane a stream; each leaves its verdict in LDS and every
-                 * lane reads all four after the sync (no cross-lane vote) */
-                for (uint32_t s = w.lane; s < 4; s += W::kLanes) {
-                    t.stream_bad[s] = 0;
-                }
-                w.sync();
-                if (streams == 1) {
-                    for (uint32_t s = w.lane; s < 1; s += W::kLanes) {
-                        t.stream_bad[0] = decode_huffman_stream(payload, psize, t.huffman, huf_log,
-                                                                lits, regen, t.window,
-                                                                kWindowBytes) ? 0u : 1u;
-                    }
-                } else {
-                    if (psize < 10 || regen < 6) {
-                        return CUDEC_ERR_CORRUPT_INPUT;
-                    }
-                    const uint64_t s0 = read_le(payload, 2), s1 = read_le(payload + 2, 2),
-                                   s2 = read_le(payload + 4, 2);
-                    const uint64_t bytes = psize - 6;
-                    if (s0 + s1 + s2 >= bytes) {
-                        return CUDEC_ERR_CORRUPT_INPUT;
-                    }
-                    const uint64_t seg = (regen + 3) / 4;
-                    for (uint32_t s = w.lane; s < 4; s += W::kLanes) {
-                        const uint64_t from = 6 + (s > 0 ? s0 : 0) + (s > 1 ? s1 : 0) + (s > 2 ? s2 : 0);
-                        const uint64_t len = s == 0 ? s0 : s == 1 ? s1 : s == 2 ? s2 : bytes - s0 - s1 - s2;
-                        const uint64_t n = s < 3 ? seg : regen - 3 * seg;
-                        t.stream_bad[s] = decode_huffman_stream(
-                                              payload + from, len, t.huffman, huf_log,
-                                              lits + s * seg, n, t.window + s * (kWindowBytes / 4),
-                                              kWindowBytes / 4) ? 0u : 1u;
-                    }
-                }
-                w.sync();
-                if ((t.stream_bad[0] | t.stream_bad[1] | t.stream_bad[2] | t.stream_bad[3]) != 0) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                lit = lits;
                 lused = lh + csize;
             }
 
@@ -1108,20 +965,21 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
             if (left == 0) {
                 return CUDEC_ERR_CORRUPT_INPUT;
             }
-            uint32_t count = sec[0];
+            const uint64_t sh = f.u64(read_le(sec, left < 4 ? (uint32_t)left : 4));
+            uint32_t count = (uint32_t)sh & 255u;
             uint32_t cb = 1;
             if (count >= 128) {
                 if (count < 255) {
                     if (left < 2) {
                         return CUDEC_ERR_CORRUPT_INPUT;
                     }
-                    count = ((count - 128) << 8) + sec[1];
+                    count = ((count - 128) << 8) + ((uint32_t)(sh >> 8) & 255u);
                     cb = 2;
                 } else {
                     if (left < 3) {
                         return CUDEC_ERR_CORRUPT_INPUT;
                     }
-                    count = sec[1] + ((uint32_t)sec[2] << 8) + 0x7F00u;
+                    count = ((uint32_t)(sh >> 8) & 0xFFFFu) + 0x7F00u;
                     cb = 3;
                 }
             }
@@ -1133,130 +991,21 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
                 if (left <= cb) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                const uint32_t modes = sec[cb];
+                const uint32_t modes = (uint32_t)(sh >> (8 * cb)) & 255u;
                 if ((modes & 3u) != 0) {
                     return CUDEC_ERR_CORRUPT_INPUT;
                 }
-                sec += cb + 1;
-                left -= cb + 1;
-                uint64_t u = 0;
-                if (!load_seq_table(w, modes >> 6, sec, left, kLitLenMax, kLitLenLog, kLitLenDefault,
-                                    35, 6, ll, t.counts, t.next, u)) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                sec += u;
-                left -= u;
-                if (!load_seq_table(w, (modes >> 4) & 3u, sec, left, kOffsetMax, kOffsetLog,
-                                    kOffsetDefault, 28, 5, of, t.counts, t.next, u)) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                sec += u;
-                left -= u;
-                if (!load_seq_table(w, (modes >> 2) & 3u, sec, left, kMatchLenMax, kMatchLenLog,
-                                    kMatchLenDefault, 52, 6, ml, t.counts, t.next, u)) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                sec += u;
-                left -= u;
-
-                /* the sequences (RFC 8878 3.1.1.3.2.2 and 4.1) */
-                BackBitsT<typename W::Same> in;
-                if (left == 0 || !in.start(sec, left)) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                stage_wave(w, in, t.window, kWindowBytes);
-                uint32_t sl = 0, so = 0, sm = 0;
-                if (!in.read(ll.log, sl) || !in.read(of.log, so) || !in.read(ml.log, sm)) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                const uint32_t nl = 1u << ll.log, no = 1u << of.log, nm = 1u << ml.log;
-                int pending = CUDEC_OK; /* the first execution error, reported
-                                           once the whole block decodes */
-                typename W::Records recs;
-                uint32_t cnt = 0;     /* sequences in the batch */
-                uint64_t bo = o;      /* the batch's first output byte */
-                for (uint32_t k = 0; k < count; k++) {
-                    if (k != 0 && (k & (kBatch - 1)) == 0) {
-                        stage_wave(w, in, t.window, kWindowBytes);
-                    }
-                    if (sl >= nl || so >= no || sm >= nm) {
-                        return CUDEC_ERR_CORRUPT_INPUT;
-                    }
-                    const FseCell cl = load_cell(w, ll.cells, sl), co = load_cell(w, of.cells, so),
-                                  cm = load_cell(w, ml.cells, sm);
-                    if (cl.symbol > kLitLenMax || co.symbol > kOffsetMax || cm.symbol > kMatchLenMax) {
-                        return CUDEC_ERR_CORRUPT_INPUT;
-                    }
-                    uint32_t eo = 0, em = 0, el = 0;
-                    if (!in.read(co.symbol, eo) || !in.read(kMatchLenBits[cm.symbol], em) ||
-                        !in.read(kLitLenBits[cl.symbol], el)) {
-                        return CUDEC_ERR_CORRUPT_INPUT;
-                    }
-                    const uint64_t value = (1ull << co.symbol) + eo;
-                    const uint32_t mlen = kMatchLenBase[cm.symbol] + em;
-                    const uint32_t llen = kLitLenBase[cl.symbol] + el;
-                    if (k + 1 < count) {
-                        uint32_t v = 0;
-                        if (!in.read(cl.bits, v)) {
-                            return CUDEC_ERR_CORRUPT_INPUT;
-                        }
-                        sl = cl.base + v;
-                        if (!in.read(cm.bits, v)) {
-                            return CUDEC_ERR_CORRUPT_INPUT;
-                        }
-                        sm = cm.base + v;
-                        if (!in.read(co.bits, v)) {
-                            return CUDEC_ERR_CORRUPT_INPUT;
-                        }
-                        so = co.base + v;
-                    }
-                    if (pending != CUDEC_OK) {
-                        continue;
-                    }
-                    /* execute: literals, repeat offset, window, capacity */
-                    if (llen > regen - lp) {
-                        pending = CUDEC_ERR_CORRUPT_INPUT;
-                        continue;
-                    }
-                    const uint64_t d = rep.resolve(value, llen);
-                    const uint64_t m = o + llen;
-                    if (d == 0 || d > m || d > h.window) {
-                        pending = CUDEC_ERR_CORRUPT_INPUT;
-                        continue;
-                    }
-                    if (m > cap || mlen > cap - m) {
-                        pending = CUDEC_ERR_OUTPUT_TOO_SMALL;
-                        continue;
-                    }
-                    recs.put(w.lane, cnt, Rec{d, llen, mlen, (uint32_t)lp, (uint32_t)(o - bo)});
-                    cnt++;
-                    lp += llen;
-                    o = m + mlen;
-                    if (cnt == kBatch) {
-                        w.sync();
-                        execute_batch(w, out, bo, lit, fill, recs, cnt);
-                        w.sync();
-                        cnt = 0;
-                        bo = o;
-                    }
-                }
-                if (!in.at_end()) {
-                    return CUDEC_ERR_CORRUPT_INPUT;
-                }
-                if (pending != CUDEC_OK) {
-                    return pending;
-                }
-                if (cnt != 0) {
-                    w.sync();
-                    execute_batch(w, out, bo, lit, fill, recs, cnt);
-                    w.sync();
+                const int sst = f.sequences(sec + cb + 1, left - cb - 1, modes, count, regen,
+                                            h.window, cap, lp, o);
+                if (sst != CUDEC_OK) {
+                    return sst;
                 }
             }
             /* the literals after the last sequence */
             if (regen - lp > cap - o) {
                 return CUDEC_ERR_OUTPUT_TOO_SMALL;
             }
-            put_literals(w, out + o, lit != nullptr ? lit + lp : nullptr, fill, regen - lp);
+            f.tail(lp, regen - lp);
             o += regen - lp;
         }
         pos += 3 + body_size;
@@ -1273,7 +1022,7 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
         if (size - pos < 4) {
             return CUDEC_ERR_CORRUPT_INPUT;
         }
-        end.checksum = (uint32_t)read_le(src + pos, 4);
+        end.checksum = (uint32_t)f.u64(read_le(src + pos, 4));
         pos += 4;
     }
     if (pos != size) {
@@ -1282,6 +1031,153 @@ ZD int decode_frame(const W& w, const ZG uint8_t* src, uint64_t size, ZG uint8_t
     end.written = o;
     return CUDEC_OK;
 }
+
+/* ------------------------------------------------------------ direct flow */
+
+#if !defined(__HIP_DEVICE_COMPILE__)
+
+/* Decodes and executes every section where walk_frame hands it on: the
+ * plain form of the frame decode, one sequence after the other, for the CPU
+ * build. */
+template <class W>
+struct DirectFlow {
+    const W& w;
+    uint8_t* out;
+    FrameTables& t;
+    uint8_t* lits;
+    SeqTable ll, of, ml;
+    uint32_t huf_log; /* 0: no Huffman table yet */
+    Repeats rep;
+    const uint8_t* lit; /* the block's literals; null: the byte `fill_byte` */
+    uint8_t fill_byte;
+    uint64_t at; /* output position */
+
+    DirectFlow(const W& wave, uint8_t* o, FrameTables& tables, uint8_t* scratch)
+        : w(wave), out(o), t(tables), lits(scratch), ll{tables.litlen, 0, false},
+          of{tables.offset, 0, false}, ml{tables.matchlen, 0, false}, huf_log(0), lit(nullptr),
+          fill_byte(0), at(0) {
+        rep.reset();
+    }
+    uint64_t u64(uint64_t v) const { return v; }
+    void put(const uint8_t* from, uint8_t fill, uint64_t n) {
+        for (uint64_t i = 0; i < n; i++) {
+            out[at + i] = from != nullptr ? from[i] : fill;
+        }
+        at += n;
+    }
+    void block(const uint8_t* from, uint8_t fill, uint64_t n) { put(from, fill, n); }
+    void literals(const uint8_t* from, uint8_t fill, uint64_t) {
+        lit = from;
+        fill_byte = fill;
+    }
+    bool huffman(const uint8_t* payload, uint64_t size, uint64_t regen, uint32_t streams,
+                 bool treeless) {
+        lit = lits;
+        return decode_huffman_section(w, payload, size, regen, streams, treeless, t.huf, t.huffman,
+                                      huf_log, t.stream_bad, t.window, kWindowBytes, lits);
+    }
+    void tail(uint64_t lp, uint64_t n) { put(lit != nullptr ? lit + lp : nullptr, fill_byte, n); }
+    int sequences(const uint8_t* sec, uint64_t left, uint32_t modes, uint32_t count,
+                  uint64_t regen, uint64_t window, uint64_t cap, uint64_t& lp, uint64_t& o) {
+        uint64_t u = 0;
+        if (!load_seq_table(w, modes >> 6, sec, left, kLitLenMax, kLitLenLog, kLitLenDefault, 35,
+                            6, ll, t.counts, t.next, u)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        sec += u;
+        left -= u;
+        if (!load_seq_table(w, (modes >> 4) & 3u, sec, left, kOffsetMax, kOffsetLog,
+                            kOffsetDefault, 28, 5, of, t.counts, t.next, u)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        sec += u;
+        left -= u;
+        if (!load_seq_table(w, (modes >> 2) & 3u, sec, left, kMatchLenMax, kMatchLenLog,
+                            kMatchLenDefault, 52, 6, ml, t.counts, t.next, u)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        sec += u;
+        left -= u;
+
+        /* the sequences (RFC 8878 3.1.1.3.2.2 and 4.1) */
+        LaneBits in;
+        if (left == 0 || !in.start(sec, left)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        uint32_t sl = 0, so = 0, sm = 0;
+        if (!in.read(ll.log, sl) || !in.read(of.log, so) || !in.read(ml.log, sm)) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        int pending = CUDEC_OK; /* the first execution error, reported
+                                   once the whole block decodes */
+        for (uint32_t k = 0; k < count; k++) {
+            const FseCell cl = ll.cells[sl], co = of.cells[so], cm = ml.cells[sm];
+            uint32_t eo = 0, em = 0, el = 0;
+            if (!in.read(co.symbol, eo) || !in.read(kMatchLenBits[cm.symbol], em) ||
+                !in.read(kLitLenBits[cl.symbol], el)) {
+                return CUDEC_ERR_CORRUPT_INPUT;
+            }
+            const uint64_t value = (1ull << co.symbol) + eo;
+            const uint32_t mlen = kMatchLenBase[cm.symbol] + em;
+            const uint32_t llen = kLitLenBase[cl.symbol] + el;
+            if (k + 1 < count) {
+                uint32_t v = 0;
+                if (!in.read(cl.bits, v)) {
+                    return CUDEC_ERR_CORRUPT_INPUT;
+                }
+                sl = cl.base + v;
+                if (!in.read(cm.bits, v)) {
+                    return CUDEC_ERR_CORRUPT_INPUT;
+                }
+                sm = cm.base + v;
+                if (!in.read(co.bits, v)) {
+                    return CUDEC_ERR_CORRUPT_INPUT;
+                }
+                so = co.base + v;
+            }
+            if (pending != CUDEC_OK) {
+                continue;
+            }
+            /* execute: literals, repeat offset, window, capacity */
+            if (llen > regen - lp) {
+                pending = CUDEC_ERR_CORRUPT_INPUT;
+                continue;
+            }
+            const uint64_t d = rep.resolve(value, llen);
+            const uint64_t m = o + llen;
+            if (d == 0 || d > m || d > window) {
+                pending = CUDEC_ERR_CORRUPT_INPUT;
+                continue;
+            }
+            if (m > cap || mlen > cap - m) {
+                pending = CUDEC_ERR_OUTPUT_TOO_SMALL;
+                continue;
+            }
+            put(lit != nullptr ? lit + lp : nullptr, fill_byte, llen);
+            for (uint32_t i = 0; i < mlen; i++) {
+                out[m + i] = out[m + i - d];
+            }
+            at += mlen;
+            lp += llen;
+            o = m + mlen;
+        }
+        if (!in.at_end()) {
+            return CUDEC_ERR_CORRUPT_INPUT;
+        }
+        return pending;
+    }
+};
+
+/* Decodes one frame of `size` bytes into out[0, cap). `lits` is scratch of
+ * kBlockCeiling bytes for Huffman-coded literals. */
+template <class W>
+inline int decode_frame(const W& w, const uint8_t* src, uint64_t size, uint8_t* out, uint64_t cap,
+                        FrameTables& t, uint8_t* lits, FrameEnd& end) {
+    DirectFlow<W> f(w, out, t, lits);
+    return walk_frame(f, src, size, cap, end);
+}
+
+#endif
 
 }  // namespace zstd
 }  // namespace cudec_amd
