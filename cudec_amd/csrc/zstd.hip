@@ -11,17 +11,22 @@
  * other beyond the slots, so a frame's time is the longer of the two.
  *
  * What bounds it is the FSE chain: a sequence's three states give the bits
- * that give the next states. The entropy wave spends a lane on each of the
- * three fields (every quad of lanes does the same): one LDS read takes the
- * three cells, sums over the quad place each lane's bits, and two reads of
- * the staged bitstream give its extra bits and its next state, two LDS round
- * trips and about 45 instructions a sequence. Everything that does not feed
- * the next state (code baselines, repeat offsets, limits, positions) is done
- * per 64 sequences, a lane each. Measured alone, a sequence costs 390 cycles
- * of FSE chain, 208 of finishing and 211 of copies on the other wave. One
- * wave a frame with one sequence decoded and executed after the other took
- * 13.72 ms for 4096 frames of 64 KiB and 284 ms for 20 000 uneven frames;
- * this takes 6.27 and 78.9 ms.
+ * that give the next states. The entropy wave spends two lanes on each of the
+ * three fields, one on the next state and one on the extra bits: sums over a
+ * quad say where each lane's bits end, a shift of the 64 stream bits on top
+ * (read while the sums are made) gives them, and one LDS read the next cell,
+ * about 45 instructions and 287 cycles a sequence. (Bits read from LDS where
+ * the sums say took a second round trip and 388 cycles; every lane keeping
+ * the 128 bits on top and choosing words of them, 62 instructions and 338.)
+ * Everything that does not feed the next state (code baselines, repeat
+ * offsets, limits, positions) is done per 64 sequences, a lane each: 37
+ * cycles a sequence, the repeat offsets as a scan over maps (one after the
+ * other on the scalar unit they took 190). The copies on the other wave take
+ * about 200.
+ *
+ * One wave a frame with one sequence decoded and executed after the other
+ * took 13.72 ms for 8192 frames of 64 KiB and 284 ms for 2000 frames of
+ * 1 KiB to 4 MiB; this takes 4.94 and 56.0 ms.
  *
  * The first error in stream order decides a frame: the entropy wave's
  * verdicts travel as jobs, behind the literals that precede them.
@@ -30,6 +35,7 @@
  * lanes a frame (xxhash.h), over every frame that decoded and carries one:
  * one frame's XXH64 is a serial chain of stripes, so frames in parallel is
  * what fills the device. */
+#include <cstddef>
 #include <mutex>
 
 #include "common.h"
@@ -82,9 +88,11 @@ struct alignas(16) Job {
 };
 static_assert(sizeof(Job) % 16 == 0, "slots keep their alignment");
 
-/* An FSE cell of a sequence field in one word: symbol (6 bits), state bits
- * (4), extra bits of the symbol's code (5), next-state base (16). */
-constexpr uint32_t kCellBits = 6, kCellExtra = 10, kCellBase = 16;
+/* An FSE cell of a sequence field in one word: extra bits of the symbol's
+ * code (a byte), state bits (a byte, so that a quad's cells add up to a sum
+ * of each: at most 63 and 26), symbol (6 bits), next-state base. */
+constexpr uint32_t kCellBits = 8, kCellSymbol = 16, kCellBase = 22;
+constexpr uint32_t kCellSums = 0xFFFF, kCellExtras = 0xFF;
 constexpr uint32_t kCodes = (zstd::kLitLenMax + 1) + (zstd::kMatchLenMax + 1);
 
 /* Staged bitstream of one batch: at most 712 bytes (zstd::kWindowBytes). */
@@ -100,6 +108,7 @@ struct alignas(16) EntropyLds {
 constexpr uint32_t kHeaderStage = 512; /* of the window: table descriptions */
 static_assert(kHeaderStage + (1u << zstd::kLitLenLog) <= zstd::kWindowBytes,
               "a field's symbol order lies behind the descriptions");
+static_assert(offsetof(EntropyLds, window) >= 712 + 16, "what words_below may read");
 static_assert(zstd::kBatch == kWave, "a batch holds a sequence a lane");
 
 struct alignas(16) CopyLds : RingLds<kRing> {
@@ -117,6 +126,7 @@ struct alignas(16) FrameLds {
     Job job[kJobs];
     uint32_t published; /* jobs written */
     uint32_t consumed;  /* jobs done */
+    uint32_t unused;
     uint32_t broken;    /* a wait ran out, and no wave waits any more */
 };
 static_assert(sizeof(FrameLds) <= 20480, "eight blocks share a CU's 160 KiB");
@@ -129,20 +139,46 @@ __device__ __forceinline__ uint32_t lds_at(const T* p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const T*)p;
 }
 
-/* Lane `from` of every quad, on its whole quad. */
+/* Lane kFrom of every quad, on its whole quad. */
 template <uint32_t kFrom>
 __device__ __forceinline__ uint32_t quad(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kFrom * 0x55, 0xF, 0xF, true);
 }
 
-/* n (0..31) bits of the staged stream from window bit `at` on, in stream
- * order lowest first. A position before the window (a stream that ran out:
- * its batch is refused) reads the window's start. */
-__device__ __forceinline__ uint32_t window_bits(uint32_t window, int at, uint32_t n) {
-    const uint32_t p = at < 0 ? 0u : (uint32_t)at;
-    const uint32_t a = window + ((p >> 5) << 2);
-    const uint32_t lo = *(lds_u32*)(uintptr_t)a, hi = *(lds_u32*)(uintptr_t)(a + 4);
-    return __builtin_amdgcn_ubfe(__builtin_amdgcn_alignbit(hi, lo, p & 31), 0, n);
+/* The 128 bits of the staged stream up to the 32-bit word that holds window
+ * bit `at` - 1. A stream that ran out (its batch is refused) reads what lies
+ * before the window: a batch takes at most 712 bytes, and the tables before
+ * it are larger. */
+struct Words {
+    uint32_t w0, w1, w2, w3;
+    int first; /* window bit of w0's lowest */
+};
+__device__ __forceinline__ Words words_below(uint32_t window, int at) {
+    const int word = (at - 1) >> 5;
+    const uint32_t a = window + (uint32_t)(4 * word);
+    return Words{*(lds_u32*)(uintptr_t)(a - 12), *(lds_u32*)(uintptr_t)(a - 8),
+                 *(lds_u32*)(uintptr_t)(a - 4), *(lds_u32*)(uintptr_t)a, 32 * word - 96};
+}
+/* The three words that hold the 64 bits below window bit `at` and more. */
+struct Top {
+    uint32_t w0, w1, w2;
+    __device__ __forceinline__ uint64_t bits(int at) const {
+        return (uint64_t)__builtin_amdgcn_alignbit(w2, w1, (uint32_t)at) << 32 |
+               __builtin_amdgcn_alignbit(w1, w0, (uint32_t)at);
+    }
+};
+__device__ __forceinline__ Top top_below(uint32_t window, int at) {
+    const uint32_t a = window + (uint32_t)(at >> 3 & ~3);
+    return Top{*(lds_u32*)(uintptr_t)(a - 8), *(lds_u32*)(uintptr_t)(a - 4),
+               *(lds_u32*)(uintptr_t)a};
+}
+/* n (0..31) of them from window bit `from` on. */
+__device__ __forceinline__ uint32_t bits_of(const Words& w, int from, uint32_t n) {
+    const uint32_t p = (uint32_t)(from - w.first);
+    const bool far = (p & 64) != 0, odd = (p & 32) != 0;
+    const uint32_t a = far ? w.w2 : w.w0, b = far ? w.w3 : w.w1, c = far ? 0u : w.w2;
+    return __builtin_amdgcn_ubfe(
+        __builtin_amdgcn_alignbit(odd ? c : b, odd ? b : a, p & 31), 0, n);
 }
 
 /* Builds a field's cells from counts[0..last] at accuracy `log` (RFC 8878
@@ -209,12 +245,40 @@ __device__ __forceinline__ bool build_cells(EntropyLds& e, uint32_t* cells, uint
             }
             const uint32_t bits = log - zstd::high_bit(state);
             const uint32_t extra = codes == nullptr ? s : codes[s] >> 24;
-            cells[c] = s | bits << kCellBits | extra << kCellExtra |
+            cells[c] = extra | bits << kCellBits | s << kCellSymbol |
                        ((state << bits) - size) << kCellBase;
         }
         wave_order();
     }
     return true;
+}
+
+/* The three repeat offsets after some sequences, in terms of those before
+ * them: a distance (kFarthest for every one beyond, past any window
+ * and refused), or kRepeat<i> less the ones that code 3 without literals
+ * took off the offset i before (64 at most in a batch). */
+struct Repeats {
+    uint32_t a, b, c;
+};
+constexpr uint32_t kRepeat0 = 0x80000100u, kRepeat1 = 0x90000100u, kRepeat2 = 0xA0000100u;
+constexpr uint32_t kFarthest = 0x7FFFFFFFu; /* no distance looks like a reference */
+static_assert(zstd::kWindowMax < kFarthest, "refused");
+__device__ __forceinline__ uint32_t of_repeats(uint32_t v, uint32_t a, uint32_t b, uint32_t c) {
+    const uint32_t i = v >> 28;
+    const uint32_t at = i == 8 ? a : i == 9 ? b : c;
+    return (int32_t)v < 0 ? at + (v & 0x0FFFFFFFu) - 0x100u : v;
+}
+/* r after what the lane that DPP pattern kCtrl names has composed so far;
+ * unchanged on lanes without one. */
+template <int kCtrl, int kRows>
+__device__ __forceinline__ Repeats repeats_after(const Repeats& r) {
+    const uint32_t a = (uint32_t)__builtin_amdgcn_update_dpp((int)kRepeat0, (int)r.a, kCtrl, kRows,
+                                                             0xF, false);
+    const uint32_t b = (uint32_t)__builtin_amdgcn_update_dpp((int)kRepeat1, (int)r.b, kCtrl, kRows,
+                                                             0xF, false);
+    const uint32_t c = (uint32_t)__builtin_amdgcn_update_dpp((int)kRepeat2, (int)r.c, kCtrl, kRows,
+                                                             0xF, false);
+    return Repeats{of_repeats(r.a, a, b, c), of_repeats(r.b, a, b, c), of_repeats(r.c, a, b, c)};
 }
 
 /* One sequence field's table. */
@@ -302,7 +366,7 @@ struct EntropyFlow {
             if (s > max_symbol) {
                 return false;
             }
-            f.cells[0] = s | (f.codes == nullptr ? s : f.codes[s] >> 24) << kCellExtra;
+            f.cells[0] = s << kCellSymbol | (f.codes == nullptr ? s : f.codes[s] >> 24);
             wave_order();
             f.log = 0;
             f.present = true;
@@ -372,13 +436,23 @@ struct EntropyFlow {
         }
         int bits = 8 * (int)(left - 1) + (int)zstd::high_bit(marker);
 
-        /* this lane's field: 0 literal length, 1 match length, 2 (and 3)
-         * offset; masks of what precedes its bits */
+        /* this lane's field (0 literal length, 1 match length, 2 offset) and
+         * its part of it: lanes 0 to 2 the next state, 4 to 6 the extra bits */
         const uint32_t f = (lane & 3) < 2 ? lane & 3 : 2;
+        const bool states = (lane & 4) == 0, is_of = f == 2;
         const uint32_t table = f == 0 ? lds_at(e.litlen) : f == 1 ? lds_at(e.matchlen)
                                                                    : lds_at(e.offset);
-        const uint32_t is_of = f == 2 ? ~0u : 0u, is_ll = f == 0 ? ~0u : 0u;
-        uint32_t state = 0;
+        /* what of the three cells' bits lies up to the end of this lane's
+         * own: the offset's extra bits come first, then the match length's,
+         * then the literal length's, then the states of literal length,
+         * match length and offset */
+        const uint32_t upto0 = states || f == 0 ? (states ? kCellSums : kCellExtras) : 0;
+        const uint32_t upto1 = states    ? (f >= 1 ? kCellSums : kCellExtras)
+                               : f <= 1 ? kCellExtras
+                                        : 0;
+        const uint32_t upto2 = states && f == 2 ? kCellSums : kCellExtras;
+        const uint32_t own = states ? kCellBits : 0;
+        uint32_t cell = 0; /* of the next sequence */
         int pending = CUDEC_OK; /* the first execution error, reported once
                                    the whole block decodes */
         uint32_t k = 0;
@@ -394,10 +468,12 @@ struct EntropyFlow {
             if (k == 0) {
                 /* the initial states: literal length, offset, match length */
                 const uint32_t n = f == 0 ? ll.log : f == 1 ? ml.log : of.log;
-                const uint32_t upto = f == 0   ? ll.log
-                                      : f == 2 ? ll.log + of.log
-                                               : ll.log + of.log + ml.log;
-                state = window_bits(win, base + bits - (int)upto, n);
+                const uint32_t end = f == 0    ? ll.log
+                                     : f == 2 ? ll.log + of.log
+                                              : ll.log + of.log + ml.log;
+                const uint32_t state =
+                    bits_of(words_below(win, base + bits), base + bits - (int)end, n);
+                cell = *(lds_u32*)(uintptr_t)(table + 4 * state);
                 bits -= (int)(ll.log + of.log + ml.log);
                 if (bits < 0) {
                     return CUDEC_ERR_CORRUPT_INPUT;
@@ -405,29 +481,37 @@ struct EntropyFlow {
             }
             const uint32_t cnt = count - k < kWave ? count - k : kWave;
             Job& j = slot();
-            const uint32_t raw = lds_at(j.ll) + 4 * f;
+            /* the extra bits' lanes write; the others to a word of no use */
+            uint32_t raw = states ? lds_at(&l.unused) : lds_at(j.ll) + 4 * f;
+            const uint32_t stride = states ? 0 : 12;
             int at = base + bits; /* window bit above the next one */
+            Top top = top_below(win, at);
+            uint32_t last = 0;
             for (uint32_t s = 0; s < cnt; s++) {
-                const uint32_t cell = *(lds_u32*)(uintptr_t)(table + 4 * state);
-                const uint32_t sym = cell & 63;
-                const uint32_t extra = (cell >> kCellExtra) & 31;
+                last = cell;
+                /* bits from `at` down to the end of this lane's own */
+                const uint32_t sums = (quad<0>(cell) & upto0) + (quad<1>(cell) & upto1) +
+                                      (quad<2>(cell) & upto2);
+                const uint32_t end = (sums & kCellExtras) + (sums >> kCellBits);
+                const uint32_t n = __builtin_amdgcn_ubfe(cell, own, 5);
+                uint32_t v = __builtin_amdgcn_ubfe((uint32_t)(top.bits(at) >> ((64 - end) & 63)), 0, n);
+                if (__ballot(end > 64) != 0) {
+                    v = bits_of(words_below(win, at), at - (int)end, n);
+                }
+                at -= (int)__builtin_amdgcn_readlane(end, 2); /* the last of them */
+                top = top_below(win, at);
+                /* the next cell, its address from the state's lane */
+                const uint32_t next = table + 4 * ((cell >> kCellBase) + v);
+                const uint32_t word = is_of ? (1u << n) + v : (cell & (63u << kCellSymbol)) | v;
+                cell = *(lds_u32*)(uintptr_t)(uint32_t)__builtin_amdgcn_update_dpp(
+                    (int)next, (int)next, 0x114, 0xF, 0xA, false); /* row_shr:4 on every other four */
+                *(lds_u32*)(uintptr_t)raw = word;
+                raw += stride;
+            }
+            if (k + cnt == count) {
                 /* no state is read after the block's last sequence */
-                const uint32_t sb = k + s + 1 == count ? 0u : (cell >> kCellBits) & 15;
-                /* the offset's extra bits come first, then the match
-                 * length's, then the literal length's; the states: literal
-                 * length, match length, offset */
-                const uint32_t x0 = quad<0>(extra), x1 = quad<1>(extra), x2 = quad<2>(extra);
-                const uint32_t s0 = quad<0>(sb), s1 = quad<1>(sb), s2 = quad<2>(sb);
-                const uint32_t before = x2 + (x1 & ~is_of) + (x0 & is_ll);
-                const uint32_t extras = x0 + x1 + x2;
-                const uint32_t states = s0 + (s1 & ~is_ll) + (s2 & is_of);
-                const uint32_t ex = window_bits(win, at - (int)before, extra);
-                at -= (int)extras;
-                const uint32_t nx = window_bits(win, at - (int)states, sb);
-                at -= (int)(s0 + s1 + s2);
-                state = (cell >> kCellBase) + nx;
-                const uint32_t value = (is_of != 0 ? 1u << (sym & 31) : sym << 16) + ex;
-                *(lds_u32*)(uintptr_t)(raw + 12 * s) = value;
+                at += (int)((quad<0>(last) >> kCellBits & 15) + (quad<1>(last) >> kCellBits & 15) +
+                            (quad<2>(last) >> kCellBits & 15));
             }
             bits = (int)uniform32((uint32_t)(at - base));
             if (bits < 0) {
@@ -465,33 +549,32 @@ struct EntropyFlow {
             in ? (l.e.code[zstd::kLitLenMax + 1 + (c1 <= zstd::kMatchLenMax ? c1 : 0)] & 0xFFFFFF) +
                      (v1 & 0xFFFF)
                : 0;
-        /* repeat offsets (RFC 8878 3.1.1.5), one sequence after the other on
-         * the scalar unit; zero: an error */
-        const uint64_t no_literals = __ballot(llen == 0);
-        uint32_t dist = 0;
-        uint32_t a = r0, b = r1, c = r2;
-        for (uint32_t i = 0; i < cnt; i++) {
-            const uint32_t v = __builtin_amdgcn_readlane(value, i);
-            uint32_t d;
-            if (v > 3) {
-                d = v - 3;
-                c = b;
-                b = a;
-                a = d;
-            } else {
-                const uint32_t which = v - 1 + (uint32_t)((no_literals >> i) & 1);
-                d = which == 0 ? a : which == 1 ? b : which == 2 ? c : a - 1;
-                if (which != 0 && d != 0) {
-                    c = which == 1 ? c : b;
-                    b = a;
-                    a = d;
-                }
-            }
-            dist = lane == i ? d : dist;
+        /* repeat offsets (RFC 8878 3.1.1.5): each sequence maps the three
+         * offsets before it to the three after it, its own distance first;
+         * an inclusive scan composes the maps (Repeats). Zero: an error. */
+        const uint32_t which = value - 1 + (llen == 0 ? 1u : 0u);
+        Repeats r = {kRepeat0, kRepeat1, kRepeat2};
+        if (in && value > 3) {
+            const uint32_t d = value - 3;
+            r = Repeats{d < kFarthest ? d : kFarthest, kRepeat0, kRepeat1};
+        } else if (in && which != 0) {
+            r = Repeats{which == 1   ? kRepeat1
+                        : which == 2 ? kRepeat2
+                                     : kRepeat0 - 1,
+                        kRepeat0, which == 1 ? kRepeat2 : kRepeat1};
         }
-        r0 = a;
-        r1 = b;
-        r2 = c;
+        r = repeats_after<0x111, 0xF>(r); /* row_shr:1, 2, 4, 8 */
+        r = repeats_after<0x112, 0xF>(r);
+        r = repeats_after<0x114, 0xF>(r);
+        r = repeats_after<0x118, 0xF>(r);
+        r = repeats_after<0x142, 0xA>(r); /* row_bcast:15, 31 */
+        r = repeats_after<0x143, 0xC>(r);
+        r = Repeats{of_repeats(r.a, r0, r1, r2), of_repeats(r.b, r0, r1, r2),
+                    of_repeats(r.c, r0, r1, r2)};
+        const uint32_t dist = r.a;
+        r0 = uniform32(__builtin_amdgcn_readlane(r.a, kWave - 1));
+        r1 = uniform32(__builtin_amdgcn_readlane(r.b, kWave - 1));
+        r2 = uniform32(__builtin_amdgcn_readlane(r.c, kWave - 1));
         /* positions: a block's regenerated literals and output fit 32 bits
          * whatever the lengths claim (64 of at most 2^17 + 2^16 each) */
         const uint32_t lit_incl = wave_inclusive_sum(llen, lane);

@@ -91,6 +91,34 @@ def test_sequences_at_the_edges(host, level):  # noqa: F811
     assert np.all(st[0::2] == libs.OK) and np.all(st[1::2] == libs.TOO_SMALL)
 
 
+def test_wide_sequences_and_repeats(host):  # noqa: F811
+    """Sequences of more than 64 bits (far sources, long runs on both sides),
+    and copies without literals whose distance steps down by one or returns
+    to one of the last three."""
+    rng = np.random.default_rng(23)
+    far = bytearray(rng.integers(0, 256, 1_700_000, dtype=np.uint8).tobytes())
+    for i in range(70):
+        far += rng.integers(0, 256, 5000 + 97 * i, dtype=np.uint8).tobytes()
+        at = len(far) - 1_600_000 + 1013 * i
+        far += far[at:at + 9000 + 131 * i]
+    steps = bytearray(rng.integers(0, 256, 4000, dtype=np.uint8).tobytes())
+    back = [1500, 700, 300]
+    for i in range(600):
+        if i % 3 == 0:
+            steps += rng.integers(0, 256, i % 5, dtype=np.uint8).tobytes()
+        k = int(rng.integers(0, 4))
+        d = back[k] if k < 3 else back[0] - 1
+        back = [d] + [b for b in back if b != d][:2]
+        at = len(steps) - d
+        steps += steps[at:at + min(d, 20 + i % 40)]
+    cases = []
+    for name, data in (("far", bytes(far)), ("steps", bytes(steps))):
+        for level in (1, 12, 19):
+            cases.append((f"{name} at {level}", libs.zstd_compress(data, level, checksum=1),
+                          len(data)))
+    assert np.all(check(host, cases) == libs.OK)
+
+
 def test_literals_at_the_edges(host):  # noqa: F811
     rng = np.random.default_rng(5)
     cases = []
