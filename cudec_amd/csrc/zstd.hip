@@ -5,7 +5,7 @@
  * The entropy wave walks the frame (zstd_decode.h, walk_frame), builds the
  * FSE tables and decodes the sequences, 64 at a time, into jobs: slots in
  * LDS that the copy wave takes in order. The copy wave decodes the
- * Huffman-coded literals (one lane a stream) into the block's 128 KiB slot
+ * Huffman-coded literals (16 lanes a stream) into the block's 128 KiB slot
  * in global scratch and executes the sequences through an LDS ring
  * (execute.h, the same code that writes LZ4 output). Neither waits for the
  * other beyond the slots, so a frame's time is the longer of the two.
@@ -26,7 +26,11 @@
  *
  * One wave a frame with one sequence decoded and executed after the other
  * took 13.72 ms for 8192 frames of 64 KiB and 284 ms for 2000 frames of
- * 1 KiB to 4 MiB; this takes 4.94 and 56.0 ms.
+ * 1 KiB to 4 MiB; this takes 2.70 and 33.6 ms (4.94 and 56.0 with a lane a
+ * Huffman stream). A frame's time is now the entropy wave's: per 64 KiB of
+ * text-like data 0.82 M cycles of FSE chain, 0.11 M of tables, 0.10 M of
+ * finishing and 0.02 M of staging, against 0.16 M of literals and 0.53 M of
+ * copies on the other.
  *
  * The first error in stream order decides a frame: the entropy wave's
  * verdicts travel as jobs, behind the literals that precede them.
@@ -49,17 +53,6 @@ namespace {
 
 constexpr int kVerifyBlock = 256;
 constexpr uint64_t kPoolKeep = 512ull << 20; /* scratch kept between launches */
-
-/* The Wave policy of the shared Huffman code. */
-struct Wave {
-    static constexpr uint32_t kLanes = kWave;
-    uint32_t lane;
-    __device__ void sync() const { wave_order(); }
-    /* a reader every lane runs on the same stream */
-    struct Same {
-        static __device__ uint64_t fix64(uint64_t v) { return v; }
-    };
-};
 
 /* What the decode leaves for the checksum pass, per frame. */
 struct FrameCheck {
@@ -113,10 +106,14 @@ static_assert(zstd::kBatch == kWave, "a batch holds a sequence a lane");
 
 struct alignas(16) CopyLds : RingLds<kRing> {
     CoverLds cover;
-    uint16_t huffman[zstd::kHufCells];
-    zstd::HufScratch huf;
-    uint32_t stream_bad[4];
-    alignas(16) uint8_t stage[zstd::kWindowBytes + 16]; /* literals of a group; Huffman windows */
+    alignas(16) uint16_t huffman[zstd::kHufCells];
+    /* of a Huffman tree description */
+    uint8_t weights[256];
+    uint32_t weight_cells[1u << zstd::kWeightLogMax];
+    uint32_t first[16]; /* per weight: its next code's cell */
+    int16_t counts[zstd::kWeightSymbolMax + 1];
+    uint16_t next[zstd::kWeightSymbolMax + 1];
+    alignas(16) uint8_t stage[zstd::kWindowBytes + 16]; /* literals of a group; a description */
 };
 constexpr uint32_t kLitStage = zstd::kWindowBytes - 16; /* literal bytes of a group */
 
@@ -189,12 +186,12 @@ __device__ __forceinline__ uint32_t bits_of(const Words& w, int from, uint32_t n
  * cell's rank among its symbol's comes from ballots on the symbol's bits.
  * `order` is scratch of 1 << log bytes. False if the counts do not fill the
  * table exactly. */
-__device__ __forceinline__ bool build_cells(EntropyLds& e, uint32_t* cells, uint8_t* order,
-                                            uint32_t last, uint32_t log, const uint32_t* codes,
-                                            uint32_t lane) {
+__device__ __forceinline__ bool build_cells(const int16_t* counts, uint16_t* next,
+                                            uint32_t* cells, uint8_t* order, uint32_t last,
+                                            uint32_t log, const uint32_t* codes, uint32_t lane) {
     const uint32_t size = 1u << log;
     const uint32_t mask = size - 1;
-    const int count = lane <= last ? e.counts[lane] : 0;
+    const int count = lane <= last ? counts[lane] : 0;
     const uint64_t lows = __ballot(count < 0);
     const uint32_t low = (uint32_t)__builtin_popcountll(lows);
     const uint32_t mine = count > 0 ? (uint32_t)count : 0;
@@ -208,7 +205,7 @@ __device__ __forceinline__ bool build_cells(EntropyLds& e, uint32_t* cells, uint
         cells[size - 1 - (uint32_t)__builtin_popcountll(lows & below)] = lane;
     }
     if (lane <= last) {
-        e.next[lane] = (uint16_t)(count < 0 ? 1 : count);
+        next[lane] = (uint16_t)(count < 0 ? 1 : count);
     }
     for (uint32_t t = 0; t < mine; t++) {
         order[incl - mine + t] = (uint8_t)lane;
@@ -236,12 +233,12 @@ __device__ __forceinline__ bool build_cells(EntropyLds& e, uint32_t* cells, uint
             const uint64_t set = __ballot(((s >> b) & 1) != 0);
             same &= ((s >> b) & 1) != 0 ? set : ~set;
         }
-        const uint32_t first = e.next[s];
+        const uint32_t first = next[s];
         const uint32_t state = first + (uint32_t)__builtin_popcountll(same & below);
         wave_order();
         if (c < size) {
             if ((same >> lane) == 1) { /* the symbol's last cell here */
-                e.next[s] = (uint16_t)(state + 1);
+                next[s] = (uint16_t)(state + 1);
             }
             const uint32_t bits = log - zstd::high_bit(state);
             const uint32_t extra = codes == nullptr ? s : codes[s] >> 24;
@@ -389,7 +386,8 @@ struct EntropyFlow {
             used = uniform32((uint32_t)u);
         }
         wave_order();
-        if (!build_cells(l.e, f.cells, &l.e.window[kHeaderStage], last, log, f.codes, lane)) {
+        if (!build_cells(l.e.counts, l.e.next, f.cells, &l.e.window[kHeaderStage], last, log,
+                         f.codes, lane)) {
             used = 0;
             return false;
         }
@@ -602,6 +600,366 @@ struct EntropyFlow {
     }
 };
 
+/* ----------------------------------------------------------- literals */
+
+/* Reads a Huffman tree description (RFC 8878 4.2.1) and fills the decode
+ * table, as zstd::read_huffman_table does one step after the other: cell
+ * index = the next table_log bits; symbol in the low byte, code length in the
+ * high byte. The description is staged; only the FSE-compressed weights are
+ * read in sequence. False if it is refused. */
+__device__ __forceinline__ bool read_tree(CopyLds& w, gcu8* src, uint64_t size, uint32_t& table_log,
+                                          uint32_t& used, uint32_t lane) {
+    if (size == 0) {
+        return false;
+    }
+    const uint32_t staged = size < 160 ? (uint32_t)size : 160;
+    const uint8_t* head = w.stage + stage_into<1>(w.stage, src, staged, 0, staged, lane);
+    const uint32_t header = uniform32(head[0]);
+    const uint32_t payload = header >= 128 ? (header - 126) / 2 : header;
+    if (payload + 1 > size) {
+        return false;
+    }
+    used = payload + 1;
+    uint32_t written = 0;
+    if (header >= 128) {
+        written = header - 127;
+        for (uint32_t i = lane; i < written; i += kWave) {
+            const uint32_t b = head[1 + i / 2];
+            w.weights[i] = (uint8_t)((i & 1) == 0 ? b >> 4 : b & 15u);
+        }
+    } else {
+        uint32_t last = 0, log = 0;
+        uint64_t description = 0;
+        if (!zstd::read_fse_description((const ZL uint8_t*)(head + 1), payload,
+                                        zstd::kWeightSymbolMax, zstd::kWeightLogMax,
+                                        (ZL int16_t*)w.counts, last, log, description)) {
+            return false;
+        }
+        last = uniform32(last);
+        log = uniform32(log);
+        wave_order();
+        if (!build_cells(w.counts, w.next, w.weight_cells, w.stage + 512, last, log, nullptr,
+                         lane)) {
+            return false;
+        }
+        const uint32_t from = 1 + uniform32((uint32_t)description);
+        const uint32_t mark = from > payload ? 0 : uniform32(head[payload]);
+        if (mark == 0) {
+            return false;
+        }
+        /* two states in turn; when a state's update needs more bits than
+         * remain, its symbol and the other state's close the list */
+        const uint32_t base = lds_at(head + from);
+        uint32_t bits = 8 * (payload - from) + zstd::high_bit(mark);
+        if (bits < 2 * log) {
+            return false;
+        }
+        const uint32_t a0 = base & ~3u, skew = 8 * (base & 3);
+        const auto take = [&](uint32_t n) {
+            bits -= n;
+            const uint32_t p = bits + skew, a = a0 + (p >> 5 << 2);
+            return uniform32(__builtin_amdgcn_ubfe(
+                __builtin_amdgcn_alignbit(*(lds_u32*)(uintptr_t)(a + 4), *(lds_u32*)(uintptr_t)a,
+                                          p & 31),
+                0, n));
+        };
+        uint32_t one = take(log), other = take(log);
+        for (;;) {
+            const uint32_t cell = uniform32(w.weight_cells[one]);
+            w.weights[written++] = (uint8_t)(cell >> kCellSymbol & 63);
+            const uint32_t n = cell >> kCellBits & 15;
+            if (written == 255) {
+                return false;
+            }
+            if (n > bits) {
+                w.weights[written++] = (uint8_t)(w.weight_cells[other] >> kCellSymbol & 63);
+                break;
+            }
+            one = other;
+            other = (cell >> kCellBase) + take(n);
+        }
+    }
+    wave_order();
+    /* symbol 64 r + lane on this lane */
+    uint32_t weight[4], sum = 0;
+    bool over = false;
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++) {
+        const uint32_t i = r * kWave + lane;
+        weight[r] = i < written ? w.weights[i] : 0;
+        over |= weight[r] > zstd::kHufLogMax;
+        sum += (1u << weight[r]) >> 1;
+    }
+    if (__ballot(over) != 0) {
+        return false;
+    }
+    const uint32_t total =
+        uniform32(__builtin_amdgcn_readlane(wave_inclusive_sum(sum, lane), kWave - 1));
+    if (total == 0) {
+        return false;
+    }
+    const uint32_t log = zstd::high_bit(total) + 1;
+    if (log > zstd::kHufLogMax) {
+        return false;
+    }
+    const uint32_t rest = (1u << log) - total;
+    const uint32_t last_weight = zstd::high_bit(rest) + 1;
+    if ((1u << (last_weight - 1)) != rest) {
+        return false;
+    }
+    /* codes of weight 1 (the longest) take the lowest cells, then weight 2,
+     * ...; within a weight, symbols in increasing order */
+    uint32_t at = 0;
+    uint32_t begin = 0; /* of weight `lane` */
+    for (uint32_t k = 1; k <= log; k++) {
+        uint32_t have = 0;
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+            if (r * kWave + lane == written) {
+                weight[r] = last_weight;
+            }
+            have += (uint32_t)__builtin_popcountll(__ballot(weight[r] == k));
+        }
+        if (k == 1 && have < 2) {
+            return false;
+        }
+        begin = lane == k ? at : begin;
+        at += have << (k - 1);
+    }
+    if (lane < 16) {
+        w.first[lane] = begin;
+    }
+    wave_order();
+    const uint64_t below = (1ull << lane) - 1;
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++) {
+        if (r * kWave > written) {
+            break;
+        }
+        const uint32_t wt = weight[r];
+        uint64_t same = ~0ull;
+#pragma unroll
+        for (uint32_t b = 0; b < 4; b++) {
+            const uint64_t set = __ballot(((wt >> b) & 1) != 0);
+            same &= ((wt >> b) & 1) != 0 ? set : ~set;
+        }
+        const uint32_t span = (1u << wt) >> 1;
+        const uint32_t to = w.first[wt] + (uint32_t)__builtin_popcountll(same & below) * span;
+        wave_order();
+        if ((same >> lane) == 1) { /* the weight's last symbol here */
+            w.first[wt] = to + span;
+        }
+        const uint32_t cell = (r * kWave + lane) | (log + 1 - wt) << 8;
+        /* short spans by their own lane, long ones by all */
+        uint64_t wide = __ballot(span >= 32);
+        if (span == 1) {
+            w.huffman[to] = (uint16_t)cell;
+        } else if (span < 32) {
+            for (uint32_t j = 0; j < span; j += 2) {
+                *(uint32_t*)&w.huffman[to + j] = cell | cell << 16;
+            }
+        }
+        while (wide != 0) {
+            const uint32_t i = (uint32_t)__builtin_ctzll(wide);
+            wide &= wide - 1;
+            const uint32_t c = __builtin_amdgcn_readlane(cell, i);
+            const uint32_t n = __builtin_amdgcn_readlane(span, i);
+            const uint32_t t = __builtin_amdgcn_readlane(to, i);
+            for (uint32_t j = 2 * lane; j < n; j += 2 * kWave) {
+                *(uint32_t*)&w.huffman[t + j] = c | c << 16;
+            }
+        }
+        wave_order();
+    }
+    table_log = log;
+    return true;
+}
+
+/* Up to eight codes from stream bit p down. Twelve bytes hold them: 89 bits
+ * below p at least, eight codes of 11 bits at most. A stream's first bytes
+ * follow a frame's, a block's and a section's header and a tree or a jump
+ * table, 14 bytes at least, so the load stays in the frame. */
+struct Codes {
+    uint64_t acc; /* the next bits on top */
+    uint32_t low; /* the bits below, on top */
+    uint32_t taken;
+    __device__ __forceinline__ void load(gcu8* src, int p) {
+        const int end = (p + 7) >> 3;
+        uint32_t v[3];
+        __builtin_memcpy(v, (const void*)(src + (end - 12)), 12);
+        const uint32_t skip = (uint32_t)(8 * end - p);
+        const uint64_t tail = (uint64_t)v[0] << skip;
+        acc = ((uint64_t)v[2] << 32 | v[1]) << skip | tail >> 32;
+        low = (uint32_t)tail;
+        taken = 0;
+    }
+    __device__ __forceinline__ uint32_t index(uint32_t shift) const {
+        return (uint32_t)(acc >> 32) >> shift;
+    }
+    __device__ __forceinline__ void drop(uint32_t n) {
+        acc <<= n;
+        taken += n;
+    }
+    /* after four codes: the bits below follow */
+    __device__ __forceinline__ void refill() {
+        acc |= (uint64_t)low << 32 >> ((64 - taken) & 63);
+    }
+};
+
+/* From stream bit p code by code until p is `stop` or less; counts them. */
+__device__ __forceinline__ int walk_codes(gcu8* src, const uint16_t* table, uint32_t shift, int p,
+                                          int stop, uint32_t& count) {
+    while (p > stop) {
+        Codes c;
+        c.load(src, p);
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) {
+            if (j == 4) {
+                c.refill();
+            }
+            const uint32_t bits = p > stop ? (uint32_t)table[c.index(shift)] >> 8 : 0;
+            count += p > stop ? 1 : 0;
+            c.drop(bits);
+            p -= (int)bits;
+        }
+    }
+    return p;
+}
+
+/* A Huffman-coded literals section's payload (RFC 8878 3.1.1.3.1), as
+ * zstd::decode_huffman_section decodes it a lane a stream: the tree
+ * description unless treeless (log holds the table of the block before, 0:
+ * none), then one or four streams of `regen` symbols in all.
+ *
+ * A stream is a chain of table lookups, about 110 cycles a symbol. Prefix
+ * codes synchronise by themselves: a decoder started at any bit soon finds
+ * code boundaries of the real chain. So a stream is cut into 16 segments (64
+ * for a single stream), and each lane starts 24 longest codes before its own
+ * and walks to its end; then a lane whose start is not where the lane before
+ * it ended walks again from there, until all agree. (The first lane is right
+ * at once, and each round makes at least one more so; codes that never
+ * synchronise take as long as one lane would.) Segments are multiples of
+ * table_log, so codes of one length agree at once. Counts give each segment's
+ * place, and a second walk writes the symbols, eight a store.
+ *
+ * A 64 KiB frame's literals took 1.18 M cycles with a lane a stream and the
+ * tree read in sequence; 0.16 M so.
+ *
+ * A stream is right if its chain ends on bit 0 with the symbols it should
+ * have: a code that takes bits from below bit 0 ends below it, whatever they
+ * are. */
+__device__ __forceinline__ bool huffman_section(CopyLds& w, gcu8* payload, uint64_t psize,
+                                                uint32_t regen, uint32_t streams, bool treeless,
+                                                uint32_t& log, gu8* lits, uint32_t lane) {
+    if (!treeless) {
+        uint32_t used = 0, tree_log = 0;
+        if (!read_tree(w, payload, psize, tree_log, used, lane)) {
+            return false;
+        }
+        log = tree_log;
+        payload += used;
+        psize -= used;
+    } else if (log == 0) {
+        return false;
+    }
+    if (psize == 0) {
+        return false;
+    }
+    const uint32_t lanes = streams == 1 ? kWave : kWave / 4;
+    const uint32_t k = lane & (lanes - 1);
+    gcu8* src = payload;
+    uint32_t size = (uint32_t)psize, n = regen, to = 0;
+    if (streams != 1) {
+        if (psize < 10 || regen < 6) {
+            return false;
+        }
+        uint32_t jump[3];
+        for (uint32_t i = 0; i < 3; i++) {
+            jump[i] = uniform32(payload[2 * i] | (uint32_t)payload[2 * i + 1] << 8);
+        }
+        const uint32_t bytes = (uint32_t)psize - 6;
+        if (jump[0] + jump[1] + jump[2] >= bytes) {
+            return false;
+        }
+        const uint32_t g = lane / lanes, seg = (regen + 3) / 4;
+        src += 6 + (g > 0 ? jump[0] : 0) + (g > 1 ? jump[1] : 0) + (g > 2 ? jump[2] : 0);
+        size = g == 0   ? jump[0]
+               : g == 1 ? jump[1]
+               : g == 2 ? jump[2]
+                        : bytes - jump[0] - jump[1] - jump[2];
+        to = g * seg;
+        n = g < 3 ? seg : regen - 3 * seg;
+    }
+    const uint32_t mark = size == 0 ? 0 : src[size - 1];
+    if (__ballot(mark == 0) != 0) {
+        return false;
+    }
+    const uint32_t shift = 32 - log;
+    const int bits = 8 * (int)(size - 1) + (int)zstd::high_bit(mark);
+    const int least = 64 / (int)log + 1;
+    int codes = (bits + (int)(lanes * log) - 1) / (int)(lanes * log);
+    codes = codes < least ? least : codes;
+    const int per = codes * (int)log;
+    const int hi = bits - (int)k * per;
+    const int lo = hi - per > 0 ? hi - per : 0;
+    /* where this lane's codes begin: a guess, but for the first lane */
+    int begin = hi + 24 * (int)log < bits ? hi + 24 * (int)log : bits;
+    uint32_t count = 0;
+    begin = hi <= 0 ? 0 : walk_codes(src, w.huffman, shift, begin, hi, count);
+    count = 0;
+    int end = walk_codes(src, w.huffman, shift, begin, lo, count);
+    for (;;) {
+        const int before =
+            __builtin_amdgcn_update_dpp(bits, end, 0x138, 0xF, 0xF, false); /* wave_shr:1 */
+        const int should = k == 0 ? bits : before;
+        if (__ballot(should != begin) == 0) {
+            break;
+        }
+        if (should != begin) {
+            begin = should;
+            count = 0;
+            end = walk_codes(src, w.huffman, shift, begin, lo, count);
+        }
+    }
+    const uint32_t incl = wave_inclusive_sum(count, lane);
+    const uint32_t group = lane - k; /* symbols of the streams before */
+    const uint32_t earlier = (uint32_t)__shfl((int)(incl - count), (int)group);
+    if (__ballot(k == lanes - 1 && (end != 0 || incl - earlier != n)) != 0) {
+        return false;
+    }
+    gu8* out = lits + to + (incl - count - earlier);
+    int p = begin;
+    while (count != 0) {
+        Codes c;
+        c.load(src, p);
+        uint32_t word[2] = {0, 0};
+#pragma unroll
+        for (uint32_t j = 0; j < 8; j++) {
+            if (j == 4) {
+                c.refill();
+            }
+            const uint32_t cell = w.huffman[c.index(shift)];
+            const uint32_t n_bits = j < count ? cell >> 8 : 0;
+            word[j / 4] |= (cell & 0xFF) << (8 * (j & 3));
+            c.drop(n_bits);
+        }
+        p -= (int)c.taken;
+        if (count >= 8) {
+            __builtin_memcpy((void*)out, word, 8);
+            out += 8;
+            count -= 8;
+        } else {
+            const uint64_t rest = (uint64_t)word[1] << 32 | word[0];
+            for (uint32_t j = 0; j < count; j++) {
+                out[j] = (uint8_t)(rest >> (8 * j));
+            }
+            count = 0;
+        }
+    }
+    wave_order();
+    return true;
+}
+
 /* ------------------------------------------------------------ copies */
 
 /* The copy wave's place in a frame's output. */
@@ -769,7 +1127,6 @@ __global__ void __launch_bounds__(kFrameBlock) __attribute__((amdgpu_waves_per_e
         return;
     }
     CopyLds& w = l.c;
-    const Wave wave{lane};
     gu8* lits = (gu8*)(lits_base + (size_t)blockIdx.x * zstd::kBlockCeiling);
     CopyState s{nullptr, 0, 0, 0, 0, lits};
     uint64_t chunk = 0;
@@ -825,11 +1182,8 @@ __global__ void __launch_bounds__(kFrameBlock) __attribute__((amdgpu_waves_per_e
                 }
             } else if (kind == kJobHuffman) {
                 s.lit = lits;
-                if (!zstd::decode_huffman_section(wave, (const ZG uint8_t*)(uintptr_t)a, b, num, x,
-                                                  y != 0, *(ZL zstd::HufScratch*)&w.huf,
-                                                  (ZL uint16_t*)w.huffman, huf_log,
-                                                  (ZL uint32_t*)w.stream_bad, (ZL uint8_t*)w.stage,
-                                                  zstd::kWindowBytes, (ZG uint8_t*)lits)) {
+                if (!huffman_section(w, (gcu8*)(uintptr_t)a, b, num, x, y != 0, huf_log, lits,
+                                     lane)) {
                     status = CUDEC_ERR_CORRUPT_INPUT;
                 }
                 status = (int)uniform32((uint32_t)status);

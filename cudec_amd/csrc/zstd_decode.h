@@ -1,5 +1,6 @@
-/* Zstandard frame decode (RFC 8878), one frame per chunk, written once for
- * the device kernel and for a CPU build of the same code (tests).
+/* Zstandard frame decode (RFC 8878), one frame per chunk: the frame walk that
+ * the device kernel and a CPU build share, and the whole decode as the CPU
+ * build (tests) runs it.
  *
  * The frame decode is a serial process: a block's literals section comes
  * first (raw, run-length, or Huffman-coded in one or four streams), then its
@@ -12,11 +13,11 @@
  * walk_frame reads a frame's and its blocks' headers and decides their
  * verdicts in order; what the sections hold it hands to a Flow. The device
  * kernel's Flow (zstd.hip) passes literals and copies on to a second wave
- * and decodes the sequences with the whole wave; the Flow here (DirectFlow)
- * decodes and executes everything on the spot, one sequence after the other,
- * as the CPU build does. The Huffman parts, shared by both, take a Wave
- * policy (kLanes, lane, sync): a wave of 64 lanes on the device, one lane on
- * the host; their lanes exchange results only through memory after a sync().
+ * and decodes the sequences with the whole wave; it shares walk_frame, the
+ * FSE descriptions and the code tables. The Flow here (DirectFlow) decodes
+ * and executes everything on the spot, one sequence after the other, and the
+ * kernel is held to its results. It takes a Wave policy (kLanes, lane,
+ * sync): one lane on the host.
  *
  * Accepted frames and verdicts follow the reference's v1 subset
  * (docs/MASTERPLAN.md:1172-1305, tests/zstd_twin_driver.h:178-390): one

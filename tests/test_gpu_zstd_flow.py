@@ -9,7 +9,8 @@ status, size and bytes on every frame, whatever is around.
   batch holds (64) and one more or less, literal runs around what a group
   stages, matches around what a group writes, sources in the ring and before
   it;
-* literals around the sizes where streams and their windows split;
+* literals around the sizes where streams split, of codes that synchronise and
+  of codes that hardly do, and damaged ones;
 * more frames than there are blocks, from a byte up, at odd output offsets.
 """
 import random
@@ -129,7 +130,19 @@ def test_literals_at_the_edges(host):  # noqa: F811
             data = rng.choice(alphabet, size, p=w / w.sum()).astype(np.uint8).tobytes()
             cases.append((f"{size} of {alphabet}", libs.zstd_compress(data, 1, checksum=0),
                           size))
-    assert np.all(check(host, cases) == libs.OK)
+        for alphabet in (3, 128, 192):  # codes of one length, or nearly: slow to synchronise
+            data = rng.integers(0, alphabet, size, dtype=np.uint8).tobytes()
+            cases.append((f"{size} even of {alphabet}", libs.zstd_compress(data, 1, checksum=0),
+                          size))
+    st = check(host, cases)
+    assert np.all(st == libs.OK)
+    broken = []
+    for name, frame, size in cases:
+        for at in (len(frame) - 2, len(frame) - 5, len(frame) // 2):
+            bad = bytearray(frame)
+            bad[max(at, 0)] ^= 1 << (size % 8)
+            broken.append((f"{name} byte {at}", bytes(bad), size))
+    assert libs.CORRUPT in set(int(v) for v in check(host, broken))
 
 
 def test_more_frames_than_blocks(host):  # noqa: F811
