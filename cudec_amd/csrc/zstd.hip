@@ -15,7 +15,7 @@
  * three fields, one on the next state and one on the extra bits: sums over a
  * quad say where each lane's bits end, a shift of the 64 stream bits on top
  * (read while the sums are made) gives them, and one LDS read the next cell,
- * about 45 instructions and 287 cycles a sequence. (Bits read from LDS where
+ * about 36 instructions and 254 cycles a sequence. (Bits read from LDS where
  * the sums say took a second round trip and 388 cycles; every lane keeping
  * the 128 bits on top and choosing words of them, 62 instructions and 338.)
  * Everything that does not feed the next state (code baselines, repeat
@@ -26,9 +26,9 @@
  *
  * One wave a frame with one sequence decoded and executed after the other
  * took 13.72 ms for 8192 frames of 64 KiB and 284 ms for 2000 frames of
- * 1 KiB to 4 MiB; this takes 2.70 and 33.6 ms (4.94 and 56.0 with a lane a
+ * 1 KiB to 4 MiB; this takes 2.37 and 26.7 ms (4.94 and 56.0 with a lane a
  * Huffman stream). A frame's time is now the entropy wave's: per 64 KiB of
- * text-like data 0.82 M cycles of FSE chain, 0.11 M of tables, 0.10 M of
+ * text-like data 0.70 M cycles of FSE chain, 0.11 M of tables, 0.10 M of
  * finishing and 0.02 M of staging, against 0.16 M of literals and 0.53 M of
  * copies on the other.
  *
@@ -90,13 +90,13 @@ constexpr uint32_t kCodes = (zstd::kLitLenMax + 1) + (zstd::kMatchLenMax + 1);
 
 /* Staged bitstream of one batch: at most 712 bytes (zstd::kWindowBytes). */
 struct alignas(16) EntropyLds {
+    uint32_t offset[1u << zstd::kOffsetLog];
+    alignas(16) uint8_t window[zstd::kWindowBytes + 16]; /* read with constant offsets, so early */
     uint32_t litlen[1u << zstd::kLitLenLog];
     uint32_t matchlen[1u << zstd::kMatchLenLog];
-    uint32_t offset[1u << zstd::kOffsetLog];
     uint32_t code[kCodes]; /* baseline, extra bits above it (24) */
     int16_t counts[zstd::kMatchLenMax + 1];
     uint16_t next[zstd::kMatchLenMax + 1];
-    alignas(16) uint8_t window[zstd::kWindowBytes + 16];
 };
 constexpr uint32_t kHeaderStage = 512; /* of the window: table descriptions */
 static_assert(kHeaderStage + (1u << zstd::kLitLenLog) <= zstd::kWindowBytes,
@@ -437,7 +437,7 @@ struct EntropyFlow {
         /* this lane's field (0 literal length, 1 match length, 2 offset) and
          * its part of it: lanes 0 to 2 the next state, 4 to 6 the extra bits */
         const uint32_t f = (lane & 3) < 2 ? lane & 3 : 2;
-        const bool states = (lane & 4) == 0, is_of = f == 2;
+        const bool states = (lane & 4) == 0;
         const uint32_t table = f == 0 ? lds_at(e.litlen) : f == 1 ? lds_at(e.matchlen)
                                                                    : lds_at(e.offset);
         /* what of the three cells' bits lies up to the end of this lane's
@@ -450,6 +450,9 @@ struct EntropyFlow {
                                         : 0;
         const uint32_t upto2 = states && f == 2 ? kCellSums : kCellExtras;
         const uint32_t own = states ? kCellBits : 0;
+        /* what a value is: 1 << extra bits plus these for the offset, the
+         * code above these for the lengths */
+        const uint32_t one = f == 2 ? 1 : 0, code = f == 2 ? 0 : 63u << kCellSymbol;
         uint32_t cell = 0; /* of the next sequence */
         int pending = CUDEC_OK; /* the first execution error, reported once
                                    the whole block decodes */
@@ -484,32 +487,31 @@ struct EntropyFlow {
             const uint32_t stride = states ? 0 : 12;
             int at = base + bits; /* window bit above the next one */
             Top top = top_below(win, at);
-            uint32_t last = 0;
-            for (uint32_t s = 0; s < cnt; s++) {
-                last = cell;
+            uint32_t end, s = cnt;
+            do {
                 /* bits from `at` down to the end of this lane's own */
-                const uint32_t sums = (quad<0>(cell) & upto0) + (quad<1>(cell) & upto1) +
-                                      (quad<2>(cell) & upto2);
-                const uint32_t end = (sums & kCellExtras) + (sums >> kCellBits);
+                end = __builtin_amdgcn_sad_u8((quad<0>(cell) & upto0) + (quad<1>(cell) & upto1) +
+                                                  (quad<2>(cell) & upto2),
+                                              0, 0);
                 const uint32_t n = __builtin_amdgcn_ubfe(cell, own, 5);
-                uint32_t v = __builtin_amdgcn_ubfe((uint32_t)(top.bits(at) >> ((64 - end) & 63)), 0, n);
-                if (__ballot(end > 64) != 0) {
+                uint32_t v = __builtin_amdgcn_ubfe((uint32_t)(top.bits(at) >> ((64 - end) & 63)),
+                                                   0, n);
+                if (__builtin_expect(__ballot(end > 64) != 0, 0)) {
                     v = bits_of(words_below(win, at), at - (int)end, n);
                 }
                 at -= (int)__builtin_amdgcn_readlane(end, 2); /* the last of them */
                 top = top_below(win, at);
                 /* the next cell, its address from the state's lane */
                 const uint32_t next = table + 4 * ((cell >> kCellBase) + v);
-                const uint32_t word = is_of ? (1u << n) + v : (cell & (63u << kCellSymbol)) | v;
+                const uint32_t word = (cell & code) | ((one << n) + v);
                 cell = *(lds_u32*)(uintptr_t)(uint32_t)__builtin_amdgcn_update_dpp(
                     (int)next, (int)next, 0x114, 0xF, 0xA, false); /* row_shr:4 on every other four */
                 *(lds_u32*)(uintptr_t)raw = word;
                 raw += stride;
-            }
+            } while (--s != 0);
             if (k + cnt == count) {
                 /* no state is read after the block's last sequence */
-                at += (int)((quad<0>(last) >> kCellBits & 15) + (quad<1>(last) >> kCellBits & 15) +
-                            (quad<2>(last) >> kCellBits & 15));
+                at += (int)(__builtin_amdgcn_readlane(end, 2) - __builtin_amdgcn_readlane(end, 4));
             }
             bits = (int)uniform32((uint32_t)(at - base));
             if (bits < 0) {
