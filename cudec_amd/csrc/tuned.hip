@@ -1574,6 +1574,12 @@ __device__ __forceinline__ void decode_alone(WaveLds& w, uint32_t idx, const voi
 }
 
 
+/* Whether a queued batch has no chunk that its plan pipelines: the queue
+ * holds those first, so the first of the others has place 0. */
+__device__ __forceinline__ bool none_piped(const Queue* q) {
+    return uniform32(q->bin_base[kBins]) == 0;
+}
+
 /* The persistent decoder. A block takes the queue's pipelined chunks first,
  * all four waves on one chunk (above); a barrier opens every chunk, so that
  * no control word is reset while another wave may still read it. The queue
@@ -1594,6 +1600,9 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
     const uint32_t wave = uniform32(threadIdx.x / kWave);
     QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
     uint32_t idx;
+    if (kSubs != 0 && none_piped(q)) {
+        return; /* alone_batch follows and takes them all */
+    }
     if (wave == 0 && lane == 0) {
         l.broken = 0;
     }
@@ -1648,17 +1657,24 @@ __global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu
 
 /* The persistent decoder of launches where every chunk runs on one wave:
  * those are bound by throughput and gain from a fifth wave per SIMD (96
- * VGPRs). */
+ * VGPRs): 16 384 token chunks of 64 KiB in 2.69 ms against 3.05 by
+ * piped_batch's split blocks. Only the queue build knows whether a batch has
+ * chunks to pipeline, so it `follows` a piped_batch that leaves batches
+ * without one untouched, and leaves the others (an empty launch is about 5
+ * us) to that. */
 constexpr int kAloneBlock = 2 * kWave;
 template <int kFormat, uint32_t kSubs, bool kParseOnly>
 __global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_eu(5)))
     alone_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
                 const size_t* caps, size_t n, cudec_chunk_result* results, Queue* q,
-                const uint32_t* order) {
+                const uint32_t* order, bool follows) {
     __shared__ WaveLds w[kAloneBlock / kWave];
     const uint32_t lane = __lane_id();
     QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
     const uint32_t wave = uniform32(threadIdx.x / kWave);
+    if (follows && !none_piped(q)) {
+        return;
+    }
     const uint32_t idx = queue_pop<kSubs>(
         q, n, cursor, lane, (uint64_t)blockIdx.x * (kAloneBlock / kWave) + wave);
     decode_alone<kFormat, kSubs, kParseOnly>(w[wave], idx, srcs,
@@ -1863,6 +1879,7 @@ struct Launch {
     bool pipes;
     bool direct;
     size_t grid;
+    size_t alone_grid; /* of the one-wave kernel that follows, or 0 */
 };
 
 /* A launch of few chunks leaves most of the chip idle whatever it does, and
@@ -1882,15 +1899,19 @@ Launch plan_launch(const DeviceState& dev, int f, size_t n) {
     if (n <= 2 * pipe_blocks && std::memcmp(&r.plan, &usual, sizeof(Plan)) == 0) {
         r.plan = plan_from_threshold(kFewPipeMinCost);
     }
+    bool all = true;
     r.pipes = false;
     for (int w = 0; w < kBins / 64; w++) {
         r.pipes = r.pipes || r.plan.two_wave[w] != 0;
+        all = all && r.plan.two_wave[w] == ~0ull;
     }
     const size_t per = r.pipes ? 1 : kAloneBlock / kWave; /* chunks a block starts with */
-    const size_t blocks = r.pipes ? pipe_blocks : (size_t)dev.cus * (size_t)dev.alone_blocks_per_cu[f];
+    const size_t alone_blocks = (size_t)dev.cus * (size_t)dev.alone_blocks_per_cu[f];
+    const size_t blocks = r.pipes ? pipe_blocks : alone_blocks;
     const size_t wanted = (n + per - 1) / per;
     r.direct = wanted <= blocks;
     r.grid = r.direct ? wanted : blocks;
+    r.alone_grid = !r.pipes || all || r.direct ? 0 : alone_blocks;
     return r;
 }
 
@@ -1915,16 +1936,18 @@ hipError_t queue_and_decode(const Launch& launch, int format, const void* const*
                            order, plan);
     }
     /* pipelined blocks, each of which splits into one-wave decoders when it
-     * meets a one-wave chunk; or, where the plan pipelines no chunk, the
-     * one-wave kernel */
+     * meets a one-wave chunk, unless the batch has no other; or, where it has
+     * none or the plan pipelines no chunk, the one-wave kernel */
     const int f = format == kFormatSnappy ? 1 : 0;
-    const int waves = launch.pipes ? (int)kPipeWaves : kAloneBlock / (int)kWave;
-    const size_t grid = launch.grid;
-    const dim3 gd((unsigned)grid), bd((unsigned)(waves * (int)kWave));
-    const bool many = (uint64_t)n >= kSubQueueMinPerWave * (uint64_t)waves * (uint64_t)grid;
-    const int subs = launch.direct ? 2 : many ? 1 : 0;
-    const int shape = (parse_only ? 16 : 0) | (f ? 8 : 0) | (launch.pipes ? 0 : 4) | subs;
-    switch (shape) {
+    for (int pass = 0; pass < (launch.alone_grid != 0 ? 2 : 1); pass++) {
+        const bool follows = pass != 0, pipes = launch.pipes && !follows;
+        const int waves = pipes ? (int)kPipeWaves : kAloneBlock / (int)kWave;
+        const size_t grid = follows ? launch.alone_grid : launch.grid;
+        const dim3 gd((unsigned)grid), bd((unsigned)(waves * (int)kWave));
+        const bool many = (uint64_t)n >= kSubQueueMinPerWave * (uint64_t)waves * (uint64_t)grid;
+        const int subs = launch.direct ? 2 : many ? 1 : 0;
+        const int shape = (parse_only ? 16 : 0) | (f ? 8 : 0) | (pipes ? 0 : 4) | subs;
+        switch (shape) {
 #define CUDEC_PIPED(kShape, kFmt, kS, kP)                                                 \
     case kShape:                                                                          \
         hipLaunchKernelGGL((piped_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
@@ -1932,23 +1955,24 @@ hipError_t queue_and_decode(const Launch& launch, int format, const void* const*
         break;                                                                            \
     case kShape + 4:                                                                      \
         hipLaunchKernelGGL((alone_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
-                           src_sizes, dsts, caps, n, results, q, order);                  \
+                           src_sizes, dsts, caps, n, results, q, order, follows);         \
         break;
-        CUDEC_PIPED(0, kFormatLz4, 1, false)
-        CUDEC_PIPED(1, kFormatLz4, kSubQueues, false)
-        CUDEC_PIPED(2, kFormatLz4, 0, false)
-        CUDEC_PIPED(8, kFormatSnappy, 1, false)
-        CUDEC_PIPED(9, kFormatSnappy, kSubQueues, false)
-        CUDEC_PIPED(10, kFormatSnappy, 0, false)
-        CUDEC_PIPED(16, kFormatLz4, 1, true)
-        CUDEC_PIPED(17, kFormatLz4, kSubQueues, true)
-        CUDEC_PIPED(18, kFormatLz4, 0, true)
-        CUDEC_PIPED(24, kFormatSnappy, 1, true)
-        CUDEC_PIPED(25, kFormatSnappy, kSubQueues, true)
-        CUDEC_PIPED(26, kFormatSnappy, 0, true)
+            CUDEC_PIPED(0, kFormatLz4, 1, false)
+            CUDEC_PIPED(1, kFormatLz4, kSubQueues, false)
+            CUDEC_PIPED(2, kFormatLz4, 0, false)
+            CUDEC_PIPED(8, kFormatSnappy, 1, false)
+            CUDEC_PIPED(9, kFormatSnappy, kSubQueues, false)
+            CUDEC_PIPED(10, kFormatSnappy, 0, false)
+            CUDEC_PIPED(16, kFormatLz4, 1, true)
+            CUDEC_PIPED(17, kFormatLz4, kSubQueues, true)
+            CUDEC_PIPED(18, kFormatLz4, 0, true)
+            CUDEC_PIPED(24, kFormatSnappy, 1, true)
+            CUDEC_PIPED(25, kFormatSnappy, kSubQueues, true)
+            CUDEC_PIPED(26, kFormatSnappy, 0, true)
 #undef CUDEC_PIPED
-        default:
-            return hipErrorInvalidValue;
+            default:
+                return hipErrorInvalidValue;
+        }
     }
     return hipGetLastError();
 }

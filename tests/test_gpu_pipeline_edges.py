@@ -138,6 +138,29 @@ def test_launch_sizes_exact(fmt, n):
     check_against_oracle(fmt, "tuned", streams, caps)
 
 
+@pytest.mark.parametrize("fmt", ["lz4", "snappy"])
+@pytest.mark.parametrize("big", [0, 1])
+@pytest.mark.parametrize("n", [2049, 90000])
+def test_queued_batches_with_and_without_a_large_chunk(fmt, n, big):
+    """Batches that need the queue, of one and of many chunks a wave, whose
+    chunks are all below the pipelining threshold or all but one: the first
+    kind goes to the one-wave kernel, the second to the split blocks."""
+    from cudec_amd import workload
+    codec = workload.CODEC_LZ4 if fmt == "lz4" else workload.CODEC_SNAPPY
+    rng = np.random.default_rng(n + big)
+    base = workload.build(codec, rng.integers(1, 300, 40), rng.integers(0, 3, 40),
+                          rng.integers(1, 1 << 60, 40))
+    streams = [base.compressed(i % 40) for i in range(n)]
+    caps = [int(base.sizes[i % 40]) for i in range(n)]
+    if big:
+        large = workload.build(codec, [200000], [0], [1])
+        streams[n // 2], caps[n // 2] = large.compressed(0), 200000
+    streams[5] = streams[5][:-1]
+    caps[7] -= 1
+    print(f"[queued] {fmt} {n} chunks, {big} large", flush=True)
+    check_against_oracle(fmt, "tuned", streams, caps)
+
+
 def snappy_element(lit, off, length):
     out = bytearray()
     if lit:
