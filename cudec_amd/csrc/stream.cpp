@@ -5,15 +5,20 @@
  * ValidateStreamArgs 196-216, StampNotDecoded 218-230, DecodeStreamCtx
  * 238-488, the entry points 492-593, CopyWaveToHost 163-184).
  *
- * This implementation's shape: the call is split into waves sized by a
- * staging budget charged to its largest chunk (so a hostile size mix cannot
- * inflate staging). Staging is double-buffered -- two pinned source slots,
- * two device source slots, and for host output two device destination and
- * two pinned destination slots -- so the host-side pack of wave w+1 and the
- * host-side unpack of wave w-1 overlap the device decode of wave w on the
- * context's one stream. Host output comes back as one asynchronous copy per
- * wave into pinned memory, then exactly bytes_written bytes per chunk go to
- * the caller. Everything grows on demand and is kept for the next call. */
+ * This implementation's shape: the call is split into waves, of a staging
+ * budget charged to its largest chunk (so a hostile size mix cannot inflate
+ * staging) and, in large calls, of an eighth of its chunks. Up to four waves
+ * are in hand, each with a stream and staging of its own (pinned and device
+ * source, and for host output device and pinned destination): while the
+ * device takes one in, decodes another and gives a third back, host threads
+ * pack the next and unpack an earlier one. Host output comes back as one
+ * asynchronous copy per wave into pinned memory, then exactly bytes_written
+ * bytes per chunk go to the caller. Everything but the threads grows on
+ * demand and is kept for the next call.
+ *
+ * What bounds it is the copies between the caller's memory and pinned memory
+ * (277 MB for 2048 chunks of 16 to 256 KiB, 95 in and 182 out), which one
+ * thread and one wave did in a row with the transfers: 18.3 ms, 5.5 so. */
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -22,6 +27,7 @@
 
 #include "cudec.h"
 #include "hip_owner.h"
+#include "host_copy.h"
 
 namespace cudec_amd {
 
@@ -32,26 +38,29 @@ constexpr size_t kStreamMaxChunks = static_cast<size_t>(INT32_MAX) * 64;
  * destination on the host-output path), against the largest chunk. */
 constexpr size_t kWaveBudget = size_t{1} << 30;
 constexpr size_t kWaveChunksMax = 16384;
+/* Waves of a large call: enough to overlap, and none so small that its
+ * launch and its largest chunk take longer than its transfers. */
+constexpr size_t kWavesWanted = 8;
+constexpr size_t kWaveBytesMin = size_t{24} << 20;
+constexpr int kSlots = 4;
 
 struct Slot {
+    Stream stream;
     PinnedRegion p_src;
     DeviceRegion d_src;
     PinnedRegion p_meta;
     DeviceRegion d_meta;
     DeviceRegion d_dst;
     PinnedRegion p_dst;
-    Event staged;  /* the H2D of this slot's pinned source has completed */
     Event landed;  /* this slot's results and output are in pinned memory */
-    bool staged_pending = false;
     bool landed_pending = false;
-    size_t begin = 0, count = 0;
+    size_t begin = 0, count = 0, meta_stride = 0;
 };
 
 }  // namespace cudec_amd
 
 struct cudec_stream_ctx {
-    cudec_amd::Stream stream;
-    cudec_amd::Slot slot[2];
+    cudec_amd::Slot slot[cudec_amd::kSlots];
     cudec_amd::DeviceRegion d_results;
     cudec_amd::PinnedRegion p_results;
     bool poisoned = false;
@@ -88,7 +97,7 @@ void stamp(cudec_chunk_result* r, size_t n, cudec_status st) {
 }
 
 size_t choose_wave(const size_t* src_sizes, const size_t* caps, size_t n, bool host_out) {
-    size_t biggest = 1;
+    size_t biggest = 1, total = 0;
     for (size_t i = 0; i < n; i++) {
         size_t b = src_sizes[i];
         if (host_out) {
@@ -97,6 +106,7 @@ size_t choose_wave(const size_t* src_sizes, const size_t* caps, size_t n, bool h
         if (b > biggest) {
             biggest = b;
         }
+        total = SIZE_MAX - total < b ? SIZE_MAX : total + b;
     }
     size_t wave = kWaveBudget / biggest;
     if (wave == 0) {
@@ -105,30 +115,39 @@ size_t choose_wave(const size_t* src_sizes, const size_t* caps, size_t n, bool h
     if (wave > kWaveChunksMax) {
         wave = kWaveChunksMax;
     }
-    return wave > n ? n : wave;
+    size_t parts = total / kWaveBytesMin;
+    parts = parts < 1 ? 1 : parts > kWavesWanted ? kWavesWanted : parts;
+    const size_t part = (n + parts - 1) / parts;
+    return wave > part ? part : wave;
 }
 
 /* Unpacks one landed host-output wave: exactly bytes_written bytes per chunk
  * into the caller's buffer. A device-reported length beyond the chunk's
  * capacity is a device fault, never a copy length (src/stream.cpp:163-184). */
 cudec_status unpack_wave(const Slot& s, cudec_chunk_result* pres, void* const* dst_ptrs,
-                         const size_t* caps) {
+                         const size_t* caps, CopyCrew& crew) {
     const unsigned char* base = static_cast<const unsigned char*>(s.p_dst.data());
-    size_t off = 0;
-    for (size_t j = 0; j < s.count; j++) {
-        const size_t i = s.begin + j;
-        cudec_chunk_result& r = pres[i];
-        const size_t bw = static_cast<size_t>(r.bytes_written);
-        if (bw > caps[i]) {
-            r.status = static_cast<int32_t>(CUDEC_ERR_CUDA);
-            r.reserved = 0;
-            r.bytes_written = 0;
-            return CUDEC_ERR_CUDA;
+    const unsigned char* dd = static_cast<const unsigned char*>(s.d_dst.data());
+    const void* const* m_dst = reinterpret_cast<const void* const*>(
+        static_cast<const unsigned char*>(s.p_meta.data()) + 2 * s.meta_stride);
+    size_t good = 0;
+    while (good < s.count && pres[s.begin + good].bytes_written <= caps[s.begin + good]) {
+        good++;
+    }
+    crew.each(good, [&](size_t j) {
+        const cudec_chunk_result& r = pres[s.begin + j];
+        if (r.status == CUDEC_OK && r.bytes_written != 0) {
+            std::memcpy(dst_ptrs[s.begin + j],
+                        base + (static_cast<const unsigned char*>(m_dst[j]) - dd),
+                        static_cast<size_t>(r.bytes_written));
         }
-        if (r.status == CUDEC_OK && bw != 0) {
-            std::memcpy(dst_ptrs[i], base + off, bw);
-        }
-        off += caps[i];
+    });
+    if (good != s.count) {
+        cudec_chunk_result& r = pres[s.begin + good];
+        r.status = static_cast<int32_t>(CUDEC_ERR_CUDA);
+        r.reserved = 0;
+        r.bytes_written = 0;
+        return CUDEC_ERR_CUDA;
     }
     return CUDEC_OK;
 }
@@ -141,7 +160,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     stamp(h_results, n, CUDEC_ERR_CUDA);
     const size_t wave = choose_wave(h_src_sizes, dst_caps, n, host_out);
     const size_t waves = (n + wave - 1) / wave;
-    size_t max_src = 1, max_dst = 1;
+    size_t max_src = 1, max_dst = 1, total = 0;
     for (size_t w = 0; w < waves; w++) {
         const size_t b = w * wave, e = b + wave < n ? b + wave : n;
         size_t ws = 0, wd = 0;
@@ -159,7 +178,13 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
         }
         max_src = ws > max_src ? ws : max_src;
         max_dst = wd > max_dst ? wd : max_dst;
+        total = SIZE_MAX - total < ws ? SIZE_MAX : total + ws;
+        total = SIZE_MAX - total < wd ? SIZE_MAX : total + wd;
     }
+    /* two slots where four would stage more than two full budgets */
+    const size_t most = kWaveBudget / 2;
+    const size_t slots = max_src > most || max_dst > most - max_src ? 2 : kSlots;
+    const size_t used = waves < slots ? waves : slots;
     if (n > SIZE_MAX / sizeof(cudec_chunk_result)) {
         return CUDEC_ERR_CORRUPT_INPUT;
     }
@@ -167,14 +192,13 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     const size_t meta_bytes = 4 * meta_stride;
     const size_t res_bytes = n * sizeof(cudec_chunk_result);
     bool ok = true;
-    for (int k = 0; k < 2 && ok; k++) {
+    for (size_t k = 0; k < used && ok; k++) {
         Slot& s = ctx.slot[k];
         ok = s.p_src.reserve(max_src) == hipSuccess && s.d_src.reserve(max_src) == hipSuccess &&
              s.p_meta.reserve(meta_bytes) == hipSuccess &&
              s.d_meta.reserve(meta_bytes) == hipSuccess &&
              (!host_out || (s.d_dst.reserve(max_dst) == hipSuccess &&
                             s.p_dst.reserve(max_dst) == hipSuccess));
-        s.staged_pending = false;
         s.landed_pending = false;
     }
     ok = ok && ctx.d_results.reserve(res_bytes) == hipSuccess &&
@@ -185,20 +209,14 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     }
     cudec_chunk_result* pres = static_cast<cudec_chunk_result*>(ctx.p_results.data());
     stamp(pres, n, CUDEC_ERR_CUDA);
-    hipStream_t st = ctx.stream.get();
     cudec_status failure = CUDEC_OK;
+    CopyCrew crew(total);
 
     for (size_t w = 0; w < waves && failure == CUDEC_OK; w++) {
-        Slot& s = ctx.slot[w & 1];
-        /* the slot's previous wave: its pinned source must be uploaded, and
-         * on the host-output path its output unpacked, before reuse */
-        if (s.staged_pending) {
-            if (hipEventSynchronize(s.staged.get()) != hipSuccess) {
-                failure = CUDEC_ERR_CUDA;
-                break;
-            }
-            s.staged_pending = false;
-        }
+        Slot& s = ctx.slot[w % slots];
+        hipStream_t st = s.stream.get();
+        /* the slot's previous wave must have landed, and on the host-output
+         * path its output be unpacked, before reuse */
         if (s.landed_pending) {
             if (hipEventSynchronize(s.landed.get()) != hipSuccess) {
                 failure = CUDEC_ERR_CUDA;
@@ -206,7 +224,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
             }
             s.landed_pending = false;
             if (host_out) {
-                failure = unpack_wave(s, pres, dst_ptrs, dst_caps);
+                failure = unpack_wave(s, pres, dst_ptrs, dst_caps, crew);
                 if (failure != CUDEC_OK) {
                     break;
                 }
@@ -214,6 +232,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
         }
         s.begin = w * wave;
         s.count = (s.begin + wave < n ? s.begin + wave : n) - s.begin;
+        s.meta_stride = meta_stride;
         unsigned char* ps = static_cast<unsigned char*>(s.p_src.data());
         unsigned char* ds = static_cast<unsigned char*>(s.d_src.data());
         unsigned char* dd = static_cast<unsigned char*>(s.d_dst.data());
@@ -225,9 +244,6 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
         size_t so = 0, dof = 0;
         for (size_t j = 0; j < s.count; j++) {
             const size_t i = s.begin + j;
-            if (h_src_sizes[i] != 0) {
-                std::memcpy(ps + so, h_src_ptrs[i], h_src_sizes[i]);
-            }
             m_src[j] = ds + so;
             m_size[j] = h_src_sizes[i];
             m_cap[j] = dst_caps[i];
@@ -239,15 +255,19 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
             }
             so += h_src_sizes[i];
         }
+        crew.each(s.count, [&](size_t j) {
+            if (m_size[j] != 0) {
+                std::memcpy(ps + (static_cast<const unsigned char*>(m_src[j]) - ds),
+                            h_src_ptrs[s.begin + j], m_size[j]);
+            }
+        });
         unsigned char* dm = static_cast<unsigned char*>(s.d_meta.data());
         cudec_chunk_result* dres = static_cast<cudec_chunk_result*>(ctx.d_results.data()) + s.begin;
         if ((so != 0 && hipMemcpyAsync(ds, ps, so, hipMemcpyHostToDevice, st) != hipSuccess) ||
-            hipMemcpyAsync(dm, pm, meta_bytes, hipMemcpyHostToDevice, st) != hipSuccess ||
-            hipEventRecord(s.staged.get(), st) != hipSuccess) {
+            hipMemcpyAsync(dm, pm, meta_bytes, hipMemcpyHostToDevice, st) != hipSuccess) {
             failure = CUDEC_ERR_CUDA;
             break;
         }
-        s.staged_pending = true;
         const cudec_status launched = cudec_lz4_decompress_batch(
             reinterpret_cast<const void* const*>(dm),
             reinterpret_cast<const size_t*>(dm + meta_stride),
@@ -268,26 +288,27 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
         }
         s.landed_pending = true;
     }
-    /* drain: nothing of this call outlives it */
-    if (hipStreamSynchronize(st) != hipSuccess && failure == CUDEC_OK) {
-        failure = CUDEC_ERR_CUDA;
-    }
-    if (hipGetLastError() != hipSuccess && failure == CUDEC_OK) {
-        failure = CUDEC_ERR_CUDA;
-    }
     /* unpack the waves still in flight, in order */
-    for (size_t w = (waves >= 2 ? waves - 2 : 0); w < waves && failure == CUDEC_OK; w++) {
-        Slot& s = ctx.slot[w & 1];
+    for (size_t w = (waves > slots ? waves - slots : 0); w < waves && failure == CUDEC_OK; w++) {
+        Slot& s = ctx.slot[w % slots];
         if (s.landed_pending && s.begin == w * wave) {
             s.landed_pending = false;
-            if (host_out) {
-                failure = unpack_wave(s, pres, dst_ptrs, dst_caps);
+            if (hipEventSynchronize(s.landed.get()) != hipSuccess) {
+                failure = CUDEC_ERR_CUDA;
+            } else if (host_out) {
+                failure = unpack_wave(s, pres, dst_ptrs, dst_caps, crew);
             }
         }
     }
-    for (int k = 0; k < 2; k++) {
-        ctx.slot[k].staged_pending = false;
+    /* drain: nothing of this call outlives it */
+    for (size_t k = 0; k < used; k++) {
+        if (hipStreamSynchronize(ctx.slot[k].stream.get()) != hipSuccess && failure == CUDEC_OK) {
+            failure = CUDEC_ERR_CUDA;
+        }
         ctx.slot[k].landed_pending = false;
+    }
+    if (hipGetLastError() != hipSuccess && failure == CUDEC_OK) {
+        failure = CUDEC_ERR_CUDA;
     }
     std::memcpy(h_results, pres, res_bytes);
     if (failure == CUDEC_ERR_CUDA) {
@@ -321,13 +342,11 @@ cudec_status cudec_stream_ctx_create(cudec_stream_ctx** out_ctx) {
     if (ctx == nullptr) {
         return CUDEC_ERR_CUDA;
     }
-    if (make_stream(ctx->stream) != hipSuccess ||
-        make_sync_event(ctx->slot[0].staged) != hipSuccess ||
-        make_sync_event(ctx->slot[0].landed) != hipSuccess ||
-        make_sync_event(ctx->slot[1].staged) != hipSuccess ||
-        make_sync_event(ctx->slot[1].landed) != hipSuccess) {
-        delete ctx;
-        return CUDEC_ERR_CUDA;
+    for (Slot& s : ctx->slot) {
+        if (make_stream(s.stream) != hipSuccess || make_sync_event(s.landed) != hipSuccess) {
+            delete ctx;
+            return CUDEC_ERR_CUDA;
+        }
     }
     *out_ctx = ctx;
     return CUDEC_OK;
@@ -364,8 +383,8 @@ void cudec_stream_ctx_destroy(cudec_stream_ctx* ctx) {
     if (ctx == nullptr) {
         return;
     }
-    if (ctx->stream.get() != nullptr) {
-        (void)hipStreamSynchronize(ctx->stream.get());
+    for (Slot& s : ctx->slot) {
+        (void)hipStreamSynchronize(s.stream.get());
     }
     delete ctx;
 }
