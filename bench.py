@@ -460,7 +460,7 @@ def committed_traffic():
 
 def chunk_latency_leg(seed):
     """Idle latency of one chunk per size bin: a batch of one token-process
-    chunk, decoded by the tuned launch on two pipelined waves and on one
+    chunk, decoded by the tuned launch on a pipelined block and on one
     wave, median of 10 event-timed launches after 2 warmups. A request's
     latency cannot fall below its largest chunk's."""
     import numpy as np
@@ -618,7 +618,7 @@ def main():
         bins = sorted({cudec_amd.cost_bin(int(c), int(u))
                        for c, u in zip(batch.comp_size, batch.sizes)})
         tuning = {"knob": "lanes per chunk for each cost bin (cost = 2 x capacity - "
-                          "compressed): 128 = two pipelined waves, 64 = one wave; a threshold "
+                          "compressed): 128 = a pipelined block, 64 = one wave; a threshold "
                           "sweep, then each occupied octave moved to the other lane count when "
                           "that gains 1%",
                   "plan": {str(b): lanes[b] for b in bins},

@@ -97,9 +97,9 @@ hipError_t launch_plain(int format, const void* const* srcs,
 /* The current device's decode plan of one format (tuned.hip): for each of
  * the 256 cost bins (cost = capacity + (capacity - compressed size), four
  * bins per octave, bin 0 the costliest), the lanes that decode a chunk of
- * that bin, 128 (two pipelined waves) or 64 (one wave). A threshold sets
- * the plan that puts chunks costing at least min_cost on two waves (0:
- * every chunk, UINT64_MAX none); get_pipe_min_cost reports the threshold
+ * that bin: 128 stands for a pipelined block of four waves, 64 for one wave.
+ * A threshold sets the plan that pipelines chunks costing at least min_cost
+ * (0: every chunk, UINT64_MAX none); get_pipe_min_cost reports the threshold
  * last set. */
 constexpr int kCostBins = 256;
 hipError_t set_pipe_min_cost(int format, uint64_t min_cost);

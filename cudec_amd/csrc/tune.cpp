@@ -1,11 +1,11 @@
-/* Autotuners of the tuned batch launch: which chunks decode on two waves
- * (parse and execute pipelined) and which on one.
+/* Autotuners of the tuned batch launch: which chunks decode on a pipelined
+ * block of four waves (named 128 lanes) and which on one wave (64).
  *
  * Chunks fall into cost bins (cost = capacity + (capacity - compressed
  * size)); a format's decode plan names the lanes per chunk of every bin.
- * Two waves shorten one chunk's critical path (large chunks bound a
- * launch); one wave keeps twice as many chunks in flight (batches of small
- * chunks are throughput-bound). cudec_mi355x_autotune_lz4 sweeps threshold
+ * A block shortens one chunk's critical path (large chunks bound a
+ * launch); one wave keeps five times as many chunks in flight (batches of
+ * small chunks are throughput-bound). cudec_mi355x_autotune_lz4 sweeps threshold
  * plans; cudec_mi355x_autotune_plan refines the best threshold plan octave
  * by octave. Both decode the caller's batch per candidate after a warmup
  * and keep the fastest for the current device. */

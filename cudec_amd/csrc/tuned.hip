@@ -3,43 +3,47 @@
  * Work distribution: four small kernels bin the chunks by decode cost
  * (capacity + (capacity - compressed size), the output plus what matches
  * add to it; four bins per octave) into a device queue. A per-device,
- * per-format decode plan names, for each cost bin, the lanes that decode
- * one of its chunks: 128 (both waves of a block, as a software pipeline)
- * or 64 (one wave). The queue holds the two-wave chunks first, then the
- * one-wave ones, each class costliest first. A persistent grid of two-wave
+ * per-format decode plan names, for each cost bin, how one of its chunks is
+ * decoded: pipelined on a block of four waves (named 128 in the plan) or on
+ * one wave (64). The queue holds the pipelined chunks first, then the
+ * one-wave ones, each class costliest first. A persistent grid of four-wave
  * blocks pulls chunks from it; once the queue reaches the one-wave class,
- * a block splits into two independent one-wave decoders.
+ * a block splits into four independent one-wave decoders. A batch without a
+ * pipelined chunk goes to a kernel of one-wave decoders alone, and a launch
+ * with a resident block for every chunk takes them without the queue.
  *
- * Per chunk, the stream is decoded in windows of candidate positions
- * staged in LDS:
+ * Per chunk, the stream is decoded in windows of source bytes staged in LDS:
  *   1. stage     -- compressed bytes from the window start are loaded as
  *                   aligned 16-byte blocks (a block holding any byte of the
  *                   chunk never leaves the chunk's pages);
- *   2. speculate -- every lane parses 16 (two-wave form) or 8 (one-wave
- *                   form) candidate positions as if a sequence
- *                   (LZ4) or element (Snappy) started there, and records
- *                   where the next one would start;
- *   3. walk      -- a scalar walk follows the true chain from position 0
- *                   through those links (v_readlane): up to 64 members, one
- *                   per lane;
- *   4. resolve   -- a wavefront prefix sum places each member's output and
+ *   2. find      -- where the window's sequences (LZ4) or elements (Snappy),
+ *                   its members, start. A pipelined block walks 64 segments
+ *                   of the window at once, a lane each ("pipelined blocks"
+ *                   below). A lone wave parses eight candidate positions a
+ *                   lane as if a member started there, and follows the true
+ *                   chain through their links by pointer doubling: its
+ *                   windows hold 512 bytes, and the segment walk there is
+ *                   1 to 3% faster on chunks of 64 KiB and 20% slower on
+ *                   chunks of 1 to 4 KiB (0.76 against 0.92 ms for 100 003);
+ *   3. resolve   -- of 64 members, a lane each: a wavefront prefix sum places
+ *                   each member's output and
  *                   the exact validation ladder (src/lz4_block.h:95-258,
  *                   src/snappy_block.h:288-435) runs per lane; the first
  *                   member in stream order that rejects, ends the stream,
  *                   or would overflow the group ends the group, so a chunk's
  *                   status is the sequential ladder's;
- *   5. execute   -- output goes through an LDS ring: literals by member
- *                   lanes; matches whose sources are final by member lanes
- *                   (batched 16-byte history loads); the rest in stream
+ *   4. execute   -- output goes through an LDS ring (execute.h): literals by
+ *                   member lanes; matches whose sources are final by member
+ *                   lanes (batched 16-byte history loads); the rest in stream
  *                   order with the wave fanned out over the bytes;
- *   6. flush     -- completed ring bytes leave as aligned 16-byte stores;
+ *   5. flush     -- completed ring bytes leave as aligned 16-byte stores;
  *                   only a chunk's first and last partial blocks use byte
  *                   stores, so exactly bytes_written bytes are stored.
- * Steps 1-4 read only the source and decide every status; steps 5-6 only
- * write. In the two-wave form one wave runs 1-4 on window i + 1 while the
- * other runs 5-6 on window i. A sequence the window cannot hold (a length
- * with two or more extension bytes, a Snappy literal over 256 bytes) is
- * decided by the exact scalar ladder and copied wave-wide, global to global.
+ * Steps 1-3 read only the source and decide every status; steps 4-5 only
+ * write. In a pipelined block one wave runs 1-2 and three take turns at 3-5.
+ * A member the window cannot hold (a long run of extension bytes, a Snappy
+ * literal over 256 bytes) is decided by the exact scalar ladder and copied
+ * wave-wide, global to global.
  */
 #include <cstdlib>
 #include <cstring>
@@ -73,7 +77,7 @@ constexpr uint64_t kDefaultPipeMinCost[2] = {128u << 10, 64u << 10};
 /* ... and in launches of few chunks (plan_launch): below this one wave is
  * as fast (a 4 KiB token page alone: 36 us on one wave, 40 pipelined). */
 constexpr uint64_t kFewPipeMinCost = 8u << 10;
-/* Queue keys: a chunk's class (two-wave first), then its cost bin. */
+/* Queue keys: a chunk's class (pipelined first), then its cost bin. */
 constexpr int kKeys = 2 * kBins;
 
 static_assert(2 + 269 + 3 <= stage_bytes(0), "a window's last candidate fits the stage");
@@ -119,7 +123,7 @@ struct Queue {
 };
 
 /* A decode plan: bit b (of word b / 64) set when cost bin b decodes on
- * two pipelined waves, clear for one wave. Passed to the kernels by value. */
+ * a pipelined block, clear for one wave. Passed to the kernels by value. */
 struct Plan {
     uint64_t two_wave[kBins / 64];
 };
@@ -1709,7 +1713,7 @@ constexpr size_t kFixedMaxChunks = CUDEC_MI355X_NOALLOC_MAX_CHUNKS;
 constexpr size_t kFixedBytes = sizeof(Queue) + sizeof(uint32_t) * kFixedMaxChunks;
 static __device__ __align__(256) uint8_t scratch[kFixedBytes];
 
-/* The plan that puts chunks costing at least min_cost on two waves: every
+/* The plan that pipelines chunks costing at least min_cost: every
  * bin up to the bin of a chunk whose cost is exactly min_cost (costlier
  * bins have smaller numbers). 0 takes every bin, UINT64_MAX none. */
 Plan plan_from_threshold(uint64_t min_cost) {

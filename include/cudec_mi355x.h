@@ -44,12 +44,14 @@ size_t cudec_mi355x_max_batch_chunks(void);
  * size): the output, plus what matches add to it. Costs fall into
  * CUDEC_MI355X_COST_BINS bins, four per octave, bin 0 the costliest
  * (cudec_mi355x_cost_bin). A format's decode plan names, for each bin, the
- * lanes that decode one of its chunks: 128 (two waves of a block, one
- * parsing the next window while the other executes the current one) or 64
- * (one wave). Inside one launch the two-wave chunks start first, then the
- * one-wave ones, each costliest first. Output bytes and results never
+ * lanes that decode one of its chunks: 128 stands for a pipelined block (one
+ * wave finds where sequences start, three others resolve and execute them),
+ * 64 for one wave. Inside one launch the pipelined chunks start first, then
+ * the one-wave ones, each costliest first. Output bytes and results never
  * depend on the plan. Plans are per device and per format, process-wide;
- * the default puts chunks costing at least 512 KiB on two waves. */
+ * the default pipelines chunks costing at least 128 KiB (LZ4) or 64 KiB
+ * (Snappy), and under it launches of few chunks (up to two a resident
+ * block) pipeline those costing at least 8 KiB. */
 #define CUDEC_MI355X_COST_BINS 256
 #define CUDEC_MI355X_FORMAT_LZ4 0
 #define CUDEC_MI355X_FORMAT_SNAPPY 1
@@ -64,8 +66,8 @@ cudec_status cudec_mi355x_set_decode_plan(int format, const uint16_t* h_lanes_pe
 cudec_status cudec_mi355x_decode_plan(int format, uint16_t* h_lanes_per_bin);
 
 /* A format's plan by threshold: chunks whose cost is at least min_cost
- * bytes decode on two waves, cheaper ones on one; 0 puts every chunk on
- * two waves, SIZE_MAX none. The getters return the threshold last set
+ * bytes are pipelined, cheaper ones decode on one wave; 0 pipelines every
+ * chunk, SIZE_MAX none. The getters return the threshold last set
  * (a plan set per bin since then is read with cudec_mi355x_decode_plan).
  * The LZ4 setting applies to cudec_lz4_decompress_batch only, the Snappy
  * one to cudec_snappy_decompress_batch only. */
