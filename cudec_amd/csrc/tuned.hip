@@ -917,18 +917,27 @@ static_assert(kPipeHistory + kCopiers * kPipeBatch + 64 <= kPipeRing &&
               "running groups and their history share the ring");
 static_assert(kPipeBatch <= 64 * kWave, "CoverLds marks a batch");
 
-/* Bytes of a lane's segment: the window is 64 of them. A chunk's first
- * window, and one after a window cut short, is a small one, so that its
- * members reach the copiers early. */
+/* Bytes of a lane's segment: the window is 64 of them. A window takes as
+ * many steps as the longest wrong chain in it (about 85 members of LZ4 token
+ * data), whatever its size, so a wider one is parsed faster by the byte: one
+ * 1 MiB chunk in 2.32 ms with segments of 64, 1.44 with 128, 1.30 with 192
+ * and 1.28 with 320 (the copiers bound it then). LDS sets the line: four
+ * blocks a CU at 128, three at 192, and a full chip needs the fourth (the
+ * uneven LZ4 batch: 17.5 ms, 20.1 with 192 and 21.7 with 64 and three waves
+ * on five blocks). So LZ4 launches that have a block of three a CU for every
+ * chunk take 192 (16 chunks of 4 KiB to 1 MiB: 1.44 -> 1.31 ms; 700 of 256
+ * KiB: 0.57 -> 0.52), all others 128. Snappy's chains meet sooner and gain
+ * nothing (700 of 256 KiB: 0.79 ms, 0.82 with 192). A chunk's first window,
+ * and one after a window cut short, is a small one, so that its members
+ * reach the copiers early. */
 constexpr uint32_t kSegment = 128;
+constexpr uint32_t kSegmentWide = 192;
 constexpr uint32_t kSegmentFirst = 32;
-constexpr uint32_t kPipeStage = stage_bytes(kSegment * kWave) + 16;
 constexpr uint32_t stage_rounds(uint32_t bytes) { return (bytes / 16 + 1 + kWave - 1) / kWave; }
-constexpr uint32_t kStageRounds = stage_rounds(stage_bytes(kSegment * kWave));
 constexpr uint32_t kStageRoundsFirst = stage_rounds(stage_bytes(kSegmentFirst * kWave));
 static_assert(stage_rounds(stage_bytes(kCandSplit * kWave)) == 1, "one-wave stage");
 /* Members listed of one window; a window that holds more ends there. */
-constexpr uint32_t kListMax = 1280;
+constexpr uint32_t list_max(uint32_t segment) { return 10 * segment; }
 constexpr uint32_t kListEnd = 0xFFFFu; /* a listed position at the source end */
 
 struct PipeWindow {
@@ -948,12 +957,14 @@ struct PipeClaim {
 };
 constexpr uint32_t kNoWindow = 0xFFFFFFFFu;
 
+template <uint32_t kSeg>
 struct alignas(16) PipeLds {
+    static constexpr uint32_t kSegment = kSeg;
     union {
         struct {
             RingLds<kPipeRing> w;
-            uint8_t stage[2][kPipeStage];
-            uint16_t list[2][kListMax + 2];
+            alignas(16) uint8_t stage[2][stage_bytes(kSeg * kWave) + 16];
+            uint16_t list[2][list_max(kSeg) + 2];
             CoverLds cover[kCopiers];
         } pipe;                       /* pipelined */
         WaveLds split[kPipeWaves];    /* one chunk a wave, once the block splits */
@@ -971,13 +982,15 @@ struct alignas(16) PipeLds {
     uint32_t done_dp;     /* output position they reach (low 32 bits) */
     uint32_t broken;      /* a wait ran out, and no wave waits any more */
 };
-static_assert(sizeof(PipeLds) <= 40960, "four blocks share a CU's 160 KiB");
+static_assert(sizeof(PipeLds<kSegment>) <= 40960, "four blocks share a CU's 160 KiB");
+static_assert(sizeof(PipeLds<kSegmentWide>) <= 54608, "three blocks");
 
 /* A copier's group among the groups at once (execute_group's Order). */
+template <class L>
 struct InTurn {
     static constexpr bool kInTurn = true;
     static constexpr uint32_t kHistory = kPipeHistory;
-    PipeLds& l;
+    L& l;
     uint32_t k;
     /* everything below is final: done_dp is at most two groups behind */
     __device__ uint64_t final_below(uint64_t d0) const {
@@ -1051,7 +1064,7 @@ __device__ __forceinline__ uint32_t walk_step(const uint8_t* cw, uint32_t p, uin
 /* Walks the window's chain (see above) from its first byte and lists its
  * members; returns where it goes on: a window position, or kWalkStop | the
  * last listed member, whose end the window cannot tell. */
-template <int kFormat>
+template <int kFormat, uint32_t kMost>
 __device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segment,
                                                 uint32_t limit, uint32_t lim, uint16_t* list,
                                                 uint32_t& count, uint32_t lane) {
@@ -1100,17 +1113,17 @@ __device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segm
     uint32_t p = entry;
     uint32_t next = 0; /* the member after a full list, on its lane */
     while (p < end) {
-        if (i < kListMax) {
+        if (i < kMost) {
             list[i] = (uint16_t)p;
-        } else if (i == kListMax) {
+        } else if (i == kMost) {
             next = p;
         }
         i++;
         p = walk_step<kFormat>(cw, p, limit, lim);
     }
-    if (total > kListMax) {
-        count = kListMax;
-        const uint64_t holder = __ballot(incl - mine <= kListMax && kListMax < incl);
+    if (total > kMost) {
+        count = kMost;
+        const uint64_t holder = __ballot(incl - mine <= kMost && kMost < incl);
         return uniform32(__builtin_amdgcn_readlane(next, __builtin_ctzll(holder)));
     }
     count = total;
@@ -1119,9 +1132,11 @@ __device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segm
 
 /* The parser's side of a chunk: window after window into the two window
  * slots, a slot again once the groups of its window have finished. */
-template <int kFormat>
-__device__ __forceinline__ void run_parser(PipeLds& l, gcu8* src, uint64_t src_size, uint64_t cap,
+template <int kFormat, class L>
+__device__ __forceinline__ void run_parser(L& l, gcu8* src, uint64_t src_size, uint64_t cap,
                                            uint32_t lane) {
+    constexpr uint32_t kSeg = L::kSegment;
+    constexpr uint32_t kStageRounds = stage_rounds(stage_bytes(kSeg * kWave));
     uint64_t base = 0;
     if (kFormat == kFormatSnappy) {
         uint64_t declared = 0;
@@ -1158,13 +1173,14 @@ __device__ __forceinline__ void run_parser(PipeLds& l, gcu8* src, uint64_t src_s
             segment > kSegmentFirst
                 ? stage_into<kStageRounds>(stage, src, src_size, base, limit, lane)
                 : stage_into<kStageRoundsFirst>(stage, src, src_size, base, limit, lane);
-        const uint32_t touch = touch_ahead(src, src_size, base, limit, kSegment, lane);
+        const uint32_t touch = touch_ahead(src, src_size, base, limit, kSeg, lane);
         const uint8_t* cw = stage + delta;
         uint32_t count = 0;
-        const uint32_t next = walk_window<kFormat>(cw, segment, limit, lim, list, count, lane);
+        const uint32_t next =
+            walk_window<kFormat, list_max(kSeg)>(cw, segment, limit, lim, list, count, lane);
         bool last = false;
         uint64_t next_base = base + next;
-        segment = kSegment;
+        segment = kSeg;
         if ((next & kWalkStop) != 0) {
             /* only where the member ends matters here (the copiers decide
              * what it is worth): the exact ladder, with room for any output */
@@ -1210,9 +1226,9 @@ __device__ __forceinline__ void run_parser(PipeLds& l, gcu8* src, uint64_t src_s
  * `c` on, and executes it. The copier whose claim decides the chunk's end
  * returns true, with the status and the bytes produced. kParseOnly: claims
  * only. */
-template <int kFormat, bool kParseOnly>
-__device__ __forceinline__ bool run_copier(PipeLds& l, uint32_t c, gcu8* src, uint64_t src_size,
-                                           gu8* dst, uint64_t cap, int& status, uint64_t& produced,
+template <int kFormat, bool kParseOnly, class L>
+__device__ __forceinline__ bool run_copier(L& l, uint32_t c, gcu8* src, uint64_t src_size, gu8* dst,
+                                           uint64_t cap, int& status, uint64_t& produced,
                                            uint32_t lane) {
     lds_flag* broken = (lds_flag*)&l.broken;
     lds_flag* claim = (lds_flag*)&l.claim;
@@ -1226,7 +1242,7 @@ __device__ __forceinline__ bool run_copier(PipeLds& l, uint32_t c, gcu8* src, ui
             status = CUDEC_ERR_CUDA;
             return true;
         }
-        const InTurn turn{l, k};
+        const InTurn<L> turn{l, k};
         uint64_t dp = uniform64(l.next.dp);
         uint64_t flushed = uniform64(l.next.flushed);
         uint64_t ring_lo = uniform64(l.next.ring_lo);
@@ -1590,16 +1606,18 @@ __device__ __forceinline__ bool none_piped(const Queue* q) {
  * holds every pipelined chunk before the others, so once a block meets one
  * of the others it splits for good into four one-wave decoders.
  *
- * Four blocks fill a CU's LDS, sixteen waves at 128 VGPRs each. kSubs:
+ * Four blocks fill a CU's LDS, sixteen waves at 128 VGPRs each (three with
+ * kSegmentWide, twelve waves). kSubs:
  * decode sub-queues, kSubQueues for launches of many chunks per wave, 0 for
  * launches with a resident block for every chunk, else 1 (the single
  * counter, whose code keeps the fewest scalar registers live). */
-template <int kFormat, uint32_t kSubs, bool kParseOnly>
-__global__ void __launch_bounds__(kPipeBlock) __attribute__((amdgpu_waves_per_eu(4)))
+template <int kFormat, uint32_t kSubs, bool kParseOnly, uint32_t kSeg = kSegment>
+__global__ void __launch_bounds__(kPipeBlock)
+    __attribute__((amdgpu_waves_per_eu(kSeg == kSegment ? 4 : 3)))
     piped_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
                 const size_t* caps, size_t n, cudec_chunk_result* results, Queue* q,
                 const uint32_t* order, Plan plan) {
-    __shared__ PipeLds l;
+    __shared__ PipeLds<kSeg> l;
     const uint32_t lane = __lane_id();
     const uint32_t wave = uniform32(threadIdx.x / kWave);
     QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
@@ -1692,6 +1710,7 @@ __global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_e
 struct DeviceState {
     int cus = 0;
     int pipe_blocks_per_cu[2] = {0, 0};  /* piped_batch, per format */
+    int wide_blocks_per_cu = 0;          /* LZ4's piped_batch in kSegmentWide's windows */
     int alone_blocks_per_cu[2] = {0, 0}; /* alone_batch */
     Plan plan[2];                /* per format (kFormatLz4, kFormatSnappy) */
     uint64_t min_cost[2];        /* the threshold each plan was last set from */
@@ -1763,6 +1782,15 @@ hipError_t device_state(DeviceState** out) {
             }
             d.alone_blocks_per_cu[f] = per > 0 ? per : 1;
         }
+        int wide = 0;
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &wide,
+            reinterpret_cast<const void*>(&piped_batch<kFormatLz4, 0, false, kSegmentWide>),
+            kPipeBlock, 0);
+        if (e != hipSuccess) {
+            return e;
+        }
+        d.wide_blocks_per_cu = wide > 0 ? wide : 1;
         for (int f = 0; f < 2; f++) {
             d.plan[f] = plan_from_threshold(kDefaultPipeMinCost[f]);
             d.min_cost[f] = kDefaultPipeMinCost[f];
@@ -1882,6 +1910,7 @@ struct Launch {
     Plan plan;
     bool pipes;
     bool direct;
+    bool wide;         /* LZ4, direct and pipelined: in kSegmentWide's windows */
     size_t grid;
     size_t alone_grid; /* of the one-wave kernel that follows, or 0 */
 };
@@ -1914,6 +1943,8 @@ Launch plan_launch(const DeviceState& dev, int f, size_t n) {
     const size_t blocks = r.pipes ? pipe_blocks : alone_blocks;
     const size_t wanted = (n + per - 1) / per;
     r.direct = wanted <= blocks;
+    r.wide = f == 0 && r.pipes && r.direct &&
+             n <= (size_t)dev.cus * (size_t)dev.wide_blocks_per_cu;
     r.grid = r.direct ? wanted : blocks;
     r.alone_grid = !r.pipes || all || r.direct ? 0 : alone_blocks;
     return r;
@@ -1949,7 +1980,7 @@ hipError_t queue_and_decode(const Launch& launch, int format, const void* const*
         const size_t grid = follows ? launch.alone_grid : launch.grid;
         const dim3 gd((unsigned)grid), bd((unsigned)(waves * (int)kWave));
         const bool many = (uint64_t)n >= kSubQueueMinPerWave * (uint64_t)waves * (uint64_t)grid;
-        const int subs = launch.direct ? 2 : many ? 1 : 0;
+        const int subs = launch.wide ? 3 : launch.direct ? 2 : many ? 1 : 0;
         const int shape = (parse_only ? 16 : 0) | (f ? 8 : 0) | (pipes ? 0 : 4) | subs;
         switch (shape) {
 #define CUDEC_PIPED(kShape, kFmt, kS, kP)                                                 \
@@ -1961,6 +1992,15 @@ hipError_t queue_and_decode(const Launch& launch, int format, const void* const*
         hipLaunchKernelGGL((alone_batch<kFmt, kS, kP>), gd, bd, 0, stream, srcs,          \
                            src_sizes, dsts, caps, n, results, q, order, follows);         \
         break;
+#define CUDEC_WIDE(kShape, kP)                                                            \
+    case kShape:                                                                          \
+        hipLaunchKernelGGL((piped_batch<kFormatLz4, 0, kP, kSegmentWide>), gd, bd, 0,     \
+                           stream, srcs, src_sizes, dsts, caps, n, results, q, order,     \
+                           plan);                                                         \
+        break;
+            CUDEC_WIDE(3, false)
+            CUDEC_WIDE(19, true)
+#undef CUDEC_WIDE
             CUDEC_PIPED(0, kFormatLz4, 1, false)
             CUDEC_PIPED(1, kFormatLz4, kSubQueues, false)
             CUDEC_PIPED(2, kFormatLz4, 0, false)

@@ -138,6 +138,33 @@ def test_launch_sizes_exact(fmt, n):
     check_against_oracle(fmt, "tuned", streams, caps)
 
 
+@pytest.mark.parametrize("launch", ["tuned-pipe", "tuned"])
+@pytest.mark.parametrize("copies", [1, 768, 769])
+def test_lz4_wide_windows_exact(launch, copies):
+    """Launches of up to three blocks a CU take windows of 12 KiB of at most
+    1920 members: sources around one and two of them behind the first 2 KiB,
+    of the shortest sequences and of ones that jump, alone and on both sides
+    of the line between the two widths."""
+    streams = []
+    for size in (12287, 12288, 12289, 14335, 14336, 14337, 26623, 26625, 60000):
+        for longest in (4, 19, 300):
+            w = Writer(size + longest)
+            while len(w.out) + 40 < size:
+                near = w.rng.random() < 0.7
+                w.put(int(w.rng.integers(0, 2)) if near else int(w.rng.integers(0, 400)),
+                      int(w.rng.integers(1, 30 if near else 60000)),
+                      int(w.rng.integers(4, longest + 1)))
+            streams.append(w.done(max(12, min(size - len(w.out) - 1, 14))))
+    caps = [len(oracle_decode("lz4", s, 1 << 22)[1]) for s in streams]
+    streams += [streams[1][:-3], streams[7][:9000], streams[11]]
+    caps += [caps[1], caps[7], caps[11] - 1]
+    if copies > 1:
+        streams = [streams[i % len(streams)] for i in range(copies)]
+        caps = [caps[i % len(caps)] for i in range(copies)]
+    print(f"[wide windows] {len(streams)} chunks, {launch}", flush=True)
+    check_against_oracle("lz4", launch, streams, caps)
+
+
 @pytest.mark.parametrize("fmt", ["lz4", "snappy"])
 @pytest.mark.parametrize("big", [0, 1])
 @pytest.mark.parametrize("n", [2049, 90000])
