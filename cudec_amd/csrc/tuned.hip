@@ -934,6 +934,7 @@ constexpr uint32_t kSegment = 128;
 constexpr uint32_t kSegmentWide = 192;
 constexpr uint32_t kSegmentFirst = 32;
 constexpr uint32_t stage_rounds(uint32_t bytes) { return (bytes / 16 + 1 + kWave - 1) / kWave; }
+constexpr uint32_t kStageRoundsUsual = stage_rounds(stage_bytes(kSegment * kWave));
 constexpr uint32_t kStageRoundsFirst = stage_rounds(stage_bytes(kSegmentFirst * kWave));
 static_assert(stage_rounds(stage_bytes(kCandSplit * kWave)) == 1, "one-wave stage");
 /* Members listed of one window; a window that holds more ends there. */
@@ -1170,8 +1171,10 @@ __device__ __forceinline__ void run_parser(L& l, gcu8* src, uint64_t src_size, u
         segment = spread < segment ? spread : segment;
         const uint32_t limit = stage_bytes(segment * kWave);
         const uint32_t delta =
-            segment > kSegmentFirst
+            kSeg > kSegment && segment > kSegment
                 ? stage_into<kStageRounds>(stage, src, src_size, base, limit, lane)
+            : segment > kSegmentFirst
+                ? stage_into<kStageRoundsUsual>(stage, src, src_size, base, limit, lane)
                 : stage_into<kStageRoundsFirst>(stage, src, src_size, base, limit, lane);
         const uint32_t touch = touch_ahead(src, src_size, base, limit, kSeg, lane);
         const uint8_t* cw = stage + delta;
@@ -1180,7 +1183,9 @@ __device__ __forceinline__ void run_parser(L& l, gcu8* src, uint64_t src_size, u
             walk_window<kFormat, list_max(kSeg)>(cw, segment, limit, lim, list, count, lane);
         bool last = false;
         uint64_t next_base = base + next;
-        segment = kSeg;
+        /* a wide window only behind one that was not cut short: what it stages
+         * past a cut is staged in vain */
+        segment = segment < kSegment ? kSegment : kSeg;
         if ((next & kWalkStop) != 0) {
             /* only where the member ends matters here (the copiers decide
              * what it is worth): the exact ladder, with room for any output */
