@@ -925,7 +925,7 @@ static_assert(kPipeBatch <= 64 * kWave, "CoverLds marks a batch");
  * blocks a CU at 128, three at 192, and a full chip needs the fourth (the
  * uneven LZ4 batch: 17.5 ms, 20.1 with 192 and 21.7 with 64 and three waves
  * on five blocks). So LZ4 launches that have a block of three a CU for every
- * chunk take 192 (16 chunks of 4 KiB to 1 MiB: 1.44 -> 1.31 ms; 700 of 256
+ * chunk take 192 (16 chunks of 4 KiB to 1 MiB: 1.46 -> 1.34 ms; 700 of 256
  * KiB: 0.57 -> 0.52), all others 128. Snappy's chains meet sooner and gain
  * nothing (700 of 256 KiB: 0.79 ms, 0.82 with 192). A chunk's first window,
  * and one after a window cut short, is a small one, so that its members
