@@ -20,8 +20,9 @@
  * the 128 bits on top and choosing words of them, 62 instructions and 338.)
  * Everything that does not feed the next state (code baselines, repeat
  * offsets, limits, positions) is done per 64 sequences, a lane each: 37
- * cycles a sequence, the repeat offsets as a scan over maps (one after the
- * other on the scalar unit they took 190). The copies on the other wave take
+ * cycles a sequence, the repeat offsets as a scan over maps of three bytes (one
+ * after the other on the scalar unit they took 190 cycles a sequence; as maps
+ * that held the distances 8192 frames of 64 KiB took 2.34 ms, and 2.27 so). The copies on the other wave take
  * about 200.
  *
  * One wave a frame with one sequence decoded and executed after the other
@@ -250,32 +251,49 @@ __device__ __forceinline__ bool build_cells(const int16_t* counts, uint16_t* nex
     return true;
 }
 
-/* The three repeat offsets after some sequences, in terms of those before
- * them: a distance (kFarthest for every one beyond, past any window
- * and refused), or kRepeat<i> less the ones that code 3 without literals
- * took off the offset i before (64 at most in a batch). */
+/* The three repeat offsets after some sequences of a batch, in terms of those
+ * before them, a byte each: the offset before that it comes from (0 to 2), or
+ * kOwn and the lane of the sequence that brought a distance of its own;
+ * beside it, how often code 3 without literals took one off (64 at most). The
+ * distances themselves stay where they are, so they may be any of 32 bits:
+ * the window of a single-segment frame is its content size, and offset code
+ * 31 names distances up to 2^32 - 4 that are decoded. */
 struct Repeats {
-    uint32_t a, b, c;
+    uint32_t from, less;
 };
-constexpr uint32_t kRepeat0 = 0x80000100u, kRepeat1 = 0x90000100u, kRepeat2 = 0xA0000100u;
-constexpr uint32_t kFarthest = 0x7FFFFFFFu; /* no distance looks like a reference */
-static_assert(zstd::kWindowMax < kFarthest, "refused");
-__device__ __forceinline__ uint32_t of_repeats(uint32_t v, uint32_t a, uint32_t b, uint32_t c) {
-    const uint32_t i = v >> 28;
-    const uint32_t at = i == 8 ? a : i == 9 ? b : c;
-    return (int32_t)v < 0 ? at + (v & 0x0FFFFFFFu) - 0x100u : v;
-}
+static_assert(zstd::kOffsetMax < 32, "every distance fits 32 bits");
+constexpr uint32_t kSame = 0x020100, kOwn = 0x80;
 /* r after what the lane that DPP pattern kCtrl names has composed so far;
  * unchanged on lanes without one. */
 template <int kCtrl, int kRows>
 __device__ __forceinline__ Repeats repeats_after(const Repeats& r) {
-    const uint32_t a = (uint32_t)__builtin_amdgcn_update_dpp((int)kRepeat0, (int)r.a, kCtrl, kRows,
-                                                             0xF, false);
-    const uint32_t b = (uint32_t)__builtin_amdgcn_update_dpp((int)kRepeat1, (int)r.b, kCtrl, kRows,
-                                                             0xF, false);
-    const uint32_t c = (uint32_t)__builtin_amdgcn_update_dpp((int)kRepeat2, (int)r.c, kCtrl, kRows,
-                                                             0xF, false);
-    return Repeats{of_repeats(r.a, a, b, c), of_repeats(r.b, a, b, c), of_repeats(r.c, a, b, c)};
+    const uint32_t from = (uint32_t)__builtin_amdgcn_update_dpp((int)kSame, (int)r.from, kCtrl,
+                                                                kRows, 0xF, false);
+    const uint32_t less =
+        (uint32_t)__builtin_amdgcn_update_dpp(0, (int)r.less, kCtrl, kRows, 0xF, false);
+    /* v_perm selectors: the byte of the one before that it comes from, or, of
+     * its own, itself (4 to 6) */
+    const uint32_t own = __umul24((r.from >> 7) & 0x010101u, 0xFFu);
+    const uint32_t pick = (own & 0x060504u) | (~own & r.from);
+    return Repeats{__builtin_amdgcn_perm(r.from, from, pick),
+                   r.less + __builtin_amdgcn_perm(0u, less, pick)};
+}
+
+/* The offset that byte 0 of a map stands for, given those before the batch
+ * and, if it is one of the batch's own, that. */
+__device__ __forceinline__ uint32_t offset_of(uint32_t from, uint32_t less, uint32_t own,
+                                              uint32_t b0, uint32_t b1, uint32_t b2) {
+    uint32_t d = b0;
+    if ((from & 1) != 0) {
+        d = b1;
+    }
+    if ((from & 2) != 0) {
+        d = b2;
+    }
+    if ((from & kOwn) != 0) {
+        d = own;
+    }
+    return d - (less & 0xFF);
 }
 
 /* One sequence field's table. */
@@ -552,29 +570,34 @@ struct EntropyFlow {
         /* repeat offsets (RFC 8878 3.1.1.5): each sequence maps the three
          * offsets before it to the three after it, its own distance first;
          * an inclusive scan composes the maps (Repeats). Zero: an error. */
-        const uint32_t which = value - 1 + (llen == 0 ? 1u : 0u);
-        Repeats r = {kRepeat0, kRepeat1, kRepeat2};
-        if (in && value > 3) {
-            const uint32_t d = value - 3;
-            r = Repeats{d < kFarthest ? d : kFarthest, kRepeat0, kRepeat1};
-        } else if (in && which != 0) {
-            r = Repeats{which == 1   ? kRepeat1
-                        : which == 2 ? kRepeat2
-                                     : kRepeat0 - 1,
-                        kRepeat0, which == 1 ? kRepeat2 : kRepeat1};
-        }
+        const uint32_t which = in ? value - 1 + (llen == 0 ? 1u : 0u) : 0;
+        const bool own = in && value > 3;
+        /* of 0 to 3: the first from {0, 1, 2, 0}, the third from {2, 2, 1, 1}
+         * by v_perm, the second 1 or 0 */
+        const uint32_t old = __builtin_amdgcn_perm(0x01010202u, 0x00020100u,
+                                                   __umul24(which & 3, 0x10001u) + 0x0C040C00u) |
+                             (which == 0 ? 0x100u : 0u);
+        Repeats r = {own ? 0x010000u | kOwn | lane : old, which == 3 && !own ? 1u : 0u};
         r = repeats_after<0x111, 0xF>(r); /* row_shr:1, 2, 4, 8 */
         r = repeats_after<0x112, 0xF>(r);
         r = repeats_after<0x114, 0xF>(r);
         r = repeats_after<0x118, 0xF>(r);
         r = repeats_after<0x142, 0xA>(r); /* row_bcast:15, 31 */
         r = repeats_after<0x143, 0xC>(r);
-        r = Repeats{of_repeats(r.a, r0, r1, r2), of_repeats(r.b, r0, r1, r2),
-                    of_repeats(r.c, r0, r1, r2)};
-        const uint32_t dist = r.a;
-        r0 = uniform32(__builtin_amdgcn_readlane(r.a, kWave - 1));
-        r1 = uniform32(__builtin_amdgcn_readlane(r.b, kWave - 1));
-        r2 = uniform32(__builtin_amdgcn_readlane(r.c, kWave - 1));
+        const uint32_t brought = value - 3;
+        const uint32_t mine = (uint32_t)__shfl((int)brought, (int)(r.from & (kWave - 1)));
+        /* (read before the choice: a choice of members becomes a load at a
+         * chosen scratch address, 600 cycles) */
+        const uint32_t b0 = uniform32(r0), b1 = uniform32(r1), b2 = uniform32(r2);
+        const uint32_t dist = offset_of(r.from, r.less, mine, b0, b1, b2);
+        const uint32_t from = uniform32(__builtin_amdgcn_readlane(r.from, kWave - 1));
+        const uint32_t less = uniform32(__builtin_amdgcn_readlane(r.less, kWave - 1));
+        r0 = offset_of(from, less, __builtin_amdgcn_readlane(brought, from & (kWave - 1)), b0, b1,
+                       b2);
+        r1 = offset_of(from >> 8, less >> 8,
+                       __builtin_amdgcn_readlane(brought, (from >> 8) & (kWave - 1)), b0, b1, b2);
+        r2 = offset_of(from >> 16, less >> 16,
+                       __builtin_amdgcn_readlane(brought, (from >> 16) & (kWave - 1)), b0, b1, b2);
         /* positions: a block's regenerated literals and output fit 32 bits
          * whatever the lengths claim (64 of at most 2^17 + 2^16 each) */
         const uint32_t lit_incl = wave_inclusive_sum(llen, lane);
