@@ -6,7 +6,6 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
-#include <functional>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -47,8 +46,10 @@ public:
     CopyCrew& operator=(const CopyCrew&) = delete;
 
     /* work(i) for every i below n, on any of the threads; work does not
-     * throw. Returns when all are done. */
-    void each(size_t n, const std::function<void(size_t)>& work) {
+     * throw. Returns when all are done. Allocates nothing: it runs while
+     * transfers are in flight, where a failure has to drain them first. */
+    template <class Work>
+    void each(size_t n, const Work& work) {
         if (threads_.empty()) {
             for (size_t i = 0; i < n; i++) {
                 work(i);
@@ -58,13 +59,14 @@ public:
         {
             std::lock_guard<std::mutex> hold(lock_);
             work_ = &work;
+            call_ = [](const void* w, size_t i) { (*static_cast<const Work*>(w))(i); };
             count_ = n;
             next_.store(0);
             busy_ = threads_.size();
             round_++;
         }
         wake_.notify_all();
-        claim(n, work);
+        claim(n, call_, work_);
         std::unique_lock<std::mutex> hold(lock_);
         idle_.wait(hold, [this] { return busy_ == 0; });
     }
@@ -73,9 +75,11 @@ private:
     static constexpr size_t kBytesPerHelper = size_t{8} << 20;
     static constexpr size_t kMostHelpers = 7;
 
-    void claim(size_t n, const std::function<void(size_t)>& work) {
+    using Call = void (*)(const void* work, size_t i);
+
+    void claim(size_t n, Call call, const void* work) {
         for (size_t i = next_.fetch_add(1); i < n; i = next_.fetch_add(1)) {
-            work(i);
+            call(work, i);
         }
     }
     void help() {
@@ -88,9 +92,10 @@ private:
             }
             seen = round_;
             const size_t n = count_;
-            const std::function<void(size_t)>& work = *work_;
+            const Call call = call_;
+            const void* const work = work_;
             hold.unlock();
-            claim(n, work);
+            claim(n, call, work);
             hold.lock();
             if (--busy_ == 0) {
                 idle_.notify_one();
@@ -100,7 +105,8 @@ private:
 
     std::mutex lock_;
     std::condition_variable wake_, idle_;
-    const std::function<void(size_t)>* work_ = nullptr;
+    const void* work_ = nullptr;
+    Call call_ = nullptr;
     size_t count_ = 0, round_ = 0, busy_ = 0;
     std::atomic<size_t> next_{0};
     bool quit_ = false;

@@ -152,6 +152,29 @@ cudec_status unpack_wave(const Slot& s, cudec_chunk_result* pres, void* const* d
     return CUDEC_OK;
 }
 
+/* Waits, at the latest where the call ends, whichever way it does, for
+ * everything its slots' streams hold: nothing of a call outlives it. */
+class Drain {
+public:
+    Drain(cudec_stream_ctx& ctx, size_t used) : ctx_(ctx), used_(used) {}
+    ~Drain() { (void)now(); }
+    Drain(const Drain&) = delete;
+    Drain& operator=(const Drain&) = delete;
+
+    hipError_t now() {
+        hipError_t first = hipSuccess;
+        for (; used_ != 0; used_--) {
+            const hipError_t e = hipStreamSynchronize(ctx_.slot[used_ - 1].stream.get());
+            first = first == hipSuccess ? e : first;
+        }
+        return first;
+    }
+
+private:
+    cudec_stream_ctx& ctx_;
+    size_t used_;
+};
+
 cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
                            const size_t* h_src_sizes, void* const* dst_ptrs,
                            const size_t* dst_caps, size_t n, cudec_mem_space space,
@@ -210,6 +233,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     cudec_chunk_result* pres = static_cast<cudec_chunk_result*>(ctx.p_results.data());
     stamp(pres, n, CUDEC_ERR_CUDA);
     cudec_status failure = CUDEC_OK;
+    Drain drain(ctx, used);
     CopyCrew crew(total);
 
     for (size_t w = 0; w < waves && failure == CUDEC_OK; w++) {
@@ -300,11 +324,10 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
             }
         }
     }
-    /* drain: nothing of this call outlives it */
+    if (drain.now() != hipSuccess && failure == CUDEC_OK) {
+        failure = CUDEC_ERR_CUDA;
+    }
     for (size_t k = 0; k < used; k++) {
-        if (hipStreamSynchronize(ctx.slot[k].stream.get()) != hipSuccess && failure == CUDEC_OK) {
-            failure = CUDEC_ERR_CUDA;
-        }
         ctx.slot[k].landed_pending = false;
     }
     if (hipGetLastError() != hipSuccess && failure == CUDEC_OK) {
