@@ -60,7 +60,8 @@ struct Slot {
 }  // namespace cudec_amd
 
 struct cudec_stream_ctx {
-    cudec_amd::Slot slot[cudec_amd::kSlots];
+    cudec_amd::Slot slot[cudec_amd::kSlots]; /* the first has its stream; the others on first use */
+    int device = 0;                          /* the streams' */
     cudec_amd::DeviceRegion d_results;
     cudec_amd::PinnedRegion p_results;
     bool poisoned = false;
@@ -152,6 +153,29 @@ cudec_status unpack_wave(const Slot& s, cudec_chunk_result* pres, void* const* d
     return CUDEC_OK;
 }
 
+/* Gives a slot its stream and event, on the context's device. */
+hipError_t open_slot(Slot& s, int device) {
+    if (s.stream && s.landed) {
+        return hipSuccess;
+    }
+    int now = 0;
+    hipError_t e = hipGetDevice(&now);
+    if (e == hipSuccess && now != device) {
+        e = hipSetDevice(device);
+    }
+    if (e == hipSuccess && !s.stream) {
+        e = make_stream(s.stream);
+    }
+    if (e == hipSuccess) {
+        e = make_sync_event(s.landed);
+    }
+    if (now != device) {
+        const hipError_t back = hipSetDevice(now);
+        e = e == hipSuccess ? back : e;
+    }
+    return e;
+}
+
 /* Waits, at the latest where the call ends, whichever way it does, for
  * everything its slots' streams hold: nothing of a call outlives it. */
 class Drain {
@@ -217,7 +241,8 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     bool ok = true;
     for (size_t k = 0; k < used && ok; k++) {
         Slot& s = ctx.slot[k];
-        ok = s.p_src.reserve(max_src) == hipSuccess && s.d_src.reserve(max_src) == hipSuccess &&
+        ok = open_slot(s, ctx.device) == hipSuccess &&
+             s.p_src.reserve(max_src) == hipSuccess && s.d_src.reserve(max_src) == hipSuccess &&
              s.p_meta.reserve(meta_bytes) == hipSuccess &&
              s.d_meta.reserve(meta_bytes) == hipSuccess &&
              (!host_out || (s.d_dst.reserve(max_dst) == hipSuccess &&
@@ -365,11 +390,10 @@ cudec_status cudec_stream_ctx_create(cudec_stream_ctx** out_ctx) {
     if (ctx == nullptr) {
         return CUDEC_ERR_CUDA;
     }
-    for (Slot& s : ctx->slot) {
-        if (make_stream(s.stream) != hipSuccess || make_sync_event(s.landed) != hipSuccess) {
-            delete ctx;
-            return CUDEC_ERR_CUDA;
-        }
+    if (hipGetDevice(&ctx->device) != hipSuccess ||
+        open_slot(ctx->slot[0], ctx->device) != hipSuccess) {
+        delete ctx;
+        return CUDEC_ERR_CUDA;
     }
     *out_ctx = ctx;
     return CUDEC_OK;
@@ -407,7 +431,9 @@ void cudec_stream_ctx_destroy(cudec_stream_ctx* ctx) {
         return;
     }
     for (Slot& s : ctx->slot) {
-        (void)hipStreamSynchronize(s.stream.get());
+        if (s.stream) {
+            (void)hipStreamSynchronize(s.stream.get());
+        }
     }
     delete ctx;
 }

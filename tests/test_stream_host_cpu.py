@@ -1,0 +1,93 @@
+"""What the streaming call makes and keeps, and in which order it moves bytes:
+cudec_amd/csrc/stream.cpp over a stand-in for the HIP runtime on the CPU
+(tests/stream_host.cpp), where a chunk decodes to its own bytes.
+
+* a context makes the streams that its calls need, no more;
+* results and bytes of calls of one and of many waves."""
+import ctypes
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from tests import libs
+
+BUILD = os.path.join(libs.ROOT, "tests", "_build")
+RES = np.dtype([("status", "<i4"), ("reserved", "<u4"), ("bytes_written", "<u8")])
+MIB = 1 << 20
+HOST = 0
+
+
+@pytest.fixture(scope="module")
+def lib():
+    os.makedirs(BUILD, exist_ok=True)
+    out = os.path.join(BUILD, "libstream_host.so")
+    subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-Wall", "-Wextra", "-Werror", "-fPIC",
+                    "-shared", "-pthread", "-Wl,-Bsymbolic", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(libs.ROOT, "include"),
+                    "-I", os.path.join(libs.ROOT, "cudec_amd", "csrc"), "-I/opt/rocm/include",
+                    "-o", out, os.path.join(libs.ROOT, "tests", "stream_host.cpp")], check=True)
+    lib = ctypes.CDLL(out)
+    vp, sz = ctypes.c_void_p, ctypes.c_size_t
+    lib.cudec_stream_ctx_create.argtypes = [ctypes.POINTER(vp)]
+    lib.cudec_stream_ctx_destroy.argtypes = [vp]
+    lib.cudec_stream_ctx_destroy.restype = None
+    lib.cudec_lz4_decompress_stream_ctx.argtypes = [vp, vp, vp, vp, vp, sz, ctypes.c_int, vp]
+    lib.host_stream_counts.argtypes = [vp]
+    lib.host_stream_counts.restype = None
+    return lib
+
+
+def counts(lib):
+    c = np.zeros(5, np.uint64)
+    lib.host_stream_counts(c.ctypes.data)
+    return dict(zip(("streams", "events", "held", "most", "open"), (int(v) for v in c)))
+
+
+class Context:
+    def __init__(self, lib):
+        self.lib, self.h = lib, ctypes.c_void_p()
+        assert lib.cudec_stream_ctx_create(ctypes.byref(self.h)) == 0
+
+    def run(self, src, sizes, dst, caps):
+        """Pointers and sizes as lists; (status, results)."""
+        n = len(sizes)
+        a = [np.array(v, dtype=np.uint64) for v in (src, sizes, dst, caps)]
+        res = np.zeros(n, RES)
+        st = self.lib.cudec_lz4_decompress_stream_ctx(
+            self.h, *(v.ctypes.data for v in a), n, HOST, res.ctypes.data)
+        return st, res
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        self.lib.cudec_stream_ctx_destroy(self.h)
+
+
+def plain(ctx, n, size):
+    """A call of n chunks of `size` bytes, checked."""
+    data = np.random.default_rng(n).integers(0, 256, n * size, dtype=np.uint8)
+    out = np.zeros(n * size, np.uint8)
+    at = size * np.arange(n, dtype=np.uint64)
+    st, res = ctx.run(at + np.uint64(data.ctypes.data), [size] * n,
+                      at + np.uint64(out.ctypes.data), [size] * n)
+    assert st == 0 and np.all(res["status"] == 0) and np.all(res["bytes_written"] == size)
+    assert np.array_equal(out, data)
+
+
+# chunks of 1 MiB in and out: 24 MiB a wave at least, four waves at once
+@pytest.mark.parametrize("n,streams", [(1, 1), (23, 1), (24, 2), (40, 3), (60, 4), (200, 4)])
+def test_streams_of_a_context(lib, n, streams):
+    before = counts(lib)
+    with Context(lib) as ctx:
+        made = counts(lib)
+        assert made["streams"] - before["streams"] == 1
+        assert made["events"] - before["events"] == 1
+        for _ in range(2):
+            plain(ctx, n, MIB)
+        made = counts(lib)
+        assert made["streams"] - before["streams"] == streams
+        assert made["events"] - before["events"] == streams
+    assert counts(lib)["open"] == before["open"]
