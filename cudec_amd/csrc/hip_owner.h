@@ -6,7 +6,7 @@
  * is replaced or goes out of scope; it moves but does not copy.
  * Region<Space> is a grow-only byte area in one memory space, built on a
  * Handle: reserve(n) keeps the area while it already holds n bytes and
- * otherwise replaces it with one of exactly n bytes. */
+ * otherwise replaces it with one of exactly n bytes; release() gives it back. */
 #ifndef CUDEC_AMD_HIP_OWNER_H
 #define CUDEC_AMD_HIP_OWNER_H
 
@@ -112,6 +112,11 @@ public:
             bytes_ = n;
         }
         return e;
+    }
+
+    void release() {
+        mem_.adopt(nullptr);
+        bytes_ = 0;
     }
 
 private:

@@ -153,6 +153,19 @@ cudec_status unpack_wave(const Slot& s, cudec_chunk_result* pres, void* const* d
     return CUDEC_OK;
 }
 
+/* Bytes (of the device's, and as many pinned) that the slots hold once the
+ * first `used` hold waves of src and dst bytes. */
+size_t staging(const cudec_stream_ctx& ctx, size_t used, size_t src, size_t dst) {
+    size_t sum = 0;
+    for (size_t k = 0; k < kSlots; k++) {
+        const size_t hs = ctx.slot[k].d_src.capacity(), hd = ctx.slot[k].d_dst.capacity();
+        const size_t s = k < used && src > hs ? src : hs, d = k < used && dst > hd ? dst : hd;
+        const size_t both = SIZE_MAX - s < d ? SIZE_MAX : s + d;
+        sum = SIZE_MAX - sum < both ? SIZE_MAX : sum + both;
+    }
+    return sum;
+}
+
 /* Gives a slot its stream and event, on the context's device. */
 hipError_t open_slot(Slot& s, int device) {
     if (s.stream && s.landed) {
@@ -228,10 +241,24 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
         total = SIZE_MAX - total < ws ? SIZE_MAX : total + ws;
         total = SIZE_MAX - total < wd ? SIZE_MAX : total + wd;
     }
-    /* two slots where four would stage more than two full budgets */
-    const size_t most = kWaveBudget / 2;
-    const size_t slots = max_src > most || max_dst > most - max_src ? 2 : kSlots;
-    const size_t used = waves < slots ? waves : slots;
+    /* two slots where four would stage more than two full budgets, with what
+     * the slots keep of earlier calls; that much is what a context keeps,
+     * unless a chunk of this call is larger than a budget */
+    size_t slots = kSlots;
+    size_t used = waves < slots ? waves : slots;
+    const size_t wave_dst = host_out ? max_dst : 0;
+    if (staging(ctx, used, max_src, wave_dst) > 2 * kWaveBudget) {
+        slots = 2;
+        used = waves < slots ? waves : slots;
+        if (staging(ctx, used, max_src, wave_dst) > 2 * kWaveBudget) {
+            for (size_t k = slots; k < kSlots; k++) {
+                ctx.slot[k].p_src.release();
+                ctx.slot[k].d_src.release();
+                ctx.slot[k].p_dst.release();
+                ctx.slot[k].d_dst.release();
+            }
+        }
+    }
     if (n > SIZE_MAX / sizeof(cudec_chunk_result)) {
         return CUDEC_ERR_CORRUPT_INPUT;
     }

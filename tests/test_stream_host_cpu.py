@@ -3,6 +3,8 @@ cudec_amd/csrc/stream.cpp over a stand-in for the HIP runtime on the CPU
 (tests/stream_host.cpp), where a chunk decodes to its own bytes.
 
 * a context makes the streams that its calls need, no more;
+* what it keeps for the next call stays within two budgets of staging (1 GiB
+  each, or the largest chunk);
 * results and bytes of calls of one and of many waves."""
 import ctypes
 import os
@@ -91,3 +93,21 @@ def test_streams_of_a_context(lib, n, streams):
         assert made["streams"] - before["streams"] == streams
         assert made["events"] - before["events"] == streams
     assert counts(lib)["open"] == before["open"]
+
+
+@pytest.mark.parametrize("calls", ["AB", "BA", "ABAB", "CAB"])
+def test_staging_kept(lib, calls):
+    """A: four chunks of 480 MiB of room, a slot each; B: two of 900 MiB, which
+    two slots take; C: nine of 100 MiB. (A byte each of input.)"""
+    shapes = {"A": (4, 480 * MIB), "B": (2, 900 * MIB), "C": (9, 100 * MIB)}
+    src = np.full(16, 7, np.uint8)
+    out = np.empty(1920 * MIB, np.uint8)  # hardly touched
+    with Context(lib) as ctx:
+        for c in calls:
+            n, cap = shapes[c]
+            st, res = ctx.run([src.ctypes.data] * n, [1] * n,
+                              [out.ctypes.data + i * cap for i in range(n)], [cap] * n)
+            assert st == 0 and np.all(res["bytes_written"] == 1)
+            # tables and results are a few hundred bytes here
+            assert counts(lib)["held"] <= 2 * 1024 * MIB + 4096, (calls, c)
+        plain(ctx, 60, MIB)
