@@ -17,6 +17,8 @@ namespace cudec_amd {
  * (small calls, one core, threads refused) the caller does everything. */
 class CopyCrew {
 public:
+    static constexpr size_t kBytesPerHelper = size_t{8} << 20;
+
     /* `bytes`: what the call copies in all. A helper costs about 20 us to
      * start, and more than seven do not copy faster. */
     explicit CopyCrew(size_t bytes) {
@@ -72,7 +74,6 @@ public:
     }
 
 private:
-    static constexpr size_t kBytesPerHelper = size_t{8} << 20;
     static constexpr size_t kMostHelpers = 7;
 
     using Call = void (*)(const void* work, size_t i);

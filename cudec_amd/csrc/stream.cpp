@@ -21,9 +21,11 @@
  * thread and one wave did in a row with the transfers: 18.3 ms, 5.5 so. */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <new>
+#include <vector>
 
 #include "cudec.h"
 #include "hip_owner.h"
@@ -97,7 +99,76 @@ void stamp(cudec_chunk_result* r, size_t n, cudec_status st) {
     }
 }
 
-size_t choose_wave(const size_t* src_sizes, const size_t* caps, size_t n, bool host_out) {
+/* Whether a host destination of the call lies over the source of a later
+ * chunk or over another destination: programs decode within one arena, or
+ * many chunks into one buffer of which they want the last, or none. (Over its
+ * own source or an earlier one is no matter: those are read by then.) 3 ns a
+ * chunk where buffers ascend, up to 140 where they lie in any order. */
+bool buffers_meet(const void* const* src, const size_t* src_sizes, void* const* dst,
+                  const size_t* caps, size_t n) {
+    struct Range {
+        uintptr_t begin, end;
+        size_t chunk;
+    };
+    const auto range = [](const void* p, size_t len, size_t i) {
+        const uintptr_t b = reinterpret_cast<uintptr_t>(p);
+        return Range{b, UINTPTR_MAX - b < len ? UINTPTR_MAX : b + len, i};
+    };
+    size_t total = 0;
+    for (size_t i = 0; i < n && total < CopyCrew::kBytesPerHelper; i++) {
+        total += src_sizes[i] < CopyCrew::kBytesPerHelper ? src_sizes[i]
+                                                          : CopyCrew::kBytesPerHelper;
+        total += caps[i] < CopyCrew::kBytesPerHelper ? caps[i] : CopyCrew::kBytesPerHelper;
+    }
+    if (total < CopyCrew::kBytesPerHelper) {
+        return false; /* one wave and one thread in any case */
+    }
+    std::vector<Range> out;
+    out.reserve(n);
+    for (size_t i = 0; i < n; i++) {
+        if (caps[i] != 0) {
+            out.push_back(range(dst[i], caps[i], i));
+        }
+    }
+    if (out.empty()) {
+        return false;
+    }
+    const auto before = [](const Range& x, const Range& y) { return x.begin < y.begin; };
+    if (!std::is_sorted(out.begin(), out.end(), before)) {
+        std::sort(out.begin(), out.end(), before);
+    }
+    for (size_t k = 1; k < out.size(); k++) {
+        if (out[k].begin < out[k - 1].end) {
+            return true;
+        }
+    }
+    /* from the last one that ends at or before the source, which is near the
+     * one of the source before where buffers ascend */
+    size_t steps = 4 * n; /* sources that cover ever so many destinations: true */
+    size_t k = 0;
+    for (size_t i = 0; i < n; i++) {
+        const Range s = range(src[i], src_sizes[i], i);
+        if (s.begin == s.end || s.begin >= out.back().end || s.end <= out.front().begin) {
+            continue;
+        }
+        if (out[k].begin > s.begin || (k + 4 < out.size() && out[k + 4].begin <= s.begin)) {
+            const auto o = std::upper_bound(out.begin(), out.end(), s, before);
+            k = o == out.begin() ? 0 : static_cast<size_t>(o - out.begin()) - 1;
+        }
+        while (k < out.size() - 1 && out[k].end <= s.begin) {
+            k++;
+        }
+        for (size_t j = k; j < out.size() && out[j].begin < s.end; j++) {
+            if (out[j].end > s.begin && (out[j].chunk < i || steps-- == 0)) {
+                return true;
+            }
+        }
+    }
+    return false;
+}
+
+size_t choose_wave(const size_t* src_sizes, const size_t* caps, size_t n, bool host_out,
+                   bool in_order) {
     size_t biggest = 1, total = 0;
     for (size_t i = 0; i < n; i++) {
         size_t b = src_sizes[i];
@@ -116,7 +187,7 @@ size_t choose_wave(const size_t* src_sizes, const size_t* caps, size_t n, bool h
     if (wave > kWaveChunksMax) {
         wave = kWaveChunksMax;
     }
-    size_t parts = total / kWaveBytesMin;
+    size_t parts = in_order ? 1 : total / kWaveBytesMin;
     parts = parts < 1 ? 1 : parts > kWavesWanted ? kWavesWanted : parts;
     const size_t part = (n + parts - 1) / parts;
     return wave > part ? part : wave;
@@ -218,7 +289,13 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
                            cudec_chunk_result* h_results) {
     const bool host_out = space == CUDEC_MEM_HOST;
     stamp(h_results, n, CUDEC_ERR_CUDA);
-    const size_t wave = choose_wave(h_src_sizes, dst_caps, n, host_out);
+    /* buffers that meet keep the order that a call has with one thread and two
+     * slots: a wave is as large as the budget lets it be, it is read whole
+     * before its first byte is written, and chunks are written one after the
+     * other */
+    const bool in_order =
+        host_out && buffers_meet(h_src_ptrs, h_src_sizes, dst_ptrs, dst_caps, n);
+    const size_t wave = choose_wave(h_src_sizes, dst_caps, n, host_out, in_order);
     const size_t waves = (n + wave - 1) / wave;
     size_t max_src = 1, max_dst = 1, total = 0;
     for (size_t w = 0; w < waves; w++) {
@@ -244,7 +321,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     /* two slots where four would stage more than two full budgets, with what
      * the slots keep of earlier calls; that much is what a context keeps,
      * unless a chunk of this call is larger than a budget */
-    size_t slots = kSlots;
+    size_t slots = in_order ? 2 : kSlots;
     size_t used = waves < slots ? waves : slots;
     const size_t wave_dst = host_out ? max_dst : 0;
     if (staging(ctx, used, max_src, wave_dst) > 2 * kWaveBudget) {
@@ -286,7 +363,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     stamp(pres, n, CUDEC_ERR_CUDA);
     cudec_status failure = CUDEC_OK;
     Drain drain(ctx, used);
-    CopyCrew crew(total);
+    CopyCrew crew(in_order ? 0 : total);
 
     for (size_t w = 0; w < waves && failure == CUDEC_OK; w++) {
         Slot& s = ctx.slot[w % slots];

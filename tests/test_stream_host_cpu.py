@@ -5,6 +5,9 @@ cudec_amd/csrc/stream.cpp over a stand-in for the HIP runtime on the CPU
 * a context makes the streams that its calls need, no more;
 * what it keeps for the next call stays within two budgets of staging (1 GiB
   each, or the largest chunk);
+* host buffers of one call that lie over each other: what a call of one wave
+  gives, every source read before the first byte is written and chunks written
+  in order;
 * results and bytes of calls of one and of many waves."""
 import ctypes
 import os
@@ -111,3 +114,67 @@ def test_staging_kept(lib, calls):
             # tables and results are a few hundred bytes here
             assert counts(lib)["held"] <= 2 * 1024 * MIB + 4096, (calls, c)
         plain(ctx, 60, MIB)
+
+
+def streams_of(lib, ctx_calls):
+    before = counts(lib)["streams"]
+    with Context(lib) as ctx:
+        ctx_calls(ctx)
+        return counts(lib)["streams"] - before
+
+
+# (over its own source or an earlier one, it does not matter when it is written)
+@pytest.mark.parametrize("n,ahead,streams", [(200, 110, 1), (200, 1, 1), (60, 59, 1),
+                                             (200, -110, 4), (200, -1, 4), (200, 0, 4)])
+def test_outputs_over_sources(lib, n, ahead, streams):
+    """Chunk i's output lies where chunk i + ahead's input does."""
+    pad = max(0, -ahead)
+    arena = np.random.default_rng(5).integers(0, 256, (n + abs(ahead)) * MIB, dtype=np.uint8)
+    want = arena.copy()
+    for i in range(n):
+        want[(i + pad + ahead) * MIB:][:MIB] = arena[(i + pad) * MIB:][:MIB]
+    src = [arena.ctypes.data + (i + pad) * MIB for i in range(n)]
+    dst = [arena.ctypes.data + (i + pad + ahead) * MIB for i in range(n)]
+
+    def call(ctx):
+        st, res = ctx.run(src, [MIB] * n, dst, [MIB] * n)
+        assert st == 0 and np.all(res["bytes_written"] == MIB)
+    made = streams_of(lib, call)
+    assert np.array_equal(arena, want)
+    assert made == streams
+
+
+@pytest.mark.parametrize("step", [0, 1000])
+def test_outputs_over_outputs(lib, step):
+    """All outputs in one buffer, or each a little further on: the last chunk
+    over each byte is what stays."""
+    n = 200
+    data = np.random.default_rng(6).integers(0, 256, n * MIB, dtype=np.uint8)
+    out = np.zeros(MIB + n * step, np.uint8)
+    want = out.copy()
+    for i in range(n):
+        want[i * step:i * step + MIB] = data[i * MIB:(i + 1) * MIB]
+    with Context(lib) as ctx:
+        st, _ = ctx.run([data.ctypes.data + i * MIB for i in range(n)], [MIB] * n,
+                        [out.ctypes.data + i * step for i in range(n)], [MIB] * n)
+    assert st == 0 and np.array_equal(out, want)
+
+
+def test_buffers_side_by_side(lib):
+    """Inputs and outputs in turn, in any order, some of them empty: none lies
+    over another, and the call overlaps its waves."""
+    n = 200
+    arena = np.random.default_rng(7).integers(0, 256, 2 * n * MIB, dtype=np.uint8)
+    order = np.random.default_rng(8).permutation(n)
+    for places in (np.arange(n), order):
+        want = arena.copy()
+        for p in places:
+            want[(2 * p + 1) * MIB:][:MIB] = arena[2 * p * MIB:][:MIB]
+        src = [arena.ctypes.data + 2 * int(p) * MIB for p in places] + [0, 0]
+        dst = [s + MIB for s in src[:n]] + [0, arena.ctypes.data]
+
+        def call(ctx):
+            st, res = ctx.run(src, [MIB] * n + [0, 0], dst, [MIB] * n + [0, 0])
+            assert st == 0
+        assert streams_of(lib, call) == 4
+        assert np.array_equal(arena, want)
