@@ -1,0 +1,105 @@
+/* Decode plans: how the chunks of each cost bin are decoded. Internal, host
+ * code but for the cost's key. */
+#ifndef CUDEC_AMD_PLAN_H
+#define CUDEC_AMD_PLAN_H
+
+#include <stddef.h>
+#include <stdint.h>
+
+#if defined(__HIPCC__)
+#define CUDEC_HD __host__ __device__
+#else
+#define CUDEC_HD
+#endif
+
+namespace cudec_amd {
+
+constexpr uint32_t kOctaveBits = 2; /* cost bins per octave: 4 */
+constexpr int kBins = 64 << kOctaveBits;
+
+/* Default plans (LZ4, Snappy): chunks costing at least this (capacity +
+ * capacity - compressed) are pipelined. */
+constexpr uint64_t kDefaultPipeMinCost[2] = {128u << 10, 64u << 10};
+/* ... and in launches of few chunks: below this one wave is as fast (a 4 KiB
+ * token page alone: 36 us on one wave, 40 pipelined). */
+constexpr uint64_t kFewPipeMinCost = 8u << 10;
+
+/* Order-preserving key of a cost below 2^63: the octave and the next
+ * kOctaveBits bits below its leading one (costs below 2^kOctaveBits are
+ * their own key). */
+CUDEC_HD inline uint32_t cost_key(uint64_t cost) {
+    if (cost < (1u << kOctaveBits)) {
+        return (uint32_t)cost;
+    }
+    const uint32_t lg = 63u - (uint32_t)__builtin_clzll(cost);
+    return lg << kOctaveBits |
+           (uint32_t)((cost >> (lg - kOctaveBits)) & ((1u << kOctaveBits) - 1));
+}
+
+/* A decode plan: bit b (of word b / 64) set when cost bin b decodes on
+ * a pipelined block, clear for one wave. Passed to the kernels by value. */
+struct Plan {
+    uint64_t two_wave[kBins / 64];
+};
+
+CUDEC_HD inline bool plan_two_wave(const Plan& p, uint32_t bin) {
+    return ((p.two_wave[bin >> 6] >> (bin & 63)) & 1u) != 0;
+}
+
+/* The plan that pipelines chunks costing at least min_cost: every
+ * bin up to the bin of a chunk whose cost is exactly min_cost (costlier
+ * bins have smaller numbers). 0 takes every bin, UINT64_MAX none. */
+inline Plan plan_from_threshold(uint64_t min_cost) {
+    Plan p = {};
+    const int32_t last = min_cost == 0 ? kBins - 1
+                         : min_cost == UINT64_MAX ? -1
+                                                  : (int32_t)(kBins - 1 - cost_key(min_cost));
+    for (int32_t b = 0; b <= last; b++) {
+        p.two_wave[b >> 6] |= 1ull << (b & 63);
+    }
+    return p;
+}
+
+/* A format's plan on one device. */
+struct DecodePlan {
+    Plan plan;
+    uint64_t min_cost; /* the threshold last set */
+    bool chosen;       /* the caller (or a tuner for it) has set a plan */
+
+    static DecodePlan usual(int format) {
+        return {plan_from_threshold(kDefaultPipeMinCost[format]), kDefaultPipeMinCost[format],
+                false};
+    }
+    void set_threshold(uint64_t cost) {
+        plan = plan_from_threshold(cost);
+        min_cost = cost;
+        chosen = true;
+    }
+    void set_bins(const uint16_t* lanes) {
+        plan = {};
+        for (int b = 0; b < kBins; b++) {
+            if (lanes[b] == 128) {
+                plan.two_wave[b >> 6] |= 1ull << (b & 63);
+            }
+        }
+        chosen = true;
+    }
+    /* What a launch of n chunks follows. A launch of few chunks leaves most
+     * of the chip idle whatever it does, and takes as long as its largest
+     * chunk: unless a plan was chosen, all its chunks from kFewPipeMinCost on
+     * are pipelined (16 token chunks of 4 KiB to 1 MiB: 1.45 ms, against 2.38
+     * with the threshold alone), up to two chunks a resident block. A chosen
+     * plan is followed as it is, also one that equals the default. */
+    Plan of_launch(size_t n, size_t blocks) const {
+        return !chosen && n <= 2 * blocks ? plan_from_threshold(kFewPipeMinCost) : plan;
+    }
+};
+
+/* The current device's plan of a format, whole, for a tuner that puts it
+ * back; false when there is no device (tuned.hip). */
+bool read_plan(int format, DecodePlan* plan);
+bool write_plan(int format, const DecodePlan& plan);
+
+}  // namespace cudec_amd
+
+#endif /* CUDEC_AMD_PLAN_H */

@@ -16,6 +16,7 @@
 #include "cudec_mi355x.h"
 #include "cudec_snappy.h"
 #include "hip_owner.h"
+#include "plan.h"
 
 namespace cudec_amd {
 namespace {
@@ -87,18 +88,18 @@ extern "C" cudec_status cudec_mi355x_autotune_lz4(
         return CUDEC_ERR_INVALID_ARGUMENT;
     }
     try {
-        size_t previous = 0;
-        cudec_status st = cudec_mi355x_lz4_pipeline_threshold(&previous);
-        if (st != CUDEC_OK) {
-            return st;
+        DecodePlan previous;
+        if (!read_plan(CUDEC_MI355X_FORMAT_LZ4, &previous)) {
+            return CUDEC_ERR_CUDA;
         }
+        cudec_status st = CUDEC_OK;
         const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
         Event t0, t1;
         if (make_timing_event(t0) != hipSuccess || make_timing_event(t1) != hipSuccess) {
             return CUDEC_ERR_CUDA;
         }
         float best = -1.0f;
-        size_t best_cost = previous;
+        size_t best_cost = kCandidates[0];
         for (int c = 0; c < CUDEC_MI355X_TUNE_CANDIDATES; c++) {
             st = cudec_mi355x_set_lz4_pipeline_threshold(kCandidates[c]);
             if (st != CUDEC_OK) {
@@ -112,14 +113,14 @@ extern "C" cudec_status cudec_mi355x_autotune_lz4(
                 st = cudec_lz4_decompress_batch(d_src_ptrs, d_src_sizes, d_dst_ptrs,
                                                 d_dst_capacities, chunk_count, d_results, stream);
                 if (st != CUDEC_OK) {
-                    (void)cudec_mi355x_set_lz4_pipeline_threshold(previous);
+                    (void)write_plan(CUDEC_MI355X_FORMAT_LZ4, previous);
                     return st;
                 }
                 float ms = 0.0f;
                 if (hipEventRecord(t1.get(), s) != hipSuccess ||
                     hipEventSynchronize(t1.get()) != hipSuccess ||
                     hipEventElapsedTime(&ms, t0.get(), t1.get()) != hipSuccess) {
-                    (void)cudec_mi355x_set_lz4_pipeline_threshold(previous);
+                    (void)write_plan(CUDEC_MI355X_FORMAT_LZ4, previous);
                     return CUDEC_ERR_CUDA;
                 }
                 if (r > 0 && (fastest < 0.0f || ms < fastest)) {

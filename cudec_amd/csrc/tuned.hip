@@ -45,14 +45,13 @@
  * literal over 256 bytes) is decided by the exact scalar ladder and copied
  * wave-wide, global to global.
  */
-#include <cstdlib>
-#include <cstring>
 #include <mutex>
 
 #include "common.h"
 #include "cudec_mi355x.h"
 #include "execute.h"
 #include "ladder.h"
+#include "plan.h"
 
 namespace cudec_amd {
 namespace {
@@ -68,15 +67,7 @@ constexpr uint32_t kCandSplit = 8;
 constexpr uint32_t stage_bytes(uint32_t window) { return window + 304u; }
 constexpr uint32_t kStageBuf = stage_bytes(kCandSplit * 64) + 16;
 constexpr uint32_t kStop = 0xFFFFu;       /* link of an unresolvable candidate */
-constexpr uint32_t kOctaveBits = 2;       /* cost bins per octave: 4 */
-constexpr int kBins = 64 << kOctaveBits;
 static_assert(kBins == kCostBins, "the plan API names every bin");
-/* Default plans: chunks costing at least this (capacity + capacity -
- * compressed) are pipelined. */
-constexpr uint64_t kDefaultPipeMinCost[2] = {128u << 10, 64u << 10};
-/* ... and in launches of few chunks (plan_launch): below this one wave is
- * as fast (a 4 KiB token page alone: 36 us on one wave, 40 pipelined). */
-constexpr uint64_t kFewPipeMinCost = 8u << 10;
 /* Queue keys: a chunk's class (pipelined first), then its cost bin. */
 constexpr int kKeys = 2 * kBins;
 
@@ -121,16 +112,6 @@ struct Queue {
     uint32_t bin_base[kKeys];
     uint32_t bin_cursor[kKeys];
 };
-
-/* A decode plan: bit b (of word b / 64) set when cost bin b decodes on
- * a pipelined block, clear for one wave. Passed to the kernels by value. */
-struct Plan {
-    uint64_t two_wave[kBins / 64];
-};
-
-__host__ __device__ inline bool plan_two_wave(const Plan& p, uint32_t bin) {
-    return ((p.two_wave[bin >> 6] >> (bin & 63)) & 1u) != 0;
-}
 
 /* Loads one dword per lane, `step` bytes apart, of what follows the `bytes`
  * staged at sp (every one inside the source), so that the next window's
@@ -1445,18 +1426,6 @@ __global__ void queue_reset(Queue* q) {
     }
 }
 
-/* Order-preserving key of a cost below 2^63: the octave and the next
- * kOctaveBits bits below its leading one (costs below 2^kOctaveBits are
- * their own key). */
-__host__ __device__ inline uint32_t cost_key(uint64_t cost) {
-    if (cost < (1u << kOctaveBits)) {
-        return (uint32_t)cost;
-    }
-    const uint32_t lg = 63u - (uint32_t)__builtin_clzll(cost);
-    return lg << kOctaveBits |
-           (uint32_t)((cost >> (lg - kOctaveBits)) & ((1u << kOctaveBits) - 1));
-}
-
 /* Bin of a chunk by its decode cost, compressed size plus capacity: a
  * chunk's time follows the bytes it produces (a 4 MiB run of short-offset
  * matches compresses to a few hundred KiB yet decodes as long as 4 MiB of
@@ -1717,8 +1686,7 @@ struct DeviceState {
     int pipe_blocks_per_cu[2] = {0, 0};  /* piped_batch, per format */
     int wide_blocks_per_cu = 0;          /* LZ4's piped_batch in kSegmentWide's windows */
     int alone_blocks_per_cu[2] = {0, 0}; /* alone_batch */
-    Plan plan[2];                /* per format (kFormatLz4, kFormatSnappy) */
-    uint64_t min_cost[2];        /* the threshold each plan was last set from */
+    DecodePlan plan[2];          /* per format (kFormatLz4, kFormatSnappy) */
     hipMemPool_t pool = nullptr; /* made on the first allocating launch */
     bool pool_tried = false;
     void* fixed = nullptr;       /* this device's address of fixed_scratch */
@@ -1737,19 +1705,6 @@ constexpr size_t kFixedMaxChunks = CUDEC_MI355X_NOALLOC_MAX_CHUNKS;
 constexpr size_t kFixedBytes = sizeof(Queue) + sizeof(uint32_t) * kFixedMaxChunks;
 static __device__ __align__(256) uint8_t scratch[kFixedBytes];
 
-/* The plan that pipelines chunks costing at least min_cost: every
- * bin up to the bin of a chunk whose cost is exactly min_cost (costlier
- * bins have smaller numbers). 0 takes every bin, UINT64_MAX none. */
-Plan plan_from_threshold(uint64_t min_cost) {
-    Plan p = {};
-    const int32_t last = min_cost == 0 ? kBins - 1
-                         : min_cost == UINT64_MAX ? -1
-                                                  : (int32_t)(kBins - 1 - cost_key(min_cost));
-    for (int32_t b = 0; b <= last; b++) {
-        p.two_wave[b >> 6] |= 1ull << (b & 63);
-    }
-    return p;
-}
 DeviceState g_devices[kMaxDevices];
 std::mutex g_devices_lock;
 
@@ -1797,8 +1752,7 @@ hipError_t device_state(DeviceState** out) {
         }
         d.wide_blocks_per_cu = wide > 0 ? wide : 1;
         for (int f = 0; f < 2; f++) {
-            d.plan[f] = plan_from_threshold(kDefaultPipeMinCost[f]);
-            d.min_cost[f] = kDefaultPipeMinCost[f];
+            d.plan[f] = DecodePlan::usual(f);
         }
         /* this device is current: its own copy of the fixed scratch */
         d.fixed_status = hipGetSymbolAddress(&d.fixed, HIP_SYMBOL(scratch));
@@ -1848,8 +1802,7 @@ hipError_t set_pipe_min_cost(int format, uint64_t min_cost) {
         return e;
     }
     std::lock_guard<std::mutex> hold(g_devices_lock);
-    dev->plan[format] = plan_from_threshold(min_cost);
-    dev->min_cost[format] = min_cost;
+    dev->plan[format].set_threshold(min_cost);
     return hipSuccess;
 }
 
@@ -1860,25 +1813,39 @@ hipError_t get_pipe_min_cost(int format, uint64_t* min_cost) {
         return e;
     }
     std::lock_guard<std::mutex> hold(g_devices_lock);
-    *min_cost = dev->min_cost[format];
+    *min_cost = dev->plan[format].min_cost;
     return hipSuccess;
 }
 
 hipError_t set_decode_plan(int format, const uint16_t* lanes) {
-    Plan p = {};
-    for (int b = 0; b < kBins; b++) {
-        if (lanes[b] == 128) {
-            p.two_wave[b >> 6] |= 1ull << (b & 63);
-        }
-    }
     DeviceState* dev = nullptr;
     const hipError_t e = device_state(&dev);
     if (e != hipSuccess) {
         return e;
     }
     std::lock_guard<std::mutex> hold(g_devices_lock);
-    dev->plan[format] = p;
+    dev->plan[format].set_bins(lanes);
     return hipSuccess;
+}
+
+bool read_plan(int format, DecodePlan* plan) {
+    DeviceState* dev = nullptr;
+    if (device_state(&dev) != hipSuccess) {
+        return false;
+    }
+    std::lock_guard<std::mutex> hold(g_devices_lock);
+    *plan = dev->plan[format];
+    return true;
+}
+
+bool write_plan(int format, const DecodePlan& plan) {
+    DeviceState* dev = nullptr;
+    if (device_state(&dev) != hipSuccess) {
+        return false;
+    }
+    std::lock_guard<std::mutex> hold(g_devices_lock);
+    dev->plan[format] = plan;
+    return true;
 }
 
 hipError_t get_decode_plan(int format, uint16_t* lanes) {
@@ -1890,7 +1857,7 @@ hipError_t get_decode_plan(int format, uint16_t* lanes) {
     Plan p;
     {
         std::lock_guard<std::mutex> hold(g_devices_lock);
-        p = dev->plan[format];
+        p = dev->plan[format].plan;
     }
     for (int b = 0; b < kBins; b++) {
         lanes[b] = plan_two_wave(p, (uint32_t)b) ? 128 : 64;
@@ -1920,22 +1887,15 @@ struct Launch {
     size_t alone_grid; /* of the one-wave kernel that follows, or 0 */
 };
 
-/* A launch of few chunks leaves most of the chip idle whatever it does, and
- * takes as long as its largest chunk: under the default plan all its chunks
- * are pipelined (16 token chunks of 4 KiB to 1 MiB: 1.45 ms, against 2.38
- * with the threshold alone), up to two chunks a resident block. The queue's
- * four kernels and the scratch allocation cost about 35 us, so a launch
- * that has a resident block for each chunk takes them in their own order. */
+/* The queue's four kernels and the scratch allocation cost about 35 us, so a
+ * launch that has a resident block for each chunk takes them in their own
+ * order. */
 Launch plan_launch(const DeviceState& dev, int f, size_t n) {
     Launch r;
+    const size_t pipe_blocks = (size_t)dev.cus * (size_t)dev.pipe_blocks_per_cu[f];
     {
         std::lock_guard<std::mutex> hold(g_devices_lock);
-        r.plan = dev.plan[f];
-    }
-    const size_t pipe_blocks = (size_t)dev.cus * (size_t)dev.pipe_blocks_per_cu[f];
-    const Plan usual = plan_from_threshold(kDefaultPipeMinCost[f]);
-    if (n <= 2 * pipe_blocks && std::memcmp(&r.plan, &usual, sizeof(Plan)) == 0) {
-        r.plan = plan_from_threshold(kFewPipeMinCost);
+        r.plan = dev.plan[f].of_launch(n, pipe_blocks);
     }
     bool all = true;
     r.pipes = false;

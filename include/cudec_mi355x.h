@@ -51,7 +51,9 @@ size_t cudec_mi355x_max_batch_chunks(void);
  * depend on the plan. Plans are per device and per format, process-wide;
  * the default pipelines chunks costing at least 128 KiB (LZ4) or 64 KiB
  * (Snappy), and under it launches of few chunks (up to two a resident
- * block) pipeline those costing at least 8 KiB. */
+ * block) pipeline those costing at least 8 KiB. A plan that a caller has
+ * set, here or through an autotuner, is what every launch follows from then
+ * on, also one that equals the default. */
 #define CUDEC_MI355X_COST_BINS 256
 #define CUDEC_MI355X_FORMAT_LZ4 0
 #define CUDEC_MI355X_FORMAT_SNAPPY 1

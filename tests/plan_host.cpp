@@ -1,0 +1,30 @@
+/* cudec_amd/csrc/plan.h built for the CPU: TEST INFRASTRUCTURE ONLY. */
+#include "plan.h"
+
+#include <cstring>
+
+extern "C" {
+
+/* The plan (kBins / 64 words) that a launch of n chunks follows on a device
+ * of `blocks` resident blocks; how: 0 nothing set, 1 a threshold, 2 the bins
+ * that this threshold gives. */
+void host_plan(int format, int how, uint64_t threshold, uint64_t n, uint64_t blocks,
+               uint64_t* words, uint64_t* min_cost) {
+    using namespace cudec_amd;
+    DecodePlan d = DecodePlan::usual(format);
+    if (how == 1) {
+        d.set_threshold(threshold);
+    } else if (how == 2) {
+        const Plan p = plan_from_threshold(threshold);
+        uint16_t lanes[kBins];
+        for (int b = 0; b < kBins; b++) {
+            lanes[b] = plan_two_wave(p, (uint32_t)b) ? 128 : 64;
+        }
+        d.set_bins(lanes);
+    }
+    const Plan p = d.of_launch(n, blocks);
+    std::memcpy(words, p.two_wave, sizeof(p.two_wave));
+    *min_cost = d.min_cost;
+}
+
+}  // extern "C"
