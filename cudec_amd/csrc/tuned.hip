@@ -1,6 +1,6 @@
 /* The tuned launch form of the LZ4 and Snappy batch decoders for gfx950.
  *
- * Work distribution: four small kernels bin the chunks by decode cost
+ * Work distribution: three small kernels bin the chunks by decode cost
  * (capacity + (capacity - compressed size), the output plus what matches
  * add to it; four bins per octave) into a device queue. A per-device,
  * per-format decode plan names, for each cost bin, how one of its chunks is
@@ -99,7 +99,8 @@ constexpr uint32_t kSubStride = 1024; /* uint32 words: 4 KiB apart */
 constexpr uint64_t kSubQueueMinPerWave = 16; /* chunks per wave for kSubQueues */
 
 /* A wave's place in the decode queue: the sub-queue it draws from and how
- * many sub-queues it has not yet found drained. */
+ * many sub-queues it has not yet found drained; of the one queue, the
+ * positions before those it hands out, which waves started with. */
 struct QueueCursor {
     uint32_t sub;
     uint32_t left;
@@ -109,8 +110,8 @@ struct QueueCursor {
 struct Queue {
     uint32_t next[kSubQueues * kSubStride];
     uint32_t bin_count[kKeys];
-    uint32_t bin_base[kKeys];
     uint32_t bin_cursor[kKeys];
+    uint32_t piped; /* chunks of the pipelined class */
 };
 
 /* Loads one dword per lane, `step` bytes apart, of what follows the `bytes`
@@ -1469,27 +1470,35 @@ __global__ void queue_count(const size_t* sizes, const size_t* caps, size_t n, Q
     }
 }
 
-__global__ void queue_scan(Queue* q) {
-    if (threadIdx.x == 0) {
-        uint32_t acc = 0;
-        for (int b = 0; b < kKeys; b++) {
-            q->bin_base[b] = acc;
-            acc += q->bin_count[b];
-        }
-    }
-}
+constexpr int kFillBlock = 256;
+static_assert(kKeys == 2 * kFillBlock, "a thread of queue_fill adds up two keys");
 
 /* Each chunk's place in the order: its bin's base, the block's range in
  * that bin (one global atomic per bin the block holds) and its rank in the
- * block (an LDS atomic). */
-__global__ void queue_fill(const size_t* sizes, const size_t* caps, size_t n, Queue* q,
-                           uint32_t* order, Plan plan) {
+ * block (an LDS atomic). Every block adds the counts up for itself: a kernel
+ * that did it once, on one thread, took 7 us and the gap to the next one. */
+__global__ void __launch_bounds__(kFillBlock)
+    queue_fill(const size_t* sizes, const size_t* caps, size_t n, Queue* q, uint32_t* order,
+               Plan plan) {
     __shared__ uint32_t local[kKeys];
     __shared__ uint32_t range[kKeys];
-    for (uint32_t t = threadIdx.x; t < kKeys; t += blockDim.x) {
-        local[t] = 0;
+    __shared__ uint32_t waves[kFillBlock / kWave];
+    const uint32_t k = 2 * threadIdx.x;
+    const uint32_t c0 = q->bin_count[k], c1 = q->bin_count[k + 1];
+    const uint32_t incl = wave_inclusive_sum(c0 + c1, __lane_id());
+    if (__lane_id() == kWave - 1) {
+        waves[threadIdx.x / kWave] = incl;
     }
+    local[k] = 0;
+    local[k + 1] = 0;
     __syncthreads();
+    uint32_t base = incl - c0 - c1; /* of key k */
+    for (uint32_t w = 0; w < threadIdx.x / kWave; w++) {
+        base += waves[w];
+    }
+    if (blockIdx.x == 0 && k == (uint32_t)kBins) {
+        q->piped = base;
+    }
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t b = 0, rank = 0;
     if (i < n) {
@@ -1497,14 +1506,15 @@ __global__ void queue_fill(const size_t* sizes, const size_t* caps, size_t n, Qu
         rank = atomicAdd(&local[b], 1u);
     }
     __syncthreads();
-    for (uint32_t t = threadIdx.x; t < kKeys; t += blockDim.x) {
-        if (local[t] != 0) {
-            range[t] = atomicAdd(&q->bin_cursor[t], local[t]);
-        }
+    if (local[k] != 0) {
+        range[k] = base + atomicAdd(&q->bin_cursor[k], local[k]);
+    }
+    if (local[k + 1] != 0) {
+        range[k + 1] = base + c0 + atomicAdd(&q->bin_cursor[k + 1], local[k + 1]);
     }
     __syncthreads();
     if (i < n) {
-        order[q->bin_base[b] + range[b] + rank] = (uint32_t)i;
+        order[range[b] + rank] = (uint32_t)i;
     }
 }
 
@@ -1525,7 +1535,8 @@ __device__ __forceinline__ uint32_t queue_pop(Queue* q, size_t n, QueueCursor& c
         return first && own < n ? (uint32_t)own : (uint32_t)n;
     }
     if (kSubs == 1) {
-        return uniform32(atomicAdd(&q->next[0], lane == 0 ? 1u : 0u));
+        return c.sub >= n ? (uint32_t)n
+                          : uniform32(c.sub + atomicAdd(&q->next[0], lane == 0 ? 1u : 0u));
     }
     while (c.left != 0) {
         const uint32_t i =
@@ -1569,9 +1580,9 @@ __device__ __forceinline__ void decode_alone(WaveLds& w, uint32_t idx, const voi
 
 
 /* Whether a queued batch has no chunk that its plan pipelines: the queue
- * holds those first, so the first of the others has place 0. */
+ * holds those first. */
 __device__ __forceinline__ bool none_piped(const Queue* q) {
-    return uniform32(q->bin_base[kBins]) == 0;
+    return uniform32(q->piped) == 0;
 }
 
 /* The persistent decoder. A block takes the queue's pipelined chunks first,
@@ -1656,8 +1667,12 @@ __global__ void __launch_bounds__(kPipeBlock)
  * VGPRs): 16 384 token chunks of 64 KiB in 2.69 ms against 3.05 by
  * piped_batch's split blocks. Only the queue build knows whether a batch has
  * chunks to pipeline, so it `follows` a piped_batch that leaves batches
- * without one untouched, and leaves the others (an empty launch is about 5
- * us) to that. */
+ * without one untouched, and leaves the others to that: an empty launch is
+ * about 2 us, and up to 8 with the gap before the next. (With that launch, a
+ * kernel to add the queue's counts up and 5120 waves whatever the batch, 1500
+ * chunks of 512 bytes took 113 us, 2500 of 64 KiB 816 and 20 000 of 512 bytes
+ * 329; they take 46, 686 and 273. Before there were two kernels: 88, 856 and
+ * 310.) */
 constexpr int kAloneBlock = 2 * kWave;
 template <int kFormat, uint32_t kSubs, bool kParseOnly>
 __global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_eu(5)))
@@ -1671,8 +1686,17 @@ __global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_e
     if (follows && !none_piped(q)) {
         return;
     }
-    const uint32_t idx = queue_pop<kSubs>(
-        q, n, cursor, lane, (uint64_t)blockIdx.x * (kAloneBlock / kWave) + wave);
+    const uint64_t own = (uint64_t)blockIdx.x * (kAloneBlock / kWave) + wave;
+    uint32_t idx;
+    if (kSubs == 1) {
+        /* of the one queue, every wave starts with a position of its own: up
+         * to 5120 pops of about 12 ns each fewer at one counter, and none at
+         * all where every chunk has a wave */
+        idx = own < n ? (uint32_t)own : (uint32_t)n;
+        cursor.sub = gridDim.x * (uint32_t)(kAloneBlock / kWave);
+    } else {
+        idx = queue_pop<kSubs>(q, n, cursor, lane, own);
+    }
     decode_alone<kFormat, kSubs, kParseOnly>(w[wave], idx, srcs,
                                              src_sizes, dsts, caps, n, results, q, order, cursor,
                                              lane);
@@ -1887,9 +1911,10 @@ struct Launch {
     size_t alone_grid; /* of the one-wave kernel that follows, or 0 */
 };
 
-/* The queue's four kernels and the scratch allocation cost about 35 us, so a
+/* The queue's three kernels and the scratch allocation cost about 25 us, so a
  * launch that has a resident block for each chunk takes them in their own
- * order. */
+ * order. The one-wave kernel that follows has no more waves than there are
+ * chunks: a wave that finds nothing costs the others a pop's time. */
 Launch plan_launch(const DeviceState& dev, int f, size_t n) {
     Launch r;
     const size_t pipe_blocks = (size_t)dev.cus * (size_t)dev.pipe_blocks_per_cu[f];
@@ -1911,7 +1936,8 @@ Launch plan_launch(const DeviceState& dev, int f, size_t n) {
     r.wide = f == 0 && r.pipes && r.direct &&
              n <= (size_t)dev.cus * (size_t)dev.wide_blocks_per_cu;
     r.grid = r.direct ? wanted : blocks;
-    r.alone_grid = !r.pipes || all || r.direct ? 0 : alone_blocks;
+    const size_t pairs = (n + kAloneBlock / kWave - 1) / (kAloneBlock / kWave);
+    r.alone_grid = !r.pipes || all || r.direct ? 0 : pairs < alone_blocks ? pairs : alone_blocks;
     return r;
 }
 
@@ -1926,12 +1952,11 @@ hipError_t queue_and_decode(const Launch& launch, int format, const void* const*
     Queue* q = static_cast<Queue*>(work);
     uint32_t* order = launch.direct ? nullptr : reinterpret_cast<uint32_t*>(q + 1);
     if (!launch.direct) {
-        const unsigned tb = 256;
+        const unsigned tb = kFillBlock;
         const unsigned nb = (unsigned)((n + tb - 1) / tb);
         hipLaunchKernelGGL(queue_reset, dim3(1), dim3(kKeys), 0, stream, q);
         hipLaunchKernelGGL(queue_count, dim3(nb), dim3(tb), 0, stream, src_sizes, caps, n, q,
                            plan);
-        hipLaunchKernelGGL(queue_scan, dim3(1), dim3(1), 0, stream, q);
         hipLaunchKernelGGL(queue_fill, dim3(nb), dim3(tb), 0, stream, src_sizes, caps, n, q,
                            order, plan);
     }
@@ -2005,11 +2030,10 @@ hipError_t cost_order(const size_t* sizes, const size_t* caps, size_t n, void* w
     const Plan plan{};
     Queue* q = static_cast<Queue*>(work);
     uint32_t* out = reinterpret_cast<uint32_t*>(q + 1);
-    const unsigned tb = 256;
+    const unsigned tb = kFillBlock;
     const unsigned nb = (unsigned)((n + tb - 1) / tb);
     hipLaunchKernelGGL(queue_reset, dim3(1), dim3(kKeys), 0, stream, q);
     hipLaunchKernelGGL(queue_count, dim3(nb), dim3(tb), 0, stream, sizes, caps, n, q, plan);
-    hipLaunchKernelGGL(queue_scan, dim3(1), dim3(1), 0, stream, q);
     hipLaunchKernelGGL(queue_fill, dim3(nb), dim3(tb), 0, stream, sizes, caps, n, q, out, plan);
     *order = out;
     return hipGetLastError();

@@ -9,6 +9,8 @@ chunk: statuses, sizes, bytes and the poison beyond them.
   entry, whose second call is smaller and must not see the first's queue, and
   both decoding entries captured into a graph, where the scratch is a graph
   allocation or the fixed array;
+* the one-wave kernel around one and two chunks for each of its waves, and
+  batches with chunks in every cost bin there is from nothing to 4 MiB;
 * the streams of the copy, slow-sequence and chain tests, which have a block
   each there and so the wide windows, in the usual ones;
 * matches on both sides of the piece that a pipelined block expands at once
@@ -205,3 +207,33 @@ def test_edges_in_the_usual_windows(made, request):
     with plan_by_threshold("lz4", 0):
         check_against_oracle("lz4", "tuned", streams + [last_literals(bytes(9))] * fill,
                              caps + [9] * fill, names + ["fill"] * fill)
+
+
+@pytest.mark.parametrize("fmt", ["lz4", "snappy"])
+@pytest.mark.parametrize("n", [2049, 5119, 5120, 5121, 5122, 10239, 10240, 10241])
+def test_chunks_for_each_wave(fmt, n):
+    rng = np.random.default_rng(n)
+    codec = workload.CODEC_LZ4 if fmt == "lz4" else workload.CODEC_SNAPPY
+    base = workload.build(codec, rng.integers(1, 600, 60), rng.integers(0, 3, 60),
+                          rng.integers(1, 1 << 60, 60))
+    which = rng.integers(0, 60, n)
+    streams = [base.compressed(int(i)) for i in which]
+    caps = [int(base.sizes[i]) for i in which]
+    streams[3], caps[n - 2] = streams[3][:-1], 0
+    print(f"[one wave] {fmt} {n} chunks", flush=True)
+    with plan_by_threshold(fmt, 1 << 40):
+        check_against_oracle(fmt, "tuned", streams, caps)
+
+
+@pytest.mark.parametrize("fmt", ["lz4", "snappy"])
+@pytest.mark.parametrize("threshold", [16 << 10, 1 << 40])
+def test_every_cost_bin(fmt, threshold):
+    codec = workload.CODEC_LZ4 if fmt == "lz4" else workload.CODEC_SNAPPY
+    sizes = [int(1.18 ** k) for k in range(93)]  # 1 byte to 4 MiB, a few a bin
+    b = workload.build(codec, sizes, [k % 3 for k in range(93)], range(1, 94))
+    streams = [b.compressed(k) for k in range(93)] + [b.compressed(0), b"" if fmt == "lz4" else bytes(1)] + [b.compressed(20)] * 2400
+    caps = sizes + [0, 0] + [sizes[20]] * 2400
+    order = np.random.default_rng(4).permutation(len(streams))
+    print(f"[cost bins] {fmt} {len(streams)} chunks, threshold {threshold}", flush=True)
+    with plan_by_threshold(fmt, threshold):
+        check_against_oracle(fmt, "tuned", [streams[i] for i in order], [caps[i] for i in order])
