@@ -39,11 +39,11 @@ CUDEC_HD inline uint32_t cost_key(uint64_t cost) {
 /* A decode plan: bit b (of word b / 64) set when cost bin b decodes on
  * a pipelined block, clear for one wave. Passed to the kernels by value. */
 struct Plan {
-    uint64_t two_wave[kBins / 64];
+    uint64_t pipes[kBins / 64];
 };
 
-CUDEC_HD inline bool plan_two_wave(const Plan& p, uint32_t bin) {
-    return ((p.two_wave[bin >> 6] >> (bin & 63)) & 1u) != 0;
+CUDEC_HD inline bool plan_pipes(const Plan& p, uint32_t bin) {
+    return ((p.pipes[bin >> 6] >> (bin & 63)) & 1u) != 0;
 }
 
 /* The plan that pipelines chunks costing at least min_cost: every
@@ -55,7 +55,7 @@ inline Plan plan_from_threshold(uint64_t min_cost) {
                          : min_cost == UINT64_MAX ? -1
                                                   : (int32_t)(kBins - 1 - cost_key(min_cost));
     for (int32_t b = 0; b <= last; b++) {
-        p.two_wave[b >> 6] |= 1ull << (b & 63);
+        p.pipes[b >> 6] |= 1ull << (b & 63);
     }
     return p;
 }
@@ -79,7 +79,7 @@ struct DecodePlan {
         plan = {};
         for (int b = 0; b < kBins; b++) {
             if (lanes[b] == 128) {
-                plan.two_wave[b >> 6] |= 1ull << (b & 63);
+                plan.pipes[b >> 6] |= 1ull << (b & 63);
             }
         }
         chosen = true;

@@ -1445,7 +1445,7 @@ __device__ __forceinline__ uint32_t cost_bin(uint64_t src_size, uint64_t cap) {
 /* Queue key of a chunk: its class under the plan, then its bin. */
 __device__ __forceinline__ uint32_t queue_key(const Plan& plan, uint64_t src_size, uint64_t cap) {
     const uint32_t bin = cost_bin(src_size, cap);
-    return plan_two_wave(plan, bin) ? bin : kBins + bin;
+    return plan_pipes(plan, bin) ? bin : kBins + bin;
 }
 
 /* Chunks per cost bin. A block counts its chunks in LDS and adds one
@@ -1639,7 +1639,7 @@ __global__ void __launch_bounds__(kPipeBlock)
         gu8* dst = global_bytes(dsts[chunk]);
         const uint64_t src_size = uniform64(src_sizes[chunk]);
         const uint64_t cap = uniform64(caps[chunk]);
-        if (!plan_two_wave(plan, cost_bin(src_size, cap))) {
+        if (!plan_pipes(plan, cost_bin(src_size, cap))) {
             break;
         }
         if (wave == 0) {
@@ -1884,7 +1884,7 @@ hipError_t get_decode_plan(int format, uint16_t* lanes) {
         p = dev->plan[format].plan;
     }
     for (int b = 0; b < kBins; b++) {
-        lanes[b] = plan_two_wave(p, (uint32_t)b) ? 128 : 64;
+        lanes[b] = plan_pipes(p, (uint32_t)b) ? 128 : 64;
     }
     return hipSuccess;
 }
@@ -1925,8 +1925,8 @@ Launch plan_launch(const DeviceState& dev, int f, size_t n) {
     bool all = true;
     r.pipes = false;
     for (int w = 0; w < kBins / 64; w++) {
-        r.pipes = r.pipes || r.plan.two_wave[w] != 0;
-        all = all && r.plan.two_wave[w] == ~0ull;
+        r.pipes = r.pipes || r.plan.pipes[w] != 0;
+        all = all && r.plan.pipes[w] == ~0ull;
     }
     const size_t per = r.pipes ? 1 : kAloneBlock / kWave; /* chunks a block starts with */
     const size_t alone_blocks = (size_t)dev.cus * (size_t)dev.alone_blocks_per_cu[f];

@@ -18,12 +18,12 @@ void host_plan(int format, int how, uint64_t threshold, uint64_t n, uint64_t blo
         const Plan p = plan_from_threshold(threshold);
         uint16_t lanes[kBins];
         for (int b = 0; b < kBins; b++) {
-            lanes[b] = plan_two_wave(p, (uint32_t)b) ? 128 : 64;
+            lanes[b] = plan_pipes(p, (uint32_t)b) ? 128 : 64;
         }
         d.set_bins(lanes);
     }
     const Plan p = d.of_launch(n, blocks);
-    std::memcpy(words, p.two_wave, sizeof(p.two_wave));
+    std::memcpy(words, p.pipes, sizeof(p.pipes));
     *min_cost = d.min_cost;
 }
 
