@@ -95,6 +95,64 @@ struct DecodePlan {
     }
 };
 
+/* Waves of a block of piped_batch and of alone_batch (tuned.hip). */
+constexpr uint32_t kPipeWaves = 4;
+constexpr uint32_t kAloneWaves = 2;
+
+/* Blocks that a device holds at once, on all its CUs together. */
+struct Resident {
+    size_t piped; /* of piped_batch */
+    size_t wide;  /* of its build for wide windows; 0: the format has none */
+    size_t alone; /* of alone_batch */
+};
+
+/* Chunks per wave from which the queue hands out its order through
+ * sub-queues (tuned.hip). */
+constexpr uint64_t kSubQueueMinPerWave = 16;
+
+/* How one launch runs: its plan, whether any chunk may be pipelined, its
+ * grid, and whether every chunk has a resident block (or wave) of its own,
+ * so that it needs no queue and no scratch. */
+struct Launch {
+    Plan plan;
+    bool pipes;
+    bool direct;
+    bool wide;         /* direct and pipelined: in kSegmentWide's windows */
+    bool many;         /* through sub-queues */
+    size_t grid;
+    size_t alone_grid; /* of the one-wave kernel that follows, or 0 */
+};
+
+/* The queue's three kernels and the scratch allocation cost about 25 us, so a
+ * launch that has a resident block for each chunk takes them in their own
+ * order. The one-wave kernel that follows has no more waves than there are
+ * chunks: a wave that finds nothing costs the others a pop's time. Whether
+ * the order goes through sub-queues is settled for both kernels by the first
+ * one's waves, which are the fewer (65 536 chunks on 256 CUs): by its own
+ * 5120 the second would leave 65 536 to 81 919 small chunks to one counter
+ * (80 000 of 512 bytes: 1014 us, 346 so). */
+inline Launch plan_launch(const DecodePlan& set, const Resident& at, size_t n) {
+    Launch r;
+    r.plan = set.of_launch(n, at.piped);
+    bool all = true;
+    r.pipes = false;
+    for (int w = 0; w < kBins / 64; w++) {
+        r.pipes = r.pipes || r.plan.pipes[w] != 0;
+        all = all && r.plan.pipes[w] == ~0ull;
+    }
+    const size_t per = r.pipes ? 1 : kAloneWaves; /* chunks a block starts with */
+    const size_t blocks = r.pipes ? at.piped : at.alone;
+    const size_t wanted = (n + per - 1) / per;
+    r.direct = wanted <= blocks;
+    r.wide = r.pipes && r.direct && n <= at.wide;
+    r.grid = r.direct ? wanted : blocks;
+    r.many = (uint64_t)n >=
+             kSubQueueMinPerWave * (r.pipes ? kPipeWaves : kAloneWaves) * (uint64_t)r.grid;
+    const size_t pairs = (n + kAloneWaves - 1) / kAloneWaves;
+    r.alone_grid = !r.pipes || all || r.direct ? 0 : pairs < at.alone ? pairs : at.alone;
+    return r;
+}
+
 /* The current device's plan of a format, whole, for a tuner that puts it
  * back; false when there is no device (tuned.hip). */
 bool read_plan(int format, DecodePlan* plan);

@@ -96,7 +96,6 @@ constexpr uint32_t kPipeHistory = kPipeRing - 3 * kPipeBatch - 64;
  * queue: its exact costliest-first order matters more there. */
 constexpr uint32_t kSubQueues = 8;
 constexpr uint32_t kSubStride = 1024; /* uint32 words: 4 KiB apart */
-constexpr uint64_t kSubQueueMinPerWave = 16; /* chunks per wave for kSubQueues */
 
 /* A wave's place in the decode queue: the sub-queue it draws from and how
  * many sub-queues it has not yet found drained; of the one queue, the
@@ -891,7 +890,6 @@ __device__ __forceinline__ int chunk_begin(gcu8* src, uint64_t src_size, uint64_
  * its start): a follower can overwrite nothing that a running group reads,
  * and everything older than that history was flushed to memory by groups
  * that have finished, because unfinished ones span at most two groups. */
-constexpr uint32_t kPipeWaves = 4;
 constexpr uint32_t kCopiers = kPipeWaves - 1;
 constexpr int kPipeBlock = kPipeWaves * kWave;
 static_assert(kPipeHistory + kCopiers * kPipeBatch + 64 <= kPipeRing &&
@@ -1673,27 +1671,27 @@ __global__ void __launch_bounds__(kPipeBlock)
  * chunks of 512 bytes took 113 us, 2500 of 64 KiB 816 and 20 000 of 512 bytes
  * 329; they take 46, 686 and 273. Before there were two kernels: 88, 856 and
  * 310.) */
-constexpr int kAloneBlock = 2 * kWave;
+constexpr int kAloneBlock = kAloneWaves * kWave;
 template <int kFormat, uint32_t kSubs, bool kParseOnly>
 __global__ void __launch_bounds__(kAloneBlock) __attribute__((amdgpu_waves_per_eu(5)))
     alone_batch(const void* const* srcs, const size_t* src_sizes, void* const* dsts,
                 const size_t* caps, size_t n, cudec_chunk_result* results, Queue* q,
                 const uint32_t* order, bool follows) {
-    __shared__ WaveLds w[kAloneBlock / kWave];
+    __shared__ WaveLds w[kAloneWaves];
     const uint32_t lane = __lane_id();
     QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
     const uint32_t wave = uniform32(threadIdx.x / kWave);
     if (follows && !none_piped(q)) {
         return;
     }
-    const uint64_t own = (uint64_t)blockIdx.x * (kAloneBlock / kWave) + wave;
+    const uint64_t own = (uint64_t)blockIdx.x * kAloneWaves + wave;
     uint32_t idx;
     if (kSubs == 1) {
         /* of the one queue, every wave starts with a position of its own: up
          * to 5120 pops of about 12 ns each fewer at one counter, and none at
          * all where every chunk has a wave */
         idx = own < n ? (uint32_t)own : (uint32_t)n;
-        cursor.sub = gridDim.x * (uint32_t)(kAloneBlock / kWave);
+        cursor.sub = gridDim.x * kAloneWaves;
     } else {
         idx = queue_pop<kSubs>(q, n, cursor, lane, own);
     }
@@ -1899,46 +1897,14 @@ uint32_t host_cost_bin(uint64_t src_size, uint64_t cap) {
 
 namespace {
 
-/* How one launch runs: its plan, whether any chunk may be pipelined, its
- * grid, and whether every chunk has a resident block (or wave) of its own,
- * so that it needs no queue and no scratch. */
-struct Launch {
-    Plan plan;
-    bool pipes;
-    bool direct;
-    bool wide;         /* LZ4, direct and pipelined: in kSegmentWide's windows */
-    size_t grid;
-    size_t alone_grid; /* of the one-wave kernel that follows, or 0 */
-};
-
-/* The queue's three kernels and the scratch allocation cost about 25 us, so a
- * launch that has a resident block for each chunk takes them in their own
- * order. The one-wave kernel that follows has no more waves than there are
- * chunks: a wave that finds nothing costs the others a pop's time. */
-Launch plan_launch(const DeviceState& dev, int f, size_t n) {
-    Launch r;
-    const size_t pipe_blocks = (size_t)dev.cus * (size_t)dev.pipe_blocks_per_cu[f];
-    {
-        std::lock_guard<std::mutex> hold(g_devices_lock);
-        r.plan = dev.plan[f].of_launch(n, pipe_blocks);
-    }
-    bool all = true;
-    r.pipes = false;
-    for (int w = 0; w < kBins / 64; w++) {
-        r.pipes = r.pipes || r.plan.pipes[w] != 0;
-        all = all && r.plan.pipes[w] == ~0ull;
-    }
-    const size_t per = r.pipes ? 1 : kAloneBlock / kWave; /* chunks a block starts with */
-    const size_t alone_blocks = (size_t)dev.cus * (size_t)dev.alone_blocks_per_cu[f];
-    const size_t blocks = r.pipes ? pipe_blocks : alone_blocks;
-    const size_t wanted = (n + per - 1) / per;
-    r.direct = wanted <= blocks;
-    r.wide = f == 0 && r.pipes && r.direct &&
-             n <= (size_t)dev.cus * (size_t)dev.wide_blocks_per_cu;
-    r.grid = r.direct ? wanted : blocks;
-    const size_t pairs = (n + kAloneBlock / kWave - 1) / (kAloneBlock / kWave);
-    r.alone_grid = !r.pipes || all || r.direct ? 0 : pairs < alone_blocks ? pairs : alone_blocks;
-    return r;
+/* How a launch of n chunks runs now. */
+Launch launch_of(const DeviceState& dev, int f, size_t n) {
+    const size_t cus = (size_t)dev.cus;
+    const Resident at{cus * (size_t)dev.pipe_blocks_per_cu[f],
+                      f == 0 ? cus * (size_t)dev.wide_blocks_per_cu : 0,
+                      cus * (size_t)dev.alone_blocks_per_cu[f]};
+    std::lock_guard<std::mutex> hold(g_devices_lock);
+    return plan_launch(dev.plan[f], at, n);
 }
 
 /* Launches the persistent decoder on `stream`; parse_only launches its
@@ -1966,11 +1932,10 @@ hipError_t queue_and_decode(const Launch& launch, int format, const void* const*
     const int f = format == kFormatSnappy ? 1 : 0;
     for (int pass = 0; pass < (launch.alone_grid != 0 ? 2 : 1); pass++) {
         const bool follows = pass != 0, pipes = launch.pipes && !follows;
-        const int waves = pipes ? (int)kPipeWaves : kAloneBlock / (int)kWave;
+        const int waves = (int)(pipes ? kPipeWaves : kAloneWaves);
         const size_t grid = follows ? launch.alone_grid : launch.grid;
         const dim3 gd((unsigned)grid), bd((unsigned)(waves * (int)kWave));
-        const bool many = (uint64_t)n >= kSubQueueMinPerWave * (uint64_t)waves * (uint64_t)grid;
-        const int subs = launch.wide ? 3 : launch.direct ? 2 : many ? 1 : 0;
+        const int subs = launch.wide ? 3 : launch.direct ? 2 : launch.many ? 1 : 0;
         const int shape = (parse_only ? 16 : 0) | (f ? 8 : 0) | (pipes ? 0 : 4) | subs;
         switch (shape) {
 #define CUDEC_PIPED(kShape, kFmt, kS, kP)                                                 \
@@ -2059,7 +2024,7 @@ hipError_t launch_tuned(int format, const void* const* srcs, const size_t* src_s
         return e;
     }
     const int f = format == kFormatSnappy ? kFormatSnappy : kFormatLz4;
-    const Launch launch = plan_launch(*dev, f, n);
+    const Launch launch = launch_of(*dev, f, n);
     if (launch.direct) {
         return queue_and_decode(launch, format, srcs, src_sizes, dsts, caps, n, results, nullptr,
                                 stream, parse_only);
@@ -2101,7 +2066,7 @@ hipError_t launch_tuned_fixed(int format, const void* const* srcs, const size_t*
         return dev->fixed_status != hipSuccess ? dev->fixed_status : hipErrorInvalidSymbol;
     }
     const int f = format == kFormatSnappy ? kFormatSnappy : kFormatLz4;
-    return queue_and_decode(plan_launch(*dev, f, n), format, srcs, src_sizes, dsts, caps, n,
+    return queue_and_decode(launch_of(*dev, f, n), format, srcs, src_sizes, dsts, caps, n,
                             results, dev->fixed, stream, false);
 }
 

@@ -27,4 +27,22 @@ void host_plan(int format, int how, uint64_t threshold, uint64_t n, uint64_t blo
     *min_cost = d.min_cost;
 }
 
+/* How a launch of n chunks runs under the default plan (threshold 1) or one
+ * by threshold, on a device of these resident blocks. */
+void host_launch(int format, uint64_t threshold, uint64_t n, uint64_t piped, uint64_t wide,
+                 uint64_t alone, uint64_t* grids, int* flags) {
+    using namespace cudec_amd;
+    DecodePlan d = DecodePlan::usual(format);
+    if (threshold != 1) {
+        d.set_threshold(threshold);
+    }
+    const Launch r = plan_launch(d, Resident{piped, wide, alone}, n);
+    grids[0] = r.grid;
+    grids[1] = r.alone_grid;
+    flags[0] = r.pipes;
+    flags[1] = r.direct;
+    flags[2] = r.wide;
+    flags[3] = r.many;
+}
+
 }  // extern "C"
