@@ -50,6 +50,15 @@ static cudec_status validate(const void* const* srcs, const size_t* sizes,
     return CUDEC_OK;
 }
 
+/* A call's status; an error is not left for the program's next GPU call. */
+static cudec_status ended(hipError_t err) {
+    if (err == hipSuccess) {
+        return CUDEC_OK;
+    }
+    (void)hipGetLastError();
+    return CUDEC_ERR_CUDA;
+}
+
 static cudec_status submit(int format, int form, const void* const* srcs,
                            const size_t* sizes, void* const* dsts,
                            const size_t* caps, size_t n,
@@ -71,7 +80,7 @@ static cudec_status submit(int format, int form, const void* const* srcs,
             ? launch_tuned_fixed(format, srcs, sizes, dsts, caps, n, results, s)
             : launch_tuned(format, srcs, sizes, dsts, caps, n, results, s,
                            form == kFormParseOnly);
-    return err == hipSuccess ? CUDEC_OK : CUDEC_ERR_CUDA;
+    return ended(err);
 }
 
 }  // namespace cudec_amd
@@ -127,7 +136,7 @@ cudec_status cudec_zstd_decompress_batch(const void* const* d_src_ptrs,
     const hipError_t err = launch_zstd(d_src_ptrs, d_src_sizes, d_dst_ptrs, d_dst_capacities,
                                        chunk_count, d_results,
                                        reinterpret_cast<hipStream_t>(stream));
-    return err == hipSuccess ? CUDEC_OK : CUDEC_ERR_CUDA;
+    return ended(err);
 }
 
 cudec_status cudec_lz4_decompress_batch_plain(const void* const* d_src_ptrs,
@@ -174,7 +183,7 @@ cudec_status cudec_snappy_decompress_batch_plain(
 
 static cudec_status set_threshold(int format, size_t min_cost) {
     (void)hipGetLastError();
-    return set_pipe_min_cost(format, min_cost) == hipSuccess ? CUDEC_OK : CUDEC_ERR_CUDA;
+    return ended(set_pipe_min_cost(format, min_cost));
 }
 
 static cudec_status get_threshold(int format, size_t* min_cost) {
@@ -183,8 +192,9 @@ static cudec_status get_threshold(int format, size_t* min_cost) {
     }
     (void)hipGetLastError();
     uint64_t v = 0;
-    if (get_pipe_min_cost(format, &v) != hipSuccess) {
-        return CUDEC_ERR_CUDA;
+    const cudec_status st = ended(get_pipe_min_cost(format, &v));
+    if (st != CUDEC_OK) {
+        return st;
     }
     *min_cost = (size_t)v;
     return CUDEC_OK;
@@ -220,7 +230,7 @@ cudec_status cudec_mi355x_set_decode_plan(int format, const uint16_t* h_lanes_pe
         }
     }
     (void)hipGetLastError();
-    return set_decode_plan(format, h_lanes_per_bin) == hipSuccess ? CUDEC_OK : CUDEC_ERR_CUDA;
+    return ended(set_decode_plan(format, h_lanes_per_bin));
 }
 
 cudec_status cudec_mi355x_decode_plan(int format, uint16_t* h_lanes_per_bin) {
@@ -228,7 +238,7 @@ cudec_status cudec_mi355x_decode_plan(int format, uint16_t* h_lanes_per_bin) {
         return CUDEC_ERR_INVALID_ARGUMENT;
     }
     (void)hipGetLastError();
-    return get_decode_plan(format, h_lanes_per_bin) == hipSuccess ? CUDEC_OK : CUDEC_ERR_CUDA;
+    return ended(get_decode_plan(format, h_lanes_per_bin));
 }
 
 size_t cudec_mi355x_max_batch_chunks(void) { return kMaxBatchChunks; }

@@ -111,6 +111,7 @@ constexpr size_t kRunGap = 64 << 10;
 cudec_status decode_blocks(const unsigned char* f, const std::vector<Block>& blocks,
                            size_t block_max, bool sums, unsigned char* out, size_t cap,
                            size_t* total_out) {
+    const LastError taken;
     /* the blocks that go to the device: the compressed ones, and every one
      * when their checksums are checked there */
     std::vector<size_t> up, ci;

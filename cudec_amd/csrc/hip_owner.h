@@ -80,6 +80,17 @@ inline hipError_t make_timing_event(Event& e) {
     return e.make([](hipEvent_t* h) { return hipEventCreate(h); });
 }
 
+/* At the end of a call, takes back the error that a failed runtime call in it
+ * left with the thread: the status says that the call failed, and the
+ * program's next GPU call did not (an error that the device keeps stays). */
+class LastError {
+public:
+    LastError() = default;
+    ~LastError() { (void)hipGetLastError(); }
+    LastError(const LastError&) = delete;
+    LastError& operator=(const LastError&) = delete;
+};
+
 /* Memory spaces a Region can live in: how to get n bytes and give them back. */
 struct DeviceSpace {
     static hipError_t get(void** p, size_t n) { return hipMalloc(p, n); }

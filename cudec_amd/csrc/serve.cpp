@@ -387,6 +387,7 @@ extern "C" cudec_status cudec_mi355x_serve_lz4(
     if (stats != nullptr) {
         std::memset(stats, 0, sizeof(*stats));
     }
+    const LastError taken;
     try {
         Server s(h_src_ptrs, h_src_sizes, h_dst_caps, h_requests, request_count, hbm_budget,
                  max_inflight, h_results, h_digests, h_latency_s);

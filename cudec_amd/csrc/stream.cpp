@@ -490,6 +490,7 @@ cudec_status cudec_stream_ctx_create(cudec_stream_ctx** out_ctx) {
         return CUDEC_ERR_INVALID_ARGUMENT;
     }
     *out_ctx = nullptr;
+    const LastError taken;
     cudec_stream_ctx* ctx = new (std::nothrow) cudec_stream_ctx();
     if (ctx == nullptr) {
         return CUDEC_ERR_CUDA;
@@ -521,6 +522,7 @@ cudec_status cudec_lz4_decompress_stream_ctx(cudec_stream_ctx* ctx,
         stamp(h_results, chunk_count, CUDEC_ERR_CUDA);
         return CUDEC_ERR_CUDA;
     }
+    const LastError taken;
     try {
         return decode_stream(*ctx, h_src_ptrs, h_src_sizes, dst_ptrs, dst_caps, chunk_count,
                              dst_space, h_results);

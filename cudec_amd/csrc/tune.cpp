@@ -87,6 +87,7 @@ extern "C" cudec_status cudec_mi355x_autotune_lz4(
         h_best_min_cost == nullptr) {
         return CUDEC_ERR_INVALID_ARGUMENT;
     }
+    const LastError taken;
     try {
         DecodePlan previous;
         if (!read_plan(CUDEC_MI355X_FORMAT_LZ4, &previous)) {
@@ -163,6 +164,7 @@ extern "C" cudec_status cudec_mi355x_autotune_plan(
     const bool lz4 = format == CUDEC_MI355X_FORMAT_LZ4;
     auto set_threshold = lz4 ? cudec_mi355x_set_lz4_pipeline_threshold
                              : cudec_mi355x_set_snappy_pipeline_threshold;
+    const LastError taken;
     try {
         Timed run{lz4 ? cudec_lz4_decompress_batch : cudec_snappy_decompress_batch,
                   d_src_ptrs, d_src_sizes, d_dst_ptrs, d_dst_capacities, chunk_count, d_results,

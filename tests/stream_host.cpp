@@ -17,6 +17,8 @@ struct Counts {
 } g_counts;
 std::unordered_map<void*, size_t> g_sizes;
 int g_device = 0;
+hipError_t g_last = hipSuccess; /* the thread's last error */
+constexpr size_t kNoMemory = size_t{1} << 40;
 }  // namespace
 
 extern "C" {
@@ -29,7 +31,11 @@ hipError_t hipSetDevice(int d) {
     g_device = d;
     return hipSuccess;
 }
-hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned int) {
     *s = static_cast<hipStream_t>(std::malloc(8));
     g_counts.streams++;
@@ -62,6 +68,9 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
     return e == nullptr ? hipErrorInvalidHandle : hipSuccess;
 }
 hipError_t hipMalloc(void** p, size_t n) {
+    if (n >= kNoMemory) {
+        return g_last = hipErrorOutOfMemory;
+    }
     *p = std::malloc(n);
     g_sizes[*p] = n;
     g_counts.open++;
@@ -76,6 +85,9 @@ hipError_t hipFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned int) {
+    if (n >= kNoMemory) {
+        return g_last = hipErrorOutOfMemory;
+    }
     *p = std::malloc(n);
     g_counts.open++;
     return hipSuccess;
@@ -109,6 +121,9 @@ cudec_status cudec_lz4_decompress_batch(const void* const* src, const size_t* si
     }
     return CUDEC_OK;
 }
+
+/* What the program's next GPU call would report. */
+int host_last_error(void) { return g_last; }
 
 void host_stream_counts(uint64_t* out) { std::memcpy(out, &g_counts, sizeof(g_counts)); }
 

@@ -8,7 +8,8 @@ cudec_amd/csrc/stream.cpp over a stand-in for the HIP runtime on the CPU
 * host buffers of one call that lie over each other: what a call of one wave
   gives, every source read before the first byte is written and chunks written
   in order;
-* results and bytes of calls of one and of many waves."""
+* results and bytes of calls of one and of many waves;
+* a call whose staging cannot be had leaves no error with the thread."""
 import ctypes
 import os
 import subprocess
@@ -178,3 +179,18 @@ def test_buffers_side_by_side(lib):
             assert st == 0
         assert streams_of(lib, call) == 4
         assert np.array_equal(arena, want)
+
+
+@pytest.mark.parametrize("size,cap", [(1, 1 << 44), (1 << 44, 1)])
+def test_a_failed_call_leaves_no_error(lib, size, cap):
+    """Its status says so; the program's next GPU call did not fail."""
+    byte = np.zeros(1, np.uint8)
+    before = counts(lib)
+    with Context(lib) as ctx:
+        for _ in range(2):  # the second finds the context poisoned
+            st, res = ctx.run([byte.ctypes.data], [size], [byte.ctypes.data], [cap])
+            assert st == libs.DEVICE and np.all(res["status"] == libs.DEVICE)
+            assert lib.host_last_error() == 0
+    assert counts(lib)["open"] == before["open"] and lib.host_last_error() == 0
+    with Context(lib) as ctx:
+        plain(ctx, 3, 1000)
