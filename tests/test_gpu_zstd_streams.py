@@ -1,6 +1,7 @@
 """The Zstandard batch entry beside itself and its checksum pass, held to
 libzstd alone: two batches at once on two streams, each with scratch of its
-own, and content checksums with a bit flipped."""
+own, content checksums with a bit flipped, and batches around one and two
+frames for each resident block (2048 on 256 CUs)."""
 import random
 
 import numpy as np
@@ -61,3 +62,30 @@ def test_checksum_bits():
     torch.cuda.synchronize()
     status = db.results()["status"].reshape(-1, 33)
     assert np.all(status[:, 0] == libs.OK) and np.all(status[:, 1:] == libs.CORRUPT)
+
+
+@pytest.mark.parametrize("n", [1, 2, 2047, 2048, 2049, 4096, 4097, 5000])
+def test_frames_for_each_block(n):
+    import torch
+    from cudec_amd.device import DeviceBatch
+    rng = np.random.default_rng(n)
+    base = workload.build(workload.CODEC_ZSTD, rng.integers(1, 3000, 40), rng.integers(0, 3, 40),
+                          rng.integers(1, 1 << 60, 40))
+    which = rng.integers(0, 40, n)
+    frames = [base.compressed(int(i)) for i in which]
+    caps = [int(base.sizes[i]) for i in which]
+    want = [base.original(int(i)) for i in which]
+    bad = set(range(3, n, 11))
+    for i in bad:
+        frames[i] = frames[i][:-1]
+    db = DeviceBatch.from_streams(frames, caps, poison=0x5A)
+    db.reset_results()
+    print(f"[zstd blocks] {n} frames", flush=True)
+    assert db.run("zstd", "tuned") == 0
+    torch.cuda.synchronize()
+    res = db.results()
+    outs = db.outputs(res)
+    for i in range(n):
+        assert res["status"][i] == (libs.CORRUPT if i in bad else libs.OK), i
+        assert res["bytes_written"][i] == (0 if i in bad else caps[i])
+        assert i in bad or outs[i] == want[i], i
