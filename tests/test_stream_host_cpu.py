@@ -2,7 +2,8 @@
 cudec_amd/csrc/stream.cpp over a stand-in for the HIP runtime on the CPU
 (tests/stream_host.cpp), where a chunk decodes to its own bytes.
 
-* a context makes the streams that its calls need, no more;
+* a context that is kept has its four streams from the start, made one after
+  the other; that of a single call has those that the call uses;
 * what it keeps for the next call stays within two budgets of staging (1 GiB
   each, or the largest chunk);
 * host buffers of one call that lie over each other: what a call of one wave
@@ -40,6 +41,7 @@ def lib():
     lib.cudec_stream_ctx_destroy.argtypes = [vp]
     lib.cudec_stream_ctx_destroy.restype = None
     lib.cudec_lz4_decompress_stream_ctx.argtypes = [vp, vp, vp, vp, vp, sz, ctypes.c_int, vp]
+    lib.cudec_lz4_decompress_stream.argtypes = [vp, vp, vp, vp, sz, ctypes.c_int, vp]
     lib.host_stream_counts.argtypes = [vp]
     lib.host_stream_counts.restype = None
     return lib
@@ -72,6 +74,20 @@ class Context:
         self.lib.cudec_stream_ctx_destroy(self.h)
 
 
+class OneCall:
+    """The call that makes a context for itself."""
+    def __init__(self, lib):
+        self.lib = lib
+
+    def run(self, src, sizes, dst, caps):
+        n = len(sizes)
+        a = [np.array(v, dtype=np.uint64) for v in (src, sizes, dst, caps)]
+        res = np.zeros(n, RES)
+        st = self.lib.cudec_lz4_decompress_stream(*(v.ctypes.data for v in a), n, HOST,
+                                                  res.ctypes.data)
+        return st, res
+
+
 def plain(ctx, n, size):
     """A call of n chunks of `size` bytes, checked."""
     data = np.random.default_rng(n).integers(0, 256, n * size, dtype=np.uint8)
@@ -87,15 +103,17 @@ def plain(ctx, n, size):
 @pytest.mark.parametrize("n,streams", [(1, 1), (23, 1), (24, 2), (40, 3), (60, 4), (200, 4)])
 def test_streams_of_a_context(lib, n, streams):
     before = counts(lib)
+    plain(OneCall(lib), n, MIB)
+    made = counts(lib)
+    assert made["streams"] - before["streams"] == streams
+    assert made["events"] - before["events"] == streams
     with Context(lib) as ctx:
-        made = counts(lib)
-        assert made["streams"] - before["streams"] == 1
-        assert made["events"] - before["events"] == 1
-        for _ in range(2):
+        # none made between those of a context
+        for _ in range(3):
+            made = counts(lib)
+            assert made["streams"] - before["streams"] == streams + 4
+            assert made["events"] - before["events"] == streams + 4
             plain(ctx, n, MIB)
-        made = counts(lib)
-        assert made["streams"] - before["streams"] == streams
-        assert made["events"] - before["events"] == streams
     assert counts(lib)["open"] == before["open"]
 
 
@@ -117,11 +135,11 @@ def test_staging_kept(lib, calls):
         plain(ctx, 60, MIB)
 
 
-def streams_of(lib, ctx_calls):
+def streams_of(lib, call):
+    """Made by a call with a context of its own."""
     before = counts(lib)["streams"]
-    with Context(lib) as ctx:
-        ctx_calls(ctx)
-        return counts(lib)["streams"] - before
+    call(OneCall(lib))
+    return counts(lib)["streams"] - before
 
 
 # (over its own source or an earlier one, it does not matter when it is written)
