@@ -19,9 +19,10 @@ class CopyCrew {
 public:
     static constexpr size_t kBytesPerHelper = size_t{8} << 20;
 
-    /* `bytes`: what the call copies in all. A helper costs about 20 us to
-     * start, and more than seven do not copy faster. */
-    explicit CopyCrew(size_t bytes) {
+    /* `bytes`: what the call copies in all, of `items` of about one size. A
+     * helper costs about 20 us to start, and more than seven do not copy
+     * faster. */
+    CopyCrew(size_t bytes, size_t items) : step_(step_of(bytes, items)) {
         const size_t most = bytes / kBytesPerHelper < kMostHelpers ? bytes / kBytesPerHelper
                                                                    : kMostHelpers;
         const size_t cores = std::thread::hardware_concurrency();
@@ -78,9 +79,21 @@ private:
 
     using Call = void (*)(const void* work, size_t i);
 
+    /* Items that a thread takes at once: kClaimBytes of them, since threads
+     * that ask one counter for 1.6 KiB each wait for the counter (20 000 such
+     * chunks to the device through a kept context: 3.3 ms one by one, 1.2
+     * so; to the host 6.0 and 2.4). */
+    static constexpr size_t kClaimBytes = size_t{64} << 10;
+    static size_t step_of(size_t bytes, size_t items) {
+        const size_t each = items == 0 ? 0 : bytes / items;
+        return each >= kClaimBytes ? 1 : kClaimBytes / (each + 1) + 1;
+    }
     void claim(size_t n, Call call, const void* work) {
-        for (size_t i = next_.fetch_add(1); i < n; i = next_.fetch_add(1)) {
-            call(work, i);
+        for (size_t from = next_.fetch_add(step_); from < n; from = next_.fetch_add(step_)) {
+            const size_t to = n - from < step_ ? n : from + step_;
+            for (size_t i = from; i < to; i++) {
+                call(work, i);
+            }
         }
     }
     void help() {
@@ -104,6 +117,7 @@ private:
         }
     }
 
+    const size_t step_;
     std::mutex lock_;
     std::condition_variable wake_, idle_;
     const void* work_ = nullptr;

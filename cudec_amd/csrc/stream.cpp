@@ -371,7 +371,7 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     stamp(pres, n, CUDEC_ERR_CUDA);
     cudec_status failure = CUDEC_OK;
     Drain drain(ctx, used);
-    CopyCrew crew(in_order ? 0 : total);
+    CopyCrew crew(in_order ? 0 : total, n);
 
     for (size_t w = 0; w < waves && failure == CUDEC_OK; w++) {
         Slot& s = ctx.slot[w % slots];

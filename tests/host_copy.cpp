@@ -30,7 +30,7 @@ extern "C" {
  * every allocation refused meanwhile. hits[i] counts the calls for item i.
  * Returns the allocations refused, or -1 when a round threw. */
 int64_t host_copy_rounds(uint64_t bytes, uint64_t n, uint64_t rounds, uint32_t* hits) {
-    cudec_amd::CopyCrew crew(bytes);
+    cudec_amd::CopyCrew crew(bytes, n);
     g_refused = 0;
     g_refuse = true;
     bool threw = false;
@@ -48,6 +48,15 @@ int64_t host_copy_rounds(uint64_t bytes, uint64_t n, uint64_t rounds, uint32_t* 
     }
     g_refuse = false;
     return threw ? -1 : (int64_t)g_refused.load();
+}
+
+/* One round over n items of `bytes` bytes; owner[i] tells the threads apart. */
+void host_copy_owners(uint64_t bytes, uint64_t n, uint64_t* owner) {
+    cudec_amd::CopyCrew crew(bytes, n);
+    crew.each(n, [&](size_t i) {
+        static thread_local char here;
+        owner[i] = (uint64_t)(uintptr_t)&here;
+    });
 }
 
 }  // extern "C"
