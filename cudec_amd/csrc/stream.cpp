@@ -63,7 +63,8 @@ struct Slot {
 
 struct cudec_stream_ctx {
     cudec_amd::Slot slot[cudec_amd::kSlots];
-    int device = 0;                          /* the streams' */
+    int device = 0;    /* the streams' */
+    bool once = false; /* the context of a single call */
     cudec_amd::DeviceRegion d_results;
     cudec_amd::PinnedRegion p_results;
     bool poisoned = false;
@@ -329,8 +330,11 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     }
     /* two slots where four would stage more than two full budgets, with what
      * the slots keep of earlier calls; that much is what a context keeps,
-     * unless a chunk of this call is larger than a budget */
-    size_t slots = in_order ? 2 : kSlots;
+     * unless a chunk of this call is larger than a budget. Two as well where
+     * the staging serves this call alone: making it and giving it back takes
+     * longer than four waves in hand save (2048 chunks of 16 to 256 KiB: 20.9
+     * ms with four, 11.8 with two; 100 000 of 0.1 to 2 KiB: 17.9 and 11.9) */
+    size_t slots = in_order || ctx.once ? 2 : kSlots;
     size_t used = waves < slots ? waves : slots;
     const size_t wave_dst = host_out ? max_dst : 0;
     if (staging(ctx, used, max_src, wave_dst) > 2 * kWaveBudget) {
@@ -486,14 +490,18 @@ cudec_status decode_stream(cudec_stream_ctx& ctx, const void* const* h_src_ptrs,
     return CUDEC_OK;
 }
 
-/* A context with streams for the first `slots` slots, or null. */
-cudec_stream_ctx* make_context(size_t slots) {
+/* A context, or null: with all its streams, or, for a single call, without. */
+cudec_stream_ctx* make_context(bool once) {
     const LastError taken;
     cudec_stream_ctx* ctx = new (std::nothrow) cudec_stream_ctx();
     if (ctx != nullptr &&
-        (hipGetDevice(&ctx->device) != hipSuccess || open_slots(*ctx, slots) != hipSuccess)) {
+        (hipGetDevice(&ctx->device) != hipSuccess ||
+         open_slots(*ctx, once ? 0 : kSlots) != hipSuccess)) {
         delete ctx;
-        ctx = nullptr;
+        return nullptr;
+    }
+    if (ctx != nullptr) {
+        ctx->once = once;
     }
     return ctx;
 }
@@ -509,7 +517,7 @@ cudec_status cudec_stream_ctx_create(cudec_stream_ctx** out_ctx) {
     if (out_ctx == nullptr) {
         return CUDEC_ERR_INVALID_ARGUMENT;
     }
-    *out_ctx = make_context(kSlots);
+    *out_ctx = make_context(false);
     return *out_ctx != nullptr ? CUDEC_OK : CUDEC_ERR_CUDA;
 }
 
@@ -563,7 +571,7 @@ cudec_status cudec_lz4_decompress_stream(const void* const* h_src_ptrs,
     if (args != CUDEC_OK) {
         return args;
     }
-    cudec_stream_ctx* ctx = make_context(0);
+    cudec_stream_ctx* ctx = make_context(true);
     if (ctx == nullptr) {
         return CUDEC_ERR_CUDA;
     }

@@ -3,7 +3,8 @@ cudec_amd/csrc/stream.cpp over a stand-in for the HIP runtime on the CPU
 (tests/stream_host.cpp), where a chunk decodes to its own bytes.
 
 * a context that is kept has its four streams from the start, made one after
-  the other; that of a single call has those that the call uses;
+  the other; that of a single call has those that the call uses, two at most,
+  as much staging, and none of either is left;
 * what it keeps for the next call stays within two budgets of staging (1 GiB
   each, or the largest chunk);
 * host buffers of one call that lie over each other: what a call of one wave
@@ -44,6 +45,7 @@ def lib():
     lib.cudec_lz4_decompress_stream.argtypes = [vp, vp, vp, vp, sz, ctypes.c_int, vp]
     lib.host_stream_counts.argtypes = [vp]
     lib.host_stream_counts.restype = None
+    lib.host_stream_most_from_here.restype = None
     return lib
 
 
@@ -100,7 +102,7 @@ def plain(ctx, n, size):
 
 
 # chunks of 1 MiB in and out: 24 MiB a wave at least, four waves at once
-@pytest.mark.parametrize("n,streams", [(1, 1), (23, 1), (24, 2), (40, 3), (60, 4), (200, 4)])
+@pytest.mark.parametrize("n,streams", [(1, 1), (23, 1), (24, 2), (40, 2), (60, 2), (200, 2)])
 def test_streams_of_a_context(lib, n, streams):
     before = counts(lib)
     plain(OneCall(lib), n, MIB)
@@ -115,6 +117,17 @@ def test_streams_of_a_context(lib, n, streams):
             assert made["events"] - before["events"] == streams + 4
             plain(ctx, n, MIB)
     assert counts(lib)["open"] == before["open"]
+
+
+def test_staging_of_a_single_call(lib):
+    """Eight waves of 25 MiB in and as much out, two of them in hand."""
+    before = counts(lib)
+    assert before["held"] == 0
+    lib.host_stream_most_from_here()
+    plain(OneCall(lib), 200, MIB)
+    after = counts(lib)
+    assert 100 * MIB <= after["most"] <= 100 * MIB + 65536
+    assert after["open"] == before["open"] and after["held"] == 0
 
 
 @pytest.mark.parametrize("calls", ["AB", "BA", "ABAB", "CAB"])
@@ -143,9 +156,10 @@ def streams_of(lib, call):
 
 
 # (over its own source or an earlier one, it does not matter when it is written)
+@pytest.mark.parametrize("kept", [False, True])
 @pytest.mark.parametrize("n,ahead,streams", [(200, 110, 1), (200, 1, 1), (60, 59, 1),
-                                             (200, -110, 4), (200, -1, 4), (200, 0, 4)])
-def test_outputs_over_sources(lib, n, ahead, streams):
+                                             (200, -110, 2), (200, -1, 2), (200, 0, 2)])
+def test_outputs_over_sources(lib, n, ahead, streams, kept):
     """Chunk i's output lies where chunk i + ahead's input does."""
     pad = max(0, -ahead)
     arena = np.random.default_rng(5).integers(0, 256, (n + abs(ahead)) * MIB, dtype=np.uint8)
@@ -158,9 +172,12 @@ def test_outputs_over_sources(lib, n, ahead, streams):
     def call(ctx):
         st, res = ctx.run(src, [MIB] * n, dst, [MIB] * n)
         assert st == 0 and np.all(res["bytes_written"] == MIB)
-    made = streams_of(lib, call)
+    if kept:
+        with Context(lib) as ctx:
+            call(ctx)
+    else:
+        assert streams_of(lib, call) == streams
     assert np.array_equal(arena, want)
-    assert made == streams
 
 
 @pytest.mark.parametrize("step", [0, 1000])
@@ -195,7 +212,12 @@ def test_buffers_side_by_side(lib):
         def call(ctx):
             st, res = ctx.run(src, [MIB] * n + [0, 0], dst, [MIB] * n + [0, 0])
             assert st == 0
-        assert streams_of(lib, call) == 4
+        before = arena.copy()
+        assert streams_of(lib, call) == 2
+        assert np.array_equal(arena, want)
+        arena[:] = before
+        with Context(lib) as ctx:
+            call(ctx)
         assert np.array_equal(arena, want)
 
 
