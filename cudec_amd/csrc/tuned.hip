@@ -1042,19 +1042,83 @@ __device__ __forceinline__ uint32_t walk_step(const uint8_t* cw, uint32_t p, uin
     return walk_step_lz4(cw, p, limit);
 }
 
+/* Data whose chains do not meet. Lengths that repeat (columns of integers, a
+ * period in Snappy's elements of 64 bytes) or two or three bytes a sequence
+ * keep a wrong chain wrong for all of a window, and then every round moves
+ * most lanes on by one segment: 64 rounds, 2700 steps a window and as many
+ * LDS reads on every lane (1000 LZ4 chunks of 1 MiB of two symbols: 76.8 ms).
+ * Chains that do meet take few rounds (1 window in 100 of 1 MiB LZ4 tokens
+ * takes more than 8, of text, tables and sorted numbers more than 5). So after
+ * kWalkRounds the rest of the window is walked as the one-wave form walks
+ * (walk_dense), from every byte position, and so are the next kDenseWindows.
+ * (Smaller segments take more rounds of fewer steps, and are left to it.) */
+constexpr uint32_t kWalkRounds = 12;
+constexpr uint32_t kDenseWindows = 15;
+/* walk_dense's link table lies behind the positions it lists. */
+constexpr uint32_t kDenseTable = kCandSplit * kWave;
+constexpr uint32_t dense_max(uint32_t most) { return most - kDenseTable; }
+/* Marks of a link there: out of the walk's range, or a member whose end the
+ * window cannot tell. */
+constexpr uint32_t kLinkOut = 0x4000u, kLinkStop = 0x8000u, kLinkAt = 0x3FFFu;
+static_assert(kCandSplit * kWave + 4 + 15 + 255 * (kWalkExtra + 2) < kLinkAt, "links fit");
+
+/* Lists the chain's members from window position `from` to `end`, 64 at a
+ * time, behind the `count` listed so far, and returns as walk_window does.
+ * Every position is a candidate, eight a lane, and pointer doubling follows
+ * the chain through their links. */
+template <int kFormat, uint32_t kMost>
+__device__ __forceinline__ uint32_t walk_dense(const uint8_t* cw, uint32_t from, uint32_t end,
+                                               uint32_t limit, uint32_t lim, uint16_t* list,
+                                               uint32_t& count, uint32_t lane) {
+    uint16_t* jump = list + dense_max(kMost);
+    while (from < end && count + kWave <= dense_max(kMost)) {
+        const uint32_t range = end - from;
+        uint32_t link[kCandSplit];
+#pragma unroll
+        for (uint32_t k = 0; k < kCandSplit; k++) {
+            const uint32_t c = k * kWave + lane;
+            const uint32_t next = walk_step<kFormat>(cw, c < range ? from + c : from, limit, lim);
+            const uint32_t to = (next & ~kWalkStop) - from;
+            link[k] = (next & kWalkStop) != 0 ? kLinkStop | c
+                      : to >= range           ? kLinkOut | to
+                                              : to;
+        }
+        uint32_t found = 0, member = 0;
+        const uint32_t next = walk_doubling<kCandSplit>(link, 0, jump, found, member, lane);
+        if (lane < found) {
+            list[count + lane] = (uint16_t)(from + member);
+        }
+        count += found;
+        if ((next & kLinkStop) != 0) {
+            return kWalkStop | (from + (next & kLinkAt));
+        }
+        from += next & kLinkAt;
+    }
+    return from;
+}
+
 /* Walks the window's chain (see above) from its first byte and lists its
  * members; returns where it goes on: a window position, or kWalkStop | the
- * last listed member, whose end the window cannot tell. */
+ * last listed member, whose end the window cannot tell. `dense`: windows
+ * still to be walked from every position. */
 template <int kFormat, uint32_t kMost>
 __device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segment,
                                                 uint32_t limit, uint32_t lim, uint16_t* list,
-                                                uint32_t& count, uint32_t lane) {
+                                                uint32_t& count, uint32_t& dense, uint32_t lane) {
     const uint32_t start = lane * segment;
     const uint32_t end = start + segment < lim ? start + segment : lim;
     uint32_t entry = start;
     uint32_t exit, mine;
     bool moves = true;
-    for (;;) {
+    /* from where on the chain is walked from every position */
+    uint32_t rest = dense != 0 ? 0u : kWalkStop;
+    if (dense != 0) {
+        dense--;
+        entry = lim;
+        exit = 0;
+        mine = 0;
+    }
+    for (uint32_t round = 0; rest != 0; round++) {
         if (moves) {
             mine = 0;
             exit = entry;
@@ -1074,10 +1138,13 @@ __device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segm
          * so is where the chain goes from there */
         const uint32_t first = (uint32_t)__builtin_ctzll(moved);
         const uint32_t reached = uniform32(__builtin_amdgcn_readlane(from, first));
-        if (reached >= lim) {
-            /* the chain stops, or leaves the source, before that lane */
+        if (reached >= lim || (round >= kWalkRounds && segment >= kSegment)) {
+            /* the chain stops, or leaves the source, before that lane (or the
+             * rest is for walk_dense) */
+            rest = reached;
+            dense = reached < lim ? kDenseWindows : 0;
             if (lane >= first) {
-                entry = reached;
+                entry = lim;
                 exit = reached;
                 mine = 0;
             }
@@ -1108,6 +1175,10 @@ __device__ __forceinline__ uint32_t walk_window(const uint8_t* cw, uint32_t segm
         return uniform32(__builtin_amdgcn_readlane(next, __builtin_ctzll(holder)));
     }
     count = total;
+    if (rest < lim) {
+        return walk_dense<kFormat, kMost>(cw, rest, segment * kWave < lim ? segment * kWave : lim,
+                                          limit, lim, list, count, lane);
+    }
     return uniform32(__builtin_amdgcn_readlane(exit, kWave - 1));
 }
 
@@ -1130,6 +1201,7 @@ __device__ __forceinline__ void run_parser(L& l, gcu8* src, uint64_t src_size, u
         }
     }
     uint32_t segment = kSegmentFirst;
+    uint32_t dense = 0;
     for (uint32_t w = 0;; w++) {
         const uint32_t b = w & 1;
         const lds_flag* over = (const lds_flag*)&l.claim;
@@ -1160,7 +1232,7 @@ __device__ __forceinline__ void run_parser(L& l, gcu8* src, uint64_t src_size, u
         const uint8_t* cw = stage + delta;
         uint32_t count = 0;
         const uint32_t next =
-            walk_window<kFormat, list_max(kSeg)>(cw, segment, limit, lim, list, count, lane);
+            walk_window<kFormat, list_max(kSeg)>(cw, segment, limit, lim, list, count, dense, lane);
         bool last = false;
         uint64_t next_base = base + next;
         /* a wide window only behind one that was not cut short: what it stages
