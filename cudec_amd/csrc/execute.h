@@ -598,8 +598,10 @@ __device__ __forceinline__ void put_literal(W& w, const uint8_t* from, uint32_t 
  * bytes that followers may overwrite in the ring count as gone. */
 struct Alone {
     static constexpr bool kInTurn = false;
+    static constexpr bool kStrips = true; /* run_strips where it pays */
     __device__ uint64_t final_below(uint64_t d0) const { return d0; }
     __device__ bool wait_turn() const { return true; }
+    __device__ void pass(uint64_t) const {} /* the group's bytes are in the ring */
 };
 
 /* Lane's members a..b (as a mask) that cover bytes [from, to) of the group,
@@ -633,6 +635,64 @@ __device__ __forceinline__ uint64_t members_covering(CoverLds& c, bool active, u
 /* Matches longer than this go 16 bytes a lane (ring_match_wide) instead of
  * a byte a lane and 64 a step. */
 constexpr uint32_t kWideMatch = 256;
+
+/* Output bytes a member from which on members go one by one rather than by
+ * strips (run_strips): 312 cycles a member that waits for the one before it,
+ * about 700 a strip of 64 bytes. With 16, 24 and 40: 1000 LZ4 chunks of 1 MiB
+ * of text 8.7, 7.45 and 7.40 ms, the uneven Snappy batch 12.25, 12.25 and
+ * 12.35, Snappy's sparse bytes 2.75, 2.80 and 3.04. */
+constexpr uint32_t kStripMember = 24;
+constexpr uint32_t kStripAt = 1u << 12, kStripOffset = 1u << 14; /* what its word holds */
+static_assert(kBatchMax < kStripAt - 1 && kRing <= kStripOffset && kLaneMatch <= 64,
+              "12 bits of a match's start, 14 of its offset, 6 of its length");
+
+/* Many short matches of which each may wait for the one before (columns of
+ * numbers, few symbols): by output bytes, 64 at a time, a byte a lane. A
+ * byte's source is its member's offset back; where that is a byte of the same
+ * strip that is itself still to be copied, it is that byte's source instead,
+ * and so on: pointer doubling over the wave, at most six rounds. Every source
+ * is then final, and one read and one write copy the strip. `todo` holds the
+ * members (matches of up to 64 bytes whose sources lie in the ring); `c` says
+ * which member covers a byte.
+ *
+ * What bounds it is the latency of about four lane shuffles a strip. One chunk
+ * of 1 MiB of sorted 64-bit numbers, eight members a strip: 17.2 ms one member
+ * after the other, 7.3 so; of text 7.3 and 6.0; 5000 of 64 KiB on a wave each:
+ * 2.65 and 1.53 ms, text 1.64 and 1.53. */
+template <class W>
+__device__ __forceinline__ void run_strips(W& w, const CoverLds& c, uint32_t ring_at,
+                                           uint32_t m_rel, uint32_t offset, uint32_t match_len,
+                                           uint64_t todo, uint32_t end_rel, uint32_t lane) {
+    /* match start, offset and length in one word; none: past every byte */
+    constexpr uint32_t kAt = kStripAt - 1;
+    const uint32_t info = ((todo >> lane) & 1) != 0
+                              ? m_rel | offset << 12 | (match_len - 1) << 26
+                              : kAt;
+    for (uint32_t s = 0; s < end_rel; s += kWave) {
+        const uint64_t starts = c.starts[s / kWave];
+        const uint32_t member = c.before[s / kWave] +
+                                (uint32_t)__builtin_popcountll(starts & (~0ull >> (63 - lane))) - 1;
+        const uint32_t mine = (uint32_t)__shfl((int)info, (int)(member & (kWave - 1)));
+        const int pos = (int)(s + lane);
+        const int i = pos - (int)(mine & kAt);
+        const bool copies = i >= 0 && i <= (int)(mine >> 26);
+        int from = copies ? pos - (int)((mine >> 12) & (kStripOffset - 1)) : pos;
+        for (;;) {
+            const int at = from - (int)s;
+            const int further = __shfl(from, at & (int)(kWave - 1));
+            const bool moves = at >= 0 && further != from;
+            if (__ballot(moves) == 0) {
+                break;
+            }
+            from = moves ? further : from;
+        }
+        if (copies) {
+            w.ring[(ring_at + (uint32_t)pos) & (W::kSize - 1)] =
+                w.ring[(ring_at + (uint32_t)from) & (W::kSize - 1)];
+        }
+        wave_order();
+    }
+}
 
 /* Executes group g of the window staged at cw into the ring at output
  * positions [dp, dp + g.end_rel), flushes whole 16-byte blocks (all of them
@@ -789,6 +849,11 @@ __device__ __forceinline__ bool execute_group(W& w, CoverLds& cover_lds, const u
         const uint64_t before = below == 0 ? 0 : 1ull << (63 - __builtin_clzll(below));
         const uint64_t tied = __ballot((waits_for & before) != 0) | ~(once_mask | again_mask);
         undone &= ~todo;
+        if (Order::kStrips && (todo & ~(once_mask | again_mask)) == 0 &&
+            (uint32_t)__builtin_popcountll(todo) * kStripMember > g.end_rel) {
+            run_strips(w, cover_lds, ring_at, m_rel, offset, match_len, todo, g.end_rel, lane);
+            todo = 0;
+        }
         while (todo != 0) {
             const uint32_t j = __builtin_ctzll(todo);
             clear_bit(todo, j);
@@ -857,6 +922,7 @@ __device__ __forceinline__ bool execute_group(W& w, CoverLds& cover_lds, const u
         later = 0;
     }
     dp = D1;
+    order.pass(D1);
     const uintptr_t a_end = done ? da + dp : ((da + dp) & ~(uintptr_t)15);
     const uint64_t to = a_end > da + flushed ? (uint64_t)(a_end - da) : flushed;
     if (to > flushed) {

@@ -1040,6 +1040,12 @@ __device__ __forceinline__ void fill_bytes(gu8* to, uint32_t fill, uint32_t n, u
     wave_order();
 }
 
+/* The copy wave's groups go without strips: it is the entropy wave that a
+ * frame of short matches waits for, and their registers cost the kernel 3%. */
+struct AloneInOrder : Alone {
+    static constexpr bool kStrips = false;
+};
+
 /* A batch of cnt sequences, as groups that the ring and the literals' stage
  * hold; a sequence that fits neither goes global to global. */
 __device__ __forceinline__ void run_sequences(CopyLds& w, CopyState& s, const Job& j, uint32_t cnt,
@@ -1085,7 +1091,7 @@ __device__ __forceinline__ void run_sequences(CopyLds& w, CopyState& s, const Jo
         g.terminal = false;
         g.end_rel = uniform32(__builtin_amdgcn_readlane(out_incl, take - 1));
         execute_group(w, w.cover, w.stage + delta, g, s.dst, s.cap, s.dp, s.flushed, s.ring_lo,
-                      false, lane, Alone{});
+                      false, lane, AloneInOrder{});
         lp += lits;
         i += take;
     }
