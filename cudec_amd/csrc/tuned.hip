@@ -1071,12 +1071,16 @@ __device__ __forceinline__ uint32_t walk_step(const uint8_t* cw, uint32_t p, uin
  * keep a wrong chain wrong for all of a window, and then every round moves
  * most lanes on by one segment: 64 rounds, 2700 steps a window and as many
  * LDS reads on every lane (1000 LZ4 chunks of 1 MiB of two symbols: 76.8 ms).
- * Chains that do meet take few rounds (1 window in 100 of 1 MiB LZ4 tokens
- * takes more than 8, of text, tables and sorted numbers more than 5). So after
- * kWalkRounds the rest of the window is walked as the one-wave form walks
- * (walk_dense), from every byte position, and so are the next kDenseWindows.
- * (Smaller segments take more rounds of fewer steps, and are left to it.) */
-constexpr uint32_t kWalkRounds = 12;
+ * Chains that do meet take few rounds (1 window in 80 of 1 MiB LZ4 tokens
+ * takes more than 8, 1 in 650 more than 10 and 1 in 6000 more than 12; of text,
+ * tables and sorted numbers 1 in 100 more than 5). So after kWalkRounds the rest
+ * of the window is walked as the one-wave form walks (walk_dense), from every
+ * byte position, and so are the next kDenseWindows. Those cost a chunk whose
+ * chains do meet 0.3 ms, and a launch waits for its slowest chunk, so the line
+ * lies where no such window comes: with 12 rounds 1500 token chunks of 4 KiB to
+ * 1 MiB took 1.87 ms, and 1.76 with 16 and 20. (Smaller segments take more
+ * rounds of fewer steps, and are left to it.) */
+constexpr uint32_t kWalkRounds = 20;
 constexpr uint32_t kDenseWindows = 15;
 /* walk_dense's link table lies behind the positions it lists. */
 constexpr uint32_t kDenseTable = kCandSplit * kWave;
