@@ -19,7 +19,8 @@
  *   2. find      -- where the window's sequences (LZ4) or elements (Snappy),
  *                   its members, start. A pipelined block walks 64 segments
  *                   of the window at once, a lane each ("pipelined blocks"
- *                   below). A lone wave parses eight candidate positions a
+ *                   below; where their chains do not meet, as a lone wave
+ *                   does). A lone wave parses eight candidate positions a
  *                   lane as if a member started there, and follows the true
  *                   chain through their links by pointer doubling: its
  *                   windows hold 512 bytes, and the segment walk there is
@@ -35,7 +36,8 @@
  *   4. execute   -- output goes through an LDS ring (execute.h): literals by
  *                   member lanes; matches whose sources are final by member
  *                   lanes (batched 16-byte history loads); the rest in stream
- *                   order with the wave fanned out over the bytes;
+ *                   order with the wave fanned out over the bytes, or, many
+ *                   short ones, 64 output bytes at a time;
  *   5. flush     -- completed ring bytes leave as aligned 16-byte stores;
  *                   only a chunk's first and last partial blocks use byte
  *                   stores, so exactly bytes_written bytes are stored.
@@ -1705,7 +1707,17 @@ __global__ void __launch_bounds__(kPipeBlock)
     __shared__ PipeLds<kSeg> l;
     const uint32_t lane = __lane_id();
     const uint32_t wave = uniform32(threadIdx.x / kWave);
-    QueueCursor cursor{kSubs == 0 ? 0 : blockIdx.x % (kSubs == 0 ? 1 : kSubs), kSubs};
+    /* Of the one queue, every block starts with its own position. Of a CU's
+     * four blocks the first to come is the fastest (1.76 us a KiB of a 1 MiB
+     * chunk, 2.05 on the third), and where blocks took the positions as they
+     * reached the counter, an unrelated change to the code before it gave the
+     * largest chunks to late ones (3000 chunks of 4 KiB to 1 MiB: 1.79 -> 2.14
+     * ms; 1.80 so. The uneven LZ4 batch takes 1% longer than without it). */
+    QueueCursor cursor{kSubs == 0   ? 0
+                       : kSubs == 1 ? gridDim.x
+                                    : blockIdx.x % (kSubs == 0 ? 1 : kSubs),
+                       kSubs};
+    uint32_t start = kSubs == 1 ? blockIdx.x : (uint32_t)n;
     uint32_t idx;
     if (kSubs != 0 && none_piped(q)) {
         return; /* alone_batch follows and takes them all */
@@ -1717,7 +1729,8 @@ __global__ void __launch_bounds__(kPipeBlock)
         /* every wave is done with the previous chunk's control words */
         __syncthreads();
         if (wave == 0) {
-            l.chunk_idx = queue_pop<kSubs>(q, n, cursor, lane, blockIdx.x);
+            l.chunk_idx = start < n ? start : queue_pop<kSubs>(q, n, cursor, lane, blockIdx.x);
+            start = (uint32_t)n;
             l.next.dp = 0;
             l.next.flushed = 0;
             l.next.ring_lo = 0;
@@ -1768,10 +1781,10 @@ __global__ void __launch_bounds__(kPipeBlock)
 /* The persistent decoder of launches where every chunk runs on one wave:
  * those are bound by throughput and gain from a fifth wave per SIMD (96
  * VGPRs): 16 384 token chunks of 64 KiB in 2.69 ms against 3.05 by
- * piped_batch's split blocks. Only the queue build knows whether a batch has
- * chunks to pipeline, so it `follows` a piped_batch that leaves batches
- * without one untouched, and leaves the others to that: an empty launch is
- * about 2 us, and up to 8 with the gap before the next. (With that launch, a
+ * piped_batch's split blocks, and 2.62 now. Only the queue build knows whether
+ * a batch has chunks to pipeline, so it `follows` a piped_batch that leaves
+ * batches without one untouched, and leaves the others to that: an empty launch
+ * is about 2 us, and up to 8 with the gap before the next. (With that launch, a
  * kernel to add the queue's counts up and 5120 waves whatever the batch, 1500
  * chunks of 512 bytes took 113 us, 2500 of 64 KiB 816 and 20 000 of 512 bytes
  * 329; they take 46, 686 and 273. Before there were two kernels: 88, 856 and
