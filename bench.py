@@ -476,7 +476,7 @@ def chunk_latency_leg(seed):
                                np.zeros(1, np.int32), np.array([seed + size], np.uint64))
             db = DeviceBatch(b.comp, b.comp_off, b.comp_size, b.sizes)
             row = {"bytes": size}
-            for name, t in (("two_wave_ms", 0), ("one_wave_ms", (1 << 64) - 1)):
+            for name, t in (("pipelined_ms", 0), ("one_wave_ms", (1 << 64) - 1)):
                 cudec_amd.set_pipeline_threshold("lz4", t)
                 ms = []
                 for r in range(12):

@@ -23,12 +23,12 @@
  * offsets, limits, positions) is done per 64 sequences, a lane each: 37
  * cycles a sequence, the repeat offsets as a scan over maps of three bytes (one
  * after the other on the scalar unit they took 190 cycles a sequence; as maps
- * that held the distances 8192 frames of 64 KiB took 2.34 ms, and 2.27 so). The copies on the other wave take
- * about 200.
+ * that held the distances 8192 frames of 64 KiB took 2.34 ms, and 2.25 so).
+ * The copies on the other wave take about 200.
  *
  * One wave a frame with one sequence decoded and executed after the other
  * took 13.72 ms for 8192 frames of 64 KiB and 284 ms for 2000 frames of
- * 1 KiB to 4 MiB; this takes 2.37 and 26.7 ms (4.94 and 56.0 with a lane a
+ * 1 KiB to 4 MiB; this takes 2.25 and 26.7 ms (4.94 and 56.0 with a lane a
  * Huffman stream). A frame's time is now the entropy wave's: per 64 KiB of
  * text-like data 0.70 M cycles of FSE chain, 0.11 M of tables, 0.10 M of
  * finishing and 0.02 M of staging, against 0.16 M of literals and 0.53 M of
@@ -603,8 +603,9 @@ struct EntropyFlow {
                        __builtin_amdgcn_readlane(brought, (from >> 8) & (kWave - 1)), b0, b1, b2);
         r2 = offset_of(from >> 16, less >> 16,
                        __builtin_amdgcn_readlane(brought, (from >> 16) & (kWave - 1)), b0, b1, b2);
-        /* positions: a block's regenerated literals and output fit 32 bits
-         * whatever the lengths claim (64 of at most 2^17 + 2^16 each) */
+        /* positions in 32 bits, whatever the lengths claim: a sequence of at
+         * most 65536 + 65535 literals and a match of 65539 + 65535 bytes, 64
+         * of which stay below 2^25 */
         const uint32_t lit_incl = wave_inclusive_sum(llen, lane);
         const uint32_t out_incl = wave_inclusive_sum(llen + mlen, lane);
         const uint64_t m = o + (out_incl - mlen);

@@ -110,9 +110,9 @@ ZD uint64_t read_le(const ZG uint8_t* p, uint32_t n) {
 
 /* ------------------------------------------------------------ bitstreams */
 
-/* How a reader's loaded words are held. PerLane: as loaded (a lane decoding
- * its own stream). A reader every lane runs on the same stream takes the
- * Wave policy's Same instead, which may make them one wave-uniform value. */
+/* How a reader's loaded words are held: PerLane, as loaded. The readers of
+ * this file run in the CPU build, whose Wave policy names it Same; the kernel
+ * has its own (zstd.hip). */
 struct PerLane {
     static ZD uint64_t fix64(uint64_t v) { return v; }
 };
@@ -693,7 +693,7 @@ constexpr uint32_t kBatch = 64;
  * state bits) = 712 bytes, so a window of this size staged at a batch's
  * start holds every byte its refills read. */
 constexpr uint32_t kWindowBytes = 1024;
-/* One sequence's record, for a policy that holds a batch of them. */
+/* One sequence's record, for a CPU build's policy that holds a batch of them. */
 struct Rec {
     uint64_t d;
     uint32_t ll, ml, lit, at;
